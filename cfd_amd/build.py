@@ -98,7 +98,7 @@ def build_oracle() -> None:
 def build_reference() -> bool:
     """Compiles the reference into oracle/_ref when its sources are present,
     and the Fortran shims against the reference's own module sources."""
-    if not os.path.isdir("/root/reference") or shutil.which("flang") is None:
+    if not os.path.isfile("/root/reference/mLaplace.f90") or shutil.which("flang") is None:
         return False
     _run(["make", "-s", "-C", ROOT, "-f", "oracle/Makefile.ref", "all", "shims", "shimharness"])
     return True
