@@ -517,7 +517,14 @@ int cfd_bicg_ex(int npoin, const double* spMtx, const int* spIdx, const int* spR
         XF.upload(x_fix, nfix, s);
         FI.upload(x_fixIdx, nfix, s);
         PcgWork w;
-        pcg_launch(w, npoin, A.p, I.p, R.p, D.p, X.p, B.p, XF.p, FI.p, nfix, tol, maxit, rel, s);
+        // the ELL copy (bit for bit the CSR kernels' results): its two passes
+        // over the matrix cost less than the first two iterations gain
+        EllLap ell;
+        const bool el = ell.build(npoin, nnz, R.p, I.p, spRowptr, s);
+        if (el) ell.refresh(R.p, A.p, s);
+        const EllMat em = ell.mat();
+        pcg_launch(w, npoin, A.p, I.p, R.p, D.p, X.p, B.p, XF.p, FI.p, nfix, tol, maxit, rel, s,
+                   el ? &em : nullptr);
         PcgResult res = pcg_result(w, s);
         X.download(x, npoin, s);
         CFD_HIP(hipStreamSynchronize(s));
@@ -764,7 +771,7 @@ struct cfd_session {
         refresh_patch_geometry();
         launch_masas(t, AREA.p, M.p, s);
         launch_laplace(t, X.p, Y.p, DNX.p, DNY.p, LAP.p, LDIAG.p, s);
-        if (ell_on) ell.refresh(t, LAP.p, s);
+        if (ell_on) ell.refresh(t.rowptr.p, LAP.p, s);
     }
 
     // the fused paths' ESTAB outputs (patch order)
@@ -833,7 +840,7 @@ struct cfd_session {
         }
         const PcgSystem sys[2] = {{&pcg, XPOS.p, BZERO.p, POSAUX.p, ILAUX.p, nn},
                                   {&pcg_y, YPOS.p, BZERO.p, POSAUY.p, ILAUX.p, nn}};
-        const EllMat em = ell.mat(m->t);
+        const EllMat em = ell.mat();
         pcg_launch_multi(sys, 2, np, LAP.p, m->t.idx.p, m->t.rowptr.p, LDIAG.p, tol, maxit,
                          d.pcg_rel, s, ell_on ? &em : nullptr);
         last_solves_trivial = pcg_polled_iterations(pcg) == 0.0 && pcg_polled_iterations(pcg_y) == 0.0;
@@ -964,7 +971,7 @@ struct cfd_session {
                 launch_gcl(t, M.p, WX.p, WY.p, WXO.p, WYO.p, DNX.p, DNY.p, AREA.p, AREA_OLD.p, dtmin,
                            d.gcl, s);
                 launch_laplace(t, X.p, Y.p, DNX.p, DNY.p, LAP.p, LDIAG.p, s);
-                if (ell_on) ell.refresh(t, LAP.p, s);
+                if (ell_on) ell.refresh(t.rowptr.p, LAP.p, s);
             } else {
                 geometry();
             }
@@ -1369,7 +1376,7 @@ int cfd_session_set_field(cfd_session* S, int f, const double* host_in) {
         }
         if (f == CFD_F_DT || f == CFD_F_DTL) S->dt_stale = false;  // the caller's values
         if (f == CFD_F_LAP_SPARSE && S->ell_on) {
-            S->ell.refresh(S->m->t, S->LAP.p, S->s);
+            S->ell.refresh(S->m->t.rowptr.p, S->LAP.p, S->s);
             CFD_HIP(hipStreamSynchronize(S->s));
         }
     })

@@ -550,12 +550,20 @@ void launch_transf(int nedge, const int* iset, const double* X, const double* Y,
 // ---------------------------------------------------------------------------
 // PCG (biconjGrad.f90:8-62)
 // ---------------------------------------------------------------------------
+// block partials per 256 rows: r.r and relative mode's two, r.z, p.y
+constexpr int kPcgPartials = 5;
 struct PcgWork {
     int n = 0, nblocks = 0;
     DBuf<double> r, z, y, pa, pb, partial;
     DBuf<double> scal;         // see pcg.hip for the slot meaning
-    DBuf<int> fixflag;         // n: 1 on Dirichlet nodes
-    HostPinned<double> hpin;   // host copy of scal for the polls (null: a stack copy)
+    DBuf<unsigned char> fixflag;  // n: 1 on Dirichlet nodes
+    HostPinned<double> hpin;   // two host copies of scal for the polls (null: a stack copy)
+    hipEvent_t ev[2] = {nullptr, nullptr};  // the polls' ends
+    double polled_iters = -1.0;  // iterations of the last solve, as its last poll read them
+    PcgWork() = default;
+    PcgWork(const PcgWork&) = delete;
+    PcgWork& operator=(const PcgWork&) = delete;
+    ~PcgWork();
     void ensure(int npoin);
 };
 // One system of a multi-system solve: its own work space, x, b and fixed
@@ -572,23 +580,33 @@ struct PcgSystem {
 // SpMV kernels: entry k of row i (its k-th CSR entry) at k * n + i, column
 // 0-based; rows keep their CSR lengths (entries beyond are never read), so a
 // row's products are summed in the same order as from the CSR arrays.
+// Columns are kept as 16-bit distances from the row (dcol, a sixth less of the
+// matrix's bytes) when every one fits, else as column numbers (col).
 constexpr int kEllMaxWidth = 16;
 struct EllMat {
     const double* val = nullptr;
-    const int* col = nullptr;
-    const int* rowptr = nullptr;
+    const int* col = nullptr;           // null when dcol is given
+    const short* dcol = nullptr;
+    const unsigned char* len = nullptr;  // entries per row
     int width = 0;
 };
 struct EllLap {
     int n = 0, width = 0;
     DBuf<int> col;
+    DBuf<short> dcol;
+    DBuf<unsigned char> len;
     DBuf<double> val;
     // builds the column layout; false (nothing built) when the longest row
-    // exceeds kEllMaxWidth or 1.5 times the mean row length
+    // exceeds kEllMaxWidth or 1.5 times the mean row length, or a row's
+    // length is negative
     bool build(const Tables& t, hipStream_t s);
+    // the same for any CSR matrix of n rows (rowptr, idx on the device, and
+    // the row pointer on the host)
+    bool build(int n, long long nnz, const int* rowptr, const int* idx, const int* rowptr_host,
+               hipStream_t s);
     // val from the CSR values A
-    void refresh(const Tables& t, const double* A, hipStream_t s);
-    EllMat mat(const Tables& t) const { return EllMat{val.p, col.p, t.rowptr.p, width}; }
+    void refresh(const int* rowptr, const double* A, hipStream_t s);
+    EllMat mat() const { return EllMat{val.p, col.p, dcol.p, len.p, width}; }
 };
 // Several independent solves on one matrix, interleaved on stream s with
 // shared polls; ell (when given) is the same matrix in ELL order, used by
@@ -611,7 +629,8 @@ struct PcgResult {
 // (see pcg.hip).
 void pcg_launch(PcgWork& w, int npoin, const double* A, const int* idx, const int* rowptr,
                 const double* diag, double* x, const double* b, const double* x_fix,
-                const int* x_fix_idx, int nfix, double tol, int maxit, int rel, hipStream_t s);
+                const int* x_fix_idx, int nfix, double tol, int maxit, int rel, hipStream_t s,
+                const EllMat* ell = nullptr);
 // Waits for the stream and returns the last solve's outcome.
 PcgResult pcg_result(const PcgWork& w, hipStream_t s);
 // Copy the last solve's iteration count and final r.z to device scalars

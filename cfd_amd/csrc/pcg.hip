@@ -8,14 +8,22 @@
 //     k++; r -= alfa y; z = r/diag; e = r.z; beta = e/e_old; p = beta p + z
 //     y = A p (fix rows 1e30 p); alfa = e/p.y; x += alfa p; e_old = e
 //
-// On the device one iteration is two full-grid kernels, each followed by a
-// one-block finalize that combines the block partials and updates the
-// scalars:
-//   A: x += alfa p (the previous iteration's update), r -= alfa y, z = r/diag,
-//      partials of r.z;                       finalize: e, beta, k.
-//   B: each row forms p_new = beta p_old + z for its columns on the fly, y = A
-//      p_new, stores its own p_new (double-buffered p), partials of p.y;
-//                                             finalize: alfa, the loop test.
+// On the device one iteration is two full-grid kernels:
+//   A (k_cg_a): alfa and the loop test; x += alfa p, r -= alfa y, z = r/diag,
+//      block partials of r.z;
+//   B (k_cg_b): beta; each row forms p_new = beta p_old + z for its columns on
+//      the fly, y = A p_new, stores its own p_new (double-buffered p), block
+//      partials of p.y.
+// Every block of A (of B) first combines the p.y (the r.z) partials that the
+// kernel before left, all in the same fixed order, so each has the scalars it
+// needs without a launch of its own for them; the first block stores them for
+// the kernels after (no kernel reads a scalar that it writes).  Above
+// kFoldMax partials a one-block kernel per scalar combines them instead.
+//
+// x is read and written in every second iteration only: p is double-buffered,
+// so A still has the previous iteration's p and adds both updates, in order,
+// at once (the same operations on every x; half of x's traffic).
+//
 // The scalars live in device memory.  Kernels queued after a loop has ended
 // return at once (done flag), so the host queues batches of iterations
 // between polls.  Several independent systems on one matrix (the x and y mesh
@@ -23,20 +31,20 @@
 // partials in a fixed tree, so the iteration sequence is deterministic (not
 // the serial summation order of the reference).
 //
-// Two systems on one matrix (the x and y mesh solves) iterate in lockstep
-// through paired kernels: one launch per kernel for both, with the matrix
-// entries staged once for both products, and row blocks in XCD order
-// (xcd_block: a row's neighbours' blocks mostly on the same XCD).  Each
-// system's arithmetic, logical block decomposition and partial order are
-// those of the single-system kernels, so the paired iterations are bit for
-// bit the single ones; a system that has finished is skipped inside the
-// paired kernels.
+// Two systems on one matrix (the x and y mesh solves) iterate in lockstep:
+// one launch per kernel for both, each matrix entry read once for both
+// products, and row blocks in XCD order (xcd_block: a row's neighbours' blocks
+// mostly on the same XCD).  Partials belong to logical blocks of 256 rows
+// whatever the launch shape, so a system's iterates do not depend on whether
+// it runs alone or in a pair, nor on its blocks' size; a system that has
+// finished is skipped inside the paired kernels.
 //
 // Relative mode (rel = 1): the two tests use tol^2 times the r.r and r.z of
 // the residual of the guess that is zero off the fixed nodes, so the stopping
 // point does not depend on the initial guess (warm starts compare at equal
 // tolerance).
 #include <mutex>
+#include <type_traits>
 
 #include "cfd_internal.hpp"
 #include "reduce.hpp"
@@ -47,7 +55,7 @@ namespace {
 // scal[] slots
 enum {
     S_ALFA = 0, S_BETA, S_EOLD, S_ENEW, S_PY, S_RR, S_K, S_DONE, S_STOP, S_CONV, S_TOL, S_MAXIT,
-    S_TOLR, S_TOLZ, S_NSCAL = 16
+    S_TOLR, S_TOLZ, S_ALFA0, S_NSCAL = 16
 };
 
 // The CSR entries of a block's rows [i0, i1) are one contiguous range
@@ -73,80 +81,325 @@ __device__ inline void staged_rows(const double* __restrict__ A, const int* __re
     }
 }
 
-// fixflag = 0; scalars reset (block 0)
-__global__ void k_fix_init(int n, int* __restrict__ fixflag, double* __restrict__ scal, double tol,
-                           int maxit) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) fixflag[i] = 0;
-    if (i == 0) {
-        for (int q = 0; q < S_NSCAL; ++q) scal[q] = 0.0;
-        scal[S_TOL] = tol;
-        scal[S_MAXIT] = (double)maxit;
+// One system of a launch (the kernels take one or two)
+struct CgSys {
+    double *x, *r, *z, *y, *scal;
+    double *prr, *prz, *ppy;  // block partials: residual (3 nb), r.z, p.y
+    const double* p;  // the current p
+    double* pother;   // the other buffer: the p before in A, the next p in B
+    unsigned char* fixflag;
+    const double *b, *x_fix;
+    const int* fix_idx;
+    int nfix;
+};
+// NS systems of a block: both of a pair (NS = 2), or the one of the block's
+// grid row (NS = 1, blockIdx.y)
+struct CgBoth {
+    CgSys s[2];
+};
+template <int NS>
+struct CgArgs {
+    CgSys s[NS];
+    __device__ __forceinline__ explicit CgArgs(const CgBoth& b) {
+        if (NS == 1) {
+            s[0] = b.s[blockIdx.y];
+        } else {
+            s[0] = b.s[0];
+            s[NS - 1] = b.s[1];
+        }
     }
-}
+};
 
-__global__ void k_fix_set(int nfix, const int* __restrict__ idx, const double* __restrict__ x_fix,
-                          int* __restrict__ fixflag, double* __restrict__ x) {
-    int q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= nfix) return;
-    int i = idx[q] - 1;
-    fixflag[i] = 1;
-    x[i] = 1.0 * x_fix[q];
-}
-
-// r = -1*(A x) + b with fixed rows y = 1e30 x and r(fix) = 0; r.r and, in
-// relative mode, rd.rd and rd.(rd/diag) for the residual rd of the guess that
-// is zero off the fixed nodes; the first residual test
-__global__ void __launch_bounds__(kBlock)
-k_residual(int n, const double* __restrict__ A, const int* __restrict__ idx,
-           const int* __restrict__ rowptr, const int* __restrict__ fixflag,
-           const double* __restrict__ diag, const double* __restrict__ x,
-           const double* __restrict__ b, double* __restrict__ r, int rel,
-           double* __restrict__ partials) {
-    __shared__ double sA[kSpChunk];
-    __shared__ int sI[kSpChunk];
-    const int i0 = blockIdx.x * blockDim.x, i = i0 + threadIdx.x;
-    const bool act = i < n;
-    const bool row = act && !fixflag[i];
-    double dot = 0.0, dotd = 0.0;
-    staged_rows(A, idx, rowptr[i0], rowptr[min(i0 + (int)blockDim.x, n)], row ? rowptr[i] : 0,
-                row ? rowptr[i + 1] : 0, sA, sI, [&](double a, int c) {
-                    const double xc = x[c];
-                    dot = dot + a * xc;
-                    if (rel && fixflag[c]) dotd = dotd + a * xc;
-                });
-    double v = 0.0, vdr = 0.0, vdz = 0.0;
-    if (act) {
-        double ri = 0.0;
-        if (row) {
-            ri = -1.0 * dot + b[i];
-            if (rel) {
-                const double rd = -1.0 * dotd + b[i];
-                vdr = rd * rd;
-                vdz = rd * (rd / diag[i]);
+// The sums of NS arrays of nb block partials, in the order of
+// combine_partials on one block of 256 threads (thread t adds partials t, t +
+// 256, ... to 0, then the waves' trees, then the waves in order), known to
+// every thread.  Blocks of 512 threads or more give each array its own 256
+// threads; smaller ones (256) add the arrays side by side.  nb <= kFoldMax.
+constexpr int kFoldSmall = 1024, kFoldMid = 2048, kFoldMax = 3072;
+// Loads of the partials, issued before the caller's own loads so that the sum
+// waits for nothing else.  Blocks of 256 threads: every thread its own
+// partials of every array; blocks of 1024: every thread a quarter of them,
+// handed over through LDS (12 loads in 24 registers a thread would cost the
+// kernels a wave per SIMD).
+template <int kG, int NS>
+struct Fold {
+    static constexpr int kMax = kG == 1 ? kFoldSmall : kG == 2 ? kFoldMid : kFoldMax;
+    static constexpr int kL = kMax / (kG * kBlock);
+    double v[NS][kL];
+    __device__ __forceinline__ void load(const double* part0, const double* part1, int nb) {
+#pragma unroll
+        for (int k = 0; k < NS; ++k) {
+            const double* p = k == 0 ? part0 : part1;
+#pragma unroll
+            for (int q = 0; q < kL; ++q) {
+                const int j = threadIdx.x + q * kG * kBlock;
+                v[k][q] = j < nb ? p[j] : 0.0;
             }
         }
-        r[i] = ri;
-        v = ri * ri;
     }
-    const int nb = gridDim.x;
-    block_partial(v, OpSum(), partials);
-    if (rel) {
-        block_partial(vdr, OpSum(), partials + nb);
-        block_partial(vdz, OpSum(), partials + 2 * nb);
+    // out[k]: the sum of array k
+    __device__ __forceinline__ void sum(int nb, double (&out)[NS]) {
+        __shared__ double sh[NS][kBlock / 64];
+        const int t = threadIdx.x & (kBlock - 1), g = threadIdx.x / kBlock;
+        if constexpr (kG == 1) {
+#pragma unroll
+            for (int k = 0; k < NS; ++k) {
+                double acc = 0.0;
+#pragma unroll
+                for (int q = 0; q < kL; ++q)
+                    if (t + q * kBlock < nb) acc = acc + v[k][q];
+                acc = wave_reduce(acc, OpSum());
+                if ((t & 63) == 0) sh[k][t >> 6] = acc;
+            }
+        } else {
+            __shared__ double sp[NS][kMax];
+#pragma unroll
+            for (int k = 0; k < NS; ++k)
+#pragma unroll
+                for (int q = 0; q < kL; ++q) sp[k][threadIdx.x + q * kG * kBlock] = v[k][q];
+            __syncthreads();
+            if (g < NS) {  // 256 threads per array
+                double acc = 0.0;
+#pragma unroll
+                for (int q = 0; q < kMax / kBlock; ++q)
+                    if (t + q * kBlock < nb) acc = acc + sp[g][t + q * kBlock];
+                acc = wave_reduce(acc, OpSum());
+                if ((t & 63) == 0) sh[g][t >> 6] = acc;
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < NS; ++k) {
+            double s = sh[k][0];
+#pragma unroll
+            for (int w = 1; w < kBlock / 64; ++w) s = s + sh[k][w];
+            out[k] = s;
+        }
+    }
+};
+
+// Partials of NS values per row (block_partial's tree per 256 rows): one per
+// logical block lb0 .. lb0 + kG - 1.  Every thread of the block calls this.
+template <int kG, int NS>
+__device__ __forceinline__ void cg_partials(const double (&v)[NS], double* const (&part)[NS],
+                                            int lb0, int nb) {
+    __shared__ double sh[NS][kG * (kBlock / 64)];
+    const int t = threadIdx.x;
+#pragma unroll
+    for (int k = 0; k < NS; ++k) {
+        const double w = wave_reduce(v[k], OpSum());
+        if ((t & 63) == 0) sh[k][t >> 6] = w;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < NS; ++k) {
+        const int g = t - 64 * k;  // wave k stores system k's
+        if (g < 0 || g >= kG || !part[k] || lb0 + g >= nb) continue;
+        double s = sh[k][g * (kBlock / 64)];
+#pragma unroll
+        for (int w = 1; w < kBlock / 64; ++w) s = s + sh[k][g * (kBlock / 64) + w];
+        part[k][lb0 + g] = s;
     }
 }
 
-// the first residual test (one block)
+// fixflag = 0; scalars reset (block 0)
+template <int NS>
+__global__ void k_cg_init(int n, CgBoth sys, double tol, int maxit) {
+    const CgArgs<NS> a(sys);
+    int i = blockIdx.x * blockDim.x + threadIdx.x;
+#pragma unroll
+    for (int k = 0; k < NS; ++k) {
+        if (i < n) a.s[k].fixflag[i] = 0;
+        if (i < S_NSCAL)
+            a.s[k].scal[i] = i == S_TOL ? tol : i == S_MAXIT ? (double)maxit : 0.0;
+    }
+}
+
+template <int NS>
+__global__ void k_cg_fix(CgBoth sys) {
+    const CgArgs<NS> a(sys);
+    int q = blockIdx.x * blockDim.x + threadIdx.x;
+#pragma unroll
+    for (int k = 0; k < NS; ++k) {
+        if (q >= a.s[k].nfix) continue;
+        int i = a.s[k].fix_idx[q] - 1;
+        a.s[k].fixflag[i] = 1;
+        a.s[k].x[i] = 1.0 * a.s[k].x_fix[q];
+    }
+}
+
+// The matrix rows of a kernel: f(a_ij, column j (0-based)) over row i's
+// entries in CSR order, from the CSR arrays (staged; every thread of the
+// block calls it, rows without work with on = false) or the ELL copy.
+struct CsrRows {
+    const double* A;
+    const int *idx, *rowptr;
+    template <class F>
+    __device__ __forceinline__ void visit(int n, int i0, int i, bool on, F f) const {
+        __shared__ double sA[kSpChunk];
+        __shared__ int sI[kSpChunk];
+        staged_rows(A, idx, rowptr[i0], rowptr[min(i0 + (int)blockDim.x, n)], on ? rowptr[i] : 0,
+                    on ? rowptr[i + 1] : 0, sA, sI, f);
+    }
+    template <int NS>
+    struct Ahead {  // nothing is loaded ahead
+        __device__ __forceinline__ void load(const CsrRows&, int, int, const CgArgs<NS>&, int) {}
+        __device__ __forceinline__ void dots(const CsrRows& m, int n, int i0, int i, bool work,
+                                             const bool (&row)[NS], const CgArgs<NS>& a, int first,
+                                             const double (&beta)[NS], double (&dot)[NS]) const {
+            m.visit(n, i0, i, work, [&](double aij, int c) {
+#pragma unroll
+                for (int k = 0; k < NS; ++k) {
+                    if (!row[k]) continue;
+                    const double pc = first ? a.s[k].z[c] : beta[k] * a.s[k].p[c] + a.s[k].z[c];
+                    dot[k] = dot[k] + aij * pc;
+                }
+            });
+        }
+    };
+};
+// kW: most entries of a row; kShort: columns as 16-bit distances from the
+// row; kAhead: k_cg_b loads the entries (1), and gathers their p and z too
+// (2), ahead of the scalars
+template <int kW, bool kShort, int kAhead>
+struct EllRows {
+    EllMat m;
+    static constexpr bool kDeep = kAhead == 2;
+    template <class F>
+    __device__ __forceinline__ void visit(int n, int, int i, bool on, F f) const {
+        if (!on) return;
+        const int l = m.len[i];
+#pragma unroll
+        for (int k = 0; k < kW; ++k) {
+            if (k < l) {
+                const size_t q = (size_t)k * n + i;
+                f(m.val[q], kShort ? i + (int)m.dcol[q] : m.col[q]);
+            }
+        }
+    }
+    // k_cg_b's entries of row i, loaded ahead of the scalars (slots beyond a
+    // row's length hold 0 and the row's own column, and are not added)
+    template <int NS>
+    struct Ahead {
+        int len, col[kW];
+        double val[kW];
+        double p[kDeep ? NS : 1][kDeep ? kW : 1], z[kDeep ? NS : 1][kDeep ? kW : 1];
+        __device__ __forceinline__ void load(const EllRows& r, int n, int i, const CgArgs<NS>& a,
+                                             int first) {
+            if constexpr (kAhead == 0) return;
+            len = r.m.len[i];
+#pragma unroll
+            for (int j = 0; j < kW; ++j) {
+                if (j >= r.m.width) continue;
+                const size_t q = (size_t)j * n + i;
+                val[j] = r.m.val[q];
+                col[j] = kShort ? i + (int)r.m.dcol[q] : r.m.col[q];
+            }
+            if constexpr (kDeep) {
+#pragma unroll
+                for (int j = 0; j < kW; ++j) {
+                    if (j >= r.m.width) continue;
+#pragma unroll
+                    for (int k = 0; k < NS; ++k) {
+                        z[k][j] = a.s[k].z[col[j]];
+                        if (!first) p[k][j] = a.s[k].p[col[j]];
+                    }
+                }
+            }
+        }
+        __device__ __forceinline__ void dots(const EllRows& r, int n, int, int i, bool work,
+                                             const bool (&row)[NS], const CgArgs<NS>& a, int first,
+                                             const double (&beta)[NS], double (&dot)[NS]) const {
+            if (!work) return;
+            const int len = kAhead ? this->len : (int)r.m.len[i];
+#pragma unroll
+            for (int j = 0; j < kW; ++j) {
+                if (j >= len) continue;
+                const size_t q = (size_t)j * n + i;
+                const double aij = kAhead ? val[j] : r.m.val[q];
+                const int c = kAhead ? col[j] : kShort ? i + (int)r.m.dcol[q] : r.m.col[q];
+#pragma unroll
+                for (int k = 0; k < NS; ++k) {
+                    if (!row[k]) continue;
+                    double zc, pc = 0.0;
+                    if constexpr (kDeep) {
+                        zc = z[k][j];
+                        pc = first ? zc : beta[k] * p[k][j] + zc;
+                    } else {
+                        zc = a.s[k].z[c];
+                        pc = first ? zc : beta[k] * a.s[k].p[c] + zc;
+                    }
+                    dot[k] = dot[k] + aij * pc;
+                }
+            }
+        }
+    };
+};
+
+// r = -1*(A x) + b with fixed rows y = 1e30 x and r(fix) = 0; partials of r.r
+// and, in relative mode, of rd.rd and rd.(rd/diag) for the residual rd of the
+// guess that is zero off the fixed nodes
+template <class Rows, int NS>
+__global__ void __launch_bounds__(kBlock)
+k_cg_residual(int n, Rows rows, const double* __restrict__ diag, CgBoth sys, int rel, int nb) {
+    const CgArgs<NS> a(sys);
+    const int lb = xcd_block(blockIdx.x, gridDim.x);
+    const int i0 = lb * kBlock, i = i0 + threadIdx.x;
+    const bool act = i < n;
+    bool row[NS], any = false;
+    double dot[NS], dotd[NS];
+#pragma unroll
+    for (int k = 0; k < NS; ++k) {
+        row[k] = act && !a.s[k].fixflag[i];
+        any = any || row[k];
+        dot[k] = dotd[k] = 0.0;
+    }
+    rows.visit(n, i0, i, any, [&](double aij, int c) {
+#pragma unroll
+        for (int k = 0; k < NS; ++k) {
+            if (!row[k]) continue;
+            const double xc = a.s[k].x[c];
+            dot[k] = dot[k] + aij * xc;
+            if (rel && a.s[k].fixflag[c]) dotd[k] = dotd[k] + aij * xc;
+        }
+    });
+#pragma unroll
+    for (int k = 0; k < NS; ++k) {
+        const CgSys& q = a.s[k];
+        double v = 0.0, vdr = 0.0, vdz = 0.0;
+        if (act) {
+            double ri = 0.0;
+            if (row[k]) {
+                ri = -1.0 * dot[k] + q.b[i];
+                if (rel) {
+                    const double rd = -1.0 * dotd[k] + q.b[i];
+                    vdr = rd * rd;
+                    vdz = rd * (rd / diag[i]);
+                }
+            }
+            q.r[i] = ri;
+            v = ri * ri;
+        }
+        block_partial(v, OpSum(), q.prr, lb);
+        if (rel) {
+            block_partial(vdr, OpSum(), q.prr + nb, lb);
+            block_partial(vdz, OpSum(), q.prr + 2 * nb, lb);
+        }
+    }
+}
+
+// the first residual test (block k: system k)
 __global__ void __launch_bounds__(256)
-k_fin_residual(const double* __restrict__ partials, int nb, int rel, double* __restrict__ scal) {
-    const double rr = combine_partials(partials, nb, 0.0, OpSum());
+k_cg_test(CgBoth a, int nb, int rel) {
+    const CgSys& q = a.s[blockIdx.x];
+    const double rr = combine_partials(q.prr, nb, 0.0, OpSum());
     double dr = 0.0, dz = 0.0;
     if (rel) {
-        dr = combine_partials(partials + nb, nb, 0.0, OpSum());
-        dz = combine_partials(partials + 2 * nb, nb, 0.0, OpSum());
+        dr = combine_partials(q.prr + nb, nb, 0.0, OpSum());
+        dz = combine_partials(q.prr + 2 * nb, nb, 0.0, OpSum());
     }
     if (threadIdx.x == 0) {
+        double* scal = q.scal;
         const double tol = scal[S_TOL];
         const double tolr = rel ? tol * tol * dr : tol;
         const double tolz = rel ? tol * tol * dz : tol;
@@ -162,323 +415,271 @@ k_fin_residual(const double* __restrict__ partials, int nb, int rel, double* __r
 }
 
 // first preconditioned residual: z = r/diag, partials of r.z
+template <int NS>
 __global__ void __launch_bounds__(kBlock)
-k_first_z(int n, const double* __restrict__ r, const double* __restrict__ diag,
-          double* __restrict__ z, const double* __restrict__ scal,
-          double* __restrict__ partials) {
-    if (scal[S_DONE] != 0.0) return;
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    double v = 0.0;
-    if (i < n) {
-        double zi = r[i] / diag[i];
-        z[i] = zi;
-        v = r[i] * zi;
-    }
-    block_partial(v, OpSum(), partials);
-}
-
-__global__ void __launch_bounds__(256)
-k_fin_first_z(const double* __restrict__ partials, int nb, double* __restrict__ scal) {
-    if (scal[S_DONE] != 0.0) return;
-    const double e = combine_partials(partials, nb, 0.0, OpSum());
-    if (threadIdx.x == 0) scal[S_ENEW] = e;
-}
-
-// Kernel A of an iteration (see the file header)
-__global__ void __launch_bounds__(kBlock)
-k_iter_a(int n, double* __restrict__ x, const double* __restrict__ pcur, double* __restrict__ r,
-         const double* __restrict__ y, const double* __restrict__ diag, double* __restrict__ z,
-         const double* __restrict__ scal, double* __restrict__ partials) {
-    if (scal[S_DONE] != 0.0) return;
-    const double alfa = scal[S_ALFA];
-    const bool stop = scal[S_STOP] != 0.0;
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (stop) {  // the loop test failed: only the last x update remains
-        if (i < n) x[i] = alfa * pcur[i] + x[i];
-        return;
-    }
-    double v = 0.0;
-    if (i < n) {
-        x[i] = alfa * pcur[i] + x[i];
-        double ri = -alfa * y[i] + r[i];
-        r[i] = ri;
-        double zi = ri / diag[i];
-        z[i] = zi;
-        v = ri * zi;
-    }
-    block_partial(v, OpSum(), partials);
-}
-
-__global__ void __launch_bounds__(256)
-k_fin_a(const double* __restrict__ partials, int nb, double* __restrict__ scal) {
-    if (scal[S_DONE] != 0.0) return;
-    if (scal[S_STOP] != 0.0) {
-        if (threadIdx.x == 0) {
-            scal[S_DONE] = 1.0;
-            scal[S_CONV] = fabs(scal[S_EOLD]) > scal[S_TOLZ] ? 0.0 : 1.0;
-        }
-        return;
-    }
-    const double e = combine_partials(partials, nb, 0.0, OpSum());
-    if (threadIdx.x == 0) {
-        scal[S_K] = scal[S_K] + 1.0;
-        scal[S_ENEW] = e;
-        scal[S_BETA] = e / scal[S_EOLD];
-    }
-}
-
-// Kernel B: p_new = beta p_old + z on the fly (first: p_new = z), y = A p_new
-__global__ void __launch_bounds__(kBlock)
-k_iter_b(int n, const double* __restrict__ A, const int* __restrict__ idx,
-         const int* __restrict__ rowptr, const int* __restrict__ fixflag,
-         const double* __restrict__ pold, const double* __restrict__ z, double* __restrict__ pnew,
-         double* __restrict__ y, int first, const double* __restrict__ scal,
-         double* __restrict__ partials) {
-    if (scal[S_DONE] != 0.0 || scal[S_STOP] != 0.0) return;
-    __shared__ double sA[kSpChunk];
-    __shared__ int sI[kSpChunk];
-    const double beta = scal[S_BETA];
-    const int i0 = blockIdx.x * blockDim.x, i = i0 + threadIdx.x;
-    const bool act = i < n;
-    const bool row = act && !fixflag[i];
-    double dot = 0.0;
-    staged_rows(A, idx, rowptr[i0], rowptr[min(i0 + (int)blockDim.x, n)], row ? rowptr[i] : 0,
-                row ? rowptr[i + 1] : 0, sA, sI, [&](double a, int c) {
-                    const double pc = first ? z[c] : beta * pold[c] + z[c];
-                    dot = dot + a * pc;
-                });
-    double v = 0.0;
-    if (act) {
-        double pi = first ? z[i] : beta * pold[i] + z[i];
-        double yi;
-        if (!row) {
-            yi = 1.0e30 * pi;
-        } else {
-            yi = dot;
-        }
-        pnew[i] = pi;
-        y[i] = yi;
-        v = pi * yi;
-    }
-    block_partial(v, OpSum(), partials);
-}
-
-__global__ void __launch_bounds__(256)
-k_fin_b(const double* __restrict__ partials, int nb, double* __restrict__ scal) {
-    if (scal[S_DONE] != 0.0 || scal[S_STOP] != 0.0) return;
-    const double py = combine_partials(partials, nb, 0.0, OpSum());
-    if (threadIdx.x == 0) {
-        double e = scal[S_ENEW];
-        scal[S_PY] = py;
-        scal[S_ALFA] = e / py;
-        scal[S_EOLD] = e;
-        bool more = fabs(e) > scal[S_TOLZ] && scal[S_K] < scal[S_MAXIT];
-        if (!more) scal[S_STOP] = 1.0;
-    }
-}
-
-// ---- paired systems (0 and 1): the kernels above, both systems per launch
-struct PairSys {
-    double *x, *r, *z, *y, *partial, *scal;
-    const double *pcur, *pold;
-    double* pnew;
-    const int* fixflag;
-};
-
-__global__ void __launch_bounds__(kBlock)
-k_iter_a2(int n, PairSys s0, PairSys s1, const double* __restrict__ diag) {
-    const int lb = xcd_block(blockIdx.x, gridDim.x);  // logical row block
-    const int i = lb * blockDim.x + threadIdx.x;
+k_cg_first_z(int n, const double* __restrict__ diag, CgBoth sys) {
+    const CgArgs<NS> a(sys);
+    const int i = blockIdx.x * kBlock + threadIdx.x;
 #pragma unroll
-    for (int k = 0; k < 2; ++k) {
-        const PairSys& q = k ? s1 : s0;
+    for (int k = 0; k < NS; ++k) {
+        const CgSys& q = a.s[k];
         if (q.scal[S_DONE] != 0.0) continue;  // uniform over the grid
-        const double alfa = q.scal[S_ALFA];
-        if (q.scal[S_STOP] != 0.0) {
-            if (i < n) q.x[i] = alfa * q.pcur[i] + q.x[i];
-            continue;
-        }
         double v = 0.0;
         if (i < n) {
-            q.x[i] = alfa * q.pcur[i] + q.x[i];
-            double ri = -alfa * q.y[i] + q.r[i];
-            q.r[i] = ri;
-            double zi = ri / diag[i];
+            double zi = q.r[i] / diag[i];
             q.z[i] = zi;
-            v = ri * zi;
+            v = q.r[i] * zi;
         }
-        block_partial(v, OpSum(), q.partial, lb);
+        block_partial(v, OpSum(), q.prz);
     }
 }
 
-// block k finalizes system k (k_fin_a's body)
-__global__ void __launch_bounds__(256)
-k_fin_a2(PairSys s0, PairSys s1, int nb) {
-    const PairSys& q = blockIdx.x ? s1 : s0;
-    double* scal = q.scal;
-    if (scal[S_DONE] != 0.0) return;
-    if (scal[S_STOP] != 0.0) {
-        if (threadIdx.x == 0) {
-            scal[S_DONE] = 1.0;
-            scal[S_CONV] = fabs(scal[S_EOLD]) > scal[S_TOLZ] ? 0.0 : 1.0;
-        }
-        return;
+// The scalars a kernel starts from
+struct CgScalars {
+    double alfa, alfa0, beta, eold, enew, k, done, stop, maxit, tolz;
+    __device__ __forceinline__ void load(const double* scal) {
+        alfa = scal[S_ALFA];
+        alfa0 = scal[S_ALFA0];
+        beta = scal[S_BETA];
+        eold = scal[S_EOLD];
+        enew = scal[S_ENEW];
+        k = scal[S_K];
+        done = scal[S_DONE];
+        stop = scal[S_STOP];
+        maxit = scal[S_MAXIT];
+        tolz = scal[S_TOLZ];
     }
-    const double e = combine_partials(q.partial, nb, 0.0, OpSum());
-    if (threadIdx.x == 0) {
-        scal[S_K] = scal[S_K] + 1.0;
-        scal[S_ENEW] = e;
-        scal[S_BETA] = e / scal[S_EOLD];
-    }
+};
+
+// A's step length, and whether the loop goes on
+__device__ __forceinline__ double cg_alfa(const CgScalars& c, double py, bool& more) {
+    more = fabs(c.enew) > c.tolz && c.k < c.maxit;
+    return c.enew / py;
 }
 
-// k_iter_b (not the first iteration) for both systems, A staged once
-__global__ void __launch_bounds__(kBlock)
-k_iter_b2(int n, const double* __restrict__ A, const int* __restrict__ idx,
-          const int* __restrict__ rowptr, PairSys s0, PairSys s1) {
-    const bool on0 = s0.scal[S_DONE] == 0.0 && s0.scal[S_STOP] == 0.0;
-    const bool on1 = s1.scal[S_DONE] == 0.0 && s1.scal[S_STOP] == 0.0;
-    if (!on0 && !on1) return;
-    __shared__ double sA[kSpChunk];
-    __shared__ int sI[kSpChunk];
-    const double beta0 = s0.scal[S_BETA], beta1 = s1.scal[S_BETA];
-    const int lb = xcd_block(blockIdx.x, gridDim.x);  // logical row block
-    const int i0 = lb * blockDim.x, i = i0 + threadIdx.x;
-    const bool act = i < n;
-    const bool row0 = act && !s0.fixflag[i], row1 = act && !s1.fixflag[i];
-    const bool row = (on0 && row0) || (on1 && row1);
-    double dot0 = 0.0, dot1 = 0.0;
-    staged_rows(A, idx, rowptr[i0], rowptr[min(i0 + (int)blockDim.x, n)], row ? rowptr[i] : 0,
-                row ? rowptr[i + 1] : 0, sA, sI, [&](double a, int c) {
-                    if (on0 && row0) dot0 = dot0 + a * (beta0 * s0.pold[c] + s0.z[c]);
-                    if (on1 && row1) dot1 = dot1 + a * (beta1 * s1.pold[c] + s1.z[c]);
-                });
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-        const PairSys& q = k ? s1 : s0;
-        if (!(k ? on1 : on0)) continue;  // uniform over the grid
-        double v = 0.0;
-        if (act) {
-            const double pi = (k ? beta1 : beta0) * q.pold[i] + q.z[i];
-            const double yi = (k ? row1 : row0) ? (k ? dot1 : dot0) : 1.0e30 * pi;
-            q.pnew[i] = pi;
-            q.y[i] = yi;
-            v = pi * yi;
-        }
-        block_partial(v, OpSum(), q.partial, lb);
-    }
-}
-
-// block k finalizes system k (k_fin_b's body)
-__global__ void __launch_bounds__(256)
-k_fin_b2(PairSys s0, PairSys s1, int nb) {
-    const PairSys& q = blockIdx.x ? s1 : s0;
-    double* scal = q.scal;
-    if (scal[S_DONE] != 0.0 || scal[S_STOP] != 0.0) return;
-    const double py = combine_partials(q.partial, nb, 0.0, OpSum());
-    if (threadIdx.x == 0) {
-        double e = scal[S_ENEW];
-        scal[S_PY] = py;
-        scal[S_ALFA] = e / py;
-        scal[S_EOLD] = e;
-        bool more = fabs(e) > scal[S_TOLZ] && scal[S_K] < scal[S_MAXIT];
-        if (!more) scal[S_STOP] = 1.0;
-    }
-}
-
-// ---- ELL-order SpMV variants of k_iter_b / k_iter_b2: the same rows, the
-// same per-row summation order and block decomposition, the entries read
-// coalesced from the ELL copy (no LDS staging, no barriers before the
-// block partial)
-template <int kW>
-__device__ inline double ell_row_dot(const EllMat& m, int n, int i, int len, double beta,
-                                     const double* __restrict__ pold, const double* __restrict__ z,
-                                     bool first) {
-    double dot = 0.0;
-#pragma unroll
-    for (int k = 0; k < kW; ++k) {
-        if (k < len) {
-            const size_t q = (size_t)k * n + i;
-            const double a = m.val[q];
-            const int c = m.col[q];
-            const double pc = first ? z[c] : beta * pold[c] + z[c];
-            dot = dot + a * pc;
-        }
-    }
-    return dot;
-}
-
-template <int kW>
-__global__ void __launch_bounds__(kBlock)
-k_iter_b_ell(int n, EllMat m, const int* __restrict__ fixflag, const double* __restrict__ pold,
-             const double* __restrict__ z, double* __restrict__ pnew, double* __restrict__ y,
-             int first, const double* __restrict__ scal, double* __restrict__ partials) {
-    if (scal[S_DONE] != 0.0 || scal[S_STOP] != 0.0) return;
-    const double beta = scal[S_BETA];
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    double v = 0.0;
+// Kernel A of an iteration (see the file header).  both: x takes the previous
+// iteration's update and this one's; else x is left for the next iteration,
+// unless this is the last.  kFold: the p.y partials are combined here, else
+// k_cg_fin_b has left alfa and the loop test.
+//
+// An iteration of one system / two in A and B, with the one-block kernels and x
+// in every iteration before and now (us): 32,768 rows 15.2 / 17 -> 9.4 / 10.5;
+// 131,072 rows 17.5 / 20.7 -> 11.0 / 12.9; 524,288 rows 27 / 38 -> 19.9 / 31.
+// What bounds it: below 131,072 rows the launches and one chain of dependent
+// loads in each kernel; above, the bytes (A 56 a row and system on average, B
+// 103 with the matrix, from the Infinity Cache at 524,288 rows: A 7.8 us, B 12.2).
+template <int kG, int NS, bool kFold>
+__global__ void __launch_bounds__(kG * kBlock)
+k_cg_a(int n, const double* __restrict__ diag, CgBoth sys, int nb, int both) {
+    const CgArgs<NS> a(sys);
+    const int pb = xcd_block(blockIdx.x, gridDim.x);
+    const int i = pb * (kG * kBlock) + threadIdx.x;
+    // every load of the kernel is issued before the first wait: the partials,
+    // the rows' own values, the scalars
+    Fold<kG, NS> fold;
+    if (kFold) fold.load(a.s[0].ppy, a.s[NS - 1].ppy, nb);
+    double p[NS], y[NS], r[NS], x[NS], p0[NS], d = 1.0;
     if (i < n) {
-        const bool row = !fixflag[i];
-        const double dot =
-            row ? ell_row_dot<kW>(m, n, i, m.rowptr[i + 1] - m.rowptr[i], beta, pold, z, first)
-                : 0.0;
-        const double pi = first ? z[i] : beta * pold[i] + z[i];
-        const double yi = row ? dot : 1.0e30 * pi;
-        pnew[i] = pi;
-        y[i] = yi;
-        v = pi * yi;
-    }
-    block_partial(v, OpSum(), partials);
-}
-
-template <int kW>
-__global__ void __launch_bounds__(kBlock)
-k_iter_b2_ell(int n, EllMat m, PairSys s0, PairSys s1) {
-    const bool on0 = s0.scal[S_DONE] == 0.0 && s0.scal[S_STOP] == 0.0;
-    const bool on1 = s1.scal[S_DONE] == 0.0 && s1.scal[S_STOP] == 0.0;
-    if (!on0 && !on1) return;
-    const double beta0 = s0.scal[S_BETA], beta1 = s1.scal[S_BETA];
-    const int lb = xcd_block(blockIdx.x, gridDim.x);  // logical row block
-    const int i = lb * blockDim.x + threadIdx.x;
-    const bool act = i < n;
-    const bool row0 = act && !s0.fixflag[i], row1 = act && !s1.fixflag[i];
-    double dot0 = 0.0, dot1 = 0.0;
-    if ((on0 && row0) || (on1 && row1)) {
-        const int len = m.rowptr[i + 1] - m.rowptr[i];
+        d = diag[i];
 #pragma unroll
-        for (int k = 0; k < kW; ++k) {
-            if (k < len) {
-                const size_t q = (size_t)k * n + i;
-                const double a = m.val[q];
-                const int c = m.col[q];
-                if (on0 && row0) dot0 = dot0 + a * (beta0 * s0.pold[c] + s0.z[c]);
-                if (on1 && row1) dot1 = dot1 + a * (beta1 * s1.pold[c] + s1.z[c]);
+        for (int k = 0; k < NS; ++k) {
+            const CgSys& q = a.s[k];
+            y[k] = q.y[i];
+            r[k] = q.r[i];
+            if (both) {
+                p[k] = q.p[i];
+                p0[k] = q.pother[i];
+                x[k] = q.x[i];
             }
         }
     }
+    CgScalars sc[NS];
+    bool on[NS], any = false;
 #pragma unroll
-    for (int k = 0; k < 2; ++k) {
-        const PairSys& q = k ? s1 : s0;
-        if (!(k ? on1 : on0)) continue;  // uniform over the grid
-        double v = 0.0;
-        if (act) {
-            const double pi = (k ? beta1 : beta0) * q.pold[i] + q.z[i];
-            const double yi = (k ? row1 : row0) ? (k ? dot1 : dot0) : 1.0e30 * pi;
-            q.pnew[i] = pi;
-            q.y[i] = yi;
-            v = pi * yi;
+    for (int k = 0; k < NS; ++k) {
+        sc[k].load(a.s[k].scal);
+        on[k] = sc[k].done == 0.0;
+        any = any || on[k];
+    }
+    if (!any) return;  // uniform over the grid
+    double alfa[NS], py[NS];
+    bool stop[NS];
+    if (kFold) fold.sum(nb, py);
+#pragma unroll
+    for (int k = 0; k < NS; ++k) {
+        if (kFold) {
+            bool more;
+            alfa[k] = cg_alfa(sc[k], py[k], more);
+            stop[k] = !more;
+        } else {
+            alfa[k] = sc[k].alfa;
+            stop[k] = sc[k].stop != 0.0;
         }
-        block_partial(v, OpSum(), q.partial, lb);
+    }
+    double v[NS];
+    double* part[NS];
+#pragma unroll
+    for (int k = 0; k < NS; ++k) {
+        const CgSys& q = a.s[k];
+        v[k] = 0.0;
+        part[k] = on[k] && !stop[k] ? q.prz : nullptr;
+        if (!on[k]) continue;
+        if (kFold && pb == 0 && threadIdx.x == 0) {
+            q.scal[S_PY] = py[k];
+            q.scal[S_EOLD] = sc[k].enew;
+            if (!both) q.scal[S_ALFA0] = alfa[k];
+            if (stop[k]) q.scal[S_STOP] = 1.0;
+        }
+        if (i >= n) continue;
+        if (both) q.x[i] = alfa[k] * p[k] + (sc[k].alfa0 * p0[k] + x[k]);
+        else if (stop[k]) q.x[i] = alfa[k] * q.p[i] + q.x[i];
+        if (stop[k]) continue;  // the loop test failed: only the last x update remained
+        const double ri = -alfa[k] * y[k] + r[k];
+        q.r[i] = ri;
+        const double zi = ri / d;
+        q.z[i] = zi;
+        v[k] = ri * zi;
+    }
+    cg_partials<kG, NS>(v, part, pb * kG, nb);
+}
+
+// Kernel B: p_new = beta p_old + z on the fly (first: p_new = z), y = A p_new.
+// kFold: the r.z partials are combined here, else k_cg_fin_a has left beta.
+// As in A every load that depends on no other kernel's scalar is issued
+// before the first wait; with kDeep the gathered p and z of all entries too
+// (blocks of one per CU: nothing else hides their latency).
+template <int kG, class Rows, int NS, bool kFold>
+__global__ void __launch_bounds__(kG * kBlock) __attribute__((amdgpu_waves_per_eu(kG > 1 ? 8 : 1)))
+k_cg_b(int n, Rows rows, CgBoth sys, int nb, int first) {
+    const CgArgs<NS> a(sys);
+    const int pb = xcd_block(blockIdx.x, gridDim.x);
+    const bool lead = pb == 0 && threadIdx.x == 0;
+    const int i0 = pb * (kG * kBlock), i = i0 + threadIdx.x;
+    const bool act = i < n;
+    Fold<kG, NS> fold;
+    if (kFold) fold.load(a.s[0].prz, a.s[NS - 1].prz, nb);
+    typename Rows::template Ahead<NS> ahead;
+    ahead.load(rows, n, act ? i : n - 1, a, first);
+    bool fixed[NS];
+    double zi[NS], pi[NS];
+    if (act) {
+#pragma unroll
+        for (int k = 0; k < NS; ++k) {
+            fixed[k] = a.s[k].fixflag[i];
+            zi[k] = a.s[k].z[i];
+            if (!first) pi[k] = a.s[k].p[i];
+        }
+    }
+    CgScalars sc[NS];
+    bool on[NS], any = false;
+#pragma unroll
+    for (int k = 0; k < NS; ++k) {
+        sc[k].load(a.s[k].scal);
+        on[k] = sc[k].done == 0.0 && sc[k].stop == 0.0;
+        any = any || on[k];
+        if (kFold && lead && sc[k].stop != 0.0 && sc[k].done == 0.0) {
+            a.s[k].scal[S_CONV] = fabs(sc[k].eold) > sc[k].tolz ? 0.0 : 1.0;
+            a.s[k].scal[S_DONE] = 1.0;  // read by the other blocks only beside STOP
+        }
+    }
+    if (!any) return;  // uniform over the grid
+    bool row[NS], work = false;
+    double beta[NS], e[NS], dot[NS];
+    if (kFold) fold.sum(nb, e);
+#pragma unroll
+    for (int k = 0; k < NS; ++k) {
+        row[k] = on[k] && act && !fixed[k];
+        work = work || row[k];
+        dot[k] = 0.0;
+        beta[k] = kFold ? (first ? 0.0 : e[k] / sc[k].eold) : sc[k].beta;
+        if (kFold && lead && on[k]) {
+            double* scal = a.s[k].scal;
+            scal[S_ENEW] = e[k];
+            if (!first) {
+                scal[S_BETA] = beta[k];
+                scal[S_K] = sc[k].k + 1.0;
+            }
+        }
+    }
+    ahead.dots(rows, n, i0, i, work, row, a, first, beta, dot);
+    double v[NS];
+    double* part[NS];
+#pragma unroll
+    for (int k = 0; k < NS; ++k) {
+        const CgSys& q = a.s[k];
+        v[k] = 0.0;
+        part[k] = on[k] ? q.ppy : nullptr;
+        if (!on[k] || !act) continue;
+        const double pn = first ? zi[k] : beta[k] * pi[k] + zi[k];
+        const double yi = row[k] ? dot[k] : 1.0e30 * pn;
+        q.pother[i] = pn;
+        q.y[i] = yi;
+        v[k] = pn * yi;
+    }
+    cg_partials<kG, NS>(v, part, pb * kG, nb);
+}
+
+// The scalars between A and B, and between B and A, of systems with more than
+// kFoldMax partials: block k combines system k's
+__global__ void __launch_bounds__(256)
+k_cg_fin_a(CgBoth a, int nb, int first) {
+    const CgSys& q = a.s[blockIdx.x];
+    double* scal = q.scal;
+    if (scal[S_DONE] != 0.0) return;
+    if (scal[S_STOP] != 0.0) {
+        if (threadIdx.x == 0) {
+            scal[S_DONE] = 1.0;
+            scal[S_CONV] = fabs(scal[S_EOLD]) > scal[S_TOLZ] ? 0.0 : 1.0;
+        }
+        return;
+    }
+    const double e = combine_partials(q.prz, nb, 0.0, OpSum());
+    if (threadIdx.x == 0) {
+        scal[S_ENEW] = e;
+        if (first) return;
+        scal[S_K] = scal[S_K] + 1.0;
+        scal[S_BETA] = e / scal[S_EOLD];
     }
 }
 
-// ELL column layout and values (EllLap::build / refresh)
+__global__ void __launch_bounds__(256)
+k_cg_fin_b(CgBoth a, int nb) {
+    const CgSys& q = a.s[blockIdx.x];
+    double* scal = q.scal;
+    if (scal[S_DONE] != 0.0 || scal[S_STOP] != 0.0) return;
+    const double py = combine_partials(q.ppy, nb, 0.0, OpSum());
+    if (threadIdx.x == 0) {
+        bool more;
+        CgScalars c;
+        c.load(scal);
+        const double alfa = cg_alfa(c, py, more);
+        scal[S_PY] = py;
+        scal[S_ALFA0] = scal[S_ALFA];
+        scal[S_ALFA] = alfa;
+        scal[S_EOLD] = scal[S_ENEW];
+        if (!more) scal[S_STOP] = 1.0;
+    }
+}
+
+// ELL row lengths and columns (EllLap::build), *far = 1 when a column lies
+// more than 16 bits from its row
 __global__ void k_ell_col(int n, int width, const int* __restrict__ rowptr,
-                          const int* __restrict__ idx, int* __restrict__ col) {
+                          const int* __restrict__ idx, int* __restrict__ col,
+                          short* __restrict__ dcol, unsigned char* __restrict__ len,
+                          int* __restrict__ far) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    const int b = rowptr[i], len = rowptr[i + 1] - b;
-    for (int k = 0; k < width; ++k) col[(size_t)k * n + i] = k < len ? idx[b + k] - 1 : i;
+    const int b = rowptr[i], cnt = rowptr[i + 1] - b;
+    len[i] = (unsigned char)cnt;
+    bool out = false;
+    for (int k = 0; k < width; ++k) {
+        const int c = k < cnt ? idx[b + k] - 1 : i;
+        const int d = c - i;
+        out = out || d < -32768 || d > 32767;
+        col[(size_t)k * n + i] = c;
+        dcol[(size_t)k * n + i] = (short)d;
+    }
+    if (out) *far = 1;
 }
 
 __global__ void k_ell_val(int n, int width, const int* __restrict__ rowptr,
@@ -504,6 +705,35 @@ k_fin_sum(const double* __restrict__ partials, int nb, double* __restrict__ out)
     if (threadIdx.x == 0) *out = s;
 }
 
+CgSys cg_sys(const PcgSystem& q, int cur) {
+    PcgWork& w = *q.w;
+    double* pbuf[2] = {w.pa.p, w.pb.p};
+    const size_t nb = w.nblocks;
+    return CgSys{q.x, w.r.p, w.z.p, w.y.p, w.scal.p, w.partial.p, w.partial.p + 3 * nb,
+                 w.partial.p + 4 * nb, pbuf[cur], pbuf[cur ^ 1], w.fixflag.p, q.b,
+                 q.x_fix, q.x_fix_idx, q.nfix};
+}
+
+// Rows up to which k_cg_b loads a row's entries (kAheadRows), and gathers
+// their p and z too (kDeepRows), before it has beta.  Measured per iteration,
+// one system / two: 32,768 rows 9.6 / 13.4 us with no loads ahead, 9.5 / 13.1
+// with the entries, 9.2 / 12.5 with the gathers; 131,072 rows 10.9 / 18.7,
+// 10.8 / 16.6, 10.9 / 16.4; 245,760 rows 13.8 / 23.3, 12.7 / 21.0, 13.6 / 21.6;
+// 524,288 rows (bound by bandwidth: the registers cost waves) 21.2 / 31.9,
+// 24.7 / 38.6, 24.5 / 39.3.
+constexpr int kDeepRows = 160 * 1024, kAheadRows = 256 * 1024;
+// calls f with the row reader of the matrix: the ELL copy when there is one
+template <class F>
+void with_rows(int n, const double* A, const int* idx, const int* rowptr, const EllMat* ell, F f) {
+    if (!ell) f(CsrRows{A, idx, rowptr});
+    else if (ell->width <= 8 && ell->dcol && n <= kDeepRows) f(EllRows<8, true, 2>{*ell});
+    else if (ell->width <= 8 && ell->dcol && n <= kAheadRows) f(EllRows<8, true, 1>{*ell});
+    else if (ell->width <= 8 && ell->dcol) f(EllRows<8, true, 0>{*ell});
+    else if (ell->width <= 8) f(EllRows<8, false, 0>{*ell});
+    else if (ell->dcol) f(EllRows<kEllMaxWidth, true, 0>{*ell});
+    else f(EllRows<kEllMaxWidth, false, 0>{*ell});
+}
+
 }  // namespace
 
 void pcg_initial_rr(PcgWork& w, int npoin, const double* A, const int* idx, const int* rowptr,
@@ -512,11 +742,10 @@ void pcg_initial_rr(PcgWork& w, int npoin, const double* A, const int* idx, cons
     w.ensure(npoin);
     const dim3 g(grid_for(npoin)), blk(kBlock);
     CFD_HIP(hipMemcpyAsync(w.z.p, x, sizeof(double) * npoin, hipMemcpyDeviceToDevice, s));
-    k_fix_init<<<g, blk, 0, s>>>(npoin, w.fixflag.p, w.scal.p, 1.0, 0);
-    if (nfix > 0)
-        k_fix_set<<<grid_for(nfix), blk, 0, s>>>(nfix, x_fix_idx, x_fix, w.fixflag.p, w.z.p);
-    k_residual<<<g, blk, 0, s>>>(npoin, A, idx, rowptr, w.fixflag.p, diag, w.z.p, b, w.r.p, 0,
-                                 w.partial.p);
+    const CgBoth a{{cg_sys(PcgSystem{&w, w.z.p, b, x_fix, x_fix_idx, nfix}, 0), CgSys{}}};
+    k_cg_init<1><<<g, blk, 0, s>>>(npoin, a, 1.0, 0);
+    if (nfix > 0) k_cg_fix<1><<<grid_for(nfix), blk, 0, s>>>(a);
+    k_cg_residual<CsrRows, 1><<<g, blk, 0, s>>>(npoin, CsrRows{A, idx, rowptr}, diag, a, 0, (int)g.x);
     k_fin_sum<<<1, 256, 0, s>>>(w.partial.p, (int)g.x, rr_out);
     CFD_HIP(hipGetLastError());
 }
@@ -527,27 +756,45 @@ void pcg_store_result(const PcgWork& w, double* iters, double* rz, double* itsum
     CFD_HIP(hipGetLastError());
 }
 
-bool EllLap::build(const Tables& t, hipStream_t s) {
-    n = t.npoin;
+bool EllLap::build(int npoin, long long nnz, const int* rowptr, const int* idx, const int* rowptr_host,
+                   hipStream_t s) {
+    n = npoin;
     width = 0;
-    if (n <= 0 || t.nnz <= 0) return false;
-    std::vector<int> rp(n + 1);  // the longest row, on the host (once per session)
-    t.rowptr.download(rp.data(), n + 1, s);
-    CFD_HIP(hipStreamSynchronize(s));
+    if (n <= 0 || nnz <= 0) return false;
     int w = 0;
-    for (int i = 0; i < n; ++i) w = std::max(w, rp[i + 1] - rp[i]);
-    if (w <= 0 || w > kEllMaxWidth || (double)w * n > 1.5 * (double)t.nnz) return false;
+    for (int i = 0; i < n; ++i) {
+        const int l = rowptr_host[i + 1] - rowptr_host[i];
+        if (l < 0) return false;
+        w = std::max(w, l);
+    }
+    if (w <= 0 || w > kEllMaxWidth || (double)w * n > 1.5 * (double)nnz) return false;
     width = w;
     col.alloc((size_t)w * n);
+    dcol.alloc((size_t)w * n);
+    len.alloc(n);
     val.alloc((size_t)w * n);
-    k_ell_col<<<grid_for(n), kBlock, 0, s>>>(n, w, t.rowptr.p, t.idx.p, col.p);
+    DBuf<int> far(1);
+    far.zero(s);
+    k_ell_col<<<grid_for(n), kBlock, 0, s>>>(n, w, rowptr, idx, col.p, dcol.p, len.p, far.p);
     CFD_HIP(hipGetLastError());
+    int out = 0;
+    CFD_HIP(hipMemcpyAsync(&out, far.p, sizeof(int), hipMemcpyDeviceToHost, s));
+    CFD_HIP(hipStreamSynchronize(s));
+    if (out) dcol.release();
+    else col.release();
     return true;
 }
 
-void EllLap::refresh(const Tables& t, const double* A, hipStream_t s) {
+bool EllLap::build(const Tables& t, hipStream_t s) {
+    std::vector<int> rp(t.npoin + 1);  // the row lengths, on the host (once per session)
+    t.rowptr.download(rp.data(), t.npoin + 1, s);
+    CFD_HIP(hipStreamSynchronize(s));
+    return build(t.npoin, t.nnz, t.rowptr.p, t.idx.p, rp.data(), s);
+}
+
+void EllLap::refresh(const int* rowptr, const double* A, hipStream_t s) {
     if (!width) return;
-    k_ell_val<<<grid_for(n), kBlock, 0, s>>>(n, width, t.rowptr.p, A, val.p);
+    k_ell_val<<<grid_for(n), kBlock, 0, s>>>(n, width, rowptr, A, val.p);
     CFD_HIP(hipGetLastError());
 }
 
@@ -561,17 +808,110 @@ void PcgWork::ensure(int npoin) {
     pa.alloc(npoin);
     pb.alloc(npoin);
     fixflag.alloc(npoin);
-    partial.alloc(3 * (size_t)nblocks);
+    partial.alloc(kPcgPartials * (size_t)nblocks);
     scal.alloc(S_NSCAL);
-    hpin.alloc(S_NSCAL);
+    hpin.alloc(2 * S_NSCAL);
+    for (auto& e : ev)
+        if (!e) CFD_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
 }
 
-// launches the ELL SpMV kernel of the width class that holds m.width
-template <class F8, class F16>
-static void ell_dispatch(const EllMat& m, F8 f8, F16 f16) {
-    if (m.width <= 8) f8();
-    else f16();
+PcgWork::~PcgWork() {
+    for (auto e : ev)
+        if (e) (void)hipEventDestroy(e);
 }
+
+namespace {
+
+// the scalars of the systems to the host's pinned copies
+__global__ void k_cg_poll(CgBoth a, double* h0, double* h1) {
+    const double* scal = a.s[blockIdx.x].scal;
+    (blockIdx.x ? h1 : h0)[threadIdx.x] = scal[threadIdx.x];
+}
+
+// Launches of one solve on rows of type Rows: the start, and single
+// iterations, of one system (q.s[0]) or two.
+template <class Rows>
+struct CgLaunch {
+    int n, nb;
+    Rows rows;
+    const double* diag;
+    hipStream_t s;
+    static constexpr bool kEll = !std::is_same<Rows, CsrRows>::value;
+    // Two systems up to kRowsApart rows: a grid row of blocks each, since
+    // latency and not the matrix's bytes is what an iteration costs (4,608
+    // rows 12.6 us with both in each thread); above, both in each thread,
+    // which reads the matrix once.
+    static constexpr int kRowsApart = 160 * 1024;
+    // Up to kFoldSmall partials blocks of 256 threads that each combine them
+    // all (4 loads a thread); up to kFoldMid blocks of 512 and up to kFoldMax
+    // of 1024, so that fewer blocks read them (an iteration of one system /
+    // two at 320,000 rows: 16.2 / 25.3 us with 512 threads, 17.8 / 27.9 with
+    // 1024); above, the one-block kernels (524,288 rows: 23.0 / 34.7 us with
+    // them, 19.8 / 31.2 without; 980,000 rows 38.8 / 57.5 either way).  CSR
+    // rows are staged by 256 threads.
+    bool apart(int nsys) const { return nsys == 1 || n <= kRowsApart; }
+
+    template <int NS>
+    void start_ns(const CgBoth& q, int rows_y, double tol, int maxit, int rel) const {
+        const dim3 g(nb, rows_y), blk(kBlock);
+        k_cg_init<NS><<<g, blk, 0, s>>>(n, q, tol, maxit);
+        const int nfix = std::max(q.s[0].nfix, q.s[1].nfix);
+        if (nfix > 0) k_cg_fix<NS><<<dim3(grid_for(nfix), rows_y), blk, 0, s>>>(q);
+        k_cg_residual<Rows, NS><<<g, blk, 0, s>>>(n, rows, diag, q, rel, nb);
+        k_cg_test<<<NS * rows_y, 256, 0, s>>>(q, nb, rel);
+        k_cg_first_z<NS><<<g, blk, 0, s>>>(n, diag, q);
+    }
+    void start(const CgBoth& q, int nsys, double tol, int maxit, int rel) const {
+        if (apart(nsys)) start_ns<1>(q, nsys, tol, maxit, rel);
+        else start_ns<2>(q, 1, tol, maxit, rel);
+        b(q, nsys, 1);
+    }
+    template <int NS>
+    void a_ns(const CgBoth& q, int rows_y, int both) const {
+        if (nb <= kFoldSmall) {
+            k_cg_a<1, NS, true><<<dim3(nb, rows_y), kBlock, 0, s>>>(n, diag, q, nb, both);
+        } else if (kEll && nb <= kFoldMid) {
+            k_cg_a<2, NS, true><<<dim3((nb + 1) / 2, rows_y), 2 * kBlock, 0, s>>>(n, diag, q, nb, both);
+        } else if (kEll && nb <= kFoldMax) {
+            k_cg_a<4, NS, true><<<dim3((nb + 3) / 4, rows_y), 4 * kBlock, 0, s>>>(n, diag, q, nb, both);
+        } else {
+            k_cg_a<1, NS, false><<<dim3(nb, rows_y), kBlock, 0, s>>>(n, diag, q, nb, both);
+            k_cg_fin_a<<<NS * rows_y, 256, 0, s>>>(q, nb, 0);
+        }
+    }
+    void a(const CgBoth& q, int nsys, int both) const {
+        if (apart(nsys)) a_ns<1>(q, nsys, both);
+        else a_ns<2>(q, 1, both);
+    }
+    template <int NS>
+    void b_ns(const CgBoth& q, int rows_y, int first) const {
+        if (nb <= kFoldSmall) {
+            k_cg_b<1, Rows, NS, true><<<dim3(nb, rows_y), kBlock, 0, s>>>(n, rows, q, nb, first);
+            return;
+        }
+        if constexpr (kEll) {
+            if (nb <= kFoldMid) {
+                k_cg_b<2, Rows, NS, true>
+                    <<<dim3((nb + 1) / 2, rows_y), 2 * kBlock, 0, s>>>(n, rows, q, nb, first);
+                return;
+            }
+            if (nb <= kFoldMax) {
+                k_cg_b<4, Rows, NS, true>
+                    <<<dim3((nb + 3) / 4, rows_y), 4 * kBlock, 0, s>>>(n, rows, q, nb, first);
+                return;
+            }
+        }
+        if (first) k_cg_fin_a<<<NS * rows_y, 256, 0, s>>>(q, nb, 1);
+        k_cg_b<1, Rows, NS, false><<<dim3(nb, rows_y), kBlock, 0, s>>>(n, rows, q, nb, first);
+        k_cg_fin_b<<<NS * rows_y, 256, 0, s>>>(q, nb);
+    }
+    void b(const CgBoth& q, int nsys, int first) const {
+        if (apart(nsys)) b_ns<1>(q, nsys, first);
+        else b_ns<2>(q, 1, first);
+    }
+};
+
+}  // namespace
 
 void pcg_launch_multi(const PcgSystem* sys, int nsys, int npoin, const double* A, const int* idx,
                       const int* rowptr, const double* diag, double tol, int maxit, int rel,
@@ -579,132 +919,103 @@ void pcg_launch_multi(const PcgSystem* sys, int nsys, int npoin, const double* A
     CFD_CHECK(npoin > 0, "arg: PCG needs npoin > 0");
     constexpr int kMaxSys = 2;
     CFD_CHECK(nsys >= 1 && nsys <= kMaxSys, "internal: PCG systems per launch");
-    const dim3 g(grid_for(npoin)), blk(kBlock);
-    int cur[kMaxSys] = {0, 0};  // pbuf[cur] holds the current p
-    const int nb = (int)g.x;
-    const dim3 one(1), fin(256);
-    auto iter_a = [&](int k) {
-        PcgWork& w = *sys[k].w;
-        double* pbuf[2] = {w.pa.p, w.pb.p};
-        k_iter_a<<<g, blk, 0, s>>>(npoin, sys[k].x, pbuf[cur[k]], w.r.p, w.y.p, diag, w.z.p,
-                                   w.scal.p, w.partial.p);
-        k_fin_a<<<one, fin, 0, s>>>(w.partial.p, nb, w.scal.p);
+    const int nb = (int)grid_for(npoin);
+    for (int k = 0; k < nsys; ++k) sys[k].w->ensure(npoin);
+    // pbuf[cur] holds the current p; both systems' buffers flip together
+    int cur = 1;
+    bool done[kMaxSys] = {false, nsys == 1};
+    // the systems of a launch: both, or the one that is not done
+    auto args = [&]() {
+        CgBoth q{};
+        int m = 0;
+        for (int k = 0; k < nsys; ++k)
+            if (!done[k]) q.s[m++] = cg_sys(sys[k], cur);
+        return q;
     };
-    auto iter_b = [&](int k, int first) {
-        PcgWork& w = *sys[k].w;
-        double* pbuf[2] = {w.pa.p, w.pb.p};
-        if (ell) {
-            const EllMat m = *ell;
-            ell_dispatch(
-                m,
-                [&] {
-                    k_iter_b_ell<8><<<g, blk, 0, s>>>(npoin, m, w.fixflag.p, pbuf[cur[k]], w.z.p,
-                                                      pbuf[cur[k] ^ 1], w.y.p, first, w.scal.p,
-                                                      w.partial.p);
-                },
-                [&] {
-                    k_iter_b_ell<kEllMaxWidth><<<g, blk, 0, s>>>(
-                        npoin, m, w.fixflag.p, pbuf[cur[k]], w.z.p, pbuf[cur[k] ^ 1], w.y.p, first,
-                        w.scal.p, w.partial.p);
-                });
-        } else {
-            k_iter_b<<<g, blk, 0, s>>>(npoin, A, idx, rowptr, w.fixflag.p, pbuf[cur[k]], w.z.p,
-                                       pbuf[cur[k] ^ 1], w.y.p, first, w.scal.p, w.partial.p);
-        }
-        k_fin_b<<<one, fin, 0, s>>>(w.partial.p, nb, w.scal.p);
+    auto count = [&]() { return (int)!done[0] + (int)!done[1]; };
+    // Polls: a kernel writes the scalars to the host's pinned copies (two of
+    // them, so that a poll may be waited for while the next iterations are
+    // queued); without pinned memory a copy to the stack.
+    double local[kMaxSys][S_NSCAL];
+    const bool pinned = sys[0].w->hpin.p && sys[nsys - 1].w->hpin.p;
+    auto host = [&](int k, int slot) {
+        return pinned ? sys[k].w->hpin.p + slot * S_NSCAL : local[k];
     };
-    for (int k = 0; k < nsys; ++k) {
-        PcgWork& w = *sys[k].w;
-        w.ensure(npoin);
-        k_fix_init<<<g, blk, 0, s>>>(npoin, w.fixflag.p, w.scal.p, tol, maxit);
-        if (sys[k].nfix > 0)
-            k_fix_set<<<grid_for(sys[k].nfix), blk, 0, s>>>(sys[k].nfix, sys[k].x_fix_idx,
-                                                            sys[k].x_fix, w.fixflag.p, sys[k].x);
-        k_residual<<<g, blk, 0, s>>>(npoin, A, idx, rowptr, w.fixflag.p, diag, sys[k].x, sys[k].b,
-                                     w.r.p, rel, w.partial.p);
-        k_fin_residual<<<one, fin, 0, s>>>(w.partial.p, nb, rel, w.scal.p);
-        k_first_z<<<g, blk, 0, s>>>(npoin, w.r.p, diag, w.z.p, w.scal.p, w.partial.p);
-        k_fin_first_z<<<one, fin, 0, s>>>(w.partial.p, nb, w.scal.p);
-        cur[k] = 1;
-        iter_b(k, 1);  // p0 = z0 into pbuf[0]
-        cur[k] = 0;
-    }
-    CFD_HIP(hipGetLastError());
-    bool done[kMaxSys] = {false, false}, stop[kMaxSys] = {false, false};
-    double local[kMaxSys][S_NSCAL];  // the polls' host copy where no pinned buffer exists
-    auto poll = [&]() {
-        for (int k = 0; k < nsys; ++k) {
-            double* h = sys[k].w->hpin.p ? sys[k].w->hpin.p : local[k];
-            CFD_HIP(hipMemcpyAsync(h, sys[k].w->scal.p, S_NSCAL * sizeof(double),
-                                   hipMemcpyDeviceToHost, s));
-        }
-        CFD_HIP(hipStreamSynchronize(s));
-        bool all = true;
-        for (int k = 0; k < nsys; ++k) {
-            const double* h = sys[k].w->hpin.p ? sys[k].w->hpin.p : local[k];
-            done[k] = h[S_DONE] != 0.0;
-            stop[k] = h[S_STOP] != 0.0;
-            all = all && done[k];
-        }
-        return all;
-    };
-    // two systems: the paired kernels (both p buffers flip together; a
-    // system that has stopped or finished is skipped on the device)
-    auto pair = [&](int k) {
-        PcgWork& w = *sys[k].w;
-        double* pbuf[2] = {w.pa.p, w.pb.p};
-        return PairSys{sys[k].x, w.r.p, w.z.p, w.y.p, w.partial.p, w.scal.p, pbuf[cur[k]],
-                       pbuf[cur[k]], pbuf[cur[k] ^ 1], w.fixflag.p};
-    };
-    // most warm-started mesh solves stop at the first residual test; batches
-    // grow while a solve runs on (few polls, few no-op launches)
-    int chunk = 4;
-    for (long launched = 0; !poll(); launched += chunk) {
-        if (nsys == 2 && !done[0] && !done[1] && cur[0] == cur[1]) {
-            for (int q = 0; q < chunk; ++q) {
-                const PairSys p0 = pair(0), p1 = pair(1);
-                k_iter_a2<<<g, blk, 0, s>>>(npoin, p0, p1, diag);
-                k_fin_a2<<<dim3(2), fin, 0, s>>>(p0, p1, nb);
-                if (ell) {
-                    const EllMat m = *ell;
-                    ell_dispatch(
-                        m, [&] { k_iter_b2_ell<8><<<g, blk, 0, s>>>(npoin, m, p0, p1); },
-                        [&] { k_iter_b2_ell<kEllMaxWidth><<<g, blk, 0, s>>>(npoin, m, p0, p1); });
-                } else {
-                    k_iter_b2<<<g, blk, 0, s>>>(npoin, A, idx, rowptr, p0, p1);
-                }
-                k_fin_b2<<<dim3(2), fin, 0, s>>>(p0, p1, nb);
-                cur[0] ^= 1;
-                cur[1] ^= 1;
-            }
-            CFD_HIP(hipGetLastError());
-            CFD_CHECK(launched <= 4L * maxit + 64, "PCG did not terminate");
-            chunk = std::min(chunk * 2, 16);
-            continue;
+    auto ask = [&](int slot) {
+        if (pinned) {
+            CgBoth q{};
+            for (int k = 0; k < nsys; ++k) q.s[k] = cg_sys(sys[k], cur);
+            k_cg_poll<<<nsys, S_NSCAL, 0, s>>>(q, host(0, slot), host(nsys - 1, slot));
+            CFD_HIP(hipEventRecord(sys[0].w->ev[slot], s));
+            return;
         }
         for (int k = 0; k < nsys; ++k)
-            if (!done[k] && stop[k]) iter_a(k);  // the final x update ends the solve
-        for (int q = 0; q < chunk; ++q) {
-            for (int k = 0; k < nsys; ++k) {
-                if (done[k] || stop[k]) continue;
-                iter_a(k);
-                iter_b(k, 0);
-                cur[k] ^= 1;
-            }
+            CFD_HIP(hipMemcpyAsync(local[k], sys[k].w->scal.p, sizeof(local[k]),
+                                   hipMemcpyDeviceToHost, s));
+    };
+    auto told = [&](int slot) {
+        if (pinned) CFD_HIP(hipEventSynchronize(sys[0].w->ev[slot]));
+        else CFD_HIP(hipStreamSynchronize(s));
+        for (int k = 0; k < nsys; ++k) {
+            done[k] = done[k] || host(k, slot)[S_DONE] != 0.0;
+            sys[k].w->polled_iters = host(k, slot)[S_K];
         }
+        return count() == 0;
+    };
+    with_rows(npoin, A, idx, rowptr, ell, [&](auto rows) {
+        const CgLaunch<decltype(rows)> go{npoin, nb, rows, diag, s};
+        go.start(args(), nsys, tol, maxit, rel);  // p0 = z0 into pbuf[0]
+        cur = 0;
         CFD_HIP(hipGetLastError());
-        CFD_CHECK(launched <= 4L * maxit + 64, "PCG did not terminate");
-        chunk = std::min(chunk * 2, 16);
-    }
+        int both = 0;
+        auto iterate = [&](int m) {
+            for (int q = 0; q < m; ++q) {
+                go.a(args(), count(), both);
+                go.b(args(), count(), 0);
+                cur ^= 1;
+                both ^= 1;
+            }
+            CFD_HIP(hipGetLastError());
+        };
+        // Most warm-started mesh solves stop at the first residual test;
+        // batches grow while a solve runs on (few polls, few launches after
+        // its end).  From kAsyncFrom iterations on the next batch is queued
+        // before a poll is waited for: a poll's round trip costs an idle GPU
+        // about 15 us, the batch queued in vain at the end about 50.
+        constexpr long kAsyncFrom = 128;
+        constexpr int kAsyncBatch = 8;
+        int chunk = 4, slot = 0;
+        long launched = 0;
+        ask(slot);
+        while (!told(slot)) {
+            CFD_CHECK(launched <= 4L * maxit + 64, "PCG did not terminate");
+            if (pinned && launched >= kAsyncFrom) break;
+            iterate(chunk);
+            launched += chunk;
+            chunk = std::min(chunk * 2, 16);
+            ask(slot);
+        }
+        if (count() == 0) return;
+        iterate(kAsyncBatch);
+        ask(slot);
+        for (bool end = false; !end; slot ^= 1) {
+            launched += kAsyncBatch;
+            CFD_CHECK(launched <= 4L * maxit + 64, "PCG did not terminate");
+            iterate(kAsyncBatch);
+            ask(slot ^ 1);
+            end = told(slot);
+        }
+    });
 }
 
-double pcg_polled_iterations(const PcgWork& w) { return w.hpin.p ? w.hpin.p[S_K] : -1.0; }
+double pcg_polled_iterations(const PcgWork& w) { return w.polled_iters; }
 
 void pcg_launch(PcgWork& w, int npoin, const double* A, const int* idx, const int* rowptr,
                 const double* diag, double* x, const double* b, const double* x_fix,
-                const int* x_fix_idx, int nfix, double tol, int maxit, int rel, hipStream_t s) {
+                const int* x_fix_idx, int nfix, double tol, int maxit, int rel, hipStream_t s,
+                const EllMat* ell) {
     PcgSystem sys{&w, x, b, x_fix, x_fix_idx, nfix};
-    pcg_launch_multi(&sys, 1, npoin, A, idx, rowptr, diag, tol, maxit, rel, s);
+    pcg_launch_multi(&sys, 1, npoin, A, idx, rowptr, diag, tol, maxit, rel, s, ell);
 }
 
 PcgResult pcg_result(const PcgWork& w, hipStream_t s) {
@@ -735,18 +1046,18 @@ constexpr int kNoAllocBlocks = (kNoAllocRows + kBlock - 1) / kBlock;
 constexpr size_t kAlign = 32;  // doubles: 256-byte sub-array alignment
 constexpr size_t align_up(size_t v) { return (v + kAlign - 1) / kAlign * kAlign; }
 // layout (in doubles): r, z, y, pa, pb (kNoAllocRows each), partial
-// (3 kNoAllocBlocks), scal (S_NSCAL), fixflag (kNoAllocRows int32), the CSR
-// check flag (one int32, in its own slot)
+// (kPcgPartials kNoAllocBlocks), scal (S_NSCAL), fixflag (kNoAllocRows bytes),
+// the CSR check flag (one int32, in its own slot)
 constexpr size_t kOffVec = 0;
 constexpr size_t kOffPartial = align_up(kOffVec + 5 * (size_t)kNoAllocRows);
-constexpr size_t kOffScal = align_up(kOffPartial + 3 * (size_t)kNoAllocBlocks);
+constexpr size_t kOffScal = align_up(kOffPartial + kPcgPartials * (size_t)kNoAllocBlocks);
 constexpr size_t kOffFix = align_up(kOffScal + S_NSCAL);
-constexpr size_t kOffFlag = align_up(kOffFix + kNoAllocRows / 2);
+constexpr size_t kOffFlag = align_up(kOffFix + kNoAllocRows / 8);
 constexpr size_t kScratchDoubles = align_up(kOffFlag + 1);
 
 }  // namespace
 
-// about 23 MB per device, held until the process ends
+// about 22 MB per device, held until the process ends
 static __device__ __align__(256) double scratch[kScratchDoubles];
 
 namespace {
@@ -827,9 +1138,9 @@ extern "C" int cfd_bicg_ex_noalloc(int npoin, const double* spMtx, const int* sp
         w.y.borrow(base + kOffVec + 2 * (size_t)kNoAllocRows, npoin);
         w.pa.borrow(base + kOffVec + 3 * (size_t)kNoAllocRows, npoin);
         w.pb.borrow(base + kOffVec + 4 * (size_t)kNoAllocRows, npoin);
-        w.partial.borrow(base + kOffPartial, 3 * (size_t)nb);
+        w.partial.borrow(base + kOffPartial, kPcgPartials * (size_t)nb);
         w.scal.borrow(base + kOffScal, S_NSCAL);
-        w.fixflag.borrow(reinterpret_cast<int*>(base + kOffFix), npoin);
+        w.fixflag.borrow(reinterpret_cast<unsigned char*>(base + kOffFix), npoin);
         pcg_launch(w, npoin, spMtx, spIdx, spRowptr, diagMtx, x, b, x_fix, x_fixIdx, nfix, tol,
                    maxit, rel, s);
         PcgResult res = pcg_result(w, s);

@@ -128,7 +128,7 @@ __global__ void k_ws_features(const double* __restrict__ ex, const double* __res
 // residual of E, zero on the fixed rows)
 __global__ void __launch_bounds__(kBlock)
 k_ws_galerkin(int n, const double* __restrict__ A, const int* __restrict__ idx,
-              const int* __restrict__ rowptr, const int* __restrict__ fixflag,
+              const int* __restrict__ rowptr, const unsigned char* __restrict__ fixflag,
               const float* __restrict__ out, int axis, const double* __restrict__ r,
               double* __restrict__ partials) {
     double yr = 0.0, yay = 0.0;
