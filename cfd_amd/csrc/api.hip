@@ -372,7 +372,7 @@ int cfd_smoothing(cfd_mesh* m, double* X, double* Y, const int* fixed, const dou
         CFD_ARG(order == 0 || order == 1, "order must be 0 (node order) or 1 (by colour)");
         const int np = m->t.npoin;
         CFD_ARG(order == 1 || np <= kSmoothSeqMaxNodes,
-                "order 0 walks the nodes on one lane: at most 65536 nodes (use order 1)");
+                "order 0 walks the nodes in order: at most 65536 nodes (use order 1)");
         m->smooth.build(m->t, fixed, m->s);
         CFD_ARG(m->smooth.max_elems <= 20,
                 "a node has more than 20 elements (the reference's MAX_ELEM_PER_NODE)");

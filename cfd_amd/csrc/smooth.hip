@@ -19,10 +19,12 @@
 // the mesh (node (r, 0) follows node (r-1, last) through the seam), so the
 // reference's result is inherently sequential.
 //
-// Two schedules share the per-node code below (same operations, same order,
+// Two schedules of the same per-node arithmetic (same operations, same order,
 // contraction off):
-//   order 0 - the reference's node order, one lane walking each pass: the
-//             reference's result bit for bit, for small meshes;
+//   order 0 - the reference's node order, bit for bit its result, for small
+//             meshes: one wave per pass walks the nodes, its lanes forming a
+//             node's elements (and its tries) side by side, while the waves of
+//             the next passes follow behind (k_sm_passes);
 //   order 1 - colour by colour: a greedy colouring of the node graph (no two
 //             nodes of one colour share an element, so nodes of a colour read
 //             and write disjoint data), one lane per node, colours in
@@ -248,20 +250,318 @@ k_sm_check_fin(const double* __restrict__ hpart, const double* __restrict__ anyp
     }
 }
 
-// order 0: one lane walks a pass in node order
-__global__ void k_sm_laplacian_seq(SmDev d, int npoin) {
-    if (blockIdx.x != 0 || threadIdx.x != 0) return;
-    for (int ip = 1; ip <= npoin; ++ip) sm_laplacian_node(d, ip);
+// ---------------------------------------------------------------------------
+// order 0: up to kSmWaves consecutive passes in one block, a wave per pass.
+//
+// A node's update reads its ring (the nodes that share an element with it) and
+// marks it, and changes nothing else but the node itself.  So pass w + 1 may
+// update node i as soon as pass w is past i and past every node of i's ring:
+// each wave publishes how far it is (prog), and the next one follows that far
+// behind.  Every update then reads exactly the values and marks that it would
+// read with the passes one after the other.  Wave 0 waits for nothing and wave
+// w only for wave w - 1 of its own block, so each wait ends.  On a ring by ring
+// numbering the waves run one ring and a chunk apart; on one where every node
+// has a far neighbour they run one after the other.
+//
+// Inside a wave the lanes form the qualities of the node's elements, 8, 16 or
+// 32 lanes a group, and the groups the tries (their positions are the running
+// sums that the sequential loop forms).
+//
+// Whether a sweep is the last is known when it ends, while the next ones are
+// on their way: each wave leaves its pass's positions in hist, and the result
+// is taken from the last sweep that counts.
+//
+// Bound by the instructions that a node takes (about 1,000: seven qualities,
+// fourteen divisions, the tries' positions) on the four SIMDs of one CU; the
+// positions stay in LDS while they fit.  64 x 128 cylinder (8,192 nodes, 2 + 8
+// passes): 48 ms; one lane per pass and the passes one by one took 1,524.
+// More waves than twelve (three per SIMD) add no throughput, only passes begun
+// in vain behind the last one (sixteen: 58.8 ms).
+// ---------------------------------------------------------------------------
+constexpr int kSmWaves = 12;
+struct SmSeq {
+    SmDev d;               // topology, fixed, marks, tol_move, hmin
+    const int *ring, *need;  // per esup entry its element's nodes (0-based); per node
+                             // how far the pass before has to be
+    double2 *xy, *hist;    // positions; positions after each pass of the launch
+    double* dmax;          // per pass of the launch: the largest squared move
+    int n, npass, nlap;    // passes of the launch, Laplacian ones first
+};
+
+// v of a lane that every lane names alike
+__device__ __forceinline__ double lane_of(double v, int lane) {
+    const int l = __builtin_amdgcn_readfirstlane(lane);
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l),
+                            __builtin_amdgcn_readlane(__double2loint(v), l));
+}
+// v of another lane of the row of 16 by the DPP control kCtrl (no LDS round trip)
+template <int kCtrl>
+__device__ __forceinline__ double dpp_of(double v) {
+    const int hi = __double2hiint(v), lo = __double2loint(v);
+    return __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, kCtrl, 0xf, 0xf, false),
+                            __builtin_amdgcn_update_dpp(lo, lo, kCtrl, 0xf, 0xf, false));
+}
+constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppHalfMirror = 0x141, kDppMirror = 0x140;
+
+template <bool kLds>
+__global__ void __launch_bounds__(64 * kSmWaves)
+k_sm_passes(SmSeq q) {
+    extern __shared__ double2 smem_sm[];
+    const int n = q.n, nw = (n + 63) / 64 * 2;
+    double2* xy = kLds ? smem_sm : q.xy;
+    unsigned* marks = reinterpret_cast<unsigned*>(smem_sm + (kLds ? n : 0));
+    unsigned* free_ = marks + nw;
+    volatile int* prog = reinterpret_cast<volatile int*>(free_ + nw);
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    for (int i = threadIdx.x; i < nw; i += blockDim.x) {
+        unsigned m = 0, f = 0;
+        for (int b = 0; b < 32 && 32 * i + b < n; ++b) {
+            if (q.d.smoothable[32 * i + b]) m |= 1u << b;
+            if (!q.d.fixed[32 * i + b]) f |= 1u << b;
+        }
+        marks[i] = m;
+        free_[i] = f;
+    }
+    if (kLds)
+        for (int i = threadIdx.x; i < n; i += blockDim.x) xy[i] = q.xy[i];
+    if (threadIdx.x < kSmWaves) prog[threadIdx.x] = 0;
+    __syncthreads();
+    if (w < q.npass) {
+        const bool lap = w < q.nlap;
+        const double delta = *q.d.hmin * kSmDelta;
+        double d_max = 0.0;
+        for (int c0 = 0; c0 < n; c0 += 64) {
+            const int node = c0 + lane;
+            const bool in = node < n;
+            const int b_l = in ? q.d.esup2[node] : 0, e_l = in ? q.d.esup2[node + 1] : 0;
+            if (w > 0) {
+                int need = in ? q.need[node] : 0;
+                for (int off = 32; off > 0; off >>= 1) need = max(need, __shfl_xor(need, off, 64));
+                while (prog[w - 1] < need) __builtin_amdgcn_s_sleep(2);
+                __threadfence_block();
+            }
+            unsigned long long passed = 0;
+            int next = -1, nid[3];  // the entries of the node expected next
+            const unsigned long long fr =
+                (unsigned long long)free_[c0 / 32] | ((unsigned long long)free_[c0 / 32 + 1] << 32);
+            for (;;) {
+                const volatile unsigned* mv = marks + c0 / 32;
+                const unsigned long long m =
+                    ((unsigned long long)mv[0] | ((unsigned long long)mv[1] << 32)) & fr & ~passed;
+                if (!m) break;
+                const int j = __builtin_ctzll(m);
+                passed |= (2ull << j) - 1ull;
+                const int ip = c0 + j;
+                const int b = __builtin_amdgcn_readlane(b_l, j);
+                const int cnt = __builtin_amdgcn_readlane(e_l, j) - b;
+                const int G = cnt <= 8 ? 8 : cnt <= 16 ? 16 : 32;  // lanes per group
+                const int k = lane & (G - 1), g = lane / G;
+                const bool act = k < cnt;
+                int id[3] = {ip, ip, ip};
+                if (act)
+                    for (int v = 0; v < 3; ++v)
+                        id[v] = next == j ? nid[v] : q.ring[3 * (b + k) + v];
+                if (j < 63) {  // most nodes marked: the next one's entries, in flight meanwhile
+                    next = j + 1;
+                    const int b1 = __builtin_amdgcn_readlane(b_l, next);
+                    const int k1 = lane & ((__builtin_amdgcn_readlane(e_l, next) - b1 <= 8    ? 8
+                                            : __builtin_amdgcn_readlane(e_l, next) - b1 <= 16 ? 16
+                                                                                              : 32) - 1);
+                    if (b1 + k1 < __builtin_amdgcn_readlane(e_l, next))
+                        for (int v = 0; v < 3; ++v) nid[v] = q.ring[3 * (b1 + k1) + v];
+                }
+                double cx[3], cy[3];
+#pragma unroll
+                for (int v = 0; v < 3; ++v) {
+                    const double2 c = xy[id[v]];
+                    cx[v] = c.x;
+                    cy[v] = c.y;
+                }
+                const double2 own = xy[ip];
+                // quality (sm_mu) and h (sm_h) of the lane's element with the node at x, y
+                auto corners = [&](double x, double y, double (&X)[3], double (&Y)[3]) {
+#pragma unroll
+                    for (int v = 0; v < 3; ++v) {
+                        X[v] = id[v] == ip ? x : cx[v];
+                        Y[v] = id[v] == ip ? y : cy[v];
+                    }
+                };
+                auto mu = [&](double x, double y) {
+                    double X[3], Y[3];
+                    corners(x, y, X, Y);
+                    const double area = X[1] * Y[2] + X[2] * Y[0] + X[0] * Y[1] -
+                                        (X[1] * Y[0] + X[2] * Y[1] + X[0] * Y[2]);
+                    const double l1 = (X[2] - X[1]) * (X[2] - X[1]) + (Y[2] - Y[1]) * (Y[2] - Y[1]);
+                    const double l2 = (X[0] - X[2]) * (X[0] - X[2]) + (Y[0] - Y[2]) * (Y[0] - Y[2]);
+                    const double l3 = (X[1] - X[0]) * (X[1] - X[0]) + (Y[1] - Y[0]) * (Y[1] - Y[0]);
+                    const double l = l1 + l2 + l3;
+                    return kTwoSqrt3 * area / l;
+                };
+                // smallest of the group's v where ok (init where none is smaller;
+                // NaN never is), known to the whole group
+                auto group_min = [&](double v, bool ok, double init) {
+                    double m1 = ok && v < init ? v : init;
+                    auto take = [&](double o) {
+                        if (o < m1) m1 = o;
+                    };
+                    take(dpp_of<kDppXor1>(m1));
+                    take(dpp_of<kDppXor2>(m1));
+                    take(dpp_of<kDppHalfMirror>(m1));  // quads hold one value each
+                    if (G > 8) take(dpp_of<kDppMirror>(m1));
+                    if (G > 16) take(__shfl_xor(m1, 16, 64));
+                    return m1;
+                };
+                // getMu_vec's min_idx: the first element with the smallest quality
+                // below 1 (element 0 when none is), and its quality
+                auto worst = [&](double v, double& vm) {
+                    vm = group_min(v, act, 1.0);
+                    const unsigned long long hit = __ballot(act && v < 1.0 && v == vm);
+                    const unsigned long long mine = (hit >> (g * G)) & ((1ull << G) - 1ull);
+                    if (__any(!mine)) {
+                        const double v0 = __shfl(v, g * G, 64);
+                        if (!mine) vm = v0;
+                    }
+                    return mine ? (int)__builtin_ctzll(mine) : 0;
+                };
+                double x = own.x, y = own.y;
+                if (lap) {  // laplacianSmoothing (:77-111)
+                    const double mu_old = group_min(mu(x, y), act, 1.0);
+                    const int s0 = q.d.psup2[ip], np = q.d.psup2[ip + 1] - s0;
+                    const double2 nb = xy[lane < np ? q.d.psup1[s0 + lane] - 1 : ip];
+                    double xn = 0, yn = 0;
+                    for (int v = 0; v < np; ++v) {
+                        xn = xn + __shfl(nb.x, v, 64);
+                        yn = yn + __shfl(nb.y, v, 64);
+                    }
+                    xn = xn / np;
+                    yn = yn / np;
+                    if (q.d.tol_move) {
+                        const double dX = xn - x, dY = yn - y, tm = q.d.tol_move[ip];
+                        xn = x + dX / (fabs(dX) + fabs(dY)) * tm / 2 * kSmStep;
+                        yn = y + dY / (fabs(dX) + fabs(dY)) * tm / 2 * kSmStep;
+                    }
+                    if (!(group_min(mu(xn, yn), act, 1.0) < mu_old)) {  // else restored
+                        x = xn;
+                        y = yn;
+                    }
+                } else {  // one node of an optimisation sweep (:54-63, :113-171)
+                    if (lane == 0) atomicAnd(&marks[ip >> 5], ~(1u << (ip & 31)));
+                    double v = mu(x, y);
+                    double mu_min;
+                    int mi = worst(v, mu_min);  // the same in every group
+                    if (!(mu_min < kSmTolMetric)) continue;
+                    for (int it = 0; it < kSmSteps; ++it) {
+                        const double xo = x, yo = y;
+                        // getG
+                        const double gx = (mu(xo + delta, yo) - v) / delta;
+                        const double gy = (mu(xo, yo + delta) - v) / delta;
+                        const double gxm = lane_of(gx, mi), gym = lane_of(gy, mi);
+                        const double g2 = gxm * gxm + gym * gym;
+                        // getStep
+                        double step;
+                        if (q.d.tol_move) {
+                            step = q.d.tol_move[ip] / ((fabs(gxm) + fabs(gym)) * (double)kSmSweeps);
+                        } else {
+                            double X[3], Y[3];
+                            corners(xo, yo, X, Y);
+                            const double area = X[1] * Y[2] + X[2] * Y[0] + X[0] * Y[1] -
+                                                (X[1] * Y[0] + X[2] * Y[1] + X[0] * Y[2]);
+                            const double d1 = fabs(X[2] - X[1]) + fabs(Y[2] - Y[1]);
+                            const double d2 = fabs(X[0] - X[2]) + fabs(Y[0] - Y[2]);
+                            const double d3 = fabs(X[1] - X[0]) + fabs(Y[1] - Y[0]);
+                            const double h = group_min(fabs(area) / (d1 + d2 + d3), act, 1.0);
+                            step = h * kSmStep / (fabs(gxm) + fabs(gym));
+                        }
+                        const double gg = gxm * gx + gym * gy;
+                        step = group_min((v - mu_min) / (g2 - gg), act && gg < 0, step);
+                        // the tries, a group each, in batches of 64 / G
+                        bool accepted = false;
+                        for (int t0 = 0; t0 < kSmTries && !accepted; t0 += 64 / G) {
+                            double xs = x, ys = y;
+                            for (int u = 0; u < 64 / G; ++u) {
+                                const double dx = step * gxm, dy = step * gym;
+                                if (u <= g) {
+                                    xs = xs + dx;
+                                    ys = ys + dy;
+                                }
+                                step = .5 * step;
+                            }
+                            const double nv = mu(xs, ys);
+                            double best;
+                            const int nmi = worst(nv, best);
+                            const unsigned long long ok = __ballot(best > mu_min * kSmPlus);
+                            // the first group that raised the worst element, else the
+                            // last try's position (the tries accumulate)
+                            const int sel = ok ? (int)__builtin_ctzll(ok) / G : 64 / G - 1;
+                            x = lane_of(xs, sel * G);
+                            y = lane_of(ys, sel * G);
+                            if (ok) {
+                                v = __shfl(nv, sel * G + k, 64);
+                                mi = __builtin_amdgcn_readlane(
+                                    nmi, __builtin_amdgcn_readfirstlane(sel * G));
+                                mu_min = lane_of(best, sel * G);
+                                accepted = true;
+                            }
+                        }
+                        if (!accepted) {  // restore and stop
+                            x = xo;
+                            y = yo;
+                            break;
+                        }
+                    }
+                    const double ex = x - own.x, ey = y - own.y;
+                    const double d_move = ex * ex + ey * ey;
+                    if (d_move > d_max) d_max = d_move;
+                    if (d_move > __DBL_MIN__ && act && g == 0)  // update_list (:289-298)
+#pragma unroll
+                        for (int u = 0; u < 3; ++u)
+                            if (id[u] != ip) atomicOr(&marks[id[u] >> 5], 1u << (id[u] & 31));
+                }
+                if (lane == 0) xy[ip] = make_double2(x, y);
+                __threadfence_block();  // the wave's other lanes and the next pass read it
+            }
+            if (in) q.hist[(size_t)w * n + node] = xy[node];
+            __threadfence_block();
+            if (lane == 0) prog[w] = min(c0 + 64, n);
+        }
+        if (lane == 0) q.dmax[w] = d_max;
+    }
+    __syncthreads();
+    if (kLds)
+        for (int i = threadIdx.x; i < n; i += blockDim.x) q.xy[i] = xy[i];
+    for (int i = threadIdx.x; i < n; i += blockDim.x)
+        q.d.smoothable[i] = (marks[i >> 5] >> (i & 31)) & 1u;
 }
 
-__global__ void k_sm_sweep_seq(SmDev d, int npoin, double* __restrict__ dmax) {
-    if (blockIdx.x != 0 || threadIdx.x != 0) return;
-    double d_max = 0.0;
-    for (int ip = 1; ip <= npoin; ++ip) {
-        const double dm = sm_sweep_node(d, ip);
-        if (dm > d_max) d_max = dm;
-    }
-    *dmax = d_max;
+// per node: its ring (the nodes of its elements, in esup order) and how far the
+// pass before has to be for it
+__global__ void k_sm_ring(const int* __restrict__ inpoel, const int* __restrict__ esup1,
+                          const int* __restrict__ esup2, int* __restrict__ ring,
+                          int* __restrict__ need, int n) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    int far = i;
+    for (int s = esup2[i]; s < esup2[i + 1]; ++s)
+        for (int k = 0; k < 3; ++k) {
+            const int m = inpoel[3 * (esup1[s] - 1) + k] - 1;
+            ring[3 * s + k] = m;
+            far = max(far, m);
+        }
+    need[i] = far + 1;
+}
+
+__global__ void k_sm_pack(const double* __restrict__ X, const double* __restrict__ Y,
+                          double2* __restrict__ xy, int n) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) xy[i] = make_double2(X[i], Y[i]);
+}
+
+__global__ void k_sm_unpack(const double2* __restrict__ xy, double* __restrict__ X,
+                            double* __restrict__ Y, int n) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    X[i] = xy[i].x;
+    Y[i] = xy[i].y;
 }
 
 // order 1: one lane per node of a colour
@@ -358,11 +658,59 @@ bool smooth_check(const Tables& t, SmoothPlan& plan, double* X, double* Y, doubl
     return hs[1] != 0.0;
 }
 
+// order 0 (see k_sm_passes)
+static int smooth_run_seq(const Tables& t, SmoothPlan& plan, const SmDev& d, hipStream_t s) {
+    const int n = t.npoin;
+    if (plan.ring.n != 9 * (size_t)t.nelem) {  // kept with the mesh's plan
+        plan.ring.alloc(9 * (size_t)t.nelem);
+        plan.need.alloc(n);
+        plan.xy.alloc(n);
+        plan.hist.alloc((size_t)kSmWaves * n);
+        plan.dmax_pass.alloc(kSmWaves);
+    }
+    k_sm_ring<<<grid_for(n), kBlock, 0, s>>>(t.inpoel.p, t.esup1.p, t.esup2.p, plan.ring.p,
+                                             plan.need.p, n);
+    k_sm_pack<<<grid_for(n), kBlock, 0, s>>>(d.X, d.Y, plan.xy.p, n);
+    // the positions in LDS while they fit (9,600 nodes in 160 KB)
+    const size_t base = (size_t)((n + 63) / 64 * 2) * 2 * sizeof(unsigned) + kSmWaves * sizeof(int);
+    const size_t full = base + (size_t)n * sizeof(double2);
+    int dev = 0, most = 0;
+    CFD_HIP(hipGetDevice(&dev));
+    CFD_HIP(hipDeviceGetAttribute(&most, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
+    const bool lds = full <= (size_t)most;
+    if (lds)
+        CFD_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_sm_passes<true>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)full));
+    const double tol_dist = kSmTolDist * plan.hmin;
+    const double2* result = plan.xy.p;
+    int sweep = 0, nlap = 2;
+    for (bool end = false; !end && sweep < kSmSweeps; nlap = 0) {
+        const int nsw = std::min(kSmWaves - nlap, kSmSweeps - sweep);
+        const SmSeq q{d, plan.ring.p, plan.need.p, plan.xy.p, plan.hist.p, plan.dmax_pass.p, n,
+                      nlap + nsw, nlap};
+        if (lds) k_sm_passes<true><<<1, 64 * kSmWaves, full, s>>>(q);
+        else k_sm_passes<false><<<1, 64 * kSmWaves, base, s>>>(q);
+        CFD_HIP(hipGetLastError());
+        double dmax[kSmWaves];
+        CFD_HIP(hipMemcpyAsync(dmax, plan.dmax_pass.p, sizeof(dmax), hipMemcpyDeviceToHost, s));
+        CFD_HIP(hipStreamSynchronize(s));
+        for (int k = nlap; k < nlap + nsw && !end; ++k) {
+            ++sweep;
+            end = dmax[k] < tol_dist;
+            result = plan.hist.p + (size_t)k * n;
+        }
+    }
+    k_sm_unpack<<<grid_for(n), kBlock, 0, s>>>(result, d.X, d.Y, n);
+    CFD_HIP(hipGetLastError());
+    return sweep;
+}
+
 int smooth_run(const Tables& t, SmoothPlan& plan, double* X, double* Y, const double* tol_move,
                int order, hipStream_t s) {
     const int n = t.npoin;
     SmDev d{t.inpoel.p, t.esup1.p, t.esup2.p, t.psup1.p, t.psup2.p, plan.fixed.p,
             X, Y, plan.smoothable.p, tol_move, plan.scal.p};
+    if (order == 0) return smooth_run_seq(t, plan, d, s);
     const int ncol = (int)plan.colour_ptr.size() - 1;
     auto colour_pass = [&](auto launch) {
         for (int c = 0; c < ncol; ++c) {
@@ -371,28 +719,21 @@ int smooth_run(const Tables& t, SmoothPlan& plan, double* X, double* Y, const do
         }
     };
     for (int it = 0; it < 2; ++it) {
-        if (order == 0)
-            k_sm_laplacian_seq<<<1, 1, 0, s>>>(d, n);
-        else
-            colour_pass([&](const int* nodes, int cnt) {
-                k_sm_laplacian_colour<<<grid_for(cnt), kBlock, 0, s>>>(d, nodes, cnt);
-            });
+        colour_pass([&](const int* nodes, int cnt) {
+            k_sm_laplacian_colour<<<grid_for(cnt), kBlock, 0, s>>>(d, nodes, cnt);
+        });
     }
     CFD_HIP(hipGetLastError());
     const double tol_dist = kSmTolDist * plan.hmin;
     const int nbm = std::min<int>(grid_for(n), kRedBlocks);
     int sweep = 1;
     for (; sweep <= kSmSweeps; ++sweep) {
-        if (order == 0) {
-            k_sm_sweep_seq<<<1, 1, 0, s>>>(d, n, plan.scal.p + 2);
-        } else {
-            plan.dmove.zero(s);
-            colour_pass([&](const int* nodes, int cnt) {
-                k_sm_sweep_colour<<<grid_for(cnt), kBlock, 0, s>>>(d, nodes, cnt, plan.dmove.p);
-            });
-            k_sm_max<<<nbm, kBlock, 0, s>>>(plan.dmove.p, n, plan.partials.p);
-            k_sm_max_fin<<<1, 256, 0, s>>>(plan.partials.p, nbm, plan.scal.p + 2);
-        }
+        plan.dmove.zero(s);
+        colour_pass([&](const int* nodes, int cnt) {
+            k_sm_sweep_colour<<<grid_for(cnt), kBlock, 0, s>>>(d, nodes, cnt, plan.dmove.p);
+        });
+        k_sm_max<<<nbm, kBlock, 0, s>>>(plan.dmove.p, n, plan.partials.p);
+        k_sm_max_fin<<<1, 256, 0, s>>>(plan.partials.p, nbm, plan.scal.p + 2);
         CFD_HIP(hipGetLastError());
         double dmax;
         CFD_HIP(hipMemcpyAsync(&dmax, plan.scal.p + 2, sizeof(double), hipMemcpyDeviceToHost, s));

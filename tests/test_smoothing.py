@@ -343,3 +343,52 @@ def test_smoothing_refusals():
     with pytest.raises(CfdError, match="together"):
         mc.smoothing(X, Y, fixed, dX=np.zeros(k + 1), order=1)
     mc.close()
+
+
+def _renumbered(m, seed):
+    """The mesh with its nodes in random order: neighbours far apart."""
+    p = np.random.default_rng(seed).permutation(m.npoin)
+    X, Y = np.empty(m.npoin), np.empty(m.npoin)
+    X[p], Y[p] = m.x, m.y
+    return (p[m.inpoel - 1] + 1).astype(np.int32), X, Y, p
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nr, nt, shuffle", [
+    (3, 5, False), (9, 64, False), (33, 65, False), (24, 40, True), (70, 130, False),
+    (98, 98, False),        # 9,604 nodes: about the most whose positions fit LDS
+    (90, 120, False),       # 10,800 nodes: positions in global memory
+])
+def test_reference_order_waves_bitwise(nr, nt, shuffle):
+    """Order 0's passes run side by side in one block: the chunks' edges, both
+    places of the positions, and a numbering in which every node waits for far
+    ones, bit for bit against the sequential oracle, with the sweep count."""
+    from cfd_amd.api import MeshContext
+    m = cylinder_case(nr, nt).mesh
+    inp, X, Y = m.inpoel, m.x, m.y
+    fixed = np.zeros(m.npoin, np.int32)
+    fixed[: m.nt] = fixed[-m.nt:] = 1
+    if shuffle:
+        inp, X, Y, p = _renumbered(m, nr)
+        f = np.zeros_like(fixed)
+        f[p] = fixed
+        fixed = f
+    print(f"order 0 on {m.npoin} nodes", flush=True)
+    xo, yo, n, h = orc.smoothing(inp, X.size, X, Y, fixed)
+    xg, yg, ng, hg = MeshContext(inp, m.npoin).smoothing(X, Y, fixed)
+    assert (n, h) == (ng, hg)
+    assert np.array_equal(xo.view(np.int64), xg.view(np.int64))
+    assert np.array_equal(yo.view(np.int64), yg.view(np.int64))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("k", [3, 8, 9, 16, 17, 20])
+def test_reference_order_ring_sizes_bitwise(k):
+    """One free node with k elements: every group width and its edges."""
+    from cfd_amd.api import MeshContext
+    for seed in range(4):
+        inp, X, Y, fixed = star(np.random.default_rng(100 * k + seed), k)
+        xo, yo, n, h = orc.smoothing(inp, X.size, X, Y, fixed)
+        xg, yg, ng, hg = MeshContext(inp, X.size).smoothing(X, Y, fixed)
+        assert (n, h) == (ng, hg)
+        assert np.array_equal(xo, xg) and np.array_equal(yo, yg)
