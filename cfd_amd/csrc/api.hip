@@ -6,6 +6,7 @@
 #include <cstring>
 #include <map>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -651,7 +652,16 @@ struct Renumbering {
     cfd_mesh* mesh = nullptr;       // the renumbered mesh, owned
     std::vector<int> node_old;      // node_old[i]: the caller's node at position i
     std::vector<int> elem_old;      // elem_old[q]: the caller's element at position q
-    std::vector<long long> lap_old; // the caller's CSR entry of each Laplace entry
+    std::vector<int> lap_old;       // the caller's CSR entry of each Laplace entry
+    // the three on the device, and room for one field in the caller's order
+    // (grown to the largest field that crossed the boundary)
+    DBuf<int> d_node, d_elem, d_lap;
+    DBuf<double> stage;
+    std::mutex stage_mu;  // held while a field crosses
+    double* room(size_t n) {
+        if (stage.n < n) stage.alloc(n);
+        return stage.p;
+    }
     ~Renumbering() {
         if (mesh) cfd_mesh_destroy(mesh);
     }
@@ -1124,6 +1134,14 @@ static cfd_session* create_renumbered(cfd_mesh* m, const cfd_case_desc* d) {
             CFD_CHECK(rn->lap_old[q] >= 0, "internal: renumbered Laplace entry");
         }
     }
+    auto put = [&](DBuf<int>& d, const std::vector<int>& v) {
+        d.alloc(v.size());
+        d.upload(v.data(), v.size(), s);
+    };
+    put(rn->d_node, rn->node_old);
+    put(rn->d_elem, rn->elem_old);
+    put(rn->d_lap, rn->lap_old);
+    CFD_HIP(hipStreamSynchronize(s));
     own->rn = std::move(rn);
     return own.release();
 }
@@ -1307,24 +1325,12 @@ static FieldKind field_kind(int f, int& width) {
     }
 }
 
-// in[position] -> out[caller's position] (to_caller) or back
-static void renumber_field(const Renumbering& rn, int f, const double* in, double* out,
-                           bool to_caller) {
-    int w = 1;
+// the map of field f's entities to the caller's, their number and width
+static const int* field_map(const Renumbering& rn, int f, int& n, int& w) {
     const FieldKind k = field_kind(f, w);
-    if (k == FK_LAP) {
-        for (size_t q = 0; q < rn.lap_old.size(); ++q) {
-            if (to_caller) out[rn.lap_old[q]] = in[q];
-            else out[q] = in[rn.lap_old[q]];
-        }
-        return;
-    }
-    const std::vector<int>& old = k == FK_NODE ? rn.node_old : rn.elem_old;
-    for (size_t i = 0; i < old.size(); ++i)
-        for (int c = 0; c < w; ++c) {
-            if (to_caller) out[w * (size_t)old[i] + c] = in[w * i + c];
-            else out[w * i + c] = in[w * (size_t)old[i] + c];
-        }
+    const DBuf<int>& d = k == FK_NODE ? rn.d_node : k == FK_ELEM ? rn.d_elem : rn.d_lap;
+    n = (int)d.n;
+    return d.p;
 }
 
 extern "C" {
@@ -1334,8 +1340,6 @@ int cfd_session_get_field(cfd_session* S, int f, double* host_out) {
         CFD_ARG(S && host_out, "null argument");
         long long n = 0;
         S->field(f, n);
-        std::vector<double> tmp(S->rn ? (size_t)n : 0);
-        double* host = S->rn ? tmp.data() : host_out;
         DBuf<double>* b = S->field(f, n);
         const bool estab_field = f == CFD_F_SHOC || f == CFD_F_T_SUGN1 || f == CFD_F_T_SUGN2 ||
                                  f == CFD_F_T_SUGN3;
@@ -1349,9 +1353,18 @@ int cfd_session_get_field(cfd_session* S, int f, double* host_out) {
             launch_dt_finish(S->DT.p, S->DTL.p, S->ctl.p, nullptr, false, S->ne, S->s);
             S->dt_stale = false;
         }
-        b->download(host, n, S->s);
+        const double* src = b->p;
+        std::unique_lock<std::mutex> hold;
+        if (S->rn) {  // in the caller's order, on the device
+            int m = 0, w = 1;
+            const int* map = field_map(*S->rn, f, m, w);
+            hold = std::unique_lock<std::mutex>(S->rn->stage_mu);
+            double* out = S->rn->room(n);
+            launch_scatter_field(src, out, map, m, w, S->s);
+            src = out;
+        }
+        CFD_HIP(hipMemcpyAsync(host_out, src, sizeof(double) * n, hipMemcpyDeviceToHost, S->s));
         CFD_HIP(hipStreamSynchronize(S->s));
-        if (S->rn) renumber_field(*S->rn, f, tmp.data(), host_out, true);
     })
 }
 
@@ -1360,10 +1373,17 @@ int cfd_session_set_field(cfd_session* S, int f, const double* host_in) {
         CFD_ARG(S && host_in, "null argument");
         long long n = 0;
         DBuf<double>* b = S->field(f, n);
-        std::vector<double> tmp(S->rn ? (size_t)n : 0);
-        if (S->rn) renumber_field(*S->rn, f, host_in, tmp.data(), false);
-        const double* host = S->rn ? tmp.data() : host_in;
-        b->upload(host, n, S->s);
+        std::unique_lock<std::mutex> hold;
+        if (S->rn) {
+            int m = 0, w = 1;
+            const int* map = field_map(*S->rn, f, m, w);
+            hold = std::unique_lock<std::mutex>(S->rn->stage_mu);
+            double* in = S->rn->room(n);
+            CFD_HIP(hipMemcpyAsync(in, host_in, sizeof(double) * n, hipMemcpyHostToDevice, S->s));
+            launch_gather_field(in, b->p, map, m, w, S->s);
+        } else {
+            b->upload(host_in, n, S->s);
+        }
         CFD_HIP(hipStreamSynchronize(S->s));
         if (f == CFD_F_W_X || f == CFD_F_W_Y || f == CFD_F_XPOS || f == CFD_F_YPOS) S->w_dirty = true;
         if (f == CFD_F_XPOS || f == CFD_F_YPOS) S->xpos_zero = false;

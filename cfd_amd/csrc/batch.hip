@@ -19,6 +19,7 @@
 // with the host or clears memory with hipMemsetAsync.
 #include <map>
 #include <memory>
+#include <mutex>
 
 #include "cfd_internal.hpp"
 
@@ -52,6 +53,9 @@ struct cfd_batch {
     std::vector<std::vector<double>> X_h, Y_h;
     // per case: the caller's node / element at each patch-order position
     std::vector<std::vector<int>> node_old, elem_old;
+    DBuf<int> d_node, d_elem;  // the same on the device, the cases one after the other
+    DBuf<double> stage;        // one case's field in the caller's order
+    std::mutex stage_mu;       // held while a field crosses
     // graphs: one recorded step per U buffer parity
     bool use_graph = true;
     hipGraphExec_t gexec[2] = {nullptr, nullptr};
@@ -350,6 +354,14 @@ int cfd_batch_create(cfd_batch** out, int ncases, const cfd_batch_case* cases, i
                     key[B->ebase[k] + e] = B->ebase[k] + B->elem_old[k][e];
             reorder_esup(B->t, key, s);
         }
+        for (int pass = 0; pass < 2; ++pass) {
+            std::vector<int> all;
+            for (const auto& v : pass ? B->elem_old : B->node_old) all.insert(all.end(), v.begin(), v.end());
+            DBuf<int>& d = pass ? B->d_elem : B->d_node;
+            d.alloc(all.size());
+            d.upload(all.data(), all.size(), s);
+            CFD_HIP(hipStreamSynchronize(s));
+        }
         B->bc.upload(build_bc_host(B->np, &ub), B->np, &ub, s);
         // state
         for (auto* b : {&B->Ub[0], &B->Ub[1], &B->RHS}) b->alloc(4 * (size_t)np);
@@ -478,14 +490,13 @@ int cfd_batch_get_field(cfd_batch* b, int icase, int field, double* host) {
         }
         const size_t o = node ? b->nbase[icase] : b->ebase[icase];
         const size_t n = node ? b->nbase[icase + 1] - o : b->ebase[icase + 1] - o;
-        std::vector<double> tmp(w * n);
-        CFD_HIP(hipMemcpyAsync(tmp.data(), buf->p + w * o, sizeof(double) * w * n,
-                               hipMemcpyDeviceToHost, b->s));
+        // back to the caller's numbering of the case, on the device
+        std::lock_guard<std::mutex> hold(b->stage_mu);
+        if (b->stage.n < w * n) b->stage.alloc(w * n);
+        launch_scatter_field(buf->p + w * o, b->stage.p, (node ? b->d_node.p : b->d_elem.p) + o,
+                             (int)n, w, b->s);
+        CFD_HIP(hipMemcpyAsync(host, b->stage.p, sizeof(double) * w * n, hipMemcpyDeviceToHost, b->s));
         CFD_HIP(hipStreamSynchronize(b->s));
-        // back to the caller's numbering of the case
-        const std::vector<int>& old = node ? b->node_old[icase] : b->elem_old[icase];
-        for (size_t i = 0; i < n; ++i)
-            for (int c = 0; c < w; ++c) host[w * (size_t)old[i] + c] = tmp[w * i + c];
     })
 }
 

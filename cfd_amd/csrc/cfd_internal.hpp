@@ -532,6 +532,14 @@ void launch_step_ctl(const double* partials, const int* pb, int nb, double* ctl,
 void launch_dt_finish(double* DT, double* DTL, const double* ctl, const int* ecase, bool blend,
                       int nelem, hipStream_t s);
 
+// Fields between a renumbered state and the caller's numbering: entity i of
+// the state is the caller's map[i], w doubles each (4 for U, U1, RHS; 3 for
+// the gradients).  scatter: caller[map[i]] = state[i]; gather the other way.
+void launch_scatter_field(const double* state, double* caller, const int* map, int n, int w,
+                          hipStream_t s);
+void launch_gather_field(const double* caller, double* state, const int* map, int n, int w,
+                         hipStream_t s);
+
 // meshMove.f90 FORCES (out3 = FX, FY, RM; skipped when null) and, when visc
 // is given, FORCE_VISC (ns2DComp.ALE.f90:819-893; out2 = F_VX, F_VY) in the
 // same launch; device scalars out

@@ -100,7 +100,43 @@ __global__ void k_dt_finish(double* __restrict__ DT, double* __restrict__ DTL,
     }
 }
 
+// One thread per entity.  Bound by the scattered side (32-byte records of U
+// fill a memory sector each): U of 2,097,152 nodes 64 MB in, 64 MB out.  In
+// place of a loop on the host, which took 20 of the 24 ms of reading U.
+template <int W, bool kScatter>
+__global__ void k_renumber(const double* __restrict__ in, double* __restrict__ out,
+                           const int* __restrict__ map, int n) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const size_t a = kScatter ? i : map[i], b = kScatter ? map[i] : i;
+    if constexpr (W == 4) {
+        reinterpret_cast<double4*>(out)[b] = reinterpret_cast<const double4*>(in)[a];
+    } else {
+#pragma unroll
+        for (int c = 0; c < W; ++c) out[W * b + c] = in[W * a + c];
+    }
+}
+
+template <bool kScatter>
+void renumber(const double* in, double* out, const int* map, int n, int w, hipStream_t s) {
+    if (n <= 0) return;
+    const unsigned g = grid_for(n);
+    if (w == 4) k_renumber<4, kScatter><<<g, kBlock, 0, s>>>(in, out, map, n);
+    else if (w == 3) k_renumber<3, kScatter><<<g, kBlock, 0, s>>>(in, out, map, n);
+    else k_renumber<1, kScatter><<<g, kBlock, 0, s>>>(in, out, map, n);
+    CFD_HIP(hipGetLastError());
+}
+
 }  // namespace
+
+void launch_scatter_field(const double* state, double* caller, const int* map, int n, int w,
+                          hipStream_t s) {
+    renumber<true>(state, caller, map, n, w, s);
+}
+void launch_gather_field(const double* caller, double* state, const int* map, int n, int w,
+                         hipStream_t s) {
+    renumber<false>(caller, state, map, n, w, s);
+}
 
 // ---------------------------------------------------------------------------
 // Boundary-condition table (host construction, reference list semantics)
