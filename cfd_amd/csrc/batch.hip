@@ -6,14 +6,14 @@
 // hysteresis, the clock: X_NCTL scalars per case) and its own free stream
 // (rho_inf, u_inf, v_inf: the Mach number, angle of attack and Reynolds
 // number of a sweep); every other constant is shared.  Per RK stage one
-// launch of the fused patch kernel covers every case (a resident grid loops
-// over all cases' patches, whose shape -- elements and threads per patch --
-// is a parameter the autotuner picks), followed by the halo pass.  Patches
+// launch of the fused patch kernel covers every case (a block per patch; the
+// patches' shape -- elements and threads per patch -- is a parameter the
+// autotuner picks), followed by the halo pass.  Patches
 // never straddle two cases and are built per case exactly as a single-case
 // session builds them, so each case's arithmetic and summation order are
 // those of that case run on its own: results agree bit for bit.
 //
-// A whole time step (deltat with one min partial per case chunk, step
+// A whole time step (deltat with one min partial per patch, step
 // control per case, ESTAB, the four fused stages) is recorded once into a
 // hipGraph per U buffer parity and replayed; nothing in it synchronises
 // with the host or clears memory with hipMemsetAsync.
@@ -25,14 +25,10 @@
 
 using namespace cfd;
 
-namespace {
-constexpr int kChunkElems = 8192;  // elements per deltat partial
-}
-
 struct cfd_batch {
     hipStream_t s = nullptr;
     int ncases = 0, precision = 1, itlocal = 0, nrk = 4;
-    int np = 0, ne = 0, nchunks = 0;
+    int np = 0, ne = 0;
     std::vector<int> nbase, ebase;
     std::vector<Consts> cc;  // per case
     Consts c{};              // the shared constants (case 0's free stream)
@@ -45,7 +41,7 @@ struct cfd_batch {
     DBuf<double> DTL, DT, AREA, DNX, DNY, HH, HHX, HHY, SHOC, T1, T2, T3;
     DBuf<float> DN32, NT32, FAC32;
     DBuf<double> DN6, DN64, NT64, FAC64;
-    DBuf<int> ecase, chunk, chunk_case, pb;
+    DBuf<int> ecase, pb;  // pb: each case's patches are [pb[k], pb[k+1])
     DBuf<Consts> cases;  // per case
     DBuf<double> ctl, partials, hmin;
     // host copies for re-building patches (autotuning)
@@ -56,6 +52,9 @@ struct cfd_batch {
     DBuf<int> d_node, d_elem;  // the same on the device, the cases one after the other
     DBuf<double> stage;        // one case's field in the caller's order
     std::mutex stage_mu;       // held while a field crosses
+    // With itlocal = 0 DT's clip and DTL (DTMIN everywhere) are formed when a
+    // caller reads them: no kernel of a step does
+    bool dt_stale = false;
     // graphs: one recorded step per U buffer parity
     bool use_graph = true;
     hipGraphExec_t gexec[2] = {nullptr, nullptr};
@@ -84,7 +83,7 @@ struct cfd_batch {
         o.nt = nt;
         o.fac = fac;
         o.area = AREA.p;
-        o.dtl = DTL.p;
+        o.dtl = itlocal ? DTL.p : nullptr;
         o.inv_perm = patches.inv_perm.p;
         o.cte = c.cte;
         o.ecase = ecase.p;
@@ -117,10 +116,13 @@ struct cfd_batch {
         build_patches_batch(patches, ncases, ip.data(), xs.data(), ys.data(), nes.data(), nps.data(),
                             pe, block, s);
         patches.cases = cases.p;
-        if (precision == 1)
-            patch_make_persistent<float>(patches, false);
-        else
-            patch_make_persistent<double>(patches, false);
+        std::vector<int> base(1, 0);
+        for (int k = 0; k < ncases; ++k) base.push_back(base.back() + (nes[k] + pe - 1) / pe);
+        CFD_CHECK(base.back() == patches.npatch, "internal: batch patches");
+        pb.alloc(base.size());
+        pb.upload(base.data(), base.size(), s);
+        partials.alloc(std::max<size_t>(grid_for(ne), patches.npatch));
+        CFD_HIP(hipStreamSynchronize(s));
         refresh_patch_geometry();
         drop_graphs();
     }
@@ -128,15 +130,16 @@ struct cfd_batch {
     // One time step of every case (ns2DComp.ALE.f90:140-182 on a fixed mesh)
     void step_body() {
         const double* dtmin = ctl.p + CFD_S_DTMIN;
-        launch_deltat_chunks(t, c, AREA.p, T.p, VX.p, VY.p, WX.p, WY.p, DT.p, chunk.p, nchunks,
-                             partials.p, chunk_case.p, cases.p, s);
-        launch_step_ctl(partials.p, pb.p, nchunks, ctl.p, ncases, itlocal, 0, 0.0, 0.0, s);
-        launch_dt_finish(DT.p, DTL.p, ctl.p, ecase.p, itlocal != 0, ne, s);
+        // fixed meshes at rest: W is zero and not read
+        launch_deltat_patch(patches, c, AREA.p, T.p, VX.p, VY.p, nullptr, nullptr, DT.p, partials.p,
+                            s);
+        launch_step_ctl(partials.p, pb.p, patches.npatch, ctl.p, ncases, itlocal, 0, 0.0, 0.0, s);
+        if (itlocal) launch_dt_finish(DT.p, DTL.p, ctl.p, ecase.p, true, ne, s);
         if (precision == 1)
-            launch_estab_patch(t, patches, c, U(), T.p, GAMM.p, VX.p, VY.p, WX.p, WY.p, DNX.p,
+            launch_estab_patch(t, patches, c, U(), T.p, GAMM.p, VX.p, VY.p, nullptr, nullptr, DNX.p,
                                DNY.p, nullptr, dtmin, elem32(), s);
         else
-            launch_estab_patch(t, patches, c, U(), T.p, GAMM.p, VX.p, VY.p, WX.p, WY.p, DNX.p,
+            launch_estab_patch(t, patches, c, U(), T.p, GAMM.p, VX.p, VY.p, nullptr, nullptr, DNX.p,
                                DNY.p, DN6.p, dtmin, elem64(), s);
         PatchIn<float> in32{U(), T.p, nullptr, nullptr, DN32.p,
                             FAC32.p, NT32.p};
@@ -175,9 +178,17 @@ struct cfd_batch {
             }
             ucur ^= 1;  // U = U1
         }
+        if (n > 0 && !itlocal) dt_stale = true;
+    }
+
+    void finish_dt() {
+        if (!dt_stale) return;
+        launch_dt_finish(DT.p, DTL.p, ctl.p, ecase.p, false, ne, s);
+        dt_stale = false;
     }
 
     void init_freestream() {
+        finish_dt();  // the last step's, from the scalars cleared below
         for (int k = 0; k < ncases; ++k) {
             const size_t o = nbase[k];
             launch_freestream({U() + 4 * o, U1() + 4 * o, VX.p + o, VY.p + o, T.p + o, GAMM.p + o,
@@ -387,30 +398,16 @@ int cfd_batch_create(cfd_batch** out, int ncases, const cfd_batch_case* cases, i
             b->zero(s);
         B->X.upload(X.data(), np, s);
         B->Y.upload(Y.data(), np, s);
-        // per case: element -> case, deltat chunks inside cases, rho_inf
-        std::vector<int> ec(ne), ch(1, 0), chc, cpb(1, 0);
-        for (int k = 0; k < ncases; ++k) {
-            for (int e = B->ebase[k]; e < B->ebase[k + 1]; ++e) ec[e] = k;
-            for (int e = B->ebase[k]; e < B->ebase[k + 1]; e += kChunkElems) {
-                ch.push_back(std::min(e + kChunkElems, B->ebase[k + 1]));
-                chc.push_back(k);
-            }
-            cpb.push_back((int)ch.size() - 1);
-        }
-        B->nchunks = (int)ch.size() - 1;
+        std::vector<int> ec(ne);  // element -> case
+        for (int k = 0; k < ncases; ++k)
+            std::fill(ec.begin() + B->ebase[k], ec.begin() + B->ebase[k + 1], k);
         B->ecase.alloc(ne);
         B->ecase.upload(ec.data(), ne, s);
-        B->chunk.alloc(ch.size());
-        B->chunk.upload(ch.data(), ch.size(), s);
-        B->chunk_case.alloc(chc.size());
-        B->chunk_case.upload(chc.data(), chc.size(), s);
-        B->pb.alloc(cpb.size());
-        B->pb.upload(cpb.data(), cpb.size(), s);
         B->cases.alloc(ncases);
         B->cases.upload(B->cc.data(), ncases, s);
         B->ctl.alloc((size_t)ncases * X_NCTL);
         B->ctl.zero(s);
-        B->partials.alloc(std::max<size_t>(grid_for(ne), B->nchunks));
+        B->partials.alloc(grid_for(ne));
         B->hmin.alloc(1);
         // geometry once (fixed meshes): NORMALES, DERIV, MASAS
         B->bc.normales(B->X.p, B->Y.p, s);
@@ -488,6 +485,7 @@ int cfd_batch_get_field(cfd_batch* b, int icase, int field, double* host) {
                 launch_estab_widen(b->elem64(), b->patches.inv_perm.p, b->ne, b->SHOC.p, b->T1.p,
                                    b->T2.p, b->T3.p, b->s);
         }
+        if (field == CFD_F_DT || field == CFD_F_DTL) b->finish_dt();
         const size_t o = node ? b->nbase[icase] : b->ebase[icase];
         const size_t n = node ? b->nbase[icase + 1] - o : b->ebase[icase + 1] - o;
         // back to the caller's numbering of the case, on the device

@@ -208,17 +208,12 @@ int launch_deltat_partials(const Tables& t, const Consts& c, const double* area,
                            const double* VX, const double* VY, const double* WX, const double* WY,
                            double* DT, double* partials, hipStream_t s);
 // The same in patch order (one block per patch of ps, its node values in
-// LDS): the same DT bits, one min partial per patch; returns ps.npatch
+// LDS): the same DT bits, one min partial per patch; returns ps.npatch.  A
+// batch's patches take their case's constants.
 struct PatchSet;
 int launch_deltat_patch(const PatchSet& ps, const Consts& c, const double* area, const double* T,
                         const double* VX, const double* VY, const double* WX, const double* WY,
                         double* DT, double* partials, hipStream_t s);
-// The same with block b over the elements [chunk[b], chunk[b+1]): one min
-// partial per chunk (batches keep each chunk inside one case)
-void launch_deltat_chunks(const Tables& t, const Consts& c, const double* area, const double* T,
-                          const double* VX, const double* VY, const double* WX, const double* WY,
-                          double* DT, const int* chunk, int nchunks, double* partials,
-                          const int* chunk_case, const Consts* cases, hipStream_t s);
 // Inputs of the patch element residual (patch order, of the element type R:
 // float on the FP32 path, double on the fused FP64 path), written by ESTAB
 // in place of its element-order outputs: per element one record of nu =
@@ -318,8 +313,6 @@ constexpr int kPatchMaxNodes = 700;  // keeps the fused kernel's LDS within 64 K
 struct PatchSet {
     int npatch = 0, max_nodes = 0, nentries = 0, nhalo = 0;
     int pe = kPatchElems, block = 256;  // elements per patch, threads per patch
-    bool persistent = false;            // a resident grid loops over the patches
-    int grid[2] = {0, 0};               // its size, intermediate and final stages
     // batches: case of each patch and of each halo node, the cases' constants
     DBuf<int> pcase, hcase;
     const struct Consts* cases = nullptr;
@@ -366,10 +359,6 @@ template <class R>
 void launch_patch_stage(const Tables& t, const PatchSet& ps, const Consts& c, const BcTable& bc,
                         double rk_fact, const PatchIn<R>& in, const StageNodes& nd,
                         bool final_stage, hipStream_t s);
-// A resident grid for ps (persistent = true): as many blocks of the fused
-// kernel (element type R) as stay resident on the device at once
-template <class R>
-void patch_make_persistent(PatchSet& ps, bool fuente);
 // whether the fused kernel's LDS (node values, W, slots of slot_bytes,
 // slot ranges) fits its 64 KB budget for patches of pe elements and up to
 // max_nodes nodes

@@ -54,22 +54,12 @@ __global__ void __launch_bounds__(kBlock)
 k_deltat(const int* __restrict__ inpoel, const double* __restrict__ area, const double* __restrict__ T,
          const double* __restrict__ VX, const double* __restrict__ VY, const double* __restrict__ WX,
          const double* __restrict__ WY, double* __restrict__ DT, int nelem, double t_inf,
-         double fsafe, double* __restrict__ partials, const int* __restrict__ chunk,
-         const int* __restrict__ chunk_case, const Consts* __restrict__ cases) {
-    // grid-stride over all elements, or (chunk) block b over [chunk[b], chunk[b+1])
-    // with (cases) the constants of the chunk's case
-    if (chunk && cases) {
-        const Consts& q = cases[chunk_case[blockIdx.x]];
-        t_inf = q.t_inf;
-        fsafe = q.fsafe;
-    }
+         double fsafe, double* __restrict__ partials) {
     // grid-stride: logical blocks in XCD order (neighbouring elements' nodes
     // mostly in one L2); the min partial goes to the logical block
-    const int lb = chunk ? (int)blockIdx.x : xcd_block(blockIdx.x, gridDim.x);
-    const int beg = chunk ? chunk[blockIdx.x] + (int)threadIdx.x
-                          : (int)(lb * blockDim.x + threadIdx.x);
-    const int end = chunk ? chunk[blockIdx.x + 1] : nelem;
-    const int step = chunk ? (int)blockDim.x : (int)(gridDim.x * blockDim.x);
+    const int lb = xcd_block(blockIdx.x, gridDim.x);
+    const int beg = (int)(lb * blockDim.x + threadIdx.x);
+    const int end = nelem, step = (int)(gridDim.x * blockDim.x);
     double dmin = 1.0e20;
     for (int e = beg; e < end; e += step) {
         const int* ip = inpoel + 3 * e;
@@ -90,7 +80,9 @@ k_deltat(const int* __restrict__ inpoel, const double* __restrict__ area, const 
 
 // deltat in patch order: one block per patch, the patch's node values (T,
 // |VX - WX|, |VY - WY|) staged in LDS, each element's DT from deltat_elem
-// (the same values as k_deltat), one min partial per patch
+// (the same values as k_deltat), one min partial per patch.  Batches: the
+// constants of the patch's case (32 cases of a sweep, 3.1M triangles: 46 us,
+// against 76 in element order with 15 gathers an element).
 struct DtNode {
     double T, vu, vv;
 };
@@ -101,10 +93,16 @@ k_deltat_patch(const int* __restrict__ node_base, const int* __restrict__ elem_b
                const double* __restrict__ T, const double* __restrict__ VX,
                const double* __restrict__ VY, const double* __restrict__ WX,
                const double* __restrict__ WY, double* __restrict__ DT, double t_inf, double fsafe,
-               double* __restrict__ partials) {
+               double* __restrict__ partials, const int* __restrict__ pcase,
+               const Consts* __restrict__ cases) {
     extern __shared__ double4 smem4[];
     DtNode* sN = reinterpret_cast<DtNode*>(smem4);
     const int p = xcd_block(blockIdx.x, npatch);  // grid = npatch: logical patch
+    if (pcase) {
+        const Consts& q = cases[pcase[p]];
+        t_inf = q.t_inf;
+        fsafe = q.fsafe;
+    }
     const int nb = node_base[p], nl = node_base[p + 1] - nb;
     for (int l = threadIdx.x; l < nl; l += blockDim.x) {
         const int g = pnode[nb + l] - 1;
@@ -804,10 +802,13 @@ struct PatchDev {
 };
 
 // At most 168 VGPRs, so that 3 waves per SIMD stay resident (the LDS of the
-// default patch shapes allows 3 blocks of 256 threads per CU): the FP64
-// fixed-mesh stages fit without spilling (174 VGPRs would leave 2 waves),
-// the FP64 moving-mesh stages spill 24 B per thread and still run faster
-// than at 188 VGPRs and 2 waves
+// default patch shapes allows 3 blocks of 256 threads per CU): the FP64 stages
+// take 144 (fixed mesh) and 164 (moving mesh) and spill nothing.  One patch
+// per block and no loop over patches: a resident grid's loop kept the block's
+// constants alive across patches (168 VGPRs, 24 B of spills on moving meshes)
+// and cost the FP64 launches 7 us of 160 (intermediate) and 17 of 192 (final),
+// ESTAB 16 of 155, and a 32-case batch's FP32 stages 6 of 92, at 4.2M and 3.1M
+// triangles, with the same results.
 template <class R, bool kFuente, bool kFinal>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(3)))
 k_patch_stage(PatchDev pd, ElemConstsP<R> kc, PatchIn<R> in, StageDev a) {
@@ -819,79 +820,74 @@ k_patch_stage(PatchDev pd, ElemConstsP<R> kc, PatchIn<R> in, StageDev a) {
     V4* sC = reinterpret_cast<V4*>(sW + (kFuente ? maxn : 0));    // 3*pe
     double* sT = reinterpret_cast<double*>(sC + 3 * pe);          // maxn
     uint16_t* sP = reinterpret_cast<uint16_t*>(sT + maxn);        // maxn+1
-    // one patch per block, or (resident grid) patches blockIdx.x + k gridDim.x
-    for (int p0 = blockIdx.x; p0 < pd.npatch; p0 += gridDim.x) {
-        // measured: the XCD order helps the FP32 stages (149 -> 143 us per
-        // launch at 4.2M triangles) and slows the FP64 ones (204 -> 208 us)
-        const int p = sizeof(R) == sizeof(float) && (int)gridDim.x == pd.npatch
-                          ? xcd_block(p0, pd.npatch)
-                          : p0;
-        ElemConstsP<R> kl = kc;
-        StageDev al = a;
-        if (pd.pcase) {  // the constants of this patch's case, rounded as the host rounds them
-            const Consts& q = pd.cases[pd.pcase[p]];
-            kl.g = (R)q.gama;
-            kl.Cv = (R)q.fcv;
-            kl.lambda_ref = (R)q.fk;
-            kl.mu_ref = (R)q.fmu;
-            kl.T_inf = (R)q.t_inf;
-            kl.viscous = q.fmu > 2.2250738585072014e-308 ? 1 : 0;
-            al.fr = q.fr;
-        }
-        const int nb = pd.node_base[p], nl = pd.node_base[p + 1] - nb, nint = pd.n_int[p];
-        const long long e0 = pd.elem_base[p];
-        const int nep = pd.elem_base[p + 1] - pd.elem_base[p];
-        for (int l = threadIdx.x; l < nl; l += blockDim.x) {
-            const int g = pd.pnode[nb + l] - 1;
-            sU[l] = ld4(in.U + 4 * (long long)g);
-            sT[l] = in.T[g];
-            if (kFuente) sW[l] = make_double2(in.WX[g], in.WY[g]);
-        }
-        for (int l = threadIdx.x; l <= nl; l += blockDim.x) sP[l] = pd.lptr[nb + p + l];
-        __syncthreads();
-        for (int q = threadIdx.x; q < nep; q += blockDim.x) {
-            const long long e = e0 + q;
-            const uint64_t w = (uint64_t)pd.loc[2 * e] | ((uint64_t)pd.loc[2 * e + 1] << 32);
-            const int ln[3] = {(int)(w & 1023u), (int)((w >> 10) & 1023u), (int)((w >> 20) & 1023u)};
-            const int ls[3] = {(int)((w >> 30) & 2047u), (int)((w >> 41) & 2047u),
-                               (int)((w >> 52) & 2047u)};
-            // P1 gradients sum to zero: the first from the other two
-            const V4 gN = *reinterpret_cast<const V4*>(in.dN + 4 * e);
-            const R Nx[3] = {-(gN.x + gN.y), gN.x, gN.y};
-            const R Ny[3] = {-(gN.z + gN.w), gN.z, gN.w};
-            const V4 t4 = *reinterpret_cast<const V4*>(in.nt + 4 * e);  // nu, tau1..3
-            const R tau[3] = {t4.y, t4.z, t4.w};
-            const double T3[3] = {sT[ln[0]], sT[ln[1]], sT[ln[2]]};
-            double wx3[3] = {0.0, 0.0, 0.0}, wy3[3] = {0.0, 0.0, 0.0};
-            if (kFuente) {
+    // measured: the XCD order helps the FP32 stages (149 -> 143 us per
+    // launch at 4.2M triangles) and slows the FP64 ones (204 -> 208 us)
+    const int p = sizeof(R) == sizeof(float) ? xcd_block(blockIdx.x, pd.npatch)
+                                             : (int)blockIdx.x;
+    ElemConstsP<R> kl = kc;
+    StageDev al = a;
+    if (pd.pcase) {  // the constants of this patch's case, rounded as the host rounds them
+        const Consts& q = pd.cases[pd.pcase[p]];
+        kl.g = (R)q.gama;
+        kl.Cv = (R)q.fcv;
+        kl.lambda_ref = (R)q.fk;
+        kl.mu_ref = (R)q.fmu;
+        kl.T_inf = (R)q.t_inf;
+        kl.viscous = q.fmu > 2.2250738585072014e-308 ? 1 : 0;
+        al.fr = q.fr;
+    }
+    const int nb = pd.node_base[p], nl = pd.node_base[p + 1] - nb, nint = pd.n_int[p];
+    const long long e0 = pd.elem_base[p];
+    const int nep = pd.elem_base[p + 1] - pd.elem_base[p];
+    for (int l = threadIdx.x; l < nl; l += blockDim.x) {
+        const int g = pd.pnode[nb + l] - 1;
+        sU[l] = ld4(in.U + 4 * (long long)g);
+        sT[l] = in.T[g];
+        if (kFuente) sW[l] = make_double2(in.WX[g], in.WY[g]);
+    }
+    for (int l = threadIdx.x; l <= nl; l += blockDim.x) sP[l] = pd.lptr[nb + p + l];
+    __syncthreads();
+    for (int q = threadIdx.x; q < nep; q += blockDim.x) {
+        const long long e = e0 + q;
+        const uint64_t w = (uint64_t)pd.loc[2 * e] | ((uint64_t)pd.loc[2 * e + 1] << 32);
+        const int ln[3] = {(int)(w & 1023u), (int)((w >> 10) & 1023u), (int)((w >> 20) & 1023u)};
+        const int ls[3] = {(int)((w >> 30) & 2047u), (int)((w >> 41) & 2047u),
+                           (int)((w >> 52) & 2047u)};
+        // P1 gradients sum to zero: the first from the other two
+        const V4 gN = *reinterpret_cast<const V4*>(in.dN + 4 * e);
+        const R Nx[3] = {-(gN.x + gN.y), gN.x, gN.y};
+        const R Ny[3] = {-(gN.z + gN.w), gN.z, gN.w};
+        const V4 t4 = *reinterpret_cast<const V4*>(in.nt + 4 * e);  // nu, tau1..3
+        const R tau[3] = {t4.y, t4.z, t4.w};
+        const double T3[3] = {sT[ln[0]], sT[ln[1]], sT[ln[2]]};
+        double wx3[3] = {0.0, 0.0, 0.0}, wy3[3] = {0.0, 0.0, 0.0};
+        if (kFuente) {
 #pragma unroll
-                for (int k = 0; k < 3; ++k) {
-                    wx3[k] = sW[ln[k]].x;
-                    wy3[k] = sW[ln[k]].y;
-                }
+            for (int k = 0; k < 3; ++k) {
+                wx3[k] = sW[ln[k]].x;
+                wy3[k] = sW[ln[k]].y;
             }
-            V4 out[3];
-            elem_residual<R, kFuente>(kl, sU[ln[0]], sU[ln[1]], sU[ln[2]], T3, wx3, wy3, Nx, Ny,
-                                      in.fac[e], t4.x, tau, out);
+        }
+        V4 out[3];
+        elem_residual<R, kFuente>(kl, sU[ln[0]], sU[ln[1]], sU[ln[2]], T3, wx3, wy3, Nx, Ny,
+                                  in.fac[e], t4.x, tau, out);
 #pragma unroll
-            for (int k = 0; k < 3; ++k) sC[ls[k]] = out[k];
+        for (int k = 0; k < 3; ++k) sC[ls[k]] = out[k];
+    }
+    __syncthreads();
+    for (int l = threadIdx.x; l < nl; l += blockDim.x) {
+        double r0 = 0.0, r1 = 0.0, r2 = 0.0, r3 = 0.0;
+        for (int s = sP[l]; s < sP[l + 1]; ++s) {
+            const V4 c = sC[s];
+            r0 = r0 + (double)c.x;
+            r1 = r1 + (double)c.y;
+            r2 = r2 + (double)c.z;
+            r3 = r3 + (double)c.w;
         }
-        __syncthreads();
-        for (int l = threadIdx.x; l < nl; l += blockDim.x) {
-            double r0 = 0.0, r1 = 0.0, r2 = 0.0, r3 = 0.0;
-            for (int s = sP[l]; s < sP[l + 1]; ++s) {
-                const V4 c = sC[s];
-                r0 = r0 + (double)c.x;
-                r1 = r1 + (double)c.y;
-                r2 = r2 + (double)c.z;
-                r3 = r3 + (double)c.w;
-            }
-            if (l < nint)
-                stage_node<kFinal>(al, pd.pnode[nb + l] - 1, sU[l], r0, r1, r2, r3);
-            else
-                st4(pd.hpart + 4 * (long long)(pd.halo_base[p] + l - nint), r0, r1, r2, r3);
-        }
-        __syncthreads();  // the next patch overwrites the LDS arrays
+        if (l < nint)
+            stage_node<kFinal>(al, pd.pnode[nb + l] - 1, sU[l], r0, r1, r2, r3);
+        else
+            st4(pd.hpart + 4 * (long long)(pd.halo_base[p] + l - nint), r0, r1, r2, r3);
     }
 }
 
@@ -937,11 +933,10 @@ k_halo_stage(const int* __restrict__ hnode, const int* __restrict__ hptr,
     stage_node<kFinal>(a, g, u, r0, r1, r2, r3);
 }
 
-// ESTAB in patch order (fused paths): one patch per block (or, resident
-// grid, patches blockIdx.x + k gridDim.x); the patch's node values in LDS;
-// element q's parameters, rounded to R, written at q (coalesced).  FP64
-// gradients: the patch-order copy when the element type is double (an exact
-// copy), else the element-order arrays through perm.
+// ESTAB in patch order (fused paths): one patch per block; the patch's node
+// values in LDS; element q's parameters, rounded to R, written at q
+// (coalesced).  FP64 gradients: the patch-order copy when the element type is
+// double (an exact copy), else the element-order arrays through perm.
 struct EstabNode {
     double rho, T, vx, vy, wx, wy, gm;
 };
@@ -959,64 +954,61 @@ __global__ void __launch_bounds__(512)
 k_estab_patch(PatchDev pd, EstabIn ei, ElemP<R> o) {
     extern __shared__ double4 smem4[];
     EstabNode* sN = reinterpret_cast<EstabNode*>(smem4);  // maxn
-    for (int p0 = blockIdx.x; p0 < pd.npatch; p0 += gridDim.x) {
-        const int p = (int)gridDim.x == pd.npatch ? xcd_block(p0, pd.npatch) : p0;
-        const int cs = pd.pcase ? pd.pcase[p] : 0;
-        const Consts* cq = pd.cases ? pd.cases + cs : nullptr;
-        const double fr = cq ? cq->fr : ei.fr, tinf = cq ? cq->t_inf : ei.tinf;
-        const double rinf = cq ? cq->rho_inf : ei.rinf, cte = cq ? cq->cte : o.cte;
-        const double dtmin = ei.dtmin[(size_t)cs * o.dt_stride];
-        const int nb = pd.node_base[p], nl = pd.node_base[p + 1] - nb;
-        const long long e0 = pd.elem_base[p];
-        const int nep = pd.elem_base[p + 1] - pd.elem_base[p];
-        for (int l = threadIdx.x; l < nl; l += blockDim.x) {
-            const int g = pd.pnode[nb + l] - 1;
-            sN[l] = EstabNode{ei.U[4 * (long long)g], ei.T[g], ei.VX[g], ei.VY[g],
-                              ei.WX ? ei.WX[g] : 0.0, ei.WY ? ei.WY[g] : 0.0, ei.GAMM[g]};
-        }
-        __syncthreads();
-        for (int q = threadIdx.x; q < nep; q += blockDim.x) {
-            const long long e = e0 + q;
-            const uint64_t w = (uint64_t)pd.loc[2 * e] | ((uint64_t)pd.loc[2 * e + 1] << 32);
-            const int ln[3] = {(int)(w & 1023u), (int)((w >> 10) & 1023u), (int)((w >> 20) & 1023u)};
-            const int eo = ei.perm[e];
-            double DNX[3], DNY[3], rho[3], Tn[3], vxn[3], vyn[3], wxn[3], wyn[3], gmn[3];
-            if (ei.dN6) {  // one 48-byte record: three 16-byte loads
-                const double2* r = reinterpret_cast<const double2*>(ei.dN6 + 6 * e);
-                const double2 a = r[0], b = r[1], c = r[2];
-                DNX[0] = a.x;
-                DNX[1] = a.y;
-                DNX[2] = b.x;
-                DNY[0] = b.y;
-                DNY[1] = c.x;
-                DNY[2] = c.y;
-            } else {
-#pragma unroll
-                for (int k = 0; k < 3; ++k) {
-                    DNX[k] = ei.dNx[3 * (long long)eo + k];
-                    DNY[k] = ei.dNy[3 * (long long)eo + k];
-                }
-            }
+    const int p = xcd_block(blockIdx.x, pd.npatch);
+    const int cs = pd.pcase ? pd.pcase[p] : 0;
+    const Consts* cq = pd.cases ? pd.cases + cs : nullptr;
+    const double fr = cq ? cq->fr : ei.fr, tinf = cq ? cq->t_inf : ei.tinf;
+    const double rinf = cq ? cq->rho_inf : ei.rinf, cte = cq ? cq->cte : o.cte;
+    const double dtmin = ei.dtmin[(size_t)cs * o.dt_stride];
+    const int nb = pd.node_base[p], nl = pd.node_base[p + 1] - nb;
+    const long long e0 = pd.elem_base[p];
+    const int nep = pd.elem_base[p + 1] - pd.elem_base[p];
+    for (int l = threadIdx.x; l < nl; l += blockDim.x) {
+        const int g = pd.pnode[nb + l] - 1;
+        sN[l] = EstabNode{ei.U[4 * (long long)g], ei.T[g], ei.VX[g], ei.VY[g],
+                          ei.WX ? ei.WX[g] : 0.0, ei.WY ? ei.WY[g] : 0.0, ei.GAMM[g]};
+    }
+    __syncthreads();
+    for (int q = threadIdx.x; q < nep; q += blockDim.x) {
+        const long long e = e0 + q;
+        const uint64_t w = (uint64_t)pd.loc[2 * e] | ((uint64_t)pd.loc[2 * e + 1] << 32);
+        const int ln[3] = {(int)(w & 1023u), (int)((w >> 10) & 1023u), (int)((w >> 20) & 1023u)};
+        const int eo = ei.perm[e];
+        double DNX[3], DNY[3], rho[3], Tn[3], vxn[3], vyn[3], wxn[3], wyn[3], gmn[3];
+        if (ei.dN6) {  // one 48-byte record: three 16-byte loads
+            const double2* r = reinterpret_cast<const double2*>(ei.dN6 + 6 * e);
+            const double2 a = r[0], b = r[1], c = r[2];
+            DNX[0] = a.x;
+            DNX[1] = a.y;
+            DNX[2] = b.x;
+            DNY[0] = b.y;
+            DNY[1] = c.x;
+            DNY[2] = c.y;
+        } else {
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
-                const EstabNode& nd = sN[ln[k]];
-                rho[k] = nd.rho;
-                Tn[k] = nd.T;
-                vxn[k] = nd.vx;
-                vyn[k] = nd.vy;
-                wxn[k] = nd.wx;
-                wyn[k] = nd.wy;
-                gmn[k] = nd.gm;
+                DNX[k] = ei.dNx[3 * (long long)eo + k];
+                DNY[k] = ei.dNy[3 * (long long)eo + k];
             }
-            double sh, rrr, s2, s3;
-            estab_elem(DNX, DNY, rho, Tn, vxn, vyn, wxn, wyn, gmn, fr, tinf, rinf, dtmin, sh, rrr,
-                       s2, s3);
-            *reinterpret_cast<typename Vec4<R>::type*>(o.nt + 4 * e) =
-                make4((R)(sh * cte), (R)rrr, (R)s2, (R)s3);
-            // DTL = DTMIN in every element unless local time steps blend in DT
-            o.fac[e] = (R)(o.area[eo] * (o.dtl ? o.dtl[eo] : dtmin) / 3.0);
         }
-        __syncthreads();  // the next patch overwrites sN
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const EstabNode& nd = sN[ln[k]];
+            rho[k] = nd.rho;
+            Tn[k] = nd.T;
+            vxn[k] = nd.vx;
+            vyn[k] = nd.vy;
+            wxn[k] = nd.wx;
+            wyn[k] = nd.wy;
+            gmn[k] = nd.gm;
+        }
+        double sh, rrr, s2, s3;
+        estab_elem(DNX, DNY, rho, Tn, vxn, vyn, wxn, wyn, gmn, fr, tinf, rinf, dtmin, sh, rrr,
+                   s2, s3);
+        *reinterpret_cast<typename Vec4<R>::type*>(o.nt + 4 * e) =
+            make4((R)(sh * cte), (R)rrr, (R)s2, (R)s3);
+        // DTL = DTMIN in every element unless local time steps blend in DT
+        o.fac[e] = (R)(o.area[eo] * (o.dtl ? o.dtl[eo] : dtmin) / 3.0);
     }
 }
 
@@ -1056,7 +1048,7 @@ int launch_deltat_partials(const Tables& t, const Consts& c, const double* area,
                            double* DT, double* partials, hipStream_t s) {
     const unsigned g = std::min<unsigned>(grid_for(t.nelem), kRedBlocks);
     k_deltat<<<g, kBlock, 0, s>>>(t.inpoel.p, area, T, VX, VY, WX, WY, DT, t.nelem, c.t_inf, c.fsafe,
-                                  partials, nullptr, nullptr, nullptr);
+                                  partials);
     CFD_HIP(hipGetLastError());
     return (int)g;
 }
@@ -1081,18 +1073,10 @@ int launch_deltat_patch(const PatchSet& ps, const Consts& c, const double* area,
     const size_t lds = (size_t)ps.max_nodes * sizeof(DtNode);
     k_deltat_patch<<<ps.npatch, patch_pass_block(ps.pe), lds, s>>>(ps.node_base.p, ps.elem_base.p, ps.pnode.p,
                                                   ps.loc.p, ps.perm.p, ps.npatch, area, T, VX, VY,
-                                                  WX, WY, DT, c.t_inf, c.fsafe, partials);
+                                                  WX, WY, DT, c.t_inf, c.fsafe, partials,
+                                                  ps.cases ? ps.pcase.p : nullptr, ps.cases);
     CFD_HIP(hipGetLastError());
     return ps.npatch;
-}
-
-void launch_deltat_chunks(const Tables& t, const Consts& c, const double* area, const double* T,
-                          const double* VX, const double* VY, const double* WX, const double* WY,
-                          double* DT, const int* chunk, int nchunks, double* partials,
-                          const int* chunk_case, const Consts* cases, hipStream_t s) {
-    k_deltat<<<nchunks, kBlock, 0, s>>>(t.inpoel.p, area, T, VX, VY, WX, WY, DT, t.nelem, c.t_inf,
-                                        c.fsafe, partials, chunk, chunk_case, cases);
-    CFD_HIP(hipGetLastError());
 }
 
 void launch_deltat(const Tables& t, const Consts& c, const double* area, const double* T,
@@ -1265,8 +1249,7 @@ template <class R, bool kFuente, bool kFinal>
 static void patch_launch_t(const PatchSet& ps, const PatchDev& pd, const ElemConstsP<R>& kc,
                            const PatchIn<R>& in, const StageDev& a, hipStream_t s) {
     const size_t lds = patch_lds_bytes(pd.maxn, kFuente, pd.pe, sizeof(typename Vec4<R>::type));
-    const int grid = ps.persistent && ps.grid[kFinal] > 0 ? ps.grid[kFinal] : ps.npatch;
-    k_patch_stage<R, kFuente, kFinal><<<grid, ps.block, lds, s>>>(pd, kc, in, a);
+    k_patch_stage<R, kFuente, kFinal><<<ps.npatch, ps.block, lds, s>>>(pd, kc, in, a);
     if (ps.nhalo > 0)
         k_halo_stage<kFinal><<<grid_for(ps.nhalo), kBlock, 0, s>>>(
             ps.hnode.p, ps.hptr.p, ps.hidx.p, ps.hpart.p, in.U, a, ps.nhalo,
@@ -1310,27 +1293,6 @@ void launch_patch_stage(const Tables& t, const PatchSet& ps, const Consts& c, co
     else patch_launch_t<R, false, false>(ps, pd, kc, in, a, s);
     CFD_HIP(hipGetLastError());
 }
-
-template <class R, bool kFuente, bool kFinal>
-static int resident_blocks(const PatchSet& ps) {
-    int dev = 0, ncu = 0, per_cu = 0;
-    CFD_HIP(hipGetDevice(&dev));
-    CFD_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-    const size_t lds = patch_lds_bytes(ps.max_nodes, kFuente, ps.pe, sizeof(typename Vec4<R>::type));
-    CFD_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        &per_cu, reinterpret_cast<const void*>(k_patch_stage<R, kFuente, kFinal>), ps.block, lds));
-    return std::max(1, std::min(ps.npatch, ncu * std::max(1, per_cu)));
-}
-
-template <class R>
-void patch_make_persistent(PatchSet& ps, bool fuente) {
-    ps.persistent = true;
-    ps.grid[0] = fuente ? resident_blocks<R, true, false>(ps) : resident_blocks<R, false, false>(ps);
-    ps.grid[1] = fuente ? resident_blocks<R, true, true>(ps) : resident_blocks<R, false, true>(ps);
-}
-
-template void patch_make_persistent<float>(PatchSet&, bool);
-template void patch_make_persistent<double>(PatchSet&, bool);
 
 void launch_to_patch64(const double* dNx, const double* dNy, double* dN6, double* dN4,
                        const int* perm, int nelem, hipStream_t s) {

@@ -372,7 +372,7 @@ int cfd_session_kernel_time(cfd_session *s, int slot, double *total_ms, long lon
  * every case's results agree bit for bit with the same case run alone in a
  * session of the same precision and patch shape.  One step of every case is
  * one replay of a recorded hipGraph (cfd_batch_set_graph(b, 0): plain
- * launches); per RK stage one resident-grid launch covers every case. */
+ * launches); per RK stage one launch covers every case. */
 typedef struct cfd_batch cfd_batch;
 typedef struct {
     int nelem, npoin;
