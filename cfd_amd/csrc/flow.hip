@@ -15,7 +15,9 @@
 //
 // Floating point follows the reference expression by expression: this file
 // is compiled with -ffp-contract=off, x**2 is x*x, x**1.5d0 / x**(-.5d0) are
-// correctly rounded pow_3_2 / pow_m1_2 (crmath.hpp), x**.5d0 is sqrt().
+// correctly rounded pow_3_2 / pow_m1_2, x**.5d0 is sqrt_rn, a / b quot or, by
+// three, third (crmath.hpp: correctly rounded, quotients by one denominator
+// sharing its reciprocal).
 #include "cfd_internal.hpp"
 #include "crmath.hpp"
 #include "reduce.hpp"
@@ -32,22 +34,23 @@ __device__ __forceinline__ double deltat_elem(const double (&Tn)[3], const doubl
                                               const double (&vv)[3], double area, double t_inf,
                                               double fsafe) {
     double vumax = 0.0, vvmax = 0.0;
-    const double t_iel = (Tn[0] + Tn[1] + Tn[2]) / 3.0;
+    const double t_iel = third(Tn[0] + Tn[1] + Tn[2]);
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
         if (vu[i] > vumax) vumax = vu[i];
         if (vv[i] > vvmax) vvmax = vv[i];
     }
-    const double hh = sqrt(2.0 * area);
-    const double vel = sqrt(vumax * vumax + vvmax * vvmax);
+    const double hh = sqrt_rn(2.0 * area);
+    const double vel = sqrt_rn(vumax * vumax + vvmax * vvmax);
     const double smu = 110.0;
-    const double fmu = 0.017 * pow_3_2(t_iel / t_inf) * (t_inf + smu) / (t_iel + smu);
+    const double fmu = quot(0.017 * pow_3_2(quot(t_iel, t_inf)) * (t_inf + smu), t_iel + smu);
     const double et = fmu;
-    const double pe = (vel * hh) / (2.0 * et);
-    const double alpha = pe / 3.0 < 1.0 ? pe / 3.0 : 1.0;
-    const double deltatu = 1.0 / (4.0 * et / (hh * hh) + alpha * vel / hh);
-    const double deltatc = 1.0 / (4.0 * et / (hh * hh));
-    return fsafe / (1.0 / deltatc + 1.0 / deltatu);
+    const double pe3 = third(quot(vel * hh, 2.0 * et));
+    const double alpha = pe3 < 1.0 ? pe3 : 1.0;
+    const double visc = quot(4.0 * et, hh * hh);
+    const double deltatu = quot(1.0, visc + quot(alpha * vel, hh));
+    const double deltatc = quot(1.0, visc);
+    return quot(fsafe, quot(1.0, deltatc) + quot(1.0, deltatu));
 }
 
 __global__ void __launch_bounds__(kBlock)
@@ -145,43 +148,48 @@ __global__ void k_deltat_clip(double* __restrict__ DT, const double* __restrict_
 // element); k_estab_patch (below, with the patch structures) in patch order
 // for the fused paths.  Both run estab_elem, so both give the same values.
 // ---------------------------------------------------------------------------
+// Bound by its FP64 instructions (quotients, roots) and their latency; at 4.2M
+// triangles k_estab_patch took 139 us with every quotient its own '/' and the
+// powers through sqrt() and '/', 114 us with the shared reciprocals.
 // The element's SUPG parameters from its three nodes' values (node k of the
-// element in its connectivity order): shock capturing sh and tau1..3.
-__device__ inline void estab_elem(const double DNX[3], const double DNY[3], const double rho[3],
+// element in its connectivity order): shock capturing sh and tau1..3.  moving:
+// W is not zero (v - 0 = v, so a mesh at rest leaves it out).
+__device__ inline void estab_elem(bool moving, const double DNX[3], const double DNY[3], const double rho[3],
                                   const double Tn[3], const double vxn[3], const double vyn[3],
                                   const double wxn[3], const double wyn[3], const double gmn[3],
                                   double fr, double tinf, double rinf, double dtmin, double& sh,
                                   double& rrr, double& s2, double& s3) {
-    double gm = (gmn[0] + gmn[1] + gmn[2]) / 3.0;
+    double gm = third(gmn[0] + gmn[1] + gmn[2]);
     double tau = 0.0, h_rgne = 0.0, h_rgn = 0.0, h_jgn = 0.0;
     double r1 = rho[0], r2 = rho[1], r3 = rho[2];
-    double rho_elem = (r1 + r2 + r3) / 3.0;
-    double vx = (vxn[0] + vxn[1] + vxn[2]) / 3.0;
-    double vy = (vyn[0] + vyn[1] + vyn[2]) / 3.0;
-    double wx = (wxn[0] + wxn[1] + wxn[2]) / 3.0;
-    double wy = (wyn[0] + wyn[1] + wyn[2]) / 3.0;
-    vx = vx - wx;
-    vy = vy - wy;
-    double vel2 = sqrt(vx * vx + vy * vy);
+    double rho_elem = third(r1 + r2 + r3);
+    double vx = third(vxn[0] + vxn[1] + vxn[2]);
+    double vy = third(vyn[0] + vyn[1] + vyn[2]);
+    if (moving) {
+        vx = vx - third(wxn[0] + wxn[1] + wxn[2]);
+        vy = vy - third(wyn[0] + wyn[1] + wyn[2]);
+    }
+    double vel2 = sqrt_rn(vx * vx + vy * vy);
     double drx = r1 * DNX[0] + r2 * DNX[1] + r3 * DNX[2];
     double dry = r1 * DNY[0] + r2 * DNY[1] + r3 * DNY[2];
-    double dr2 = sqrt(drx * drx + dry * dry) + 1.0e-20;
+    double dr2 = sqrt_rn(drx * drx + dry * dry) + 1.0e-20;
     double T1 = Tn[0], T2 = Tn[1], T3 = Tn[2];
     double dtx = T1 * DNX[0] + T2 * DNX[1] + T3 * DNX[2];
     double dty = T1 * DNY[0] + T2 * DNY[1] + T3 * DNY[2];
-    double dt2 = sqrt(dtx * dtx + dty * dty) + 1.0e-20;
+    double dt2 = sqrt_rn(dtx * dtx + dty * dty) + 1.0e-20;
     // "velocity gradient" of an element constant: the rounding residue of
     // sum(dN) sets the direction (reproduced as written)
     double dux = vel2 * DNX[0] + vel2 * DNX[1] + vel2 * DNX[2];
     double duy = vel2 * DNY[0] + vel2 * DNY[1] + vel2 * DNY[2];
-    double du2 = sqrt(dux * dux + duy * duy) + 1.0e-20;
-    double rtx = dtx / dt2, rty = dty / dt2;
-    double rjx = drx / dr2, rjy = dry / dr2;
-    double rux = dux / du2, ruy = duy / du2;
-    double temp = (T1 + T2 + T3) / 3.0;
-    double cc = sqrt(gm * fr * temp);
+    double du2 = sqrt_rn(dux * dux + duy * duy) + 1.0e-20;
+    const Recip it = recip(dt2), ij = recip(dr2), iu = recip(du2);
+    double rtx = quot(dtx, it), rty = quot(dty, it);
+    double rjx = quot(drx, ij), rjy = quot(dry, ij);
+    double rux = quot(dux, iu), ruy = quot(duy, iu);
+    double temp = third(T1 + T2 + T3);
+    double cc = sqrt_rn(gm * fr * temp);
     double smu = 110.0;
-    double fmu = 0.017 * pow_3_2(temp / tinf) * (tinf + smu) / (temp + smu);
+    double fmu = quot(0.017 * pow_3_2(quot(temp, tinf)) * (tinf + smu), temp + smu);
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
         double term_1 = fabs(vx * DNX[i] + vy * DNY[i]);
@@ -193,24 +201,26 @@ __device__ inline void estab_elem(const double DNX[3], const double DNY[3], cons
         h_rgn = h_rgn + h_rgn2;
         h_jgn = h_jgn + term_2;
     }
-    tau = 1.0 / tau;
-    h_rgne = 2.0 / h_rgne;
-    h_rgn = 2.0 / h_rgn;
+    tau = quot(1.0, tau);
+    h_rgne = quot(2.0, h_rgne);
+    h_rgn = quot(2.0, h_rgn);
     if (h_rgn > 10.0) h_rgn = 0.0;
-    h_jgn = 2.0 / h_jgn;
+    h_jgn = quot(2.0, h_jgn);
     if (h_jgn > 10.0) h_jgn = 0.0;
-    double tr1 = dr2 * h_jgn / rho_elem;
-    double zzz = h_jgn / (2.0 * cc);
+    double tr1 = quot(dr2 * h_jgn, rho_elem);
+    double zzz = quot(h_jgn, 2.0 * cc);
     sh = (tr1 + tr1 * tr1) * 0.5 * (cc * cc) * zzz;
-    double resumen = 1.0 / (tau * tau) + (2.0 / dtmin) * (2.0 / dtmin);
+    const double two_dt = quot(2.0, dtmin);
+    double resumen = quot(1.0, tau * tau) + two_dt * two_dt;
     rrr = pow_m1_2(resumen);
     s2 = rrr;
     s3 = rrr;
     if (fmu != 0.0) {
-        double ts3 = (h_rgn * h_rgn) / (4.0 * fmu / rinf);
-        double ts3e = (h_rgne * h_rgne) / (4.0 * fmu / rinf);
-        s2 = pow_m1_2(resumen + 1.0 / (ts3 * ts3));
-        s3 = pow_m1_2(resumen + 1.0 / (ts3e * ts3e));
+        const Recip iv = recip(quot(4.0 * fmu, rinf));
+        double ts3 = quot(h_rgn * h_rgn, iv);
+        double ts3e = quot(h_rgne * h_rgne, iv);
+        s2 = pow_m1_2(resumen + quot(1.0, ts3 * ts3));
+        s3 = pow_m1_2(resumen + quot(1.0, ts3e * ts3e));
     }
 }
 
@@ -240,7 +250,7 @@ k_estab(const int* __restrict__ inpoel, const double* __restrict__ U, const doub
         gmn[k] = GAMM[n[k]];
     }
     double sh, rrr, s2, s3;
-    estab_elem(DNX, DNY, rho, Tn, vxn, vyn, wxn, wyn, gmn, fr, tinf, rinf, *dtminp, sh, rrr, s2,
+    estab_elem(true, DNX, DNY, rho, Tn, vxn, vyn, wxn, wyn, gmn, fr, tinf, rinf, *dtminp, sh, rrr, s2,
                s3);
     shoc[e] = sh;
     t1[e] = rrr;
@@ -293,10 +303,10 @@ __device__ inline void supg_element(const ElemConsts& k, const double (&Uv)[3][4
     }
     const double tau[3] = {tau1, tau2, tau3};
     double nu = shoc * k.cte;
-    double T_avg = (Tn[0] + Tn[1] + Tn[2]) / 3.0;
-    double pw = pow_3_2(T_avg / k.T_inf);
-    double mu = k.mu_ref * pw * (k.T_inf + 110.0) / (T_avg + 110.0);
-    double lambda = k.lambda_ref * pw * (k.T_inf + 194.0) / (T_avg + 194.0);
+    double T_avg = third(Tn[0] + Tn[1] + Tn[2]);
+    double pw = pow_3_2(quot(T_avg, k.T_inf));
+    double mu = quot(k.mu_ref * pw * (k.T_inf + 110.0), T_avg + 110.0);
+    double lambda = quot(k.lambda_ref * pw * (k.T_inf + 194.0), T_avg + 194.0);
 #pragma unroll
     for (int j = 0; j < 3; ++j)
 #pragma unroll
@@ -319,9 +329,10 @@ __device__ inline void supg_element(const ElemConsts& k, const double (&Uv)[3][4
                 th[q] = 0.0;
         }
         double rho = Uk[0];
-        double v1 = Uk[1] / rho;
-        double v2 = Uk[2] / rho;
-        double en = Uk[3] / rho;
+        const Recip ir = recip(rho);
+        double v1 = quot(Uk[1], ir);
+        double v2 = quot(Uk[2], ir);
+        double en = quot(Uk[3], ir);
         double V_sq = v1 * v1 + v2 * v2;
         double A[4];
         A[0] = Ux[1] + Uy[2];
@@ -360,23 +371,22 @@ __device__ inline void supg_element(const ElemConsts& k, const double (&Uv)[3][4
                            nu * (Nx[j] * Ux[q] + Ny[j] * Uy[q]);
         if (k.viscous) {
             const double Cv = k.Cv;
+            const Recip icr = recip(Cv * rho);
             double K1[4], K2[4];
-            K1[1] = (2.0 / 3.0) * mu * (-(2.0 * Ux[0] * v1) + 2.0 * Ux[1] + Uy[0] * v2 - Uy[2]) / rho;
-            K1[2] = mu * (-(Ux[0] * v2) + Ux[2] - Uy[0] * v1 + Uy[1]) / rho;
-            K1[3] = (1.0 / 3.0) *
+            K1[1] = quot((2.0 / 3.0) * mu * (-(2.0 * Ux[0] * v1) + 2.0 * Ux[1] + Uy[0] * v2 - Uy[2]), ir);
+            K1[2] = quot(mu * (-(Ux[0] * v2) + Ux[2] - Uy[0] * v1 + Uy[1]), ir);
+            K1[3] = quot((1.0 / 3.0) *
                     (Cv * mu * (-(Uy[0] * v1 * v2) + 3.0 * Uy[1] * v2 - 2.0 * Uy[2] * v1) -
                      Ux[0] * (Cv * mu * (3.0 * V_sq + (v1 * v1)) - 3.0 * lambda * (V_sq - en)) +
                      Ux[1] * v1 * (4.0 * Cv * mu - 3.0 * lambda) + 3.0 * Ux[2] * v2 * (Cv * mu - lambda) +
-                     3.0 * Ux[3] * lambda) /
-                    (Cv * rho);
-            K2[1] = mu * (-(Ux[0] * v2) + Ux[2] - Uy[0] * v1 + Uy[1]) / rho;
-            K2[2] = (2.0 / 3.0) * mu * (Ux[0] * v1 - Ux[1] - 2.0 * Uy[0] * v2 + 2.0 * Uy[2]) / rho;
-            K2[3] = (1.0 / 3.0) *
+                     3.0 * Ux[3] * lambda), icr);
+            K2[1] = K1[2];
+            K2[2] = quot((2.0 / 3.0) * mu * (Ux[0] * v1 - Ux[1] - 2.0 * Uy[0] * v2 + 2.0 * Uy[2]), ir);
+            K2[3] = quot((1.0 / 3.0) *
                     (Cv * mu * (-(Ux[0] * v1 * v2) - 2.0 * Ux[1] * v2 + 3.0 * Ux[2] * v1) -
                      Uy[0] * (Cv * mu * (3.0 * V_sq + (v2 * v2)) - 3.0 * lambda * (V_sq - en)) +
                      3.0 * Uy[1] * v1 * (Cv * mu - lambda) + Uy[2] * v2 * (4.0 * Cv * mu - 3.0 * lambda) +
-                     3.0 * Uy[3] * lambda) /
-                    (Cv * rho);
+                     3.0 * Uy[3] * lambda), icr);
 #pragma unroll
             for (int j = 0; j < 3; ++j)
 #pragma unroll
@@ -386,7 +396,7 @@ __device__ inline void supg_element(const ElemConsts& k, const double (&Uv)[3][4
 #pragma unroll
     for (int j = 0; j < 3; ++j)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) rt[j][q] = rt[j][q] * area * dtl / 3.0;
+        for (int q = 0; q < 4; ++q) rt[j][q] = third(rt[j][q] * area * dtl);
 }
 
 // FUENTE for one element (subrutinas.f90:1064-1078)
@@ -402,7 +412,7 @@ __device__ inline void fuente_element(const double (&Uv)[3][4], const double (&N
         Ux[q] = Uv[0][q] * Nx[0] + Uv[1][q] * Nx[1] + Uv[2][q] * Nx[2];
         Uy[q] = Uv[0][q] * Ny[0] + Uv[1][q] * Ny[1] + Uv[2][q] * Ny[2];
     }
-    double AR = area * dtl / 3.0;
+    double AR = third(area * dtl);
     double wx[3], wy[3];
 #pragma unroll
     for (int kq = 0; kq < 3; ++kq) {
@@ -553,16 +563,17 @@ template <bool kFinal>
 __device__ inline void stage_node(const StageDev& a, int i, double4 u, double r0, double r1,
                                   double r2, double r3) {
     if (kFinal && a.RHS) st4(a.RHS + 4 * (long long)i, r0, r1, r2, r3);
-    double f = a.rk_fact / a.M[i];
+    double f = quot(a.rk_fact, a.M[i]);
     double u0 = u.x - f * r0, u1 = u.y - f * r1, u2 = u.z - f * r2, u3 = u.w - f * r3;
     double gamm = a.GAMM[i];
     double rho = u0;
-    double vx = u1 / rho;
-    double vy = u2 / rho;
-    double en = u3 / rho;
+    const Recip ir = recip(rho);
+    double vx = quot(u1, ir);
+    double vy = quot(u2, ir);
+    double en = quot(u3, ir);
     double vel2 = vx * vx + vy * vy;
     double pr = rho * (gamm - 1.0) * (en - 0.5 * vel2);
-    double tt = pr / (rho * a.fr);
+    double tt = quot(pr, rho * a.fr);
     int bi = a.bcidx[i];
     if (!kFinal) {  // T after the BCs: only FIX T changes it
         if (bi >= 0 && (a.bcflags[bi] & 8)) tt = a.bcvals[8 * bi + 5];
@@ -570,7 +581,7 @@ __device__ inline void stage_node(const StageDev& a, int i, double4 u, double r0
         return;
     }
     a.P[i] = pr;
-    a.RMACH[i] = sqrt(vel2 / (tt * gamm * a.fr));
+    a.RMACH[i] = sqrt_rn(quot(vel2, tt * gamm * a.fr));
     if (bi >= 0) {
         int fl = a.bcflags[bi];
         const double* v = a.bcvals + 8 * bi;
@@ -585,7 +596,7 @@ __device__ inline void stage_node(const StageDev& a, int i, double4 u, double r0
         if (fl & 8) {                                          // FIX T
             double gm = gamm - 1.0;
             tt = v[5];
-            en = tt * a.fr / gm + 0.5 * (vx * vx + vy * vy);
+            en = quot(tt * a.fr, gm) + 0.5 * (vx * vx + vy * vy);
         }
     }
     a.RHO[i] = rho;
@@ -655,7 +666,9 @@ __device__ __forceinline__ double4 make4(double a, double b, double c, double d)
     return make_double4(a, b, c, d);
 }
 
-// reciprocal: the hardware approximation in binary32, a rounded division in FP64
+// reciprocal: the hardware approximation in binary32, a rounded division in
+// FP64 ('/' and not quot: which products of elem_residual the compiler fuses
+// into multiply-adds changes with the division's form, and the results with it)
 __device__ __forceinline__ float rcpR(float x) { return __builtin_amdgcn_rcpf(x); }
 __device__ __forceinline__ double rcpR(double x) { return 1.0 / x; }
 
@@ -689,10 +702,10 @@ __device__ inline void elem_residual(const ElemConstsP<R>& kc, const double4 u0,
     R mu = 0, kl = 0;
     if (kc.viscous) {  // Sutherland laws at the element-average temperature
         if constexpr (sizeof(R) == 8) {
-            const double Tavg = (T[0] + T[1] + T[2]) / 3.0;
-            const double pw = pow_3_2(Tavg / kc.T_inf);
-            mu = kc.mu_ref * pw * (kc.T_inf + 110.0) / (Tavg + 110.0);
-            kl = kc.lambda_ref * pw * (kc.T_inf + 194.0) / (Tavg + 194.0) / kc.Cv;
+            const double Tavg = third(T[0] + T[1] + T[2]);
+            const double pw = pow_3_2(quot(Tavg, kc.T_inf));
+            mu = quot(kc.mu_ref * pw * (kc.T_inf + 110.0), Tavg + 110.0);
+            kl = quot(quot(kc.lambda_ref * pw * (kc.T_inf + 194.0), Tavg + 194.0), kc.Cv);
         } else {
             const float Tavg = (float)((T[0] + T[1] + T[2]) * (1.0 / 3.0));
             const float x = Tavg / kc.T_inf;
@@ -1003,12 +1016,12 @@ k_estab_patch(PatchDev pd, EstabIn ei, ElemP<R> o) {
             gmn[k] = nd.gm;
         }
         double sh, rrr, s2, s3;
-        estab_elem(DNX, DNY, rho, Tn, vxn, vyn, wxn, wyn, gmn, fr, tinf, rinf, dtmin, sh, rrr,
+        estab_elem(ei.WX, DNX, DNY, rho, Tn, vxn, vyn, wxn, wyn, gmn, fr, tinf, rinf, dtmin, sh, rrr,
                    s2, s3);
         *reinterpret_cast<typename Vec4<R>::type*>(o.nt + 4 * e) =
             make4((R)(sh * cte), (R)rrr, (R)s2, (R)s3);
         // DTL = DTMIN in every element unless local time steps blend in DT
-        o.fac[e] = (R)(o.area[eo] * (o.dtl ? o.dtl[eo] : dtmin) / 3.0);
+        o.fac[e] = (R)third(o.area[eo] * (o.dtl ? o.dtl[eo] : dtmin));
     }
 }
 
