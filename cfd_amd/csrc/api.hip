@@ -877,13 +877,18 @@ struct cfd_session {
         const bool fu = fuente_needed();
         const double* wx = fu ? WX.p : nullptr;
         const double* wy = fu ? WY.p : nullptr;
-        const int nb = fused() && patches.npatch <= (int)partials.n
+        const bool in_patches = fused() && patches.npatch <= (int)partials.n;
+        const bool fold_ctl = in_patches && d.itlocal == 0 && patches.npatch <= kStepFoldMax;
+        const int nb = in_patches
                            ? launch_deltat_patch(patches, c, AREA.p, T.p, VX.p, VY.p, wx, wy,
-                                                 DT.p, partials.p, s)
+                                                 DT.p, partials.p, s, fold_ctl ? ctl.p : nullptr)
                            : launch_deltat_partials(t, c, AREA.p, T.p, VX.p, VY.p, WX.p, WY.p,
                                                     DT.p, partials.p, s);
-        launch_step_ctl(partials.p, nullptr, nb, ctl.p, 1, d.itlocal, d.motion, d.motion_amp,
-                        d.motion_omega, s);
+        const StepFold fold{partials.p, nb, ctl.p, d.itlocal, d.motion, d.motion_amp,
+                            d.motion_omega};
+        if (!fold_ctl)
+            launch_step_ctl(partials.p, nullptr, nb, ctl.p, 1, d.itlocal, d.motion, d.motion_amp,
+                            d.motion_omega, s);
         if (lazy_dt()) {
             dt_stale = true;
         } else {
@@ -896,10 +901,10 @@ struct cfd_session {
         tb(CFD_K_ESTAB);
         if (d.precision == 1)
             launch_estab_patch(t, patches, c, U(), T.p, GAMM.p, VX.p, VY.p, wx, wy, DNX.p,
-                               DNY.p, nullptr, dtmin, elem32(), s);
+                               DNY.p, nullptr, dtmin, elem32(), s, fold_ctl ? &fold : nullptr);
         else if (d.precision == 0)
             launch_estab_patch(t, patches, c, U(), T.p, GAMM.p, VX.p, VY.p, wx, wy, DNX.p,
-                               DNY.p, DN6.p, dtmin, elem64(), s);
+                               DNY.p, DN6.p, dtmin, elem64(), s, fold_ctl ? &fold : nullptr);
         else
             launch_estab(t, c, U(), T.p, GAMM.p, VX.p, VY.p, WX.p, WY.p, DNX.p, DNY.p, dtmin,
                          SHOC.p, T1.p, T2.p, T3.p, s);
@@ -920,10 +925,13 @@ struct cfd_session {
         for (int irk = 1; irk <= nrk; ++irk) {
             double rk_fact = 1.0 / (nrk + 1 - irk);
             if (fused()) {
+                const double prev = 1.0 / (nrk + 2 - irk);
                 if (d.precision == 1)
-                    launch_patch_stage(t, patches, c, bc.tab, rk_fact, in32, sn, irk == nrk, s);
+                    launch_patch_stage(t, patches, c, bc.tab, rk_fact, in32, sn, irk == nrk, s,
+                                       irk - 1, prev);
                 else
-                    launch_patch_stage(t, patches, c, bc.tab, rk_fact, in64, sn, irk == nrk, s);
+                    launch_patch_stage(t, patches, c, bc.tab, rk_fact, in64, sn, irk == nrk, s,
+                                       irk - 1, prev);
                 continue;
             }
             tb(CFD_K_ELEMENT);
@@ -1213,10 +1221,10 @@ int cfd_session_create(cfd_session** out, cfd_mesh* m, const cfd_case_desc* d) {
             CFD_HIP(hipStreamSynchronize(s));
             const int pe = d->patch_elems > 0 ? d->patch_elems
                                               : (d->precision == 1 ? kPatchElems : kPatchElems64);
-            const int blk = d->patch_block > 0 ? d->patch_block : 256;
+            const int blk = std::max(0, d->patch_block);  // 0: by the number of patches
             CFD_ARG(pe <= 682, "patch_elems must be at most 682");
             CFD_ARG(blk % 64 == 0 && blk <= 512, "patch_block must be a multiple of 64 up to 512");
-            build_patches(S->patches, inp.data(), d->X, d->Y, ne, np, pe, blk, s);
+            build_patches(S->patches, inp.data(), d->X, d->Y, ne, np, pe, blk, d->precision == 1, s);
             CFD_ARG(patch_lds_fits(S->patches.max_nodes, pe,
                                    d->precision == 1 ? sizeof(float4) : sizeof(double4)),
                     "patch_elems too large: a patch exceeds the fused kernel's 64 KB of LDS");

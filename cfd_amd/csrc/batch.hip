@@ -114,7 +114,7 @@ struct cfd_batch {
             nps[k] = nbase[k + 1] - nbase[k];
         }
         build_patches_batch(patches, ncases, ip.data(), xs.data(), ys.data(), nes.data(), nps.data(),
-                            pe, block, s);
+                            pe, block, precision == 1, s);
         patches.cases = cases.p;
         std::vector<int> base(1, 0);
         for (int k = 0; k < ncases; ++k) base.push_back(base.back() + (nes[k] + pe - 1) / pe);
@@ -148,11 +148,13 @@ struct cfd_batch {
         StageNodes sn{U(), U1(), RHS.p, T.p, VX.p, VY.p, RHO.p, E.p, P.p, RMACH.p, M.p, GAMM.p,
                       WX.p, WY.p};
         for (int irk = 1; irk <= nrk; ++irk) {
-            const double rk_fact = 1.0 / (nrk + 1 - irk);
+            const double rk_fact = 1.0 / (nrk + 1 - irk), prev = 1.0 / (nrk + 2 - irk);
             if (precision == 1)
-                launch_patch_stage(t, patches, c, bc.tab, rk_fact, in32, sn, irk == nrk, s);
+                launch_patch_stage(t, patches, c, bc.tab, rk_fact, in32, sn, irk == nrk, s,
+                                   irk - 1, prev);
             else
-                launch_patch_stage(t, patches, c, bc.tab, rk_fact, in64, sn, irk == nrk, s);
+                launch_patch_stage(t, patches, c, bc.tab, rk_fact, in64, sn, irk == nrk, s,
+                                   irk - 1, prev);
         }
     }
 
@@ -279,9 +281,9 @@ int cfd_batch_create(cfd_batch** out, int ncases, const cfd_batch_case* cases, i
         B->ne = (int)ne;
         B->c = B->cc[0];
         const int pe = patch_elems > 0 ? patch_elems : (precision == 1 ? kPatchElems : kPatchElems64);
-        const int blk = patch_block > 0 ? patch_block : 256;
+        const int blk = std::max(0, patch_block);  // 0: by the number of patches
         CFD_ARG(pe >= 1 && pe <= 682, "patch_elems must be 1..682");
-        CFD_ARG(blk % 64 == 0 && blk >= 64 && blk <= 512,
+        CFD_ARG(blk % 64 == 0 && blk <= 512,
                 "patch_block must be a multiple of 64 from 64 to 512");
         // each case numbered in patch order inside (elements in patch order,
         // each patch's nodes in turn): the same results bit for bit as the

@@ -211,9 +211,21 @@ int launch_deltat_partials(const Tables& t, const Consts& c, const double* area,
 // LDS): the same DT bits, one min partial per patch; returns ps.npatch.  A
 // batch's patches take their case's constants.
 struct PatchSet;
+// ctl (may be null): the session scalars, of which DTMIN1 and BANDERA are copied
+// aside for step control inside ESTAB (StepFold).
 int launch_deltat_patch(const PatchSet& ps, const Consts& c, const double* area, const double* T,
                         const double* VX, const double* VY, const double* WX, const double* WY,
-                        double* DT, double* partials, hipStream_t s);
+                        double* DT, double* partials, hipStream_t s, double* ctl = nullptr);
+// Step control (launch_step_ctl) inside launch_estab_patch: every block forms
+// DTMIN from deltat's partials, the first one stores the step's scalars.
+struct StepFold {
+    const double* partials;
+    int nb;
+    double* ctl;
+    int itlocal, motion;
+    double amp, omega;
+};
+constexpr int kStepFoldMax = 1024;  // partials, above: launch_step_ctl
 // Inputs of the patch element residual (patch order, of the element type R:
 // float on the FP32 path, double on the fused FP64 path), written by ESTAB
 // in place of its element-order outputs: per element one record of nu =
@@ -252,7 +264,7 @@ void launch_estab_patch(const Tables& t, const PatchSet& ps, const Consts& c, co
                         const double* T, const double* GAMM, const double* VX, const double* VY,
                         const double* WX, const double* WY, const double* dNx, const double* dNy,
                         const double* dN6_patch, const double* dtmin, const ElemP<R>& o,
-                        hipStream_t s);
+                        hipStream_t s, const StepFold* fold = nullptr);
 // SHOC, T_SUGN1..3 (element order, FP64) from the patch-order copies of o
 template <class R>
 void launch_estab_widen(const ElemP<R>& o, const int* inv_perm, int nelem, double* shoc,
@@ -306,7 +318,7 @@ void launch_stage_update(const Tables& t, const Consts& c, const BcTable& bc, do
 // node's slot range (lptr); per halo node its partial-sum entries in
 // ascending patch order.
 // ---------------------------------------------------------------------------
-// default patch shapes, 256 threads each (measured on the 1024 x 2048 O-grid)
+// default patch shapes (measured on the 1024 x 2048 O-grid)
 constexpr int kPatchElems = 512;     // FP32 path: float4 slots
 constexpr int kPatchElems64 = 384;   // FP64 path: double4 slots
 constexpr int kPatchMaxNodes = 700;  // keeps the fused kernel's LDS within 64 KB
@@ -323,10 +335,17 @@ struct PatchSet {
     DBuf<int> pnode;               // 1-based node ids, per patch
     DBuf<uint16_t> lptr;           // nl+1 per patch, at node_base[p] + p
     DBuf<int> hnode, hptr, hidx;   // halo nodes (1-based), CSR of their entries
-    DBuf<double> hpart;            // 4 per entry
+    DBuf<double> hpart;            // 4 per entry (halo_in_next: two of them)
+    // Up to kHaloInNext patches: a stage's halo nodes are formed by the next
+    // stage's patches as they load them, instead of by a launch of its own
+    bool halo_in_next = false;
+    DBuf<int4> hseg;               // per entry its node's entries (see k_patch_stage)
 };
+// block: threads per patch of the fused kernel (0: by the number of patches);
+// fp32: of the element arithmetic
 void build_patches(PatchSet& ps, const int* inpoel_host, const double* X_host,
-                   const double* Y_host, int nelem, int npoin, int pe, int block, hipStream_t s);
+                   const double* Y_host, int nelem, int npoin, int pe, int block, bool fp32,
+                   hipStream_t s);
 // The patch-order numbering of a mesh (host): elem_old[q] = the element
 // (0-based) at patch position q; node_old[i] = the node at new position i,
 // each patch's nodes in turn (interior nodes, then the halo nodes no earlier
@@ -338,7 +357,8 @@ void patch_numbering(const int* inpoel, const double* X, const double* Y, int ne
 // patches as build_patches makes them, concatenated
 void build_patches_batch(PatchSet& ps, int ncases, const int* const* inpoel_host,
                          const double* const* X_host, const double* const* Y_host,
-                         const int* nelem, const int* npoin, int pe, int block, hipStream_t s);
+                         const int* nelem, const int* npoin, int pe, int block, bool fp32,
+                         hipStream_t s);
 
 // Fused element residual + RK stage for the patch-interior nodes, then the
 // stage for the halo nodes (subrutinas.f90:679-826 with calcRHS.f90:37-141
@@ -355,10 +375,11 @@ struct PatchIn {
     const R* fac;
     const R* nt;  // per element nu, tau1, tau2, tau3 (one 16- or 32-byte record)
 };
+// stage: 0 for a step's first; prev_fact: the stage before's rk_fact
 template <class R>
 void launch_patch_stage(const Tables& t, const PatchSet& ps, const Consts& c, const BcTable& bc,
                         double rk_fact, const PatchIn<R>& in, const StageNodes& nd,
-                        bool final_stage, hipStream_t s);
+                        bool final_stage, hipStream_t s, int stage, double prev_fact);
 // whether the fused kernel's LDS (node values, W, slots of slot_bytes,
 // slot ranges) fits its 64 KB budget for patches of pe elements and up to
 // max_nodes nodes
@@ -466,7 +487,8 @@ int smooth_run(const Tables& t, SmoothPlan& plan, double* X, double* Y, const do
 // Session state helpers (state.hip), shared by the session and the batch
 // ---------------------------------------------------------------------------
 // Session scalars live on the device: the CFD_S_* slots, then work slots.
-enum { X_RAW = CFD_NSCALARS, X_FDTL, X_CA, X_SA, X_NCTL };
+// X_DTMIN1, X_BANDERA: copies that deltat leaves for step control inside ESTAB
+enum { X_RAW = CFD_NSCALARS, X_FDTL, X_CA, X_SA, X_DTMIN1, X_BANDERA, X_NCTL };
 
 // Boundary-condition table (host construction, reference list semantics)
 struct BcHost {

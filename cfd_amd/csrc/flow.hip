@@ -18,9 +18,12 @@
 // correctly rounded pow_3_2 / pow_m1_2, x**.5d0 is sqrt_rn, a / b quot or, by
 // three, third (crmath.hpp: correctly rounded, quotients by one denominator
 // sharing its reciprocal).
+#include <type_traits>
+
 #include "cfd_internal.hpp"
 #include "crmath.hpp"
 #include "reduce.hpp"
+#include "stepctl.hpp"
 
 namespace cfd {
 namespace {
@@ -97,7 +100,7 @@ k_deltat_patch(const int* __restrict__ node_base, const int* __restrict__ elem_b
                const double* __restrict__ VY, const double* __restrict__ WX,
                const double* __restrict__ WY, double* __restrict__ DT, double t_inf, double fsafe,
                double* __restrict__ partials, const int* __restrict__ pcase,
-               const Consts* __restrict__ cases) {
+               const Consts* __restrict__ cases, double* __restrict__ ctl) {
     extern __shared__ double4 smem4[];
     DtNode* sN = reinterpret_cast<DtNode*>(smem4);
     const int p = xcd_block(blockIdx.x, npatch);  // grid = npatch: logical patch
@@ -105,6 +108,10 @@ k_deltat_patch(const int* __restrict__ node_base, const int* __restrict__ elem_b
         const Consts& q = cases[pcase[p]];
         t_inf = q.t_inf;
         fsafe = q.fsafe;
+    }
+    if (ctl && blockIdx.x == 0 && threadIdx.x == 0) {
+        ctl[X_DTMIN1] = ctl[CFD_S_DTMIN1];
+        ctl[X_BANDERA] = ctl[CFD_S_BANDERA];
     }
     const int nb = node_base[p], nl = node_base[p + 1] - nb;
     for (int l = threadIdx.x; l < nl; l += blockDim.x) {
@@ -549,8 +556,8 @@ k_gather_rhs(const int* __restrict__ esup2, const double* rhs_in, const CT* __re
 }
 
 // One RK stage for one node, given its summed residual (subrutinas.f90:679-826,
-// NGAS = 0).  kFinal = false: only T is stored (the next stage's only nodal
-// input besides U); the final stage stores everything.
+// NGAS = 0).  kFinal = false: only T is formed (the next stage's only nodal
+// input besides U) and returned; the final stage stores everything.
 struct StageDev {
     double rk_fact, fr;
     const double *M, *GAMM, *WX, *WY;
@@ -559,13 +566,22 @@ struct StageDev {
     double *U1, *RHS, *T, *VX, *VY, *RHO, *E, *P, *RMACH;
 };
 
+// a node's inputs of the stage besides U
+struct NodeIn {
+    double M, gamm;
+    int bi;
+};
+__device__ __forceinline__ NodeIn node_in(const StageDev& a, int i) {
+    return NodeIn{a.M[i], a.GAMM[i], a.bcidx[i]};
+}
+
 template <bool kFinal>
-__device__ inline void stage_node(const StageDev& a, int i, double4 u, double r0, double r1,
-                                  double r2, double r3) {
+__device__ inline double stage_node(const StageDev& a, const NodeIn& n, double rk_fact, int i,
+                                    double4 u, double r0, double r1, double r2, double r3) {
     if (kFinal && a.RHS) st4(a.RHS + 4 * (long long)i, r0, r1, r2, r3);
-    double f = quot(a.rk_fact, a.M[i]);
+    double f = quot(rk_fact, n.M);
     double u0 = u.x - f * r0, u1 = u.y - f * r1, u2 = u.z - f * r2, u3 = u.w - f * r3;
-    double gamm = a.GAMM[i];
+    double gamm = n.gamm;
     double rho = u0;
     const Recip ir = recip(rho);
     double vx = quot(u1, ir);
@@ -574,11 +590,10 @@ __device__ inline void stage_node(const StageDev& a, int i, double4 u, double r0
     double vel2 = vx * vx + vy * vy;
     double pr = rho * (gamm - 1.0) * (en - 0.5 * vel2);
     double tt = quot(pr, rho * a.fr);
-    int bi = a.bcidx[i];
+    int bi = n.bi;
     if (!kFinal) {  // T after the BCs: only FIX T changes it
         if (bi >= 0 && (a.bcflags[bi] & 8)) tt = a.bcvals[8 * bi + 5];
-        a.T[i] = tt;
-        return;
+        return tt;
     }
     a.P[i] = pr;
     a.RMACH[i] = sqrt_rn(quot(vel2, tt * gamm * a.fr));
@@ -605,6 +620,14 @@ __device__ inline void stage_node(const StageDev& a, int i, double4 u, double r0
     a.E[i] = en;
     a.T[i] = tt;
     st4(a.U1 + 4 * (long long)i, rho, vx * rho, vy * rho, en * rho);
+    return tt;
+}
+// the same, T stored in either case
+template <bool kFinal>
+__device__ inline void stage_store(const StageDev& a, const NodeIn& n, int i, double4 u, double r0,
+                                   double r1, double r2, double r3) {
+    const double tt = stage_node<kFinal>(a, n, a.rk_fact, i, u, r0, r1, r2, r3);
+    if (!kFinal) a.T[i] = tt;
 }
 
 // Gather (calcRHS slots, then FUENTE slots, in esup order) + one RK stage
@@ -623,7 +646,7 @@ k_stage(const int* __restrict__ esup2, const double4* __restrict__ c_calc,
     staged_sum(c_calc, s0, s1, b, e, sbuf, r0, r1, r2, r3);
     if (kFuente) staged_sum(c_fuente, s0, s1, b, e, sbuf, r0, r1, r2, r3);
     if (!act) return;
-    stage_node<kFinal>(a, i, ld4(U + 4 * (long long)i), r0, r1, r2, r3);
+    stage_store<kFinal>(a, node_in(a, i), i, ld4(U + 4 * (long long)i), r0, r1, r2, r3);
 }
 
 // ---------------------------------------------------------------------------
@@ -800,6 +823,37 @@ __device__ inline void elem_residual(const ElemConstsP<R>& kc, const double4 u0,
     for (int j = 0; j < 3; ++j) out[j] = make4(r[j][0], r[j][1], r[j][2], r[j][3]);
 }
 
+// A halo node's partial sums (entries hidx[j0 .. j1)) in ascending patch order.
+// The first kHaloBatch entries' loads all in flight at once (a node lies in
+// 2-4 patches as a rule), then the sums in entry order.
+__device__ __forceinline__ void halo_sum(const double* __restrict__ hpart, const int* __restrict__ hidx,
+                                         int j0, int j1, double& r0, double& r1, double& r2,
+                                         double& r3) {
+    constexpr int kHaloBatch = 4;
+    double4 v[kHaloBatch];
+#pragma unroll
+    for (int q = 0; q < kHaloBatch; ++q) {
+        const int j = j0 + q;
+        v[q] = j < j1 ? ld4(hpart + 4 * (long long)hidx[j]) : make_double4(0.0, 0.0, 0.0, 0.0);
+    }
+#pragma unroll
+    for (int q = 0; q < kHaloBatch; ++q) {
+        if (j0 + q < j1) {
+            r0 = r0 + v[q].x;
+            r1 = r1 + v[q].y;
+            r2 = r2 + v[q].z;
+            r3 = r3 + v[q].w;
+        }
+    }
+    for (int j = j0 + kHaloBatch; j < j1; ++j) {
+        const double4 w = ld4(hpart + 4 * (long long)hidx[j]);
+        r0 = r0 + w.x;
+        r1 = r1 + w.y;
+        r2 = r2 + w.z;
+        r3 = r3 + w.w;
+    }
+}
+
 // Fused residual + stage, one patch per block: node values to LDS; each
 // thread computes elements of the patch into LDS slots (float4 or double4);
 // each node sums its slots in FP64, then interior nodes take the RK stage and
@@ -809,6 +863,10 @@ struct PatchDev {
     const int *elem_base, *node_base, *n_int, *halo_base, *pnode;
     const uint16_t* lptr;
     double* hpart;
+    const double* hprev;   // kPrev: the stage before's partials, and of each
+    const int4* hseg;      // entry's node its entries (-1: none), or in x -2 - h:
+    const int *hidx, *hptr;  // node h's list, longer than four
+    double prev_fact;      // and its rk_fact
     int nelem, maxn, pe, npatch;
     const int* pcase;      // batches: case of each patch (null: kc and a as given)
     const Consts* cases;
@@ -822,8 +880,18 @@ struct PatchDev {
 // and cost the FP64 launches 7 us of 160 (intermediate) and 17 of 192 (final),
 // ESTAB 16 of 155, and a 32-case batch's FP32 stages 6 of 92, at 4.2M and 3.1M
 // triangles, with the same results.
-template <class R, bool kFuente, bool kFinal>
-__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(3)))
+//
+// kPrev: the stage before has left its halo nodes as partials; each patch forms
+// the T of its own halo nodes from them (k_halo_stage's sums and formula) as it
+// loads its nodes, and no k_halo_stage runs between the stages.
+//
+// kWide: one thread per element and node of the patch (few patches): every
+// input that depends on no other thread is loaded at the start, since a launch
+// of few blocks is bound by its chain of dependent loads (us a step: 42 patches
+// 49.8 against 51.7, 340 73.0 against 75.6).
+template <class R, bool kFuente, bool kFinal, bool kPrev, bool kWide>
+__global__ void __launch_bounds__(512)
+__attribute__((amdgpu_waves_per_eu(kWide ? (sizeof(R) == 8 ? 2 : 4) : 3)))
 k_patch_stage(PatchDev pd, ElemConstsP<R> kc, PatchIn<R> in, StageDev a) {
     using V4 = typename Vec4<R>::type;
     extern __shared__ double4 smem4[];
@@ -852,25 +920,69 @@ k_patch_stage(PatchDev pd, ElemConstsP<R> kc, PatchIn<R> in, StageDev a) {
     const int nb = pd.node_base[p], nl = pd.node_base[p + 1] - nb, nint = pd.n_int[p];
     const long long e0 = pd.elem_base[p];
     const int nep = pd.elem_base[p + 1] - pd.elem_base[p];
+    struct ElemData {
+        uint64_t w;
+        V4 gN, t4;
+        R fac;
+    };
+    auto elem_load = [&](int q) {
+        const long long e = e0 + q;
+        return ElemData{(uint64_t)pd.loc[2 * e] | ((uint64_t)pd.loc[2 * e + 1] << 32),
+                        *reinterpret_cast<const V4*>(in.dN + 4 * e),
+                        *reinterpret_cast<const V4*>(in.nt + 4 * e), in.fac[e]};
+    };
+    ElemData mine{};
+    int my_g = 0;
+    NodeIn my_in{};
+    if (kWide) {
+        if ((int)threadIdx.x < nep) mine = elem_load(threadIdx.x);
+        if ((int)threadIdx.x < nint) {
+            my_g = pd.pnode[nb + threadIdx.x] - 1;
+            my_in = node_in(a, my_g);
+        }
+    }
     for (int l = threadIdx.x; l < nl; l += blockDim.x) {
         const int g = pd.pnode[nb + l] - 1;
-        sU[l] = ld4(in.U + 4 * (long long)g);
-        sT[l] = in.T[g];
+        const double4 u = ld4(in.U + 4 * (long long)g);
+        sU[l] = u;
+        if (kPrev && l >= nint) {
+            const int4 j = pd.hseg[pd.halo_base[p] + l - nint];
+            double r0 = 0.0, r1 = 0.0, r2 = 0.0, r3 = 0.0;
+            if (j.x >= 0) {
+                const int at[4] = {j.x, j.y, j.z, j.w};
+                double4 v[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    if (at[q] >= 0) v[q] = ld4(pd.hprev + 4 * (long long)at[q]);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    if (at[q] < 0) continue;
+                    r0 = r0 + v[q].x;
+                    r1 = r1 + v[q].y;
+                    r2 = r2 + v[q].z;
+                    r3 = r3 + v[q].w;
+                }
+            } else {
+                const int h = -2 - j.x;
+                halo_sum(pd.hprev, pd.hidx, pd.hptr[h], pd.hptr[h + 1], r0, r1, r2, r3);
+            }
+            sT[l] = stage_node<false>(al, node_in(a, g), pd.prev_fact, g, u, r0, r1, r2, r3);
+        } else {
+            sT[l] = in.T[g];
+        }
         if (kFuente) sW[l] = make_double2(in.WX[g], in.WY[g]);
     }
     for (int l = threadIdx.x; l <= nl; l += blockDim.x) sP[l] = pd.lptr[nb + p + l];
     __syncthreads();
-    for (int q = threadIdx.x; q < nep; q += blockDim.x) {
-        const long long e = e0 + q;
-        const uint64_t w = (uint64_t)pd.loc[2 * e] | ((uint64_t)pd.loc[2 * e + 1] << 32);
+    auto elem = [&](const ElemData& d) {
+        const uint64_t w = d.w;
         const int ln[3] = {(int)(w & 1023u), (int)((w >> 10) & 1023u), (int)((w >> 20) & 1023u)};
         const int ls[3] = {(int)((w >> 30) & 2047u), (int)((w >> 41) & 2047u),
                            (int)((w >> 52) & 2047u)};
         // P1 gradients sum to zero: the first from the other two
-        const V4 gN = *reinterpret_cast<const V4*>(in.dN + 4 * e);
+        const V4 gN = d.gN, t4 = d.t4;  // t4: nu, tau1..3
         const R Nx[3] = {-(gN.x + gN.y), gN.x, gN.y};
         const R Ny[3] = {-(gN.z + gN.w), gN.z, gN.w};
-        const V4 t4 = *reinterpret_cast<const V4*>(in.nt + 4 * e);  // nu, tau1..3
         const R tau[3] = {t4.y, t4.z, t4.w};
         const double T3[3] = {sT[ln[0]], sT[ln[1]], sT[ln[2]]};
         double wx3[3] = {0.0, 0.0, 0.0}, wy3[3] = {0.0, 0.0, 0.0};
@@ -882,10 +994,15 @@ k_patch_stage(PatchDev pd, ElemConstsP<R> kc, PatchIn<R> in, StageDev a) {
             }
         }
         V4 out[3];
-        elem_residual<R, kFuente>(kl, sU[ln[0]], sU[ln[1]], sU[ln[2]], T3, wx3, wy3, Nx, Ny,
-                                  in.fac[e], t4.x, tau, out);
+        elem_residual<R, kFuente>(kl, sU[ln[0]], sU[ln[1]], sU[ln[2]], T3, wx3, wy3, Nx, Ny, d.fac,
+                                  t4.x, tau, out);
 #pragma unroll
         for (int k = 0; k < 3; ++k) sC[ls[k]] = out[k];
+    };
+    if (kWide) {
+        if ((int)threadIdx.x < nep) elem(mine);
+    } else {
+        for (int q = threadIdx.x; q < nep; q += blockDim.x) elem(elem_load(q));
     }
     __syncthreads();
     for (int l = threadIdx.x; l < nl; l += blockDim.x) {
@@ -897,10 +1014,12 @@ k_patch_stage(PatchDev pd, ElemConstsP<R> kc, PatchIn<R> in, StageDev a) {
             r2 = r2 + (double)c.z;
             r3 = r3 + (double)c.w;
         }
-        if (l < nint)
-            stage_node<kFinal>(al, pd.pnode[nb + l] - 1, sU[l], r0, r1, r2, r3);
-        else
+        if (l < nint) {
+            const int g = kWide ? my_g : pd.pnode[nb + l] - 1;
+            stage_store<kFinal>(al, kWide ? my_in : node_in(a, g), g, sU[l], r0, r1, r2, r3);
+        } else {
             st4(pd.hpart + 4 * (long long)(pd.halo_base[p] + l - nint), r0, r1, r2, r3);
+        }
     }
 }
 
@@ -916,34 +1035,9 @@ k_halo_stage(const int* __restrict__ hnode, const int* __restrict__ hptr,
     if (hcase) a.fr = cases[hcase[h]].fr;  // batches: the node's case
     const int g = hnode[h] - 1;
     const double4 u = ld4(U + 4 * (long long)g);
-    const int j0 = hptr[h], j1 = hptr[h + 1];
-    // the first kHaloBatch entries' loads all in flight at once (a node lies
-    // in 2-4 patches as a rule), then the sums in entry order
-    constexpr int kHaloBatch = 4;
-    double4 v[kHaloBatch];
-#pragma unroll
-    for (int q = 0; q < kHaloBatch; ++q) {
-        const int j = j0 + q;
-        v[q] = j < j1 ? ld4(hpart + 4 * (long long)hidx[j]) : make_double4(0.0, 0.0, 0.0, 0.0);
-    }
     double r0 = 0.0, r1 = 0.0, r2 = 0.0, r3 = 0.0;
-#pragma unroll
-    for (int q = 0; q < kHaloBatch; ++q) {
-        if (j0 + q < j1) {
-            r0 = r0 + v[q].x;
-            r1 = r1 + v[q].y;
-            r2 = r2 + v[q].z;
-            r3 = r3 + v[q].w;
-        }
-    }
-    for (int j = j0 + kHaloBatch; j < j1; ++j) {
-        const double4 w = ld4(hpart + 4 * (long long)hidx[j]);
-        r0 = r0 + w.x;
-        r1 = r1 + w.y;
-        r2 = r2 + w.z;
-        r3 = r3 + w.w;
-    }
-    stage_node<kFinal>(a, g, u, r0, r1, r2, r3);
+    halo_sum(hpart, hidx, hptr[h], hptr[h + 1], r0, r1, r2, r3);
+    stage_store<kFinal>(a, node_in(a, g), g, u, r0, r1, r2, r3);
 }
 
 // ESTAB in patch order (fused paths): one patch per block; the patch's node
@@ -962,9 +1056,14 @@ struct EstabIn {
     double fr, tinf, rinf;
 };
 
-template <class R>
+// kCtl: step control in here, one launch less (with the forces in one block a
+// step of 42 patches 51.7 us against 60.6; as a compile-time switch, since its
+// two registers cost large launches a wave per SIMD).  DTMIN depends on the
+// last step's scalars only through the copies that deltat has made, so no block
+// reads what the first one stores.
+template <class R, bool kCtl>
 __global__ void __launch_bounds__(512)
-k_estab_patch(PatchDev pd, EstabIn ei, ElemP<R> o) {
+k_estab_patch(PatchDev pd, EstabIn ei, ElemP<R> o, StepFold fold) {
     extern __shared__ double4 smem4[];
     EstabNode* sN = reinterpret_cast<EstabNode*>(smem4);  // maxn
     const int p = xcd_block(blockIdx.x, pd.npatch);
@@ -972,7 +1071,10 @@ k_estab_patch(PatchDev pd, EstabIn ei, ElemP<R> o) {
     const Consts* cq = pd.cases ? pd.cases + cs : nullptr;
     const double fr = cq ? cq->fr : ei.fr, tinf = cq ? cq->t_inf : ei.tinf;
     const double rinf = cq ? cq->rho_inf : ei.rinf, cte = cq ? cq->cte : o.cte;
-    const double dtmin = ei.dtmin[(size_t)cs * o.dt_stride];
+    double dmin = 1.0e20;
+    if (kCtl)
+        for (int j = threadIdx.x; j < fold.nb; j += blockDim.x)
+            dmin = OpMin()(dmin, fold.partials[j]);
     const int nb = pd.node_base[p], nl = pd.node_base[p + 1] - nb;
     const long long e0 = pd.elem_base[p];
     const int nep = pd.elem_base[p + 1] - pd.elem_base[p];
@@ -981,7 +1083,24 @@ k_estab_patch(PatchDev pd, EstabIn ei, ElemP<R> o) {
         sN[l] = EstabNode{ei.U[4 * (long long)g], ei.T[g], ei.VX[g], ei.VY[g],
                           ei.WX ? ei.WX[g] : 0.0, ei.WY ? ei.WY[g] : 0.0, ei.GAMM[g]};
     }
-    __syncthreads();
+    double dtmin;
+    if (kCtl) {
+        __shared__ double s_min;
+        dmin = block_reduce(dmin, OpMin());
+        if (threadIdx.x == 0) {
+            s_min = dmin;
+            if (blockIdx.x == 0)
+                step_control(fold.ctl, dmin, fold.ctl[X_DTMIN1], fold.ctl[X_BANDERA],
+                             StepLaw{fold.itlocal, fold.motion, fold.amp, fold.omega});
+        }
+        __syncthreads();
+        dtmin = s_min;
+        double d1 = fold.ctl[X_DTMIN1], bandera = fold.ctl[X_BANDERA];
+        step_dtmin(dtmin, d1, bandera);
+    } else {
+        dtmin = ei.dtmin[(size_t)cs * o.dt_stride];
+        __syncthreads();
+    }
     for (int q = threadIdx.x; q < nep; q += blockDim.x) {
         const long long e = e0 + q;
         const uint64_t w = (uint64_t)pd.loc[2 * e] | ((uint64_t)pd.loc[2 * e + 1] << 32);
@@ -1067,27 +1186,27 @@ int launch_deltat_partials(const Tables& t, const Consts& c, const double* area,
 }
 
 // Threads per block of the patch-order element passes (deltat, ESTAB): one
-// block per patch, every thread forming the same number of elements
-// (kPassElems) when the patch shape allows it.  Two per thread: a 384-element
-// FP64 patch on 192 threads instead of 256 (where a third of the threads
-// formed one element and the rest two) took ESTAB from 171 to 164 us at 4.2M
-// triangles; one per thread (384 threads) took it to 228 us.
-constexpr int kPassElems = 2;
-constexpr int kPassMaxBlock = 512;
-inline int patch_pass_block(int pe) {
-    const int b = pe / kPassElems;
-    return pe % (64 * kPassElems) == 0 && b <= kPassMaxBlock ? b : kBlock;
+// block per patch, every thread forming the same number of elements when the
+// patch shape allows it.  Up to kPassFew patches one (too few blocks to fill the
+// chip: 59.1 against 60.6 us a step of 16k triangles, 93.3 against 95.9 of
+// 258k), above two: a 384-element FP64 patch on 192 threads took ESTAB 164 us
+// at 4.2M triangles, on 256 (a third of the threads formed one element and the
+// rest two) 171, on 384 228.
+constexpr int kPassFew = 1024, kPassMaxBlock = 512;
+inline int patch_pass_block(int pe, int npatch) {
+    const int b = pe / (npatch <= kPassFew ? 1 : 2);
+    return b % 64 == 0 && b > 0 && b <= kPassMaxBlock ? b : kBlock;
 }
 
 int launch_deltat_patch(const PatchSet& ps, const Consts& c, const double* area, const double* T,
                         const double* VX, const double* VY, const double* WX, const double* WY,
-                        double* DT, double* partials, hipStream_t s) {
+                        double* DT, double* partials, hipStream_t s, double* ctl) {
     CFD_CHECK(ps.npatch > 0 && ps.max_nodes <= kPatchMaxNodes, "internal: deltat patches");
     const size_t lds = (size_t)ps.max_nodes * sizeof(DtNode);
-    k_deltat_patch<<<ps.npatch, patch_pass_block(ps.pe), lds, s>>>(ps.node_base.p, ps.elem_base.p, ps.pnode.p,
+    k_deltat_patch<<<ps.npatch, patch_pass_block(ps.pe, ps.npatch), lds, s>>>(ps.node_base.p, ps.elem_base.p, ps.pnode.p,
                                                   ps.loc.p, ps.perm.p, ps.npatch, area, T, VX, VY,
                                                   WX, WY, DT, c.t_inf, c.fsafe, partials,
-                                                  ps.cases ? ps.pcase.p : nullptr, ps.cases);
+                                                  ps.cases ? ps.pcase.p : nullptr, ps.cases, ctl);
     CFD_HIP(hipGetLastError());
     return ps.npatch;
 }
@@ -1116,7 +1235,7 @@ void launch_estab_patch(const Tables& t, const PatchSet& ps, const Consts& c, co
                         const double* T, const double* GAMM, const double* VX, const double* VY,
                         const double* WX, const double* WY, const double* dNx, const double* dNy,
                         const double* dN6_patch, const double* dtmin,
-                        const ElemP<R>& o, hipStream_t s) {
+                        const ElemP<R>& o, hipStream_t s, const StepFold* fold) {
     CFD_CHECK(o.nt && ps.perm.p, "internal: patch outputs missing");
     CFD_CHECK(ps.max_nodes <= kPatchMaxNodes, "internal: patch beyond the node budget");
     PatchDev pd{};
@@ -1133,7 +1252,9 @@ void launch_estab_patch(const Tables& t, const PatchSet& ps, const Consts& c, co
     EstabIn ei{U, T, GAMM, VX, VY, WX, WY, dNx, dNy, dN6_patch, ps.perm.p, dtmin,
                c.fr, c.t_inf, c.rho_inf};
     const size_t lds = (size_t)ps.max_nodes * sizeof(EstabNode);
-    k_estab_patch<R><<<ps.npatch, patch_pass_block(ps.pe), lds, s>>>(pd, ei, o);
+    const int threads = patch_pass_block(ps.pe, ps.npatch);
+    if (fold) k_estab_patch<R, true><<<ps.npatch, threads, lds, s>>>(pd, ei, o, *fold);
+    else k_estab_patch<R, false><<<ps.npatch, threads, lds, s>>>(pd, ei, o, StepFold{});
     CFD_HIP(hipGetLastError());
 }
 
@@ -1150,13 +1271,13 @@ template void launch_estab_patch<float>(const Tables&, const PatchSet&, const Co
                                          const double*, const double*, const double*,
                                          const double*, const double*, const double*,
                                          const double*, const double*, const ElemP<float>&,
-                                         hipStream_t);
+                                         hipStream_t, const StepFold*);
 template void launch_estab_patch<double>(const Tables&, const PatchSet&, const Consts&,
                                           const double*, const double*, const double*,
                                           const double*, const double*, const double*,
                                           const double*, const double*, const double*,
                                           const double*, const double*, const ElemP<double>&,
-                                          hipStream_t);
+                                          hipStream_t, const StepFold*);
 template void launch_estab_widen<float>(const ElemP<float>&, const int*, int, double*, double*,
                                         double*, double*, hipStream_t);
 template void launch_estab_widen<double>(const ElemP<double>&, const int*, int, double*, double*,
@@ -1258,21 +1379,31 @@ bool patch_lds_fits(int max_nodes, int pe, size_t slot_bytes) {
     return patch_lds_bytes(max_nodes, true, pe, slot_bytes) <= 65536;
 }
 
+constexpr int kWideMax = 1024;  // patches
 template <class R, bool kFuente, bool kFinal>
 static void patch_launch_t(const PatchSet& ps, const PatchDev& pd, const ElemConstsP<R>& kc,
                            const PatchIn<R>& in, const StageDev& a, hipStream_t s) {
     const size_t lds = patch_lds_bytes(pd.maxn, kFuente, pd.pe, sizeof(typename Vec4<R>::type));
-    k_patch_stage<R, kFuente, kFinal><<<ps.npatch, ps.block, lds, s>>>(pd, kc, in, a);
-    if (ps.nhalo > 0)
+    // kWide: a thread for every element and node of a patch
+    const bool wide = ps.npatch <= kWideMax && ps.block >= pd.pe && ps.block >= pd.maxn;
+    auto go = [&](auto prev, auto wd) {
+        k_patch_stage<R, kFuente, kFinal, decltype(prev)::value, decltype(wd)::value>
+            <<<ps.npatch, ps.block, lds, s>>>(pd, kc, in, a);
+    };
+    if (pd.hprev && wide) go(std::true_type{}, std::true_type{});
+    else if (pd.hprev) go(std::true_type{}, std::false_type{});
+    else if (wide) go(std::false_type{}, std::true_type{});
+    else go(std::false_type{}, std::false_type{});
+    if (ps.nhalo > 0 && (kFinal || !ps.halo_in_next))
         k_halo_stage<kFinal><<<grid_for(ps.nhalo), kBlock, 0, s>>>(
-            ps.hnode.p, ps.hptr.p, ps.hidx.p, ps.hpart.p, in.U, a, ps.nhalo,
+            ps.hnode.p, ps.hptr.p, ps.hidx.p, pd.hpart, in.U, a, ps.nhalo,
             ps.cases ? ps.hcase.p : nullptr, ps.cases);
 }
 
 template <class R>
 void launch_patch_stage(const Tables& t, const PatchSet& ps, const Consts& c, const BcTable& bc,
                         double rk_fact, const PatchIn<R>& in, const StageNodes& nd,
-                        bool final_stage, hipStream_t s) {
+                        bool final_stage, hipStream_t s, int stage, double prev_fact) {
     ElemConstsP<R> kc;
     kc.g = (R)c.gama;
     kc.Cv = (R)c.fcv;
@@ -1288,7 +1419,14 @@ void launch_patch_stage(const Tables& t, const PatchSet& ps, const Consts& c, co
     pd.halo_base = ps.halo_base.p;
     pd.pnode = ps.pnode.p;
     pd.lptr = ps.lptr.p;
-    pd.hpart = ps.hpart.p;
+    // with halo_in_next the stages' partials alternate between two buffers
+    const size_t half = ps.halo_in_next ? ps.hpart.n / 2 : 0;
+    pd.hpart = ps.hpart.p + (stage & 1) * half;
+    pd.hprev = half && stage > 0 ? ps.hpart.p + ((stage ^ 1) & 1) * half : nullptr;
+    pd.hseg = ps.hseg.p;
+    pd.hidx = ps.hidx.p;
+    pd.hptr = ps.hptr.p;
+    pd.prev_fact = prev_fact;
     pd.nelem = t.nelem;
     pd.maxn = ps.max_nodes;
     pd.pe = ps.pe;
@@ -1316,10 +1454,10 @@ void launch_to_patch64(const double* dNx, const double* dNy, double* dN6, double
 
 template void launch_patch_stage<float>(const Tables&, const PatchSet&, const Consts&,
                                         const BcTable&, double, const PatchIn<float>&,
-                                        const StageNodes&, bool, hipStream_t);
+                                        const StageNodes&, bool, hipStream_t, int, double);
 template void launch_patch_stage<double>(const Tables&, const PatchSet&, const Consts&,
                                          const BcTable&, double, const PatchIn<double>&,
-                                         const StageNodes&, bool, hipStream_t);
+                                         const StageNodes&, bool, hipStream_t, int, double);
 
 template <class R>
 void launch_to_patch_grad(const double* dNx, const double* dNy, R* dN, const int* perm, int nelem,

@@ -7,6 +7,8 @@
 // element order: that is the order in which the reference's sequential
 // element-order scatter adds into the node, so sums are bitwise identical and
 // no atomics are needed.  All of these are HBM-bound integer/gather work.
+#include <type_traits>
+
 #include "cfd_internal.hpp"
 #include "reduce.hpp"
 #include "crmath.hpp"
@@ -301,6 +303,45 @@ k_forces_fin(int nb, const double* __restrict__ part, double* __restrict__ out,
     if (zero4 && l < 4) zero4[l] = 0.0;
 }
 
+// Both in one block, a wave per 64-edge piece and the pieces' sums in LDS: the
+// same trees in the same order, one launch instead of two.  Up to kForcesOne
+// pieces (us a step with / without: 128 edges 49.5 / 52.0, 512 edges 93.8 /
+// 94.1); above, one CU's gathers take longer than a launch (1,024 edges 232 /
+// 226, 2,048 866 / 852).
+constexpr int kForcesOne = 8;
+template <bool kPress, bool kVisc>
+__global__ void __launch_bounds__(64 * kForcesOne)
+k_forces_one(int nedge, const int* __restrict__ iset, const double* __restrict__ X,
+             const double* __restrict__ Y, const double* __restrict__ P, double xref, double yref,
+             ViscIn v, double* __restrict__ out, double* __restrict__ outv,
+             double* __restrict__ zero4) {
+    __shared__ double part[5][kForcesOne];
+    const int nb = (nedge + 63) / 64, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    for (int b = w; b < nb; b += blockDim.x >> 6) {
+        const int i = b * 64 + lane;
+        double r[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+        if (i < nedge) force_terms<kPress, kVisc>(i, iset, X, Y, P, xref, yref, v, r);
+#pragma unroll
+        for (int q = 0; q < 5; ++q) {
+            if (q < 3 && !kPress) continue;
+            if (q >= 3 && !kVisc) continue;
+            const double t = wave_reduce(r[q], OpSum());
+            if (lane == 0) part[q][b] = t;
+        }
+    }
+    __syncthreads();
+    if (w < 5 && (w < 3 ? kPress : kVisc)) {  // wave w: sum w
+        double a = 0.0;
+        for (int k = lane; k < nb; k += 64) a = a + part[w][k];
+        a = wave_reduce(a, OpSum());
+        if (lane == 0) {
+            if (w < 3) out[w] = a;
+            else outv[w - 3] = a;
+        }
+    }
+    if (zero4 && threadIdx.x < 4) zero4[threadIdx.x] = 0.0;
+}
+
 // meshMove.f90:378-389, one set
 __global__ void k_transf(int nedge, const int* __restrict__ iset, const double* __restrict__ X,
                          const double* __restrict__ Y, const double* __restrict__ cs,
@@ -382,16 +423,20 @@ void launch_forces(int nedge, const int* iset, const double* X, const double* Y,
     }
     const ViscIn v = visc ? *visc : ViscIn{};
     const int nb = (nedge + 63) / 64;
-    if (out3 && visc) {
-        k_forces_part<true, true><<<nb, 64, 0, s>>>(nedge, iset, X, Y, P, xref, yref, v, part);
-        k_forces_fin<true, true><<<1, 64, 0, s>>>(nb, part, out3, out2, zero4);
-    } else if (out3) {
-        k_forces_part<true, false><<<nb, 64, 0, s>>>(nedge, iset, X, Y, P, xref, yref, v, part);
-        k_forces_fin<true, false><<<1, 64, 0, s>>>(nb, part, out3, out2, zero4);
-    } else {
-        k_forces_part<false, true><<<nb, 64, 0, s>>>(nedge, iset, X, Y, P, xref, yref, v, part);
-        k_forces_fin<false, true><<<1, 64, 0, s>>>(nb, part, out3, out2, zero4);
-    }
+    auto go = [&](auto press, auto vis) {
+        constexpr bool kP = decltype(press)::value, kV = decltype(vis)::value;
+        if (nb <= kForcesOne) {
+            const int threads = 64 * std::max(5, nb);
+            k_forces_one<kP, kV><<<1, threads, 0, s>>>(nedge, iset, X, Y, P, xref, yref, v, out3,
+                                                       out2, zero4);
+            return;
+        }
+        k_forces_part<kP, kV><<<nb, 64, 0, s>>>(nedge, iset, X, Y, P, xref, yref, v, part);
+        k_forces_fin<kP, kV><<<1, 64, 0, s>>>(nb, part, out3, out2, zero4);
+    };
+    if (out3 && visc) go(std::true_type{}, std::true_type{});
+    else if (out3) go(std::true_type{}, std::false_type{});
+    else go(std::false_type{}, std::true_type{});
     CFD_HIP(hipGetLastError());
 }
 

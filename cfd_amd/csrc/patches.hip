@@ -192,14 +192,31 @@ void patch_numbering(const int* inpoel, const double* X, const double* Y, int ne
         if (!seen[n]) node_old.push_back(n);
 }
 
+// Up to so many patches the next stage forms a stage's halo nodes (us a step
+// with / without: 42 patches 60.8 / 67.8, 675 95.5 / 102.4; 1,363 150.4 /
+// 148.8, 10,912 972 / 849: the partials are then read by every patch around a
+// node from memory, and cost more than the launch).
+constexpr int kHaloInNext = 1024;
+// Default threads per patch: 256 (see k_patch_stage), but one per element up to
+// kWideFew patches, where there are too few blocks to fill the chip otherwise
+// (us a step: FP64 42 patches 57.8 against 60.6, 340 patches 89.6 against
+// 80.5; FP32 32 patches 55.5 against 60.4, 505 patches 75.6 against 80.9,
+// 1,022 patches 115.9 against 111.6).
+constexpr int kWideFew64 = 256, kWideFew32 = 768;
+int patch_threads(int block, int pe, int npatch, bool fp32) {
+    if (block > 0) return block;
+    if (npatch > (fp32 ? kWideFew32 : kWideFew64)) return 256;
+    return std::min(512, (pe + 63) / 64 * 64);
+}
+
 static void upload_patches(PatchSet& ps, const PatchHost& h, int ne, int pe, int block,
-                           hipStream_t s) {
+                           bool fp32, hipStream_t s) {
     const int npatch = h.npatch, nentries = h.nentries;
     std::vector<int> inv(ne);
     for (int q = 0; q < ne; ++q) inv[h.perm[q]] = q;
     ps.npatch = npatch;
     ps.pe = pe;
-    ps.block = block;
+    ps.block = patch_threads(block, pe, npatch, fp32);
     ps.max_nodes = h.max_nodes;
     ps.nentries = nentries;
     ps.nhalo = (int)h.hnode.size();
@@ -227,26 +244,42 @@ static void upload_patches(PatchSet& ps, const PatchHost& h, int ne, int pe, int
     ps.hptr.upload(h.hptr.data(), h.hptr.size(), s);
     ps.hidx.alloc(std::max(1, nentries));
     ps.hidx.upload(h.hidx.data(), nentries, s);
-    ps.hpart.alloc(4 * (size_t)std::max(1, nentries));
+    ps.halo_in_next = npatch <= kHaloInNext && nentries > 0;
+    ps.hpart.alloc((ps.halo_in_next ? 8 : 4) * (size_t)std::max(1, nentries));
+    std::vector<int4> seg;
+    if (ps.halo_in_next) {
+        seg.resize(nentries);
+        for (size_t q = 0; q < h.hnode.size(); ++q) {
+            const int b = h.hptr[q], n = h.hptr[q + 1] - b;
+            const int* at = h.hidx.data() + b;
+            const int4 v = n > 4 ? make_int4(-2 - (int)q, -1, -1, -1)
+                                 : make_int4(at[0], n > 1 ? at[1] : -1, n > 2 ? at[2] : -1,
+                                             n > 3 ? at[3] : -1);
+            for (int j = 0; j < n; ++j) seg[at[j]] = v;
+        }
+        ps.hseg.alloc(nentries);
+        ps.hseg.upload(seg.data(), nentries, s);
+    }
     CFD_HIP(hipStreamSynchronize(s));  // the host vectors go out of scope
 }
 
 static void check_shape(int pe, int block) {
     // local slots are 11-bit and local node ids 10-bit fields of the per-element word
     CFD_CHECK(pe >= 1 && 3 * pe <= 2047 && kPatchMaxNodes <= 1023, "internal: patch size");
-    CFD_CHECK(block >= 64 && block <= 512 && block % 64 == 0, "internal: patch block size");
+    CFD_CHECK(block == 0 || (block >= 64 && block <= 512 && block % 64 == 0),
+              "internal: patch block size");
 }
 
 void build_patches(PatchSet& ps, const int* inpoel, const double* X, const double* Y, int ne, int np,
-                   int pe, int block, hipStream_t s) {
+                   int pe, int block, bool fp32, hipStream_t s) {
     check_shape(pe, block);
     const PatchHost h = patches_host(inpoel, X, Y, ne, np, pe);
-    upload_patches(ps, h, ne, pe, block, s);
+    upload_patches(ps, h, ne, pe, block, fp32, s);
 }
 
 void build_patches_batch(PatchSet& ps, int ncases, const int* const* inpoel,
                          const double* const* X, const double* const* Y, const int* ne,
-                         const int* np, int pe, int block, hipStream_t s) {
+                         const int* np, int pe, int block, bool fp32, hipStream_t s) {
     check_shape(pe, block);
     // each case's patches as on its own, then concatenated: element, node,
     // patch, local-node and halo-entry numbers shifted by the cases before
@@ -283,7 +316,7 @@ void build_patches_batch(PatchSet& ps, int ncases, const int* const* inpoel,
         np_tot += np[k];
         CFD_CHECK(ne_tot < (1ll << 31) && np_tot < (1ll << 31), "arg: batch too large");
     }
-    upload_patches(ps, u, (int)ne_tot, pe, block, s);
+    upload_patches(ps, u, (int)ne_tot, pe, block, fp32, s);
     ps.pcase.alloc(std::max<size_t>(1, pcase.size()));
     ps.pcase.upload(pcase.data(), pcase.size(), s);
     ps.hcase.alloc(std::max<size_t>(1, hcase.size()));

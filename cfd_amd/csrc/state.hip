@@ -4,6 +4,7 @@
 
 #include "cfd_internal.hpp"
 #include "reduce.hpp"
+#include "stepctl.hpp"
 
 namespace cfd {
 
@@ -30,51 +31,18 @@ __global__ void k_freestream(double* __restrict__ U, double* __restrict__ U1, do
     WX[i] = -0.0;
     WY[i] = 0.0;
 }
-// Step control (ns2DComp.ALE.f90:142-166, meshMove.f90:55-70): DTMIN from
-// the deltat partials, the 1 % hysteresis against DTMIN1, the clock, the
-// local-time-step blend factor and the body's rotation increment for TRANSF.
-// BANDERA's increment after fluidStructure (ns2DComp.ALE.f90:250) is applied
-// here too: nothing in between reads it.  Block c serves case c: its
-// partials are [pb[c], pb[c+1]) (all nb when pb is null), its scalars the
-// X_NCTL slots from ctl_all + c * X_NCTL.
+// Step control (stepctl.hpp).  Block c serves case c: its partials are [pb[c],
+// pb[c+1]) (all nb when pb is null), its scalars the X_NCTL slots from ctl_all
+// + c * X_NCTL.
 __global__ void __launch_bounds__(256)
 k_step_ctl(const double* __restrict__ partials, const int* __restrict__ pb, int nb,
-           double* __restrict__ ctl_all, int itlocal, int motion, double amp, double omega) {
+           double* __restrict__ ctl_all, StepLaw law) {
     const int cs = blockIdx.x;
     const int b0 = pb ? pb[cs] : 0, b1 = pb ? pb[cs + 1] : nb;
     const double m = combine_partials(partials + b0, b1 - b0, 1.0e20, OpMin());
     if (threadIdx.x != 0) return;
     double* ctl = ctl_all + (size_t)cs * X_NCTL;
-    double dtmin = m;
-    ctl[X_RAW] = dtmin;
-    const double iter = ctl[CFD_S_ITER] + 1.0;
-    ctl[CFD_S_ITER] = iter;
-    double bandera = ctl[CFD_S_BANDERA];
-    double dtmin1 = ctl[CFD_S_DTMIN1];
-    if ((int)bandera == 1) {
-        dtmin1 = dtmin;
-        bandera = 2.0;
-    }
-    const double porc = fabs((dtmin - dtmin1) / dtmin);
-    if (100.0 * porc <= 1.0) {
-        dtmin = dtmin1;
-    } else {
-        dtmin1 = dtmin;
-        bandera = 2.0;
-    }
-    ctl[CFD_S_DTMIN1] = dtmin1;
-    ctl[CFD_S_BANDERA] = bandera + 1.0;
-    ctl[CFD_S_DTMIN] = dtmin;
-    ctl[X_FDTL] = itlocal != 0 ? 1.0 - exp(-iter * 4.6 / itlocal) : 1.0;
-    const double time = ctl[CFD_S_TIME] + dtmin;
-    ctl[CFD_S_TIME] = time;
-    // meshMove.f90:55-57,70: ampli*sin(10 t), ampli = pi/8 (motion 0)
-    const double pi = 3.141592653589793;
-    const double ang = motion == 1 ? amp * sin(omega * time) : pi / 8.0 * sin(10.0 * time);
-    const double alpha = ang - ctl[CFD_S_DISN2];
-    ctl[CFD_S_DISN2] = ang;
-    ctl[X_CA] = cos(alpha);
-    ctl[X_SA] = sin(alpha);
+    step_control(ctl, m, ctl[CFD_S_DTMIN1], ctl[CFD_S_BANDERA], law);
 }
 
 // DT clipped at 10*min(DT) (subrutinas.f90:210-216), then DTL = DTMIN, or
@@ -207,7 +175,7 @@ void launch_freestream(const NodeState& ns, const Consts& c, int n, hipStream_t 
 
 void launch_step_ctl(const double* partials, const int* pb, int nb, double* ctl, int ncases,
                      int itlocal, int motion, double amp, double omega, hipStream_t s) {
-    k_step_ctl<<<ncases, 256, 0, s>>>(partials, pb, nb, ctl, itlocal, motion, amp, omega);
+    k_step_ctl<<<ncases, 256, 0, s>>>(partials, pb, nb, ctl, StepLaw{itlocal, motion, amp, omega});
     CFD_HIP(hipGetLastError());
 }
 
