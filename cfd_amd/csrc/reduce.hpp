@@ -9,9 +9,38 @@
 
 namespace cfd {
 
+// One step of the tree: v of the lane kOff above (as far as lane 0's result
+// needs it: lanes kOff and up get some lane's value).  Half and quarter waves
+// change places in registers, the rest is DPP inside rows of 16: no step goes
+// through LDS, as a shuffle of any distance does (a tree of six of those is
+// ~0.25 us of latency, and a PCG kernel of 3-4 us waits for two).
+template <int kOff>
+__device__ __forceinline__ int lane_above(int v) {
+    typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+    if constexpr (kOff == 32) {
+        const u32x2 r = __builtin_amdgcn_permlane32_swap((unsigned)v, (unsigned)v, false, false);
+        return (int)r.y;
+    } else if constexpr (kOff == 16) {
+        const u32x2 r = __builtin_amdgcn_permlane16_swap((unsigned)v, (unsigned)v, false, false);
+        return (int)r.y;
+    } else {
+        return __builtin_amdgcn_update_dpp(v, v, 0x100 + kOff, 0xf, 0xf, false);  // row_shl
+    }
+}
+template <int kOff>
+__device__ __forceinline__ double lane_above(double v) {
+    return __hiloint2double(lane_above<kOff>(__double2hiint(v)), lane_above<kOff>(__double2loint(v)));
+}
+
+// Lanes i and i + 32, then i + 16, 8, 4, 2, 1 (the whole wave must be active)
 template <class Op>
 __device__ inline double wave_reduce(double v, Op op) {
-    for (int off = 32; off > 0; off >>= 1) v = op(v, __shfl_down(v, off, 64));
+    v = op(v, lane_above<32>(v));
+    v = op(v, lane_above<16>(v));
+    v = op(v, lane_above<8>(v));
+    v = op(v, lane_above<4>(v));
+    v = op(v, lane_above<2>(v));
+    v = op(v, lane_above<1>(v));
     return v;  // valid in lane 0
 }
 
