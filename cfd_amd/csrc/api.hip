@@ -853,7 +853,9 @@ struct cfd_session {
         const EllMat em = ell.mat();
         pcg_launch_multi(sys, 2, np, LAP.p, m->t.idx.p, m->t.rowptr.p, LDIAG.p, tol, maxit,
                          d.pcg_rel, s, ell_on ? &em : nullptr);
-        last_solves_trivial = pcg_polled_iterations(pcg) == 0.0 && pcg_polled_iterations(pcg_y) == 0.0;
+        if (ws_on && d.pcg_rel == 0)  // else nothing asks
+            last_solves_trivial =
+                pcg_polled_iterations(pcg, s) == 0.0 && pcg_polled_iterations(pcg_y, s) == 0.0;
         te(CFD_K_PCG);
         pcg_store_result(pcg, scal(CFD_S_PCG_ITX), scal(CFD_S_PCG_RZX), scal(CFD_S_PCG_ITSUM), s,
                          scal(CFD_S_PCG_UNCONV));

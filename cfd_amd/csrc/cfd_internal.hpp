@@ -582,7 +582,7 @@ struct PcgWork {
     DBuf<unsigned char> fixflag;  // n: 1 on Dirichlet nodes
     HostPinned<double> hpin;   // two host copies of scal for the polls (null: a stack copy)
     hipEvent_t ev[2] = {nullptr, nullptr};  // the polls' ends
-    double polled_iters = -1.0;  // iterations of the last solve, as its last poll read them
+    double polled_iters = -1.0;  // iterations of the last solve as its last poll read them (< 0: not polled)
     PcgWork() = default;
     PcgWork(const PcgWork&) = delete;
     PcgWork& operator=(const PcgWork&) = delete;
@@ -632,21 +632,23 @@ struct EllLap {
     EllMat mat() const { return EllMat{val.p, col.p, dcol.p, len.p, width}; }
 };
 // Several independent solves on one matrix, interleaved on stream s with
-// shared polls; ell (when given) is the same matrix in ELL order, used by
+// shared polls (small systems: a block each, without); ell (when given) is the same matrix in ELL order, used by
 // the SpMV kernels of the iterations (bit for bit the CSR kernels' results).
 void pcg_launch_multi(const PcgSystem* sys, int nsys, int npoin, const double* A, const int* idx,
                       const int* rowptr, const double* diag, double tol, int maxit, int rel,
                       hipStream_t s, const EllMat* ell = nullptr);
-// iterations of the last solve run by pcg_launch_multi on w, as its final
-// poll read them (host memory, no device access)
-double pcg_polled_iterations(const PcgWork& w);
+// iterations of the last solve run by pcg_launch_multi on w: as its final poll
+// read them (host memory), or, of a solve without polls, from the device after
+// waiting for s
+double pcg_polled_iterations(const PcgWork& w, hipStream_t s);
 struct PcgResult {
     int iters;
     double rz;
     int converged;
 };
 // One solve on stream s; the host polls the done flag between batches of
-// iterations, so the call returns once the loop has ended on the device.
+// iterations, so the call returns once the loop has ended on the device (small
+// systems: one launch, which the call does not wait for).
 // x (device) in/out; b (device); x_fix/x_fix_idx device arrays of nfix.
 // rel = 0: the reference's absolute tests against tol; rel = 1: relative
 // (see pcg.hip).

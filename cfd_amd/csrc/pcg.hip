@@ -39,6 +39,8 @@
 // it runs alone or in a pair, nor on its blocks' size; a system that has
 // finished is skipped inside the paired kernels.
 //
+// Small systems run a whole solve in one launch instead (k_cg_whole).
+//
 // Relative mode (rel = 1): the two tests use tol^2 times the r.r and r.z of
 // the residual of the guess that is zero off the fixed nodes, so the stopping
 // point does not depend on the initial guess (warm starts compare at equal
@@ -911,6 +913,284 @@ struct CgLaunch {
     }
 };
 
+
+// ---------------------------------------------------------------------------
+// Small systems: a whole solve in one launch, one block per system.  Thread t
+// of kT holds rows t, t + kT, ..., kR of them; a wave's rows s kT + 64 w ..
+// belong to logical block (s kT + 64 w) / 256, so every sum has the pieces and
+// the order of the kernels above (the same bits).  r, diag and z or y (never
+// both alive) stay in registers, p is in LDS for the gathers, the matrix in
+// registers and LDS as far as it fits.  The scalars never leave the block: no
+// launch, no round trip through memory and no poll between the iterations,
+// and a mesh that moves in steps never waits for the host.
+//
+// An iteration of one system / two against the two launches above (us): 768
+// rows 1.6 / 1.65 against 7.9 / 8.3, 2,048 rows 2.3 / 2.45, 3,072 rows 3.1 /
+// 3.3, 3,840 rows 3.8 / 4.0, 4,608 rows 5.3 / 5.7 against 7.9 / 8.35.  Bound by
+// the one CU: FP64 instructions (about 0.35 us per 512 rows), three barriers and
+// two trees (1 us).  Above kWholeRows the matrix no longer fits beside p (6,144
+// rows 8.9 / 8.9, 8,192 rows 13 / 13 against 7.8 / 8.0).
+// ---------------------------------------------------------------------------
+
+__device__ __forceinline__ double first_lane(double v) {
+    return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)),
+                            __builtin_amdgcn_readfirstlane(__double2loint(v)));
+}
+
+// a becomes {a's lower half, b's lower half}, b {a's upper, b's upper}; kRows:
+// the same of neighbouring rows of 16 lanes
+template <bool kRows>
+__device__ __forceinline__ void swap_parts(double& a, double& b) {
+    typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+    auto half = [](int u, int v) {
+        return kRows ? (u32x2)__builtin_amdgcn_permlane16_swap((unsigned)u, (unsigned)v, false, false)
+                     : (u32x2)__builtin_amdgcn_permlane32_swap((unsigned)u, (unsigned)v, false, false);
+    };
+    const u32x2 hi = half(__double2hiint(a), __double2hiint(b));
+    const u32x2 lo = half(__double2loint(a), __double2loint(b));
+    a = __hiloint2double((int)hi.x, (int)lo.x);
+    b = __hiloint2double((int)hi.y, (int)lo.y);
+}
+// wave_reduce's sums of kR values a lane, out[s * stride] for value s: after the
+// step of half waves two values share a register, after the next four
+template <int kR>
+__device__ __forceinline__ void wave_sums(double (&v)[kR], double* out, int stride) {
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int g = 0; g < kR; g += 4) {
+        double a[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) a[j] = g + j < kR ? v[g + j] : 0.0;
+        swap_parts<false>(a[0], a[1]);
+        a[0] = a[0] + a[1];
+        if (g + 2 < kR) {
+            swap_parts<false>(a[2], a[3]);
+            a[2] = a[2] + a[3];
+        }
+        swap_parts<true>(a[0], a[2]);
+        double t = a[0] + a[2];
+        t = t + lane_above<8>(t);
+        t = t + lane_above<4>(t);
+        t = t + lane_above<2>(t);
+        t = t + lane_above<1>(t);
+        // rows of 16 lanes: values g, g + 2, g + 1, g + 3
+        const int s = g + (lane >> 5) + 2 * (lane >> 4 & 1);
+        if ((lane & 15) == 0 && s < kR) out[s * stride] = t;
+    }
+}
+
+template <int kT, int kW, int kR, int kKeep, int kLds, bool kX>
+__global__ void __launch_bounds__(kT)
+k_cg_whole(int n, EllMat m, const double* __restrict__ diag, CgBoth sys, double tol, int maxit,
+           int rel) {
+    extern __shared__ double sp[];  // p (first: x), kLds values per row, a byte per row: fixed
+    __shared__ double sums[3][kR * (kT / 64)];
+    unsigned char* fixed = reinterpret_cast<unsigned char*>(sp + (kX ? 1 + kLds : 2 + kLds) * n);
+    const CgSys& q = sys.s[blockIdx.x];
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6, nb = (n + kBlock - 1) / kBlock;
+    // the waves' sums into sums[k], and all of sums[k]
+    auto put = [&](int k, double (&v)[kR]) { wave_sums(v, &sums[k][w], (kT / 64)); };
+    auto total = [&](int k) {
+        double acc = 0.0;
+        if (lane < nb) {
+            const double* p = &sums[k][4 * lane];
+            double b = p[0];
+            b = b + p[1];
+            b = b + p[2];
+            b = b + p[3];
+            acc = acc + b;
+        }
+        return first_lane(wave_reduce(acc, OpSum())) + 0.0;
+    };
+    // x in registers (kX) or in LDS
+    double x[kX ? kR : 1], d[kR], r[kR], yz[kR], v[kR];
+    double *sx = sp + n, *sv = sx + (kX ? 0 : n);
+    int fix = 0;  // bit s: row 1024 s + t is fixed
+    for (int i = t; i < n; i += kT) {
+        sp[i] = q.x[i];
+        fixed[i] = 0;
+    }
+    __syncthreads();
+    for (int f = t; f < q.nfix; f += kT) {
+        const int i = q.fix_idx[f] - 1;
+        sp[i] = 1.0 * q.x_fix[f];
+        fixed[i] = 1;
+    }
+    __syncthreads();
+    // the rows' entries: their columns as packed offsets into p, the lengths,
+    // the first kKeep values, and the next kLds in LDS; the others are read in
+    // each use, at an offset of a zero that the compiler can't see through (it
+    // would keep them all, in scratch).  Slots beyond the matrix's width repeat
+    // its last.
+    constexpr int kPairs = (kW + 1) / 2;
+    unsigned at[kR][kPairs], full = 0;  // full: rows s of the wave all of kW entries
+    unsigned long long lens = 0;
+    double kept[kR][kKeep > 0 ? kKeep : 1];
+    const int last = m.width - 1;
+#pragma unroll
+    for (int s = 0; s < kR; ++s) {
+        const int i = min(s * kT + t, n - 1);
+        lens |= (unsigned long long)m.len[i] << (4 * s);
+        if (__all(m.len[i] == kW)) full |= 1u << s;
+#pragma unroll
+        for (int j = 0; j < kW; ++j) {
+            const unsigned c = 8u * (unsigned)(i + m.dcol[min(j, last) * n + i]);
+            at[s][j / 2] = j & 1 ? at[s][j / 2] | c << 16 : c;
+            if (j < kKeep) kept[s][j] = m.val[min(j, last) * n + i];
+            else if (j < kKeep + kLds) sv[(j - kKeep) * n + i] = m.val[min(j, last) * n + i];
+        }
+    }
+    // f(in the row, a_ij, byte offset of column j's p) over the slots of the
+    // thread's row s, in order
+    auto row = [&](int s, int zero, auto all, auto f) {
+        const int i = min(s * kT + t, n - 1);
+        unsigned len = (unsigned)(lens >> (4 * s)) & 15u, o[kPairs];
+        double a[kW];
+#pragma unroll
+        for (int j = kKeep; j < kW; ++j)
+            a[j] = j < kKeep + kLds ? sv[(j - kKeep) * n + i] : m.val[min(j, last) * n + i + zero];
+#pragma unroll
+        for (int j = 0; j < kPairs; ++j) {
+            o[j] = at[s][j];
+            asm volatile("" : "+v"(o[j]));
+        }
+        asm volatile("" : "+v"(len));
+#pragma unroll
+        for (int j = 0; j < kW; ++j)
+            f(all.value || (unsigned)j < len, j < kKeep ? kept[s][j] : a[j],
+              j & 1 ? o[j / 2] >> 16 : o[j / 2] & 0xffffu);
+    };
+    auto p_at = [&](unsigned o) {
+        return *reinterpret_cast<const double*>(reinterpret_cast<const char*>(sp) + o);
+    };
+    double vr[kR], vz[kR];
+#pragma unroll
+    for (int s = 0; s < kR; ++s) {
+        const int i = s * kT + t;
+        r[s] = yz[s] = vr[s] = vz[s] = 0.0;
+        d[s] = 1.0;
+        if (i < n) {
+            if (kX) x[s] = sp[i];
+            else sx[i] = sp[i];
+            d[s] = diag[i];
+            double dot = 0.0, dotd = 0.0;
+            row(s, 0, std::false_type{}, [&](bool in, double aij, unsigned o) {
+                const double xc = p_at(o);
+                dot = in ? dot + aij * xc : dot;
+                dotd = in && fixed[o / 8] ? dotd + aij * xc : dotd;
+            });
+            if (fixed[i]) {
+                fix |= 1 << s;
+            } else {
+                const double bi = q.b[i];
+                r[s] = -1.0 * dot + bi;
+                const double rd = -1.0 * dotd + bi;
+                vr[s] = rd * rd;
+                vz[s] = rd * (rd / d[s]);
+            }
+        }
+        v[s] = r[s] * r[s];
+    }
+    put(0, v);
+    if (rel) {
+        put(1, vr);
+        put(2, vz);
+    }
+    __syncthreads();
+    const double rr = total(0);
+    const double tolr = rel ? tol * tol * total(1) : tol, tolz = rel ? tol * tol * total(2) : tol;
+    double e = rr, k = 0.0, conv = 1.0;
+    if (!(rr < tolr)) {
+        __syncthreads();  // sums are read
+#pragma unroll
+        for (int s = 0; s < kR; ++s) {
+            yz[s] = r[s] / d[s];
+            v[s] = r[s] * yz[s];
+        }
+        put(0, v);
+        __syncthreads();
+        e = total(0);
+        double beta = 0.0;
+        for (bool first = true;; first = false) {
+            // B: p = beta p + z, y = A p
+#pragma unroll
+            for (int s = 0; s < kR; ++s) {
+                const int i = s * kT + t;
+                if (i < n) sp[i] = first ? yz[s] : beta * sp[i] + yz[s];
+            }
+            __syncthreads();
+            int zero = 0;
+            asm volatile("" : "+s"(zero));
+#pragma unroll
+            for (int s = 0; s < kR; ++s) {
+                const int i = s * kT + t;
+                const double pn = sp[min(i, n - 1)];
+                double dot = 0.0;
+                const auto add = [&](bool in, double aij, unsigned o) {
+                    const double c = dot + aij * p_at(o);
+                    dot = in ? c : dot;
+                };
+                if (full >> s & 1) row(s, zero, std::true_type{}, add);
+                else row(s, zero, std::false_type{}, add);
+                yz[s] = fix >> s & 1 ? 1.0e30 * pn : dot;
+                v[s] = i < n ? pn * yz[s] : 0.0;
+            }
+            put(1, v);
+            __syncthreads();
+            // A: x += alfa p, r -= alfa y, z = r / diag
+            const double alfa = e / total(1), eold = e;
+            const bool more = fabs(e) > tolz && k < (double)maxit;
+#pragma unroll
+            for (int s = 0; s < kR; ++s) {
+                const int i = s * kT + t;
+                if (i >= n) continue;
+                double& xi = kX ? x[s] : sx[i];
+                xi = alfa * sp[i] + xi;
+            }
+            if (!more) break;
+#pragma unroll
+            for (int s = 0; s < kR; ++s) {
+                if (s * kT + t < n) r[s] = -alfa * yz[s] + r[s];
+                double ds = d[s];
+                asm volatile("" : "+v"(ds));  // else the divisor's reciprocals are kept, in scratch
+                yz[s] = r[s] / ds;
+                v[s] = r[s] * yz[s];
+            }
+            put(0, v);
+            __syncthreads();
+            e = total(0);
+            beta = e / eold;
+            k = k + 1.0;
+        }
+        conv = fabs(e) > tolz ? 0.0 : 1.0;
+    }
+#pragma unroll
+    for (int s = 0; s < kR; ++s) {
+        const int i = s * kT + t;
+        if (i < n) q.x[i] = kX ? x[s] : sx[i];
+    }
+    if (t < S_NSCAL)
+        q.scal[t] = t == S_K ? k : t == S_EOLD ? e : t == S_CONV ? conv : t == S_DONE ? 1.0
+                  : t == S_TOL ? tol : t == S_MAXIT ? (double)maxit : t == S_TOLR ? tolr
+                  : t == S_TOLZ ? tolz : t == S_RR ? rr : 0.0;
+}
+
+// The rows up to which a solve runs in k_cg_whole (33 bytes of LDS a row in
+// its largest form), and the iteration cap (one launch of at most 0.15 s)
+constexpr int kWholeRows = 4864, kWholeIters = 20000;
+
+template <int kT, int kW, int kR, int kKeep, int kLds, bool kX>
+void launch_whole(int n, const EllMat& m, const double* diag, const CgBoth& q, int nsys, double tol,
+                  int maxit, int rel, hipStream_t s) {
+    const auto kernel = k_cg_whole<kT, kW, kR, kKeep, kLds, kX>;
+    const size_t lds = (size_t)n * ((kX ? 1 + kLds : 2 + kLds) * sizeof(double) + 1);
+    if (lds > 48 * 1024)
+        CFD_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    kernel<<<nsys, kT, lds, s>>>(n, m, diag, q, tol, maxit, rel);
+    CFD_HIP(hipGetLastError());
+}
+
 }  // namespace
 
 void pcg_launch_multi(const PcgSystem* sys, int nsys, int npoin, const double* A, const int* idx,
@@ -921,6 +1201,32 @@ void pcg_launch_multi(const PcgSystem* sys, int nsys, int npoin, const double* A
     CFD_CHECK(nsys >= 1 && nsys <= kMaxSys, "internal: PCG systems per launch");
     const int nb = (int)grid_for(npoin);
     for (int k = 0; k < nsys; ++k) sys[k].w->ensure(npoin);
+    if (ell && ell->width <= 8 && ell->dcol && npoin <= kWholeRows && maxit <= kWholeIters) {
+        CgBoth q{};
+        for (int k = 0; k < nsys; ++k) {
+            q.s[k] = cg_sys(sys[k], 0);
+            sys[k].w->polled_iters = -1.0;
+        }
+        // Threads, rows a thread and where the matrix is kept, by what fits: up
+        // to 3,072 rows all of it in registers; above, values beside p in LDS,
+        // and above 4,096 rows x there too and two or three values a row read
+        // from L2 (5.3 us an iteration at 4,608 rows; 6.1 with three in LDS and
+        // x in registers, which spill; 6.8 with x in place; 8.0 in 512 threads of
+        // ten rows).
+        const int half = (npoin + 511) / 512;
+        const auto pick = [&](auto width) {
+            constexpr int kW = decltype(width)::value;
+            return half <= 2   ? launch_whole<512, kW, 2, kW, 0, true>
+                   : half <= 4 ? launch_whole<512, kW, 4, kW, 0, true>
+                   : half <= 6 ? launch_whole<512, kW, 6, kW, 0, true>
+                   : half <= 8 ? launch_whole<1024, kW, 4, 4, 3, true>
+                               : launch_whole<1024, kW, 5, 2, 2, false>;
+        };
+        const auto go = ell->width <= 7 ? pick(std::integral_constant<int, 7>{})
+                                        : pick(std::integral_constant<int, 8>{});
+        go(npoin, *ell, diag, q, nsys, tol, maxit, rel, s);
+        return;
+    }
     // pbuf[cur] holds the current p; both systems' buffers flip together
     int cur = 1;
     bool done[kMaxSys] = {false, nsys == 1};
@@ -1008,7 +1314,9 @@ void pcg_launch_multi(const PcgSystem* sys, int nsys, int npoin, const double* A
     });
 }
 
-double pcg_polled_iterations(const PcgWork& w) { return w.polled_iters; }
+double pcg_polled_iterations(const PcgWork& w, hipStream_t s) {
+    return w.polled_iters >= 0.0 ? w.polled_iters : (double)pcg_result(w, s).iters;
+}
 
 void pcg_launch(PcgWork& w, int npoin, const double* A, const int* idx, const int* rowptr,
                 const double* diag, double* x, const double* b, const double* x_fix,

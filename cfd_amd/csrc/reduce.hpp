@@ -12,8 +12,10 @@ namespace cfd {
 // One step of the tree: v of the lane kOff above (as far as lane 0's result
 // needs it: lanes kOff and up get some lane's value).  Half and quarter waves
 // change places in registers, the rest is DPP inside rows of 16: no step goes
-// through LDS, as a shuffle of any distance does (a tree of six of those is
-// ~0.25 us of latency, and a PCG kernel of 3-4 us waits for two).
+// through LDS, as a shuffle does, and a kernel that is one chain of latencies
+// waits for two such trees.  A PCG iteration (two kernels) with shuffles / so,
+// one system and two, us: 32,768 rows 8.35, 8.45 / 7.8, 8.0; 131,584 rows
+// 11.65, 14.4 / 10.95, 13.55; 524,288 rows 20.2, 31.6 / 19.05, 29.7.
 template <int kOff>
 __device__ __forceinline__ int lane_above(int v) {
     typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
