@@ -24,23 +24,15 @@ static Consts to_consts(const cfd_consts* c) { return consts_of(c); }
 // small kernels used by the entries and the session
 // ---------------------------------------------------------------------------
 namespace {
-// POS_AUX(1:NMOVE) = DPOS(ilaux), POS_AUX(NMOVE+1:NNMOVE) = 0 (meshMove.f90:79-89)
-__global__ void k_pos_aux(const int* __restrict__ ilaux, const double* __restrict__ dpos,
-                          double* __restrict__ pos, int nmove, int nn) {
-    int q = blockIdx.x * blockDim.x + threadIdx.x;
+// POS_AUX(1:NMOVE) = DPOS(ilaux), POS_AUX(NMOVE+1:NNMOVE) = 0 (meshMove.f90:79-89),
+// both axes
+__global__ void k_pos_aux(const int* __restrict__ ilaux, const double* __restrict__ dx,
+                          const double* __restrict__ dy, double* __restrict__ px,
+                          double* __restrict__ py, int nmove, int nn) {
+    const int q = blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= nn) return;
-    pos[q] = q < nmove ? dpos[ilaux[q] - 1] : 0.0;
-}
-// X += XPOS; X1 += XPOS; W = XPOS/DTMIN (meshMove.f90:99-104)
-__global__ void k_move(double* __restrict__ X, double* __restrict__ X1, double* __restrict__ W,
-                       const double* __restrict__ pos, const double* __restrict__ dtminp, int n) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const double dtmin = *dtminp;
-    double d = pos[i];
-    X[i] = X[i] + d;
-    X1[i] = X1[i] + d;
-    W[i] = d / dtmin;
+    px[q] = q < nmove ? dx[ilaux[q] - 1] : 0.0;
+    py[q] = q < nmove ? dy[ilaux[q] - 1] : 0.0;
 }
 
 }  // namespace
@@ -780,8 +772,7 @@ struct cfd_session {
                      partials.p, s);
         refresh_patch_geometry();
         launch_masas(t, AREA.p, M.p, s);
-        launch_laplace(t, X.p, Y.p, DNX.p, DNY.p, LAP.p, LDIAG.p, s);
-        if (ell_on) ell.refresh(t.rowptr.p, LAP.p, s);
+        launch_laplace(t, X.p, Y.p, DNX.p, DNY.p, LAP.p, LDIAG.p, s, ell_on ? &ell : nullptr);
     }
 
     // the fused paths' ESTAB outputs (patch order)
@@ -815,10 +806,9 @@ struct cfd_session {
     // TRANSF), so the two run interleaved.
     void mesh_solves() {
         const int nn = d.nmove + d.nfix_move;
-        if (nn > 0) {
-            k_pos_aux<<<grid_for(nn), kBlock, 0, s>>>(ILAUX.p, DXPOS.p, POSAUX.p, d.nmove, nn);
-            k_pos_aux<<<grid_for(nn), kBlock, 0, s>>>(ILAUX.p, DYPOS.p, POSAUY.p, d.nmove, nn);
-        }
+        if (nn > 0)
+            k_pos_aux<<<grid_for(nn), kBlock, 0, s>>>(ILAUX.p, DXPOS.p, DYPOS.p, POSAUX.p, POSAUY.p,
+                                                      d.nmove, nn);
         tb(CFD_K_PCG);
         const double tol = d.pcg_tol > 0.0 ? d.pcg_tol : 1.0e-10;
         const int maxit = d.pcg_maxit > 0 ? d.pcg_maxit : 1000;
@@ -857,13 +847,13 @@ struct cfd_session {
             last_solves_trivial =
                 pcg_polled_iterations(pcg, s) == 0.0 && pcg_polled_iterations(pcg_y, s) == 0.0;
         te(CFD_K_PCG);
-        pcg_store_result(pcg, scal(CFD_S_PCG_ITX), scal(CFD_S_PCG_RZX), scal(CFD_S_PCG_ITSUM), s,
-                         scal(CFD_S_PCG_UNCONV));
-        pcg_store_result(pcg_y, scal(CFD_S_PCG_ITY), scal(CFD_S_PCG_RZY), scal(CFD_S_PCG_ITSUM), s,
-                         scal(CFD_S_PCG_UNCONV));
         if (ws_on) ws.after_solves(q, s);
-        k_move<<<grid_for(np), kBlock, 0, s>>>(X.p, X1.p, WX.p, XPOS.p, scal(CFD_S_DTMIN), np);
-        k_move<<<grid_for(np), kBlock, 0, s>>>(Y.p, Y1.p, WY.p, YPOS.p, scal(CFD_S_DTMIN), np);
+        const bool old = d.gcl >= 0;
+        launch_mesh_move({&pcg, XPOS.p, X.p, X1.p, WX.p, old ? WXO.p : nullptr,
+                          scal(CFD_S_PCG_ITX), scal(CFD_S_PCG_RZX)},
+                         {&pcg_y, YPOS.p, Y.p, Y1.p, WY.p, old ? WYO.p : nullptr,
+                          scal(CFD_S_PCG_ITY), scal(CFD_S_PCG_RZY)},
+                         scal(CFD_S_PCG_ITSUM), scal(CFD_S_PCG_UNCONV), scal(CFD_S_DTMIN), np, s);
         CFD_HIP(hipGetLastError());
     }
 
@@ -947,10 +937,6 @@ struct cfd_session {
         if (fused()) te(CFD_K_ELEMENT, nrk);
 
         // fluidStructure (meshMove.f90:52-127)
-        if (d.gcl >= 0) {
-            CFD_HIP(hipMemcpyAsync(WXO.p, WX.p, sizeof(double) * np, hipMemcpyDeviceToDevice, s));
-            CFD_HIP(hipMemcpyAsync(WYO.p, WY.p, sizeof(double) * np, hipMemcpyDeviceToDevice, s));
-        }
         // FORCE_VISC as the reference's print block calls it (ns2DComp.ALE.f90:
         // 231-236): after the mesh move, with the step's velocities, pressure
         // and temperature and the shape gradients of the start of the step;
@@ -977,21 +963,21 @@ struct cfd_session {
             if (fvisc)
                 launch_forces(d.nsetedges, ISET.p, X.p, Y.p, P.p, d.xref, d.yref, nullptr, &visc,
                               scal(CFD_S_FVX), FPART.p, nullptr, s);
+        } else if (d.gcl >= 0) {  // (else the move keeps the old W)
+            CFD_HIP(hipMemcpyAsync(WXO.p, WX.p, sizeof(double) * np, hipMemcpyDeviceToDevice, s));
+            CFD_HIP(hipMemcpyAsync(WYO.p, WY.p, sizeof(double) * np, hipMemcpyDeviceToDevice, s));
         }
 
         if (d.moving == 1) {  // ns2DComp.ALE.f90:259-275
             tb(CFD_K_GEOM);
             if (d.gcl >= 0) {
-                CFD_HIP(hipMemcpyAsync(AREA_OLD.p, AREA.p, sizeof(double) * ne,
-                                       hipMemcpyDeviceToDevice, s));
                 bc.normales(X.p, Y.p, s);
                 launch_deriv(t, X.p, Y.p, AREA.p, DNX.p, DNY.p, HH.p, HHX.p, HHY.p,
-                             scal(CFD_S_HMIN), partials.p, s);
+                             scal(CFD_S_HMIN), partials.p, s, AREA_OLD.p);
                 refresh_patch_geometry();
                 launch_gcl(t, M.p, WX.p, WY.p, WXO.p, WYO.p, DNX.p, DNY.p, AREA.p, AREA_OLD.p, dtmin,
                            d.gcl, s);
-                launch_laplace(t, X.p, Y.p, DNX.p, DNY.p, LAP.p, LDIAG.p, s);
-                if (ell_on) ell.refresh(t.rowptr.p, LAP.p, s);
+                launch_laplace(t, X.p, Y.p, DNX.p, DNY.p, LAP.p, LDIAG.p, s, ell_on ? &ell : nullptr);
             } else {
                 geometry();
             }

@@ -181,15 +181,18 @@ struct Consts {
 };
 
 // deriv (subrutinas.f90:88-126); hmin_out: device double; partials holds
-// grid_for(nelem) doubles
+// grid_for(nelem) doubles; area_old (when given) receives the areas before
 void launch_deriv(const Tables& t, const double* X, const double* Y, double* area, double* dNx,
                   double* dNy, double* HH, double* HHX, double* HHY, double* hmin_out,
-                  double* partials, hipStream_t s);
+                  double* partials, hipStream_t s, double* area_old = nullptr);
 // MASAS (subrutinas.f90:128-153) as an ascending-element gather
 void launch_masas(const Tables& t, const double* area, double* M, hipStream_t s);
-// mLaplace.f90:7-58 values (structure comes from Tables)
+// mLaplace.f90:7-58 values (structure comes from Tables); ell (when given): the
+// ELL copy's values too (EllLap::refresh in the same pass)
+struct EllLap;
 void launch_laplace(const Tables& t, const double* X, const double* Y, const double* dNx,
-                    const double* dNy, double* lap, double* diag, hipStream_t s);
+                    const double* dNy, double* lap, double* diag, hipStream_t s,
+                    EllLap* ell = nullptr);
 // gcl.f90:8-46 main; mode 0 = as written, 1 = corrected y-divergence; dt is a
 // device scalar
 void launch_gcl(const Tables& t, double* M, const double* Wx, const double* Wy,
@@ -658,11 +661,19 @@ void pcg_launch(PcgWork& w, int npoin, const double* A, const int* idx, const in
                 const EllMat* ell = nullptr);
 // Waits for the stream and returns the last solve's outcome.
 PcgResult pcg_result(const PcgWork& w, hipStream_t s);
-// Copy the last solve's iteration count and final r.z to device scalars
-// (and add the count to *itsum when given, and 1 to *unconv when given and
-// the solve stopped at its iteration cap without meeting the tolerance).
-void pcg_store_result(const PcgWork& w, double* iters, double* rz, double* itsum, hipStream_t s,
-                      double* unconv = nullptr);
+// One axis of the mesh's move, and where its solve's outcome goes: X += pos,
+// X1 += pos, W = pos / dtmin (W's old values to Wold when given); the
+// iterations and the final r.z to device scalars
+struct MeshAxis {
+    const PcgWork* w;
+    const double* pos;
+    double *X, *X1, *W, *Wold;
+    double *iters, *rz;
+};
+// Both axes; the iterations are added to *itsum, and a solve that stopped at its
+// cap without meeting the tolerance adds 1 to *unconv
+void launch_mesh_move(const MeshAxis& x, const MeshAxis& y, double* itsum, double* unconv,
+                      const double* dtmin, int n, hipStream_t s);
 // r.r of the first residual test for the guess x (fixed values applied to a
 // copy; x is not changed) into the device scalar rr_out
 void pcg_initial_rr(PcgWork& w, int npoin, const double* A, const int* idx, const int* rowptr,

@@ -692,13 +692,34 @@ __global__ void k_ell_val(int n, int width, const int* __restrict__ rowptr,
     for (int k = 0; k < width; ++k) val[(size_t)k * n + i] = k < len ? A[b + k] : 0.0;
 }
 
-__global__ void k_store_result(const double* __restrict__ scal, double* __restrict__ iters,
-                               double* __restrict__ rz, double* __restrict__ itsum,
-                               double* __restrict__ unconv) {
-    *iters = scal[S_K];
-    *rz = scal[S_EOLD];
-    if (itsum) *itsum = *itsum + scal[S_K];
-    if (unconv && scal[S_CONV] == 0.0) *unconv = *unconv + 1.0;
+// meshMove.f90:99-104 for both axes in one launch, with the outcomes of their
+// solves (a launch of its own costs the step more than what it does)
+struct MoveAxis {
+    const double *scal, *pos;
+    double *X, *X1, *W, *Wold, *iters, *rz;
+};
+__global__ void k_mesh_move(MoveAxis ax, MoveAxis ay, double* __restrict__ itsum,
+                            double* __restrict__ unconv, const double* __restrict__ dtminp, int n) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const double dtmin = *dtminp;
+    if (i < n) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const MoveAxis& a = k ? ay : ax;
+            const double d = a.pos[i];
+            if (a.Wold) a.Wold[i] = a.W[i];
+            a.X[i] = a.X[i] + d;
+            a.X1[i] = a.X1[i] + d;
+            a.W[i] = d / dtmin;
+        }
+    }
+    if (i != 0) return;
+    *ax.iters = ax.scal[S_K];
+    *ax.rz = ax.scal[S_EOLD];
+    *ay.iters = ay.scal[S_K];
+    *ay.rz = ay.scal[S_EOLD];
+    *itsum = *itsum + ax.scal[S_K] + ay.scal[S_K];
+    *unconv = *unconv + (ax.scal[S_CONV] == 0.0 ? 1.0 : 0.0) + (ay.scal[S_CONV] == 0.0 ? 1.0 : 0.0);
 }
 
 __global__ void __launch_bounds__(256)
@@ -752,9 +773,12 @@ void pcg_initial_rr(PcgWork& w, int npoin, const double* A, const int* idx, cons
     CFD_HIP(hipGetLastError());
 }
 
-void pcg_store_result(const PcgWork& w, double* iters, double* rz, double* itsum, hipStream_t s,
-                      double* unconv) {
-    k_store_result<<<1, 1, 0, s>>>(w.scal.p, iters, rz, itsum, unconv);
+void launch_mesh_move(const MeshAxis& x, const MeshAxis& y, double* itsum, double* unconv,
+                      const double* dtmin, int n, hipStream_t s) {
+    auto axis = [](const MeshAxis& a) {
+        return MoveAxis{a.w->scal.p, a.pos, a.X, a.X1, a.W, a.Wold, a.iters, a.rz};
+    };
+    k_mesh_move<<<grid_for(n), kBlock, 0, s>>>(axis(x), axis(y), itsum, unconv, dtmin, n);
     CFD_HIP(hipGetLastError());
 }
 
