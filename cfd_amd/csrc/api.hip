@@ -813,6 +813,7 @@ struct cfd_session {
         const double tol = d.pcg_tol > 0.0 ? d.pcg_tol : 1.0e-10;
         const int maxit = d.pcg_maxit > 0 ? d.pcg_maxit : 1000;
         WsSolve q;
+        const EllMat em = ell.mat();
         const bool ws_now = ws_on && !(d.pcg_rel == 0 && last_solves_trivial);
         if (ws_on) {
             q.XPOS = XPOS.p;
@@ -832,6 +833,7 @@ struct cfd_session {
             q.idx = m->t.idx.p;
             q.rowptr = m->t.rowptr.p;
             q.fix_idx = ILAUX.p;
+            q.ell = ell_on ? &em : nullptr;
             q.nfix = nn;
             q.n_learned = scal(CFD_S_WS_LEARNED);
             q.n_solves = scal(CFD_S_WS_SOLVES);
@@ -840,7 +842,6 @@ struct cfd_session {
         }
         const PcgSystem sys[2] = {{&pcg, XPOS.p, BZERO.p, POSAUX.p, ILAUX.p, nn},
                                   {&pcg_y, YPOS.p, BZERO.p, POSAUY.p, ILAUX.p, nn}};
-        const EllMat em = ell.mat();
         pcg_launch_multi(sys, 2, np, LAP.p, m->t.idx.p, m->t.rowptr.p, LDIAG.p, tol, maxit,
                          d.pcg_rel, s, ell_on ? &em : nullptr);
         if (ws_on && d.pcg_rel == 0)  // else nothing asks

@@ -421,11 +421,14 @@ void mlp_forward(const MlpWeights& w, const unsigned short* X, int n, float* out
 // returns ns
 int mlp_gradient(MlpWeights& w, const unsigned short* X, const float* T, int n,
                  int tiles_per_block, hipStream_t s, int stride = 1);
-void mlp_adam(MlpWeights& w, float lr, hipStream_t s);
+// the same, then an Adam step with rate lr
+int mlp_train(MlpWeights& w, const unsigned short* X, const float* T, int n, int tiles_per_block,
+              float lr, hipStream_t s, int stride = 1);
 
 // Learned warm start of the mesh solves (warmstart.hip).  WsSolve: the two
 // solves' systems and where the session keeps its scalars.
 struct PcgWork;
+struct EllMat;
 struct WsSolve {
     double *XPOS, *YPOS;            // guesses in, solutions out
     const double *X, *Y;            // node coordinates
@@ -434,6 +437,7 @@ struct WsSolve {
     PcgWork *wx, *wy;
     const double *A, *diag, *b, *fixx, *fixy;
     const int *idx, *rowptr, *fix_idx;
+    const EllMat* ell;  // the matrix in ELL order (null: none)
     int nfix;
     double *n_learned, *n_solves, *loss;  // device scalars
 };
@@ -674,10 +678,11 @@ struct MeshAxis {
 // cap without meeting the tolerance adds 1 to *unconv
 void launch_mesh_move(const MeshAxis& x, const MeshAxis& y, double* itsum, double* unconv,
                       const double* dtmin, int n, hipStream_t s);
-// r.r of the first residual test for the guess x (fixed values applied to a
-// copy; x is not changed) into the device scalar rr_out
-void pcg_initial_rr(PcgWork& w, int npoin, const double* A, const int* idx, const int* rowptr,
-                    const double* diag, const double* x, const double* b, const double* x_fix,
-                    const int* x_fix_idx, int nfix, double* rr_out, hipStream_t s);
+// r.r of the first residual tests of two systems for the guesses sys[k].x
+// (fixed values applied to copies; the guesses are not changed) into the
+// device scalars rr_out[0], rr_out[1]; the residuals stay in the work spaces' r
+void pcg_initial_rr(const PcgSystem (&sys)[2], int npoin, const double* A, const int* idx,
+                    const int* rowptr, const double* diag, const EllMat* ell, double* rr_out,
+                    hipStream_t s);
 
 }  // namespace cfd

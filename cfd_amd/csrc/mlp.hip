@@ -294,14 +294,37 @@ __global__ void __launch_bounds__(64) k_mlp_grad(MlpDev m, const unsigned short*
     if (lane == 0) lpart[blockIdx.x] = loss;
 }
 
+// One Adam step of a parameter on the FP32 master copy (rows of W3 and b3
+// beyond the used outputs stay zero), then the weight's BF16 copy
+struct MlpAdam {
+    float *w, *mom, *vel;
+    unsigned short* wb;
+    float lr, b1, b2, eps, c1, c2;
+};
+__device__ __forceinline__ void adam_step(const MlpAdam& a, int p, float g) {
+    const bool used = !((p >= kMlpW3 && p < kMlpB3 && (p - kMlpW3) / kMlpHid >= kMlpOutUsed) ||
+                        (p >= kMlpB3 && p - kMlpB3 >= kMlpOutUsed));
+    if (used) {
+        const float mm = a.b1 * a.mom[p] + (1.f - a.b1) * g;
+        const float vv = a.b2 * a.vel[p] + (1.f - a.b2) * g * g;
+        a.mom[p] = mm;
+        a.vel[p] = vv;
+        a.w[p] = a.w[p] - a.lr * (mm * a.c1) / (sqrtf(vv * a.c2) + a.eps);
+    }
+    if (p < kMlpB3 && !(p >= kMlpB1 && p < kMlpW2) && !(p >= kMlpB2 && p < kMlpW3))
+        a.wb[p] = f2bf(a.w[p]);
+}
+
 // grad[p] = sum over blocks of gpart[b][p]; the loss likewise from lpart (as
 // column kMlpParams).  A block sums 64 columns; each of its kRedWaves waves
 // sums one contiguous range of the partial blocks, and the waves' sums are
-// added in wave order: a fixed order for a given block count.
+// added in wave order: a fixed order for a given block count.  kAdam: the
+// parameter's Adam step in the same launch.
 constexpr int kRedWaves = 16;
+template <bool kAdam>
 __global__ void __launch_bounds__(64 * kRedWaves)
 k_mlp_reduce(const float* __restrict__ gpart, const float* __restrict__ lpart, int nblocks,
-             float* __restrict__ grad, float* __restrict__ loss) {
+             float* __restrict__ grad, float* __restrict__ loss, MlpAdam adam) {
     __shared__ float sm[kRedWaves][65];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int p = blockIdx.x * 64 + lane;
@@ -321,30 +344,13 @@ k_mlp_reduce(const float* __restrict__ gpart, const float* __restrict__ lpart, i
         float t = 0.f;
 #pragma unroll
         for (int w = 0; w < kRedWaves; ++w) t += sm[w][lane];
-        if (p < kMlpParams) grad[p] = t;
-        else if (p == kMlpParams) *loss = t;
+        if (p < kMlpParams) {
+            grad[p] = t;
+            if (kAdam) adam_step(adam, p, t);
+        } else if (p == kMlpParams) {
+            *loss = t;
+        }
     }
-}
-
-// Adam on the FP32 master copy; rows of W3 and b3 beyond the used outputs
-// stay zero.  Then the BF16 copies of the weights.
-__global__ void k_mlp_adam(float* __restrict__ w, float* __restrict__ mom, float* __restrict__ vel,
-                           const float* __restrict__ grad, float lr, float b1, float b2, float eps,
-                           float c1, float c2, int nout, unsigned short* __restrict__ wb) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= kMlpParams) return;
-    const bool used = !((p >= kMlpW3 && p < kMlpB3 && (p - kMlpW3) / kMlpHid >= nout) ||
-                        (p >= kMlpB3 && p - kMlpB3 >= nout));
-    if (used) {
-        const float g = grad[p];
-        const float mm = b1 * mom[p] + (1.f - b1) * g;
-        const float vv = b2 * vel[p] + (1.f - b2) * g * g;
-        mom[p] = mm;
-        vel[p] = vv;
-        w[p] = w[p] - lr * (mm * c1) / (sqrtf(vv * c2) + eps);
-    }
-    if (p < kMlpB3 && !(p >= kMlpB1 && p < kMlpW2) && !(p >= kMlpB2 && p < kMlpW3))
-        wb[p] = f2bf(w[p]);
 }
 
 __global__ void k_mlp_to_bf16(const float* __restrict__ w, unsigned short* __restrict__ wb) {
@@ -386,8 +392,9 @@ void mlp_forward(const MlpWeights& w, const unsigned short* X, int n, float* out
     CFD_HIP(hipGetLastError());
 }
 
-int mlp_gradient(MlpWeights& w, const unsigned short* X, const float* T, int n, int tiles_per_block,
-                 hipStream_t s, int stride) {
+// gradient and loss over the samples; adam: with the Adam step
+static int gradient(MlpWeights& w, const unsigned short* X, const float* T, int n,
+                    int tiles_per_block, hipStream_t s, int stride, const MlpAdam* adam) {
     CFD_CHECK(n > 0 && tiles_per_block > 0 && stride > 0, "arg: MLP training needs nodes");
     const int ns = (n + stride - 1) / stride;  // samples 0, stride, 2 stride, ... < n
     const int nb = (ns + 16 * tiles_per_block - 1) / (16 * tiles_per_block);
@@ -395,20 +402,26 @@ int mlp_gradient(MlpWeights& w, const unsigned short* X, const float* T, int n, 
     if ((size_t)nb > w.lpart.n) w.lpart.alloc(nb);
     k_mlp_grad<<<nb, 64, 0, s>>>(mlp_dev(w), X, T, ns, stride, tiles_per_block, 1.0f / (float)ns,
                                  w.gpart.p, w.lpart.p);
-    k_mlp_reduce<<<kMlpParams / 64 + 1, 64 * kRedWaves, 0, s>>>(w.gpart.p, w.lpart.p, nb,
-                                                                  w.grad.p, w.loss.p);
+    const auto reduce = adam ? k_mlp_reduce<true> : k_mlp_reduce<false>;
+    reduce<<<kMlpParams / 64 + 1, 64 * kRedWaves, 0, s>>>(w.gpart.p, w.lpart.p, nb, w.grad.p,
+                                                          w.loss.p, adam ? *adam : MlpAdam{});
     CFD_HIP(hipGetLastError());
     return ns;
 }
 
-void mlp_adam(MlpWeights& w, float lr, hipStream_t s) {
+int mlp_gradient(MlpWeights& w, const unsigned short* X, const float* T, int n, int tiles_per_block,
+                 hipStream_t s, int stride) {
+    return gradient(w, X, T, n, tiles_per_block, s, stride, nullptr);
+}
+
+int mlp_train(MlpWeights& w, const unsigned short* X, const float* T, int n, int tiles_per_block,
+              float lr, hipStream_t s, int stride) {
     const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
     ++w.step;
     const float c1 = 1.0f / (1.0f - std::pow(b1, (float)w.step));
     const float c2 = 1.0f / (1.0f - std::pow(b2, (float)w.step));
-    k_mlp_adam<<<grid_for(kMlpParams), kBlock, 0, s>>>(w.w.p, w.m.p, w.v.p, w.grad.p, lr, b1, b2, eps,
-                                                       c1, c2, kMlpOutUsed, w.wb.p);
-    CFD_HIP(hipGetLastError());
+    const MlpAdam adam{w.w.p, w.m.p, w.v.p, w.wb.p, lr, b1, b2, eps, c1, c2};
+    return gradient(w, X, T, n, tiles_per_block, s, stride, &adam);
 }
 
 }  // namespace cfd

@@ -33,8 +33,8 @@ constexpr int kWsTrainNodes = 32768;
 constexpr int kWsAdamSteps = 4;
 
 enum {
-    W_DT1 = 0, W_DT2, W_DT3, W_SE, W_SD, W_S2, W_SC, W_BX, W_BY, W_RRPX, W_RRLX, W_RRPY,
-    W_RRLY, W_RREX, W_RREY, W_N = 16
+    W_DT1 = 0, W_DT2, W_DT3, W_SE, W_SD, W_S2, W_SC, W_BX, W_BY,  // k_max_to, k_ws_beta: in order
+    W_RRPX, W_RRPY, W_RRLX, W_RRLY, W_RREX, W_RREY, W_N = 16
 };
 
 __device__ __forceinline__ unsigned short to_bf16(float f) {  // round to nearest even
@@ -44,54 +44,54 @@ __device__ __forceinline__ unsigned short to_bf16(float f) {  // round to neares
     return (unsigned short)(u >> 16);
 }
 
-// E = dt (2 x1/dt1 - x2/dt2) for both axes
-__global__ void k_ws_extrap(const double* __restrict__ h1x, const double* __restrict__ h2x,
-                            const double* __restrict__ h1y, const double* __restrict__ h2y,
-                            const double* __restrict__ dtp, const double* __restrict__ wsc,
-                            double* __restrict__ ex, double* __restrict__ ey, int n) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const double dt = *dtp, a = 2.0 * dt / wsc[W_DT1], b = dt / wsc[W_DT2];
-    ex[i] = a * h1x[i] - b * h2x[i];
-    ey[i] = a * h1y[i] - b * h2y[i];
-}
-
 // D2 = dt (x1/dt1 - 2 x2/dt2 + x3/dt3) of one node and axis
 __device__ __forceinline__ double ws_d2(const double* h1, const double* h2, const double* h3, int i,
                                         double dt, const double* wsc) {
     return dt * (h1[i] / wsc[W_DT1] - 2.0 * h2[i] / wsc[W_DT2] + h3[i] / wsc[W_DT3]);
 }
 
-// block partials of max |D2| over both axes
+// E = dt (2 x1/dt1 - x2/dt2) for both axes; kMax: block partials of the maxima
+// over both axes of |E|, |x1 - x2| and |D2| too, gridDim.x each
+template <bool kMax>
 __global__ void __launch_bounds__(kBlock)
-k_ws_maxd2(const double* __restrict__ h1x, const double* __restrict__ h2x,
-           const double* __restrict__ h3x, const double* __restrict__ h1y,
-           const double* __restrict__ h2y, const double* __restrict__ h3y,
-           const double* __restrict__ dtp, const double* __restrict__ wsc, int n,
-           double* __restrict__ partials) {
-    const double dt = *dtp;
-    double m = 0.0;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-        m = fmax(m, fmax(fabs(ws_d2(h1x, h2x, h3x, i, dt, wsc)), fabs(ws_d2(h1y, h2y, h3y, i, dt, wsc))));
-    block_partial(m, OpMax(), partials);
+k_ws_extrap(const double* __restrict__ h1x, const double* __restrict__ h2x,
+            const double* __restrict__ h3x, const double* __restrict__ h1y,
+            const double* __restrict__ h2y, const double* __restrict__ h3y,
+            const double* __restrict__ dtp, const double* __restrict__ wsc,
+            double* __restrict__ ex, double* __restrict__ ey, int n,
+            double* __restrict__ partials) {
+    const double dt = *dtp, a = 2.0 * dt / wsc[W_DT1], b = dt / wsc[W_DT2];
+    double me = 0.0, md = 0.0, m2 = 0.0;
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+        const double u = a * h1x[i] - b * h2x[i], v = a * h1y[i] - b * h2y[i];
+        ex[i] = u;
+        ey[i] = v;
+        if (!kMax) continue;
+        me = fmax(me, fmax(fabs(u), fabs(v)));
+        md = fmax(md, fmax(fabs(h1x[i] - h2x[i]), fabs(h1y[i] - h2y[i])));
+        m2 = fmax(m2, fmax(fabs(ws_d2(h1x, h2x, h3x, i, dt, wsc)), fabs(ws_d2(h1y, h2y, h3y, i, dt, wsc))));
+    }
+    if (!kMax) return;
+    block_partial(me, OpMax(), partials);
+    block_partial(md, OpMax(), partials + gridDim.x);
+    block_partial(m2, OpMax(), partials + 2 * gridDim.x);
 }
 
-// block partials of max(|a - b|, |c - d|) (b, d may be null: zero)
+// block partials of max(|a - b|, |c - d|)
 __global__ void __launch_bounds__(kBlock)
 k_maxabs2(const double* __restrict__ a, const double* __restrict__ b, const double* __restrict__ c,
           const double* __restrict__ d, int n, double* __restrict__ partials) {
     double m = 0.0;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        const double u = fabs(a[i] - (b ? b[i] : 0.0)), v = fabs(c[i] - (d ? d[i] : 0.0));
-        m = fmax(m, fmax(u, v));
-    }
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
+        m = fmax(m, fmax(fabs(a[i] - b[i]), fabs(c[i] - d[i])));
     block_partial(m, OpMax(), partials);
 }
 
+// out[k] = the maximum of the k-th nb partials (1 when it is not positive), block k
 __global__ void __launch_bounds__(256)
 k_max_to(const double* __restrict__ partials, int nb, double* __restrict__ out) {
-    const double m = combine_partials(partials, nb, 0.0, OpMax());
-    if (threadIdx.x == 0) *out = m > 0.0 ? m : 1.0;
+    const double m = combine_partials(partials + (size_t)blockIdx.x * nb, nb, 0.0, OpMax());
+    if (threadIdx.x == 0) out[blockIdx.x] = m > 0.0 ? m : 1.0;
 }
 
 __global__ void k_ws_features(const double* __restrict__ ex, const double* __restrict__ ey,
@@ -123,14 +123,16 @@ __global__ void k_ws_features(const double* __restrict__ ex, const double* __res
     for (int k = 0; k < kMlpIn; ++k) p[k] = to_bf16(f[k]);
 }
 
-// Partials of y.r and y.(A y) over the free rows of one axis (y = the
+// Partials of y.r and y.(A y) over the free rows of axis blockIdx.y (y = the
 // network's output for that axis, taken as zero on the fixed nodes; r = the
 // residual of E, zero on the fixed rows)
 __global__ void __launch_bounds__(kBlock)
 k_ws_galerkin(int n, const double* __restrict__ A, const int* __restrict__ idx,
               const int* __restrict__ rowptr, const unsigned char* __restrict__ fixflag,
-              const float* __restrict__ out, int axis, const double* __restrict__ r,
-              double* __restrict__ partials) {
+              const float* __restrict__ out, const double* __restrict__ rx,
+              const double* __restrict__ ry, double* __restrict__ partials) {
+    const int axis = blockIdx.y;
+    const double* r = axis ? ry : rx;
     double yr = 0.0, yay = 0.0;
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         if (fixflag[i]) continue;
@@ -143,16 +145,18 @@ k_ws_galerkin(int n, const double* __restrict__ A, const int* __restrict__ idx,
         yr = yr + yi * r[i];
         yay = yay + yi * ay;
     }
-    block_partial(yr, OpSum(), partials);
-    block_partial(yay, OpSum(), partials + gridDim.x);
+    double* p = partials + 2 * (size_t)axis * gridDim.x;
+    block_partial(yr, OpSum(), p);
+    block_partial(yay, OpSum(), p + gridDim.x);
 }
 
-// beta = y.r / y.(A y) (0 when y.(A y) is not positive)
+// beta = y.r / y.(A y) (0 when y.(A y) is not positive), block k: axis k
 __global__ void __launch_bounds__(256)
 k_ws_beta(const double* __restrict__ partials, int nb, double* __restrict__ beta) {
-    const double yr = combine_partials(partials, nb, 0.0, OpSum());
-    const double yay = combine_partials(partials + nb, nb, 0.0, OpSum());
-    if (threadIdx.x == 0) *beta = yay > 0.0 ? yr / yay : 0.0;
+    const double* p = partials + 2 * (size_t)blockIdx.x * nb;
+    const double yr = combine_partials(p, nb, 0.0, OpSum());
+    const double yay = combine_partials(p + nb, nb, 0.0, OpSum());
+    if (threadIdx.x == 0) beta[blockIdx.x] = yay > 0.0 ? yr / yay : 0.0;
 }
 
 // xhat = E + beta y for both axes (beta zero: xhat = E)
@@ -167,17 +171,20 @@ __global__ void k_ws_predict(const double* __restrict__ ex, const double* __rest
     haty[i] = use_net ? ey[i] + by * (double)out[2 * (size_t)i + 1] : ey[i];
 }
 
-// x = hat when the learned first residual is smaller (a choice every block
-// makes alike); block 0 counts the choices in the session scalars
-__global__ void k_ws_select(double* __restrict__ x, const double* __restrict__ hat,
-                            const double* __restrict__ wsc, int rr_prev, int rr_learn,
-                            double* __restrict__ n_learned, double* __restrict__ n_solves, int n) {
-    const bool use = wsc[rr_learn] < wsc[rr_prev];
+// Each axis: its positions = hat when the learned first residual is smaller (a
+// choice every block makes alike); block 0 counts the choices in the session
+// scalars
+__global__ void k_ws_select(double* __restrict__ x, double* __restrict__ y,
+                            const double* __restrict__ hatx, const double* __restrict__ haty,
+                            const double* __restrict__ wsc, double* __restrict__ n_learned,
+                            double* __restrict__ n_solves, int n) {
+    const bool ux = wsc[W_RRLX] < wsc[W_RRPX], uy = wsc[W_RRLY] < wsc[W_RRPY];
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (use && i < n) x[i] = hat[i];
+    if (ux && i < n) x[i] = hatx[i];
+    if (uy && i < n) y[i] = haty[i];
     if (i == 0) {
-        *n_solves = *n_solves + 1.0;
-        if (use) *n_learned = *n_learned + 1.0;
+        *n_solves = *n_solves + 2.0;
+        *n_learned = *n_learned + (ux ? 1.0 : 0.0) + (uy ? 1.0 : 0.0);
     }
 }
 
@@ -191,12 +198,14 @@ __global__ void k_ws_target(const double* __restrict__ x, const double* __restri
     tgt[2 * (size_t)i + 1] = (float)((y[i] - ey[i]) * isc);
 }
 
-// history shift and the rates' time steps
+// history shift and the rates' time steps; *loss (when given) scaled into *dst
 __global__ void k_ws_shift(const double* __restrict__ x, const double* __restrict__ y,
                            double* __restrict__ h1x, double* __restrict__ h2x,
                            double* __restrict__ h3x, double* __restrict__ h1y,
                            double* __restrict__ h2y, double* __restrict__ h3y,
-                           const double* __restrict__ dtp, double* __restrict__ wsc, int n) {
+                           const double* __restrict__ dtp, double* __restrict__ wsc, int n,
+                           const float* __restrict__ loss, double inv_n,
+                           double* __restrict__ dst) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) {
         h3x[i] = h2x[i];
@@ -210,11 +219,8 @@ __global__ void k_ws_shift(const double* __restrict__ x, const double* __restric
         wsc[W_DT3] = wsc[W_DT2];
         wsc[W_DT2] = wsc[W_DT1];
         wsc[W_DT1] = *dtp;
+        if (loss) *dst = (double)*loss * inv_n;
     }
-}
-
-__global__ void k_copy_loss(const float* __restrict__ loss, double inv_n, double* __restrict__ dst) {
-    *dst = (double)*loss * inv_n;
 }
 
 uint64_t splitmix(uint64_t& s) {
@@ -238,7 +244,7 @@ void WarmStart::init(int npoin, double l, hipStream_t s) {
     tgt.alloc(2 * (size_t)np);
     wsc.alloc(W_N);
     wsc.zero(s);
-    partials.alloc(2 * kRedBlocks);
+    partials.alloc(4 * kRedBlocks);
     // Glorot-uniform hidden layers, zero output layer: the first prediction is E
     std::vector<float> p(kMlpParams, 0.0f);
     uint64_t seed = 20261202ull;
@@ -259,49 +265,43 @@ void WarmStart::before_solves(const WsSolve& q, hipStream_t s) {
     const unsigned g = grid_for(np);
     const int nb = std::min<int>(grid_for(np), kRedBlocks);
     net_used = use_mlp && nhist >= 3;
-    k_ws_extrap<<<g, kBlock, 0, s>>>(h1x.p, h2x.p, h1y.p, h2y.p, q.dtmin, wsc.p, ex.p, ey.p, np);
+    const auto extrap = net_used ? k_ws_extrap<true> : k_ws_extrap<false>;
+    extrap<<<nb, kBlock, 0, s>>>(h1x.p, h2x.p, h3x.p, h1y.p, h2y.p, h3y.p, q.dtmin, wsc.p, ex.p,
+                                 ey.p, np, partials.p);
+    // the first residuals of a pair of guesses, to wsc[slot] and wsc[slot + 1]
+    auto first = [&](double* gx, double* gy, int slot) {
+        const PcgSystem sys[2] = {{q.wx, gx, q.b, q.fixx, q.fix_idx, q.nfix},
+                                  {q.wy, gy, q.b, q.fixy, q.fix_idx, q.nfix}};
+        pcg_initial_rr(sys, np, q.A, q.idx, q.rowptr, q.diag, q.ell, wsc.p + slot, s);
+    };
     if (net_used) {
-        k_maxabs2<<<nb, kBlock, 0, s>>>(ex.p, nullptr, ey.p, nullptr, np, partials.p);
-        k_max_to<<<1, 256, 0, s>>>(partials.p, nb, wsc.p + W_SE);
-        k_maxabs2<<<nb, kBlock, 0, s>>>(h1x.p, h2x.p, h1y.p, h2y.p, np, partials.p);
-        k_max_to<<<1, 256, 0, s>>>(partials.p, nb, wsc.p + W_SD);
-        k_ws_maxd2<<<nb, kBlock, 0, s>>>(h1x.p, h2x.p, h3x.p, h1y.p, h2y.p, h3y.p, q.dtmin, wsc.p,
-                                         np, partials.p);
-        k_max_to<<<1, 256, 0, s>>>(partials.p, nb, wsc.p + W_S2);
+        k_max_to<<<3, 256, 0, s>>>(partials.p, nb, wsc.p + W_SE);
         k_ws_features<<<g, kBlock, 0, s>>>(ex.p, ey.p, h1x.p, h2x.p, h3x.p, h1y.p, h2y.p, h3y.p,
                                            q.X, q.Y, q.xref, q.yref, inv_l, q.dtmin, wsc.p, feat.p,
                                            np);
         mlp_forward(mlp, feat.p, np, out.p, s);
         // the energy-optimal step along the network's correction, per axis,
-        // from the residual of E (left in the work space's r by the call)
-        struct Axis { PcgWork* w; const double *e, *fix; int slot_rr, slot_b; };
-        for (const Axis a : {Axis{q.wx, ex.p, q.fixx, W_RREX, W_BX}, Axis{q.wy, ey.p, q.fixy, W_RREY, W_BY}}) {
-            pcg_initial_rr(*a.w, np, q.A, q.idx, q.rowptr, q.diag, a.e, q.b, a.fix, q.fix_idx,
-                           q.nfix, wsc.p + a.slot_rr, s);
-            k_ws_galerkin<<<nb, kBlock, 0, s>>>(np, q.A, q.idx, q.rowptr, a.w->fixflag.p, out.p,
-                                                a.slot_b == W_BX ? 0 : 1, a.w->r.p, partials.p);
-            k_ws_beta<<<1, 256, 0, s>>>(partials.p, nb, wsc.p + a.slot_b);
-        }
+        // from the residual of E (left in the work spaces' r)
+        first(ex.p, ey.p, W_RREX);
+        k_ws_galerkin<<<dim3(nb, 2), kBlock, 0, s>>>(np, q.A, q.idx, q.rowptr, q.wx->fixflag.p,
+                                                     out.p, q.wx->r.p, q.wy->r.p, partials.p);
+        k_ws_beta<<<2, 256, 0, s>>>(partials.p, nb, wsc.p + W_BX);
     }
     k_ws_predict<<<g, kBlock, 0, s>>>(ex.p, ey.p, out.p, wsc.p, net_used ? 1 : 0, hatx.p, haty.p, np);
     // first residuals of both candidates, both axes
-    pcg_initial_rr(*q.wx, np, q.A, q.idx, q.rowptr, q.diag, q.XPOS, q.b, q.fixx, q.fix_idx, q.nfix,
-                   wsc.p + W_RRPX, s);
-    pcg_initial_rr(*q.wx, np, q.A, q.idx, q.rowptr, q.diag, hatx.p, q.b, q.fixx, q.fix_idx, q.nfix,
-                   wsc.p + W_RRLX, s);
-    pcg_initial_rr(*q.wy, np, q.A, q.idx, q.rowptr, q.diag, q.YPOS, q.b, q.fixy, q.fix_idx, q.nfix,
-                   wsc.p + W_RRPY, s);
-    pcg_initial_rr(*q.wy, np, q.A, q.idx, q.rowptr, q.diag, haty.p, q.b, q.fixy, q.fix_idx, q.nfix,
-                   wsc.p + W_RRLY, s);
-    k_ws_select<<<g, kBlock, 0, s>>>(q.XPOS, hatx.p, wsc.p, W_RRPX, W_RRLX, q.n_learned, q.n_solves, np);
-    k_ws_select<<<g, kBlock, 0, s>>>(q.YPOS, haty.p, wsc.p, W_RRPY, W_RRLY, q.n_learned, q.n_solves, np);
+    first(q.XPOS, q.YPOS, W_RRPX);
+    first(hatx.p, haty.p, W_RRLX);
+    k_ws_select<<<g, kBlock, 0, s>>>(q.XPOS, q.YPOS, hatx.p, haty.p, wsc.p, q.n_learned, q.n_solves,
+                                     np);
     CFD_HIP(hipGetLastError());
     predicted = true;
 }
 
 void WarmStart::after_solves(const WsSolve& q, hipStream_t s) {
     const unsigned g = grid_for(np);
-    if (predicted && net_used) {  // train on this step's correction
+    const bool train = predicted && net_used;
+    int ns = 1;
+    if (train) {  // train on this step's correction
         const int nb = std::min<int>(grid_for(np), kRedBlocks);
         k_maxabs2<<<nb, kBlock, 0, s>>>(q.XPOS, ex.p, q.YPOS, ey.p, np, partials.p);
         k_max_to<<<1, 256, 0, s>>>(partials.p, nb, wsc.p + W_SC);
@@ -309,18 +309,16 @@ void WarmStart::after_solves(const WsSolve& q, hipStream_t s) {
         // Adam steps on evenly strided samples of about kWsTrainNodes nodes,
         // each sample shifted by a fraction of the stride
         const int stride = std::max(1, np / kWsTrainNodes);
-        int ns = 0;
         for (int k = 0; k < kWsAdamSteps; ++k) {
             const int off = (int)((long long)stride * k / kWsAdamSteps);
-            ns = mlp_gradient(mlp, feat.p + (size_t)off * kMlpIn, tgt.p + 2 * (size_t)off, np - off,
-                              2, s, stride);
-            mlp_adam(mlp, 1.0e-3f, s);
+            ns = mlp_train(mlp, feat.p + (size_t)off * kMlpIn, tgt.p + 2 * (size_t)off, np - off,
+                           2, 1.0e-3f, s, stride);
         }
-        k_copy_loss<<<1, 1, 0, s>>>(mlp.loss.p, 1.0 / ns, q.loss);
     }
     predicted = net_used = false;
     k_ws_shift<<<g, kBlock, 0, s>>>(q.XPOS, q.YPOS, h1x.p, h2x.p, h3x.p, h1y.p, h2y.p, h3y.p,
-                                    q.dtmin, wsc.p, np);
+                                    q.dtmin, wsc.p, np, train ? mlp.loss.p : nullptr, 1.0 / ns,
+                                    q.loss);
     CFD_HIP(hipGetLastError());
     nhist = std::min(nhist + 1, 3);
 }
