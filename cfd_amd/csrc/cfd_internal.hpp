@@ -467,15 +467,17 @@ void launch_normales(const BcTable& bc, int nwallnodes, const int* wnode_bc, con
 
 // Start-up mesh smoothing (smooth.hip, smoothing.f90): the colouring and
 // work space of one mesh for a given set of fixed nodes
-constexpr int kSmoothSeqMaxNodes = 65536;  // order 0 (one block) above this: refused
+constexpr int kSmoothSeqMaxNodes = 65536;  // order 0 (a wave per pass) above this: refused
 struct SmoothPlan {
     int max_elems = 0;              // most elements around one node
     double hmin = 1.0;              // H_MIN_GLOBAL of the last check
     std::vector<int> colour_ptr;    // free nodes of colour c: colour_nodes[ptr[c], ptr[c+1])
     DBuf<int> colour_nodes, fixed, smoothable;
     DBuf<double> dmove, partials, scal;
-    // order 0: rings, dependencies, positions, positions after each pass
-    DBuf<int> ring, need;
+    // order 0: rings, dependencies, positions, positions after each pass,
+    // marks between passes, the passes' progress
+    DBuf<int> ring, need, prog;
+    DBuf<unsigned> rows;
     DBuf<double2> xy, hist;
     DBuf<double> dmax_pass;
     void build(const Tables& t, const int* fixed_host, hipStream_t s);

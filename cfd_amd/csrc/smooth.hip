@@ -24,7 +24,7 @@
 //   order 0 - the reference's node order, bit for bit its result, for small
 //             meshes: one wave per pass walks the nodes, its lanes forming a
 //             node's elements (and its tries) side by side, while the waves of
-//             the next passes follow behind (k_sm_passes);
+//             the next passes, on other CUs, follow behind (k_sm_passes);
 //   order 1 - colour by colour: a greedy colouring of the node graph (no two
 //             nodes of one colour share an element, so nodes of a colour read
 //             and write disjoint data), one lane per node, colours in
@@ -34,6 +34,7 @@
 #include <algorithm>
 
 #include "cfd_internal.hpp"
+#include "crmath.hpp"
 #include "reduce.hpp"
 
 namespace cfd {
@@ -251,42 +252,54 @@ k_sm_check_fin(const double* __restrict__ hpart, const double* __restrict__ anyp
 }
 
 // ---------------------------------------------------------------------------
-// order 0: up to kSmWaves consecutive passes in one block, a wave per pass.
+// order 0: up to kSmPasses consecutive passes in one launch, a block of one wave
+// per pass, each on a CU of its own.
 //
 // A node's update reads its ring (the nodes that share an element with it) and
 // marks it, and changes nothing else but the node itself.  So pass w + 1 may
 // update node i as soon as pass w is past i and past every node of i's ring:
-// each wave publishes how far it is (prog), and the next one follows that far
-// behind.  Every update then reads exactly the values and marks that it would
-// read with the passes one after the other.  Wave 0 waits for nothing and wave
-// w only for wave w - 1 of its own block, so each wait ends.  On a ring by ring
-// numbering the waves run one ring and a chunk apart; on one where every node
-// has a far neighbour they run one after the other.
+// each block publishes how far it is (prog, after every 64 nodes) and the next
+// one follows that far behind, taking the positions and marks that it left.
+// Every update then reads exactly the values and marks that it would read with
+// the passes one after the other.  Block 0 waits for nothing and block w only
+// for block w - 1, which was started before it, so each wait ends.  On a ring by
+// ring numbering the passes run one ring and a chunk apart; on one where every
+// node has a far neighbour they run one after the other.
+//
+// Marks: a sweep that moves node i marks its ring.  Nodes after i take their
+// turn in the same sweep (the block's own marks), those before i in the next
+// one (a row of bits in memory, read once that sweep may pass them).
 //
 // Inside a wave the lanes form the qualities of the node's elements, 8, 16 or
 // 32 lanes a group, and the groups the tries (their positions are the running
-// sums that the sequential loop forms).
+// sums that the sequential loop forms) and the three points of a gradient.
 //
 // Whether a sweep is the last is known when it ends, while the next ones are
-// on their way: each wave leaves its pass's positions in hist, and the result
+// on their way: each block leaves its pass's positions in hist, and the result
 // is taken from the last sweep that counts.
 //
-// Bound by the instructions that a node takes (about 1,000: seven qualities,
-// fourteen divisions, the tries' positions) on the four SIMDs of one CU; the
-// positions stay in LDS while they fit.  64 x 128 cylinder (8,192 nodes, 2 + 8
-// passes): 48 ms; one lane per pass and the passes one by one took 1,524.
-// More waves than twelve (three per SIMD) add no throughput, only passes begun
-// in vain behind the last one (sixteen: 58.8 ms).
+// Bound by the chain of one node's update (3 us: about 700 instructions with
+// the lanes' exchanges and eight divisions in sequence), node after node, on
+// one wave; the positions stay in LDS while they fit.  64 x 128 cylinder (8,192
+// nodes, 2 + 8 passes): 29.5 ms; 42.7 with the passes as twelve waves of one
+// block (three to a SIMD share its instructions), 1,524 with one lane per pass
+// and the passes one by one.
 // ---------------------------------------------------------------------------
-constexpr int kSmWaves = 12;
+constexpr int kSmPasses = 12;
 struct SmSeq {
-    SmDev d;               // topology, fixed, marks, tol_move, hmin
+    SmDev d;               // topology, tol_move, hmin
     const int *ring, *need;  // per esup entry its element's nodes (0-based); per node
                              // how far the pass before has to be
-    double2 *xy, *hist;    // positions; positions after each pass of the launch
-    double* dmax;          // per pass of the launch: the largest squared move
+    const double2* xy;     // positions before the launch's first pass
+    double2* hist;         // positions after each pass of the launch
+    // rows of a bit per node: row 0 the marks before the first sweep, row w + 1
+    // those that pass w leaves to the next; then the free nodes
+    unsigned* rows;
+    int* prog;             // per pass: nodes done
+    double* dmax;          // per pass: the largest squared move
     int n, npass, nlap;    // passes of the launch, Laplacian ones first
 };
+__host__ __device__ constexpr int sm_words(int n) { return (n + 63) / 64 * 2; }
 
 // v of a lane that every lane names alike
 __device__ __forceinline__ double lane_of(double v, int lane) {
@@ -304,42 +317,41 @@ __device__ __forceinline__ double dpp_of(double v) {
 constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppHalfMirror = 0x141, kDppMirror = 0x140;
 
 template <bool kLds>
-__global__ void __launch_bounds__(64 * kSmWaves)
+__global__ void __launch_bounds__(64)
 k_sm_passes(SmSeq q) {
     extern __shared__ double2 smem_sm[];
-    const int n = q.n, nw = (n + 63) / 64 * 2;
-    double2* xy = kLds ? smem_sm : q.xy;
+    const int n = q.n, nw = sm_words(n), lane = threadIdx.x, w = blockIdx.x;
+    double2* own_hist = q.hist + (size_t)w * n;
+    double2* xy = kLds ? smem_sm : own_hist;
     unsigned* marks = reinterpret_cast<unsigned*>(smem_sm + (kLds ? n : 0));
-    unsigned* free_ = marks + nw;
-    volatile int* prog = reinterpret_cast<volatile int*>(free_ + nw);
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    for (int i = threadIdx.x; i < nw; i += blockDim.x) {
-        unsigned m = 0, f = 0;
-        for (int b = 0; b < 32 && 32 * i + b < n; ++b) {
-            if (q.d.smoothable[32 * i + b]) m |= 1u << b;
-            if (!q.d.fixed[32 * i + b]) f |= 1u << b;
-        }
-        marks[i] = m;
-        free_[i] = f;
-    }
-    if (kLds)
-        for (int i = threadIdx.x; i < n; i += blockDim.x) xy[i] = q.xy[i];
-    if (threadIdx.x < kSmWaves) prog[threadIdx.x] = 0;
+    const unsigned* free_ = q.rows + (size_t)(kSmPasses + 1) * nw;
+    const double2* src = w > 0 ? own_hist - n : q.xy;
+    const unsigned* in_row = q.rows + (size_t)w * nw;
+    unsigned* out_row = q.rows + (size_t)(w + 1) * nw;
+    const bool lap = w < q.nlap;
+    for (int i = lane; i < nw; i += 64) marks[i] = w <= q.nlap ? q.rows[i] : 0u;
     __syncthreads();
-    if (w < q.npass) {
-        const bool lap = w < q.nlap;
+    {
         const double delta = *q.d.hmin * kSmDelta;
+        const Recip by_delta = recip(delta);
         double d_max = 0.0;
+        int taken = 0;  // positions of the pass before that are here
         for (int c0 = 0; c0 < n; c0 += 64) {
             const int node = c0 + lane;
             const bool in = node < n;
             const int b_l = in ? q.d.esup2[node] : 0, e_l = in ? q.d.esup2[node + 1] : 0;
+            int need = in ? q.need[node] : 0;
+            for (int off = 32; off > 0; off >>= 1) need = max(need, __shfl_xor(need, off, 64));
             if (w > 0) {
-                int need = in ? q.need[node] : 0;
-                for (int off = 32; off > 0; off >>= 1) need = max(need, __shfl_xor(need, off, 64));
-                while (prog[w - 1] < need) __builtin_amdgcn_s_sleep(2);
-                __threadfence_block();
+                while (__hip_atomic_load(&q.prog[w - 1], __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_AGENT) < need)
+                    __builtin_amdgcn_s_sleep(16);
+                __threadfence();
             }
+            for (int i = taken + lane; i < need; i += 64) xy[i] = src[i];
+            taken = max(taken, need);
+            if (w > q.nlap && lane < 2) marks[c0 / 32 + lane] |= in_row[c0 / 32 + lane];
+            __syncthreads();
             unsigned long long passed = 0;
             int next = -1, nid[3];  // the entries of the node expected next
             const unsigned long long fr =
@@ -386,16 +398,22 @@ k_sm_passes(SmSeq q) {
                         Y[v] = id[v] == ip ? y : cy[v];
                     }
                 };
+                double X[3], Y[3], area;  // of the last evaluation
                 auto mu = [&](double x, double y) {
-                    double X[3], Y[3];
                     corners(x, y, X, Y);
-                    const double area = X[1] * Y[2] + X[2] * Y[0] + X[0] * Y[1] -
+                    area = X[1] * Y[2] + X[2] * Y[0] + X[0] * Y[1] -
                                         (X[1] * Y[0] + X[2] * Y[1] + X[0] * Y[2]);
                     const double l1 = (X[2] - X[1]) * (X[2] - X[1]) + (Y[2] - Y[1]) * (Y[2] - Y[1]);
                     const double l2 = (X[0] - X[2]) * (X[0] - X[2]) + (Y[0] - Y[2]) * (Y[0] - Y[2]);
                     const double l3 = (X[1] - X[0]) * (X[1] - X[0]) + (Y[1] - Y[0]) * (Y[1] - Y[0]);
                     const double l = l1 + l2 + l3;
-                    return kTwoSqrt3 * area / l;
+                    return quot(kTwoSqrt3 * area, l);
+                };
+                auto h_at = [&] {  // sm_h, from the same corners
+                    const double d1 = fabs(X[2] - X[1]) + fabs(Y[2] - Y[1]);
+                    const double d2 = fabs(X[0] - X[2]) + fabs(Y[0] - Y[2]);
+                    const double d3 = fabs(X[1] - X[0]) + fabs(Y[1] - Y[0]);
+                    return quot(fabs(area), d1 + d2 + d3);
                 };
                 // smallest of the group's v where ok (init where none is smaller;
                 // NaN never is), known to the whole group
@@ -430,8 +448,8 @@ k_sm_passes(SmSeq q) {
                     const double2 nb = xy[lane < np ? q.d.psup1[s0 + lane] - 1 : ip];
                     double xn = 0, yn = 0;
                     for (int v = 0; v < np; ++v) {
-                        xn = xn + __shfl(nb.x, v, 64);
-                        yn = yn + __shfl(nb.y, v, 64);
+                        xn = xn + lane_of(nb.x, v);
+                        yn = yn + lane_of(nb.y, v);
                     }
                     xn = xn / np;
                     yn = yn / np;
@@ -446,34 +464,45 @@ k_sm_passes(SmSeq q) {
                     }
                 } else {  // one node of an optimisation sweep (:54-63, :113-171)
                     if (lane == 0) atomicAnd(&marks[ip >> 5], ~(1u << (ip & 31)));
-                    double v = mu(x, y);
-                    double mu_min;
-                    int mi = worst(v, mu_min);  // the same in every group
+                    // The qualities v at x, y and those at x + delta and y + delta
+                    // (getG) in one evaluation: a group each
+                    const auto three = [&](double xo, double yo) {
+                        return mu(g == 1 ? xo + delta : xo, g == 2 ? yo + delta : yo);
+                    };
+                    double m = G < 32 ? three(x, y) : mu(x, y), mu_min;
+                    int mi = worst(m, mu_min);  // group 0's: its result counts
+                    mi = __builtin_amdgcn_readfirstlane(mi);
+                    mu_min = lane_of(mu_min, 0);
                     if (!(mu_min < kSmTolMetric)) continue;
                     for (int it = 0; it < kSmSteps; ++it) {
                         const double xo = x, yo = y;
+                        double v, vx, vy, h;
+                        if (G < 32) {
+                            if (it > 0) m = three(xo, yo);
+                            h = h_at();
+                            v = __shfl(m, k, 64);
+                            vx = __shfl(m, G + k, 64);
+                            vy = __shfl(m, 2 * G + k, 64);
+                        } else {
+                            v = it > 0 ? mu(xo, yo) : m;
+                            h = h_at();
+                            vx = mu(xo + delta, yo);
+                            vy = mu(xo, yo + delta);
+                        }
                         // getG
-                        const double gx = (mu(xo + delta, yo) - v) / delta;
-                        const double gy = (mu(xo, yo + delta) - v) / delta;
+                        const double gx = quot(vx - v, by_delta), gy = quot(vy - v, by_delta);
                         const double gxm = lane_of(gx, mi), gym = lane_of(gy, mi);
                         const double g2 = gxm * gxm + gym * gym;
                         // getStep
                         double step;
                         if (q.d.tol_move) {
                             step = q.d.tol_move[ip] / ((fabs(gxm) + fabs(gym)) * (double)kSmSweeps);
-                        } else {
-                            double X[3], Y[3];
-                            corners(xo, yo, X, Y);
-                            const double area = X[1] * Y[2] + X[2] * Y[0] + X[0] * Y[1] -
-                                                (X[1] * Y[0] + X[2] * Y[1] + X[0] * Y[2]);
-                            const double d1 = fabs(X[2] - X[1]) + fabs(Y[2] - Y[1]);
-                            const double d2 = fabs(X[0] - X[2]) + fabs(Y[0] - Y[2]);
-                            const double d3 = fabs(X[1] - X[0]) + fabs(Y[1] - Y[0]);
-                            const double h = group_min(fabs(area) / (d1 + d2 + d3), act, 1.0);
-                            step = h * kSmStep / (fabs(gxm) + fabs(gym));
+                        } else {  // group 0's h
+                            h = lane_of(group_min(h, act, 1.0), 0);
+                            step = quot(h * kSmStep, fabs(gxm) + fabs(gym));
                         }
                         const double gg = gxm * gx + gym * gy;
-                        step = group_min((v - mu_min) / (g2 - gg), act && gg < 0, step);
+                        step = group_min(quot(v - mu_min, g2 - gg), act && gg < 0, step);
                         // the tries, a group each, in batches of 64 / G
                         bool accepted = false;
                         for (int t0 = 0; t0 < kSmTries && !accepted; t0 += 64 / G) {
@@ -496,7 +525,6 @@ k_sm_passes(SmSeq q) {
                             x = lane_of(xs, sel * G);
                             y = lane_of(ys, sel * G);
                             if (ok) {
-                                v = __shfl(nv, sel * G + k, 64);
                                 mi = __builtin_amdgcn_readlane(
                                     nmi, __builtin_amdgcn_readfirstlane(sel * G));
                                 mu_min = lane_of(best, sel * G);
@@ -515,22 +543,41 @@ k_sm_passes(SmSeq q) {
                     if (d_move > __DBL_MIN__ && act && g == 0)  // update_list (:289-298)
 #pragma unroll
                         for (int u = 0; u < 3; ++u)
-                            if (id[u] != ip) atomicOr(&marks[id[u] >> 5], 1u << (id[u] & 31));
+                            if (id[u] != ip)
+                                atomicOr(&(id[u] > ip ? marks : out_row)[id[u] >> 5],
+                                         1u << (id[u] & 31));
                 }
                 if (lane == 0) xy[ip] = make_double2(x, y);
-                __threadfence_block();  // the wave's other lanes and the next pass read it
+                // the wave's other lanes read it: LDS takes a wave's accesses in order
+                if (kLds) asm volatile("" ::: "memory");
+                else __threadfence_block();
             }
-            if (in) q.hist[(size_t)w * n + node] = xy[node];
-            __threadfence_block();
-            if (lane == 0) prog[w] = min(c0 + 64, n);
+            if (kLds && in) own_hist[node] = xy[node];
+            __threadfence();
+            if (lane == 0)
+                __hip_atomic_store(&q.prog[w], min(c0 + 64, n), __ATOMIC_RELEASE,
+                                   __HIP_MEMORY_SCOPE_AGENT);
         }
         if (lane == 0) q.dmax[w] = d_max;
     }
-    __syncthreads();
-    if (kLds)
-        for (int i = threadIdx.x; i < n; i += blockDim.x) q.xy[i] = xy[i];
-    for (int i = threadIdx.x; i < n; i += blockDim.x)
-        q.d.smoothable[i] = (marks[i >> 5] >> (i & 31)) & 1u;
+}
+
+// Before a launch: the first sweep's marks (of the check, or what row `last`
+// was left), empty rows behind them, the free nodes, no pass begun.  A thread
+// per word.
+__global__ void k_sm_rows(const int* __restrict__ smoothable, const int* __restrict__ fixed,
+                          unsigned* __restrict__ rows, int* __restrict__ prog, int n, int last) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x, nw = sm_words(n);
+    if (i < kSmPasses) prog[i] = 0;
+    if (i >= nw) return;
+    unsigned m = 0, f = 0;
+    for (int b = 0; b < 32 && 32 * i + b < n; ++b) {
+        if (smoothable[32 * i + b]) m |= 1u << b;
+        if (!fixed[32 * i + b]) f |= 1u << b;
+    }
+    rows[i] = last > 0 ? rows[(size_t)last * nw + i] : m;
+    for (int r = 1; r <= kSmPasses; ++r) rows[(size_t)r * nw + i] = 0;
+    rows[(size_t)(kSmPasses + 1) * nw + i] = f;
 }
 
 // per node: its ring (the nodes of its elements, in esup order) and how far the
@@ -660,20 +707,21 @@ bool smooth_check(const Tables& t, SmoothPlan& plan, double* X, double* Y, doubl
 
 // order 0 (see k_sm_passes)
 static int smooth_run_seq(const Tables& t, SmoothPlan& plan, const SmDev& d, hipStream_t s) {
-    const int n = t.npoin;
+    const int n = t.npoin, nw = sm_words(n);
     if (plan.ring.n != 9 * (size_t)t.nelem) {  // kept with the mesh's plan
         plan.ring.alloc(9 * (size_t)t.nelem);
         plan.need.alloc(n);
         plan.xy.alloc(n);
-        plan.hist.alloc((size_t)kSmWaves * n);
-        plan.dmax_pass.alloc(kSmWaves);
+        plan.hist.alloc((size_t)kSmPasses * n);
+        plan.dmax_pass.alloc(kSmPasses);
+        plan.rows.alloc((size_t)(kSmPasses + 2) * nw);
+        plan.prog.alloc(kSmPasses);
     }
     k_sm_ring<<<grid_for(n), kBlock, 0, s>>>(t.inpoel.p, t.esup1.p, t.esup2.p, plan.ring.p,
                                              plan.need.p, n);
     k_sm_pack<<<grid_for(n), kBlock, 0, s>>>(d.X, d.Y, plan.xy.p, n);
     // the positions in LDS while they fit (9,600 nodes in 160 KB)
-    const size_t base = (size_t)((n + 63) / 64 * 2) * 2 * sizeof(unsigned) + kSmWaves * sizeof(int);
-    const size_t full = base + (size_t)n * sizeof(double2);
+    const size_t base = (size_t)nw * sizeof(unsigned), full = base + (size_t)n * sizeof(double2);
     int dev = 0, most = 0;
     CFD_HIP(hipGetDevice(&dev));
     CFD_HIP(hipDeviceGetAttribute(&most, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
@@ -683,18 +731,23 @@ static int smooth_run_seq(const Tables& t, SmoothPlan& plan, const SmDev& d, hip
                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)full));
     const double tol_dist = kSmTolDist * plan.hmin;
     const double2* result = plan.xy.p;
-    int sweep = 0, nlap = 2;
+    int sweep = 0, nlap = 2, last = 0;
     for (bool end = false; !end && sweep < kSmSweeps; nlap = 0) {
-        const int nsw = std::min(kSmWaves - nlap, kSmSweeps - sweep);
-        const SmSeq q{d, plan.ring.p, plan.need.p, plan.xy.p, plan.hist.p, plan.dmax_pass.p, n,
-                      nlap + nsw, nlap};
-        if (lds) k_sm_passes<true><<<1, 64 * kSmWaves, full, s>>>(q);
-        else k_sm_passes<false><<<1, 64 * kSmWaves, base, s>>>(q);
+        const int nsw = std::min(kSmPasses - nlap, kSmSweeps - sweep), np = nlap + nsw;
+        if (last > 0)  // the next passes start from the last one's positions
+            CFD_HIP(hipMemcpyAsync(plan.xy.p, result, sizeof(double2) * n, hipMemcpyDeviceToDevice, s));
+        k_sm_rows<<<grid_for(std::max(nw, kSmPasses)), kBlock, 0, s>>>(
+            plan.smoothable.p, plan.fixed.p, plan.rows.p, plan.prog.p, n, last);
+        const SmSeq q{d, plan.ring.p, plan.need.p, plan.xy.p, plan.hist.p, plan.rows.p,
+                      plan.prog.p, plan.dmax_pass.p, n, np, nlap};
+        if (lds) k_sm_passes<true><<<np, 64, full, s>>>(q);
+        else k_sm_passes<false><<<np, 64, base, s>>>(q);
         CFD_HIP(hipGetLastError());
-        double dmax[kSmWaves];
+        last = np;
+        double dmax[kSmPasses];
         CFD_HIP(hipMemcpyAsync(dmax, plan.dmax_pass.p, sizeof(dmax), hipMemcpyDeviceToHost, s));
         CFD_HIP(hipStreamSynchronize(s));
-        for (int k = nlap; k < nlap + nsw && !end; ++k) {
+        for (int k = nlap; k < np && !end; ++k) {
             ++sweep;
             end = dmax[k] < tol_dist;
             result = plan.hist.p + (size_t)k * n;

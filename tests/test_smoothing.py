@@ -360,7 +360,7 @@ def _renumbered(m, seed):
     (90, 120, False),       # 10,800 nodes: positions in global memory
 ])
 def test_reference_order_waves_bitwise(nr, nt, shuffle):
-    """Order 0's passes run side by side in one block: the chunks' edges, both
+    """Order 0's passes run side by side, a block each: the chunks' edges, both
     places of the positions, and a numbering in which every node waits for far
     ones, bit for bit against the sequential oracle, with the sweep count."""
     from cfd_amd.api import MeshContext
