@@ -27,7 +27,7 @@
 //             the next passes, on other CUs, follow behind (k_sm_passes);
 //   order 1 - colour by colour: a greedy colouring of the node graph (no two
 //             nodes of one colour share an element, so nodes of a colour read
-//             and write disjoint data), one lane per node, colours in
+//             and write disjoint data), side by side, colours in
 //             sequence.  The same per-node updates in another order: a
 //             different, equally admissible smoothing (every accepted move
 //             still raises the node's worst element).
@@ -41,7 +41,6 @@ namespace cfd {
 
 namespace {
 
-constexpr int kSmMaxE = 20;          // MAX_ELEM_PER_NODE (smoothing.f90:6)
 constexpr int kSmSweeps = 100;       // NITER
 constexpr int kSmSteps = 2;          // MITER
 constexpr int kSmTries = 8;          // NTRY
@@ -85,38 +84,12 @@ __device__ inline double sm_h(const SmDev& d, int e) {
     return fabs(area) / dd;
 }
 
-// getMu_vec (smoothing.f90:174-197): the qualities of node ip's elements in
-// esup order; *min_idx (0-based here) the first strict minimum below 1
-__device__ inline int sm_mu_vec(const SmDev& d, int ip, double* v, int* min_idx) {
-    const int b = d.esup2[ip - 1], cnt = d.esup2[ip] - b;
-    double mu_min = 1;
-    if (min_idx) *min_idx = 0;
-    for (int k = 0; k < cnt; ++k) {
-        const double mu1 = sm_mu(d, d.esup1[b + k] - 1);
-        v[k] = mu1;
-        if (min_idx && mu1 < mu_min) {
-            mu_min = mu1;
-            *min_idx = k;
-        }
-    }
-    return cnt;
-}
-
-// getMu_min (:199-215) and getH_min (:272-287)
+// getMu_min (:199-215)
 __device__ inline double sm_mu_min(const SmDev& d, int ip) {
     double m = 1;
     for (int s = d.esup2[ip - 1]; s < d.esup2[ip]; ++s) {
         const double mu1 = sm_mu(d, d.esup1[s] - 1);
         if (mu1 <= m) m = mu1;
-    }
-    return m;
-}
-
-__device__ inline double sm_h_min(const SmDev& d, int ip) {
-    double m = 1;
-    for (int s = d.esup2[ip - 1]; s < d.esup2[ip]; ++s) {
-        const double h1 = sm_h(d, d.esup1[s] - 1);
-        if (h1 < m) m = h1;
     }
     return m;
 }
@@ -149,78 +122,6 @@ __device__ void sm_laplacian_node(const SmDev& d, int ip) {
     }
 }
 
-// moveIpoin (:113-171) with getG (:217-236) and getStep (:238-270); returns
-// the squared distance moved.  The tries accumulate: a failed try is not
-// undone before the next, half as long, is added.
-__device__ double sm_move_node(const SmDev& d, int ip, double* mu_vec, int min_idx) {
-    double gx[kSmMaxE], gy[kSmMaxE];
-    const double x0 = d.X[ip - 1], y0 = d.Y[ip - 1];
-    const int cnt = d.esup2[ip] - d.esup2[ip - 1];
-    const double delta = *d.hmin * kSmDelta;
-    for (int it = 0; it < kSmSteps; ++it) {
-        const double mu_min = mu_vec[min_idx];
-        const double xo = d.X[ip - 1], yo = d.Y[ip - 1];
-        // getG: one-sided differences of every element's quality
-        d.X[ip - 1] = d.X[ip - 1] + delta;
-        sm_mu_vec(d, ip, gx, nullptr);
-        for (int k = 0; k < cnt; ++k) gx[k] = (gx[k] - mu_vec[k]) / delta;
-        d.X[ip - 1] = xo;
-        d.Y[ip - 1] = d.Y[ip - 1] + delta;
-        sm_mu_vec(d, ip, gy, nullptr);
-        for (int k = 0; k < cnt; ++k) gy[k] = (gy[k] - mu_vec[k]) / delta;
-        d.Y[ip - 1] = yo;
-        // getStep: the largest step along the worst element's gradient before
-        // another element's linearised quality falls to the worst one's
-        const double gxm = gx[min_idx], gym = gy[min_idx];
-        const double g2 = gxm * gxm + gym * gym;
-        double step = d.tol_move ? d.tol_move[ip - 1] / ((fabs(gxm) + fabs(gym)) * (double)kSmSweeps)
-                                 : sm_h_min(d, ip) * kSmStep / (fabs(gxm) + fabs(gym));
-        for (int i = 0; i < cnt; ++i) {
-            const double gg = gxm * gx[i] + gym * gy[i];
-            if (gg < 0) {
-                const double step1 = (mu_vec[i] - mu_min) / (g2 - gg);
-                if (step1 < step) step = step1;
-            }
-        }
-        bool accepted = false;
-        for (int j = 0; j < kSmTries; ++j) {
-            const double dx = step * gxm, dy = step * gym;
-            d.X[ip - 1] = d.X[ip - 1] + dx;
-            d.Y[ip - 1] = d.Y[ip - 1] + dy;
-            int mi;
-            sm_mu_vec(d, ip, mu_vec, &mi);
-            if (mu_vec[mi] > mu_min * kSmPlus) {
-                min_idx = mi;
-                accepted = true;
-                break;
-            }
-            step = .5 * step;
-        }
-        if (!accepted) {  // restore and stop
-            d.X[ip - 1] = xo;
-            d.Y[ip - 1] = yo;
-            break;
-        }
-    }
-    const double ex = d.X[ip - 1] - x0, ey = d.Y[ip - 1] - y0;
-    const double d_move = ex * ex + ey * ey;
-    if (d_move > __DBL_MIN__)  // update_list (:289-298): the neighbours again
-        for (int s = d.psup2[ip - 1]; s < d.psup2[ip]; ++s) d.smoothable[d.psup1[s] - 1] = 1;
-    return d_move;
-}
-
-// One node of an optimisation sweep (smoothing.f90:54-63); returns the
-// squared move, 0 when the node was not moved
-__device__ double sm_sweep_node(const SmDev& d, int ip) {
-    if (!(d.smoothable[ip - 1] && !d.fixed[ip - 1])) return 0.0;
-    d.smoothable[ip - 1] = 0;
-    double mu_vec[kSmMaxE];
-    int mi;
-    sm_mu_vec(d, ip, mu_vec, &mi);
-    if (mu_vec[mi] < kSmTolMetric) return sm_move_node(d, ip, mu_vec, mi);
-    return 0.0;
-}
-
 // checkMesh (:367-385): smoothable marks and per-block partials of min h
 // and of "some element below 0.85"
 __global__ void __launch_bounds__(kBlock)
@@ -250,6 +151,203 @@ k_sm_check_fin(const double* __restrict__ hpart, const double* __restrict__ anyp
         out[1] = a;
     }
 }
+
+// v of a lane that every lane names alike
+__device__ __forceinline__ double lane_of(double v, int lane) {
+    const int l = __builtin_amdgcn_readfirstlane(lane);
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l),
+                            __builtin_amdgcn_readlane(__double2loint(v), l));
+}
+// v of another lane of the row of 16 by the DPP control kCtrl (no LDS round trip)
+template <int kCtrl>
+__device__ __forceinline__ double dpp_of(double v) {
+    const int hi = __double2hiint(v), lo = __double2loint(v);
+    return __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, kCtrl, 0xf, 0xf, false),
+                            __builtin_amdgcn_update_dpp(lo, lo, kCtrl, 0xf, 0xf, false));
+}
+constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppHalfMirror = 0x141, kDppMirror = 0x140;
+
+// One node's update by a wave: lane k of each group of G lanes forms the node's
+// k-th element (esup order), the groups the tries and the three points of a
+// gradient.  pos(i) is node i's position (0-based).
+template <class Pos>
+struct SmNode {
+    const SmDev& d;
+    Pos pos;
+    int ip, id[3], G, k, g;  // the node; the lane's element; lanes a group, lane, group
+    bool act;                // the lane has an element
+    double2 own;
+    double cx[3], cy[3], X[3], Y[3], area;  // the element's corners; those of the last evaluation
+
+    static __device__ __forceinline__ int lanes(int cnt) { return cnt <= 8 ? 8 : cnt <= 16 ? 16 : 32; }
+    // ids: the nodes of the lane's element (0-based; read where it has one)
+    __device__ __forceinline__ SmNode(const SmDev& d, Pos pos, int ip, int cnt, const int (&ids)[3])
+        : d(d), pos(pos), ip(ip), G(lanes(cnt)) {
+        const int lane = threadIdx.x & 63;
+        k = lane & (G - 1);
+        g = lane / G;
+        act = k < cnt;
+#pragma unroll
+        for (int v = 0; v < 3; ++v) {
+            id[v] = act ? ids[v] : ip;
+            const double2 c = pos(id[v]);
+            cx[v] = c.x;
+            cy[v] = c.y;
+        }
+        own = pos(ip);
+    }
+    // quality (sm_mu) of the lane's element with the node at x, y
+    __device__ __forceinline__ double mu(double x, double y) {
+#pragma unroll
+        for (int v = 0; v < 3; ++v) {
+            X[v] = id[v] == ip ? x : cx[v];
+            Y[v] = id[v] == ip ? y : cy[v];
+        }
+        area = X[1] * Y[2] + X[2] * Y[0] + X[0] * Y[1] -
+               (X[1] * Y[0] + X[2] * Y[1] + X[0] * Y[2]);
+        const double l1 = (X[2] - X[1]) * (X[2] - X[1]) + (Y[2] - Y[1]) * (Y[2] - Y[1]);
+        const double l2 = (X[0] - X[2]) * (X[0] - X[2]) + (Y[0] - Y[2]) * (Y[0] - Y[2]);
+        const double l3 = (X[1] - X[0]) * (X[1] - X[0]) + (Y[1] - Y[0]) * (Y[1] - Y[0]);
+        const double l = l1 + l2 + l3;
+        return quot(kTwoSqrt3 * area, l);
+    }
+    // h (sm_h) at the corners of the last evaluation
+    __device__ __forceinline__ double h_at() const {
+        const double d1 = fabs(X[2] - X[1]) + fabs(Y[2] - Y[1]);
+        const double d2 = fabs(X[0] - X[2]) + fabs(Y[0] - Y[2]);
+        const double d3 = fabs(X[1] - X[0]) + fabs(Y[1] - Y[0]);
+        return quot(fabs(area), d1 + d2 + d3);
+    }
+    // smallest of the group's v where ok (init where none is smaller; NaN never
+    // is), known to the whole group
+    __device__ __forceinline__ double group_min(double v, bool ok, double init) const {
+        double m1 = ok && v < init ? v : init;
+        auto take = [&](double o) {
+            if (o < m1) m1 = o;
+        };
+        take(dpp_of<kDppXor1>(m1));
+        take(dpp_of<kDppXor2>(m1));
+        take(dpp_of<kDppHalfMirror>(m1));  // quads hold one value each
+        if (G > 8) take(dpp_of<kDppMirror>(m1));
+        if (G > 16) take(__shfl_xor(m1, 16, 64));
+        return m1;
+    }
+    // getMu_vec's min_idx (smoothing.f90:174-197): the first element with the
+    // smallest quality below 1 (element 0 when none is), and its quality
+    __device__ __forceinline__ int worst(double v, double& vm) const {
+        vm = group_min(v, act, 1.0);
+        const unsigned long long hit = __ballot(act && v < 1.0 && v == vm);
+        const unsigned long long mine = (hit >> (g * G)) & ((1ull << G) - 1ull);
+        if (__any(!mine)) {
+            const double v0 = __shfl(v, g * G, 64);
+            if (!mine) vm = v0;
+        }
+        return mine ? (int)__builtin_ctzll(mine) : 0;
+    }
+    // laplacianSmoothing (:77-111): the node's new position
+    __device__ __forceinline__ double2 laplacian() {
+        const double x = own.x, y = own.y;
+        const int lane = threadIdx.x & 63;
+        const double mu_old = group_min(mu(x, y), act, 1.0);
+        const int s0 = d.psup2[ip], np = d.psup2[ip + 1] - s0;
+        const double2 nb = pos(lane < np ? d.psup1[s0 + lane] - 1 : ip);
+        double xn = 0, yn = 0;
+        for (int v = 0; v < np; ++v) {
+            xn = xn + lane_of(nb.x, v);
+            yn = yn + lane_of(nb.y, v);
+        }
+        xn = xn / np;
+        yn = yn / np;
+        if (d.tol_move) {
+            const double dX = xn - x, dY = yn - y, tm = d.tol_move[ip];
+            xn = x + dX / (fabs(dX) + fabs(dY)) * tm / 2 * kSmStep;
+            yn = y + dY / (fabs(dX) + fabs(dY)) * tm / 2 * kSmStep;
+        }
+        if (group_min(mu(xn, yn), act, 1.0) < mu_old) return own;  // if worse, restored
+        return make_double2(xn, yn);
+    }
+    // One node of an optimisation sweep: moveIpoin (:113-171) with getG
+    // (:217-236) and getStep (:238-270).  False when its worst element is good
+    // enough (:54-63); else *to is where it goes.  The tries accumulate: a failed
+    // try is not undone before the next, half as long, is added.
+    __device__ __forceinline__ bool sweep(double delta, const Recip& by_delta, double2& to) {
+        double x = own.x, y = own.y;
+        // The qualities v at x, y and those at x + delta and y + delta (getG) in
+        // one evaluation: a group each
+        const auto three = [&](double xo, double yo) {
+            return mu(g == 1 ? xo + delta : xo, g == 2 ? yo + delta : yo);
+        };
+        double m = G < 32 ? three(x, y) : mu(x, y), mu_min;
+        int mi = worst(m, mu_min);  // group 0's: its result counts
+        mi = __builtin_amdgcn_readfirstlane(mi);
+        mu_min = lane_of(mu_min, 0);
+        if (!(mu_min < kSmTolMetric)) return false;
+        for (int it = 0; it < kSmSteps; ++it) {
+            const double xo = x, yo = y;
+            double v, vx, vy, h;
+            if (G < 32) {
+                if (it > 0) m = three(xo, yo);
+                h = h_at();
+                v = __shfl(m, k, 64);
+                vx = __shfl(m, G + k, 64);
+                vy = __shfl(m, 2 * G + k, 64);
+            } else {
+                v = it > 0 ? mu(xo, yo) : m;
+                h = h_at();
+                vx = mu(xo + delta, yo);
+                vy = mu(xo, yo + delta);
+            }
+            const double gx = quot(vx - v, by_delta), gy = quot(vy - v, by_delta);
+            // getStep: the largest step along the worst element's gradient before
+            // another element's linearised quality falls to the worst one's
+            const double gxm = lane_of(gx, mi), gym = lane_of(gy, mi);
+            const double g2 = gxm * gxm + gym * gym;
+            double step;
+            if (d.tol_move) {
+                step = d.tol_move[ip] / ((fabs(gxm) + fabs(gym)) * (double)kSmSweeps);
+            } else {  // group 0's h
+                h = lane_of(group_min(h, act, 1.0), 0);
+                step = quot(h * kSmStep, fabs(gxm) + fabs(gym));
+            }
+            const double gg = gxm * gx + gym * gy;
+            step = group_min(quot(v - mu_min, g2 - gg), act && gg < 0, step);
+            // the tries, a group each, in batches of 64 / G
+            bool accepted = false;
+            for (int t0 = 0; t0 < kSmTries && !accepted; t0 += 64 / G) {
+                double xs = x, ys = y;
+                for (int u = 0; u < 64 / G; ++u) {
+                    const double dx = step * gxm, dy = step * gym;
+                    if (u <= g) {
+                        xs = xs + dx;
+                        ys = ys + dy;
+                    }
+                    step = .5 * step;
+                }
+                const double nv = mu(xs, ys);
+                double best;
+                const int nmi = worst(nv, best);
+                const unsigned long long ok = __ballot(best > mu_min * kSmPlus);
+                // the first group that raised the worst element, else the last
+                // try's position
+                const int sel = ok ? (int)__builtin_ctzll(ok) / G : 64 / G - 1;
+                x = lane_of(xs, sel * G);
+                y = lane_of(ys, sel * G);
+                if (ok) {
+                    mi = __builtin_amdgcn_readlane(nmi, __builtin_amdgcn_readfirstlane(sel * G));
+                    mu_min = lane_of(best, sel * G);
+                    accepted = true;
+                }
+            }
+            if (!accepted) {  // restore and stop
+                x = xo;
+                y = yo;
+                break;
+            }
+        }
+        to = make_double2(x, y);
+        return true;
+    }
+};
 
 // ---------------------------------------------------------------------------
 // order 0: up to kSmPasses consecutive passes in one launch, a block of one wave
@@ -281,7 +379,7 @@ k_sm_check_fin(const double* __restrict__ hpart, const double* __restrict__ anyp
 // Bound by the chain of one node's update (3 us: about 700 instructions with
 // the lanes' exchanges and eight divisions in sequence), node after node, on
 // one wave; the positions stay in LDS while they fit.  64 x 128 cylinder (8,192
-// nodes, 2 + 8 passes): 29.5 ms; 42.7 with the passes as twelve waves of one
+// nodes, 2 + 8 passes): 28.7 ms; 42.7 with the passes as twelve waves of one
 // block (three to a SIMD share its instructions), 1,524 with one lane per pass
 // and the passes one by one.
 // ---------------------------------------------------------------------------
@@ -300,21 +398,6 @@ struct SmSeq {
     int n, npass, nlap;    // passes of the launch, Laplacian ones first
 };
 __host__ __device__ constexpr int sm_words(int n) { return (n + 63) / 64 * 2; }
-
-// v of a lane that every lane names alike
-__device__ __forceinline__ double lane_of(double v, int lane) {
-    const int l = __builtin_amdgcn_readfirstlane(lane);
-    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l),
-                            __builtin_amdgcn_readlane(__double2loint(v), l));
-}
-// v of another lane of the row of 16 by the DPP control kCtrl (no LDS round trip)
-template <int kCtrl>
-__device__ __forceinline__ double dpp_of(double v) {
-    const int hi = __double2hiint(v), lo = __double2loint(v);
-    return __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, kCtrl, 0xf, 0xf, false),
-                            __builtin_amdgcn_update_dpp(lo, lo, kCtrl, 0xf, 0xf, false));
-}
-constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppHalfMirror = 0x141, kDppMirror = 0x140;
 
 template <bool kLds>
 __global__ void __launch_bounds__(64)
@@ -366,188 +449,40 @@ k_sm_passes(SmSeq q) {
                 const int ip = c0 + j;
                 const int b = __builtin_amdgcn_readlane(b_l, j);
                 const int cnt = __builtin_amdgcn_readlane(e_l, j) - b;
-                const int G = cnt <= 8 ? 8 : cnt <= 16 ? 16 : 32;  // lanes per group
-                const int k = lane & (G - 1), g = lane / G;
-                const bool act = k < cnt;
+                const auto at = [xy](int i) { return xy[i]; };
+                const int G = SmNode<decltype(at)>::lanes(cnt), k = lane & (G - 1);
                 int id[3] = {ip, ip, ip};
-                if (act)
+                if (k < cnt)
+#pragma unroll
                     for (int v = 0; v < 3; ++v)
                         id[v] = next == j ? nid[v] : q.ring[3 * (b + k) + v];
+                SmNode<decltype(at)> node_(q.d, at, ip, cnt, id);
                 if (j < 63) {  // most nodes marked: the next one's entries, in flight meanwhile
                     next = j + 1;
                     const int b1 = __builtin_amdgcn_readlane(b_l, next);
-                    const int k1 = lane & ((__builtin_amdgcn_readlane(e_l, next) - b1 <= 8    ? 8
-                                            : __builtin_amdgcn_readlane(e_l, next) - b1 <= 16 ? 16
-                                                                                              : 32) - 1);
-                    if (b1 + k1 < __builtin_amdgcn_readlane(e_l, next))
+                    const int e1 = __builtin_amdgcn_readlane(e_l, next);
+                    const int k1 = lane & (SmNode<decltype(at)>::lanes(e1 - b1) - 1);
+                    if (b1 + k1 < e1)
                         for (int v = 0; v < 3; ++v) nid[v] = q.ring[3 * (b1 + k1) + v];
                 }
-                double cx[3], cy[3];
-#pragma unroll
-                for (int v = 0; v < 3; ++v) {
-                    const double2 c = xy[id[v]];
-                    cx[v] = c.x;
-                    cy[v] = c.y;
-                }
-                const double2 own = xy[ip];
-                // quality (sm_mu) and h (sm_h) of the lane's element with the node at x, y
-                auto corners = [&](double x, double y, double (&X)[3], double (&Y)[3]) {
-#pragma unroll
-                    for (int v = 0; v < 3; ++v) {
-                        X[v] = id[v] == ip ? x : cx[v];
-                        Y[v] = id[v] == ip ? y : cy[v];
-                    }
-                };
-                double X[3], Y[3], area;  // of the last evaluation
-                auto mu = [&](double x, double y) {
-                    corners(x, y, X, Y);
-                    area = X[1] * Y[2] + X[2] * Y[0] + X[0] * Y[1] -
-                                        (X[1] * Y[0] + X[2] * Y[1] + X[0] * Y[2]);
-                    const double l1 = (X[2] - X[1]) * (X[2] - X[1]) + (Y[2] - Y[1]) * (Y[2] - Y[1]);
-                    const double l2 = (X[0] - X[2]) * (X[0] - X[2]) + (Y[0] - Y[2]) * (Y[0] - Y[2]);
-                    const double l3 = (X[1] - X[0]) * (X[1] - X[0]) + (Y[1] - Y[0]) * (Y[1] - Y[0]);
-                    const double l = l1 + l2 + l3;
-                    return quot(kTwoSqrt3 * area, l);
-                };
-                auto h_at = [&] {  // sm_h, from the same corners
-                    const double d1 = fabs(X[2] - X[1]) + fabs(Y[2] - Y[1]);
-                    const double d2 = fabs(X[0] - X[2]) + fabs(Y[0] - Y[2]);
-                    const double d3 = fabs(X[1] - X[0]) + fabs(Y[1] - Y[0]);
-                    return quot(fabs(area), d1 + d2 + d3);
-                };
-                // smallest of the group's v where ok (init where none is smaller;
-                // NaN never is), known to the whole group
-                auto group_min = [&](double v, bool ok, double init) {
-                    double m1 = ok && v < init ? v : init;
-                    auto take = [&](double o) {
-                        if (o < m1) m1 = o;
-                    };
-                    take(dpp_of<kDppXor1>(m1));
-                    take(dpp_of<kDppXor2>(m1));
-                    take(dpp_of<kDppHalfMirror>(m1));  // quads hold one value each
-                    if (G > 8) take(dpp_of<kDppMirror>(m1));
-                    if (G > 16) take(__shfl_xor(m1, 16, 64));
-                    return m1;
-                };
-                // getMu_vec's min_idx: the first element with the smallest quality
-                // below 1 (element 0 when none is), and its quality
-                auto worst = [&](double v, double& vm) {
-                    vm = group_min(v, act, 1.0);
-                    const unsigned long long hit = __ballot(act && v < 1.0 && v == vm);
-                    const unsigned long long mine = (hit >> (g * G)) & ((1ull << G) - 1ull);
-                    if (__any(!mine)) {
-                        const double v0 = __shfl(v, g * G, 64);
-                        if (!mine) vm = v0;
-                    }
-                    return mine ? (int)__builtin_ctzll(mine) : 0;
-                };
-                double x = own.x, y = own.y;
-                if (lap) {  // laplacianSmoothing (:77-111)
-                    const double mu_old = group_min(mu(x, y), act, 1.0);
-                    const int s0 = q.d.psup2[ip], np = q.d.psup2[ip + 1] - s0;
-                    const double2 nb = xy[lane < np ? q.d.psup1[s0 + lane] - 1 : ip];
-                    double xn = 0, yn = 0;
-                    for (int v = 0; v < np; ++v) {
-                        xn = xn + lane_of(nb.x, v);
-                        yn = yn + lane_of(nb.y, v);
-                    }
-                    xn = xn / np;
-                    yn = yn / np;
-                    if (q.d.tol_move) {
-                        const double dX = xn - x, dY = yn - y, tm = q.d.tol_move[ip];
-                        xn = x + dX / (fabs(dX) + fabs(dY)) * tm / 2 * kSmStep;
-                        yn = y + dY / (fabs(dX) + fabs(dY)) * tm / 2 * kSmStep;
-                    }
-                    if (!(group_min(mu(xn, yn), act, 1.0) < mu_old)) {  // else restored
-                        x = xn;
-                        y = yn;
-                    }
-                } else {  // one node of an optimisation sweep (:54-63, :113-171)
+                double2 to;
+                if (lap) {
+                    to = node_.laplacian();
+                } else {
                     if (lane == 0) atomicAnd(&marks[ip >> 5], ~(1u << (ip & 31)));
-                    // The qualities v at x, y and those at x + delta and y + delta
-                    // (getG) in one evaluation: a group each
-                    const auto three = [&](double xo, double yo) {
-                        return mu(g == 1 ? xo + delta : xo, g == 2 ? yo + delta : yo);
-                    };
-                    double m = G < 32 ? three(x, y) : mu(x, y), mu_min;
-                    int mi = worst(m, mu_min);  // group 0's: its result counts
-                    mi = __builtin_amdgcn_readfirstlane(mi);
-                    mu_min = lane_of(mu_min, 0);
-                    if (!(mu_min < kSmTolMetric)) continue;
-                    for (int it = 0; it < kSmSteps; ++it) {
-                        const double xo = x, yo = y;
-                        double v, vx, vy, h;
-                        if (G < 32) {
-                            if (it > 0) m = three(xo, yo);
-                            h = h_at();
-                            v = __shfl(m, k, 64);
-                            vx = __shfl(m, G + k, 64);
-                            vy = __shfl(m, 2 * G + k, 64);
-                        } else {
-                            v = it > 0 ? mu(xo, yo) : m;
-                            h = h_at();
-                            vx = mu(xo + delta, yo);
-                            vy = mu(xo, yo + delta);
-                        }
-                        // getG
-                        const double gx = quot(vx - v, by_delta), gy = quot(vy - v, by_delta);
-                        const double gxm = lane_of(gx, mi), gym = lane_of(gy, mi);
-                        const double g2 = gxm * gxm + gym * gym;
-                        // getStep
-                        double step;
-                        if (q.d.tol_move) {
-                            step = q.d.tol_move[ip] / ((fabs(gxm) + fabs(gym)) * (double)kSmSweeps);
-                        } else {  // group 0's h
-                            h = lane_of(group_min(h, act, 1.0), 0);
-                            step = quot(h * kSmStep, fabs(gxm) + fabs(gym));
-                        }
-                        const double gg = gxm * gx + gym * gy;
-                        step = group_min(quot(v - mu_min, g2 - gg), act && gg < 0, step);
-                        // the tries, a group each, in batches of 64 / G
-                        bool accepted = false;
-                        for (int t0 = 0; t0 < kSmTries && !accepted; t0 += 64 / G) {
-                            double xs = x, ys = y;
-                            for (int u = 0; u < 64 / G; ++u) {
-                                const double dx = step * gxm, dy = step * gym;
-                                if (u <= g) {
-                                    xs = xs + dx;
-                                    ys = ys + dy;
-                                }
-                                step = .5 * step;
-                            }
-                            const double nv = mu(xs, ys);
-                            double best;
-                            const int nmi = worst(nv, best);
-                            const unsigned long long ok = __ballot(best > mu_min * kSmPlus);
-                            // the first group that raised the worst element, else the
-                            // last try's position (the tries accumulate)
-                            const int sel = ok ? (int)__builtin_ctzll(ok) / G : 64 / G - 1;
-                            x = lane_of(xs, sel * G);
-                            y = lane_of(ys, sel * G);
-                            if (ok) {
-                                mi = __builtin_amdgcn_readlane(
-                                    nmi, __builtin_amdgcn_readfirstlane(sel * G));
-                                mu_min = lane_of(best, sel * G);
-                                accepted = true;
-                            }
-                        }
-                        if (!accepted) {  // restore and stop
-                            x = xo;
-                            y = yo;
-                            break;
-                        }
-                    }
-                    const double ex = x - own.x, ey = y - own.y;
+                    if (!node_.sweep(delta, by_delta, to)) continue;
+                    const double ex = to.x - node_.own.x, ey = to.y - node_.own.y;
                     const double d_move = ex * ex + ey * ey;
                     if (d_move > d_max) d_max = d_move;
-                    if (d_move > __DBL_MIN__ && act && g == 0)  // update_list (:289-298)
+                    if (d_move > __DBL_MIN__ && node_.act && node_.g == 0)  // update_list (:289-298)
 #pragma unroll
-                        for (int u = 0; u < 3; ++u)
-                            if (id[u] != ip)
-                                atomicOr(&(id[u] > ip ? marks : out_row)[id[u] >> 5],
-                                         1u << (id[u] & 31));
+                        for (int u = 0; u < 3; ++u) {
+                            const int m = node_.id[u];
+                            if (m != ip)
+                                atomicOr(&(m > ip ? marks : out_row)[m >> 5], 1u << (m & 31));
+                        }
                 }
-                if (lane == 0) xy[ip] = make_double2(x, y);
+                if (lane == 0) xy[ip] = to;
                 // the wave's other lanes read it: LDS takes a wave's accesses in order
                 if (kLds) asm volatile("" ::: "memory");
                 else __threadfence_block();
@@ -611,20 +546,50 @@ __global__ void k_sm_unpack(const double2* __restrict__ xy, double* __restrict__
     Y[i] = xy[i].y;
 }
 
-// order 1: one lane per node of a colour
+// order 1, the Laplacian passes: one lane per node of a colour (12 us a colour of
+// 13,000 nodes; a wave per node takes 22: most of it loads of one position a
+// lane)
 __global__ void __launch_bounds__(kBlock)
 k_sm_laplacian_colour(SmDev d, const int* __restrict__ nodes, int count) {
     const int q = blockIdx.x * blockDim.x + threadIdx.x;
     if (q < count) sm_laplacian_node(d, nodes[q]);
 }
 
-__global__ void __launch_bounds__(kBlock)
-k_sm_sweep_colour(SmDev d, const int* __restrict__ nodes, int count,
-                  double* __restrict__ dmove) {
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q < count) {
-        const int ip = nodes[q];
-        dmove[ip - 1] = sm_sweep_node(d, ip);
+// order 1, a sweep: one wave per node of a colour, four a block.  A colour of
+// 13,000 nodes takes 19 us; with one lane per node, which keeps its elements'
+// qualities and gradients in scratch memory and tries one position after the
+// other, 52.
+constexpr int kColourWaves = 4;
+__global__ void __launch_bounds__(64 * kColourWaves)
+k_sm_sweep_colour(SmDev d, const int* __restrict__ nodes, int count, double* __restrict__ dmove) {
+    const int q = __builtin_amdgcn_readfirstlane(blockIdx.x * kColourWaves + (threadIdx.x >> 6));
+    if (q >= count) return;
+    const int lane = threadIdx.x & 63, ip = nodes[q] - 1;
+    if (!(d.smoothable[ip] && !d.fixed[ip])) return;
+    const int b = d.esup2[ip];
+    const auto at = [&d](int i) { return make_double2(d.X[i], d.Y[i]); };
+    const int cnt = d.esup2[ip + 1] - b, k = lane & (SmNode<decltype(at)>::lanes(cnt) - 1);
+    int id[3] = {ip, ip, ip};
+    if (k < cnt) {
+        const int* n = d.inpoel + 3 * (d.esup1[b + k] - 1);
+#pragma unroll
+        for (int v = 0; v < 3; ++v) id[v] = n[v] - 1;
+    }
+    SmNode<decltype(at)> node(d, at, ip, cnt, id);
+    if (lane == 0) d.smoothable[ip] = 0;
+    const double delta = *d.hmin * kSmDelta;
+    double2 to;
+    if (!node.sweep(delta, recip(delta), to)) return;
+    const double ex = to.x - node.own.x, ey = to.y - node.own.y;
+    const double d_move = ex * ex + ey * ey;
+    if (d_move > __DBL_MIN__ && node.act && node.g == 0)  // update_list (:289-298)
+#pragma unroll
+        for (int u = 0; u < 3; ++u)
+            if (node.id[u] != ip) d.smoothable[node.id[u]] = 1;
+    if (lane == 0) {
+        dmove[ip] = d_move;
+        d.X[ip] = to.x;
+        d.Y[ip] = to.y;
     }
 }
 
@@ -783,7 +748,8 @@ int smooth_run(const Tables& t, SmoothPlan& plan, double* X, double* Y, const do
     for (; sweep <= kSmSweeps; ++sweep) {
         plan.dmove.zero(s);
         colour_pass([&](const int* nodes, int cnt) {
-            k_sm_sweep_colour<<<grid_for(cnt), kBlock, 0, s>>>(d, nodes, cnt, plan.dmove.p);
+            k_sm_sweep_colour<<<(cnt + kColourWaves - 1) / kColourWaves, 64 * kColourWaves, 0, s>>>(
+                d, nodes, cnt, plan.dmove.p);
         });
         k_sm_max<<<nbm, kBlock, 0, s>>>(plan.dmove.p, n, plan.partials.p);
         k_sm_max_fin<<<1, 256, 0, s>>>(plan.partials.p, nbm, plan.scal.p + 2);
