@@ -272,7 +272,8 @@ typedef struct {
                                 patch, 1..682 within the kernel's 64 KB of
                                 LDS (0: 512 FP32, 384 FP64)                   */
     int patch_block;         /* threads per patch, a multiple of 64 up to 512
-                                (0: 256)                                     */
+                                (0: 256, or one per element where there are
+                                few patches)                                 */
     int renumber;            /* fused paths (precision 0, 1):
                                 0: the session keeps the caller's numbering
                                 1: the session numbers nodes and elements in
