@@ -164,7 +164,9 @@ int cfd_laplace(cfd_mesh* m, const double* X, const double* Y, const double* dNx
         double* dny = m->put("dNy", dNy, 3 * (size_t)ne);
         double* lap = m->scratch("lap", m->t.nnz);
         double* diag = m->scratch("diag", np);
-        launch_laplace(m->t, dX, dY, dnx, dny, lap, diag, m->s);
+        double* w = m->scratch("lapw", ne);
+        launch_lap_weights(m->t, dX, dY, w, m->s);
+        launch_laplace(m->t, w, dnx, dny, lap, diag, m->s);
         m->get(lap_sparse, lap, m->t.nnz);
         m->get(lap_diag, diag, np);
         m->sync();
@@ -670,7 +672,8 @@ struct cfd_session {
     DBuf<double> Ub[2];
     int ucur = 0;
     DBuf<double> RHS, T, VX, VY, WX, WY, X, Y, X1, Y1, RHO, E, P, RMACH, M, GAMM, XPOS, YPOS;
-    DBuf<double> DTL, DT, SHOC, T1, T2, T3, AREA, DNX, DNY, HH, HHX, HHY, AREA_OLD, WXO, WYO;
+    DBuf<double> DTL, DT, SHOC, T1, T2, T3, AREA, DNX, DNY, HH, HHX, HHY, AREA_OLD, WXO, WYO, LAPW;
+    DBuf<double2> GCLT;  // the elements' terms of the GCL
     DBuf<double> LAP, LDIAG, c_calc, c_fuente, DXPOS, DYPOS, POSAUX, POSAUY, BZERO, partials;
     // fused paths: shape gradients and ESTAB outputs in patch order, binary32
     // (precision 1) or FP64 (precision 0)
@@ -768,11 +771,13 @@ struct cfd_session {
     void geometry() {  // NORMALES, DERIV, MASAS, laplace (ns2DComp.ALE.f90:88-100, 259-275)
         const Tables& t = m->t;
         bc.normales(X.p, Y.p, s);
+        ElemTerms x;
+        x.lapw = LAPW.p;
         launch_deriv(t, X.p, Y.p, AREA.p, DNX.p, DNY.p, HH.p, HHX.p, HHY.p, scal(CFD_S_HMIN),
-                     partials.p, s);
+                     partials.p, s, x);
         refresh_patch_geometry();
-        launch_masas(t, AREA.p, M.p, s);
-        launch_laplace(t, X.p, Y.p, DNX.p, DNY.p, LAP.p, LDIAG.p, s, ell_on ? &ell : nullptr);
+        launch_laplace(t, LAPW.p, DNX.p, DNY.p, LAP.p, LDIAG.p, s, ell_on ? &ell : nullptr,
+                       NodeMass{M.p, AREA.p, nullptr, nullptr});
     }
 
     // the fused paths' ESTAB outputs (patch order)
@@ -974,11 +979,11 @@ struct cfd_session {
             if (d.gcl >= 0) {
                 bc.normales(X.p, Y.p, s);
                 launch_deriv(t, X.p, Y.p, AREA.p, DNX.p, DNY.p, HH.p, HHX.p, HHY.p,
-                             scal(CFD_S_HMIN), partials.p, s, AREA_OLD.p);
+                             scal(CFD_S_HMIN), partials.p, s,
+                             ElemTerms{LAPW.p, GCLT.p, AREA_OLD.p, WX.p, WY.p, WXO.p, WYO.p, d.gcl});
                 refresh_patch_geometry();
-                launch_gcl(t, M.p, WX.p, WY.p, WXO.p, WYO.p, DNX.p, DNY.p, AREA.p, AREA_OLD.p, dtmin,
-                           d.gcl, s);
-                launch_laplace(t, X.p, Y.p, DNX.p, DNY.p, LAP.p, LDIAG.p, s, ell_on ? &ell : nullptr);
+                launch_laplace(t, LAPW.p, DNX.p, DNY.p, LAP.p, LDIAG.p, s, ell_on ? &ell : nullptr,
+                               NodeMass{M.p, nullptr, GCLT.p, dtmin});
             } else {
                 geometry();
             }
@@ -1189,8 +1194,9 @@ int cfd_session_create(cfd_session** out, cfd_mesh* m, const cfd_case_desc* d) {
                         &S->WYO, &S->LDIAG, &S->DXPOS, &S->DYPOS, &S->BZERO})
             b->alloc(np);
         for (auto* b : {&S->DTL, &S->DT, &S->SHOC, &S->T1, &S->T2, &S->T3, &S->AREA, &S->HH, &S->HHX,
-                        &S->HHY, &S->AREA_OLD})
+                        &S->HHY, &S->AREA_OLD, &S->LAPW})
             b->alloc(ne);
+        if (d->moving == 1 && d->gcl >= 0) S->GCLT.alloc(ne);
         S->DNX.alloc(3 * (size_t)ne);
         S->DNY.alloc(3 * (size_t)ne);
         S->LAP.alloc(m->t.nnz);

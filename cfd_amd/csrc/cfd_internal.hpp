@@ -180,19 +180,40 @@ struct Consts {
     double gama, fr, fmu, fk, fcv, t_inf, rho_inf, u_inf, v_inf, cte, fsafe;
 };
 
+// What deriv's pass leaves for the nodes' pass besides: each element's weight in
+// laplace (lapw), and (gcl given) its terms of the GCL from W and the old W,
+// mode as launch_gcl's, and the areas before (area_old)
+struct ElemTerms {
+    double* lapw = nullptr;
+    double2* gcl = nullptr;
+    double* area_old = nullptr;
+    const double *Wx = nullptr, *Wy = nullptr, *Wxo = nullptr, *Wyo = nullptr;
+    int mode = 0;
+};
 // deriv (subrutinas.f90:88-126); hmin_out: device double; partials holds
-// grid_for(nelem) doubles; area_old (when given) receives the areas before
+// grid_for(nelem) doubles
 void launch_deriv(const Tables& t, const double* X, const double* Y, double* area, double* dNx,
                   double* dNy, double* HH, double* HHX, double* HHY, double* hmin_out,
-                  double* partials, hipStream_t s, double* area_old = nullptr);
+                  double* partials, hipStream_t s, const ElemTerms& x = ElemTerms{});
 // MASAS (subrutinas.f90:128-153) as an ascending-element gather
 void launch_masas(const Tables& t, const double* area, double* M, hipStream_t s);
+// each element's weight in laplace, from the coordinates
+void launch_lap_weights(const Tables& t, const double* X, const double* Y, double* lapw,
+                        hipStream_t s);
+// The nodes' masses in laplace's pass: MASAS (area given), or the GCL's update
+// M += dt (sums of gcl) / 2 (gcl given; dt a device scalar)
+struct NodeMass {
+    double* M = nullptr;
+    const double* area = nullptr;
+    const double2* gcl = nullptr;
+    const double* dt = nullptr;
+};
 // mLaplace.f90:7-58 values (structure comes from Tables); ell (when given): the
 // ELL copy's values too (EllLap::refresh in the same pass)
 struct EllLap;
-void launch_laplace(const Tables& t, const double* X, const double* Y, const double* dNx,
-                    const double* dNy, double* lap, double* diag, hipStream_t s,
-                    EllLap* ell = nullptr);
+void launch_laplace(const Tables& t, const double* lapw, const double* dNx, const double* dNy,
+                    double* lap, double* diag, hipStream_t s, EllLap* ell = nullptr,
+                    const NodeMass& m = NodeMass{});
 // gcl.f90:8-46 main; mode 0 = as written, 1 = corrected y-divergence; dt is a
 // device scalar
 void launch_gcl(const Tables& t, double* M, const double* Wx, const double* Wy,

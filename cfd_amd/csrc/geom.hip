@@ -16,27 +16,65 @@
 namespace cfd {
 namespace {
 
-// subrutinas.f90:99-125
+// mLaplace.f90:188-200
+__device__ inline double quality_mu(double X1, double X2, double X3, double Y1, double Y2, double Y3) {
+    const double TWOSQRT3 = 3.46410161513775;
+    double ar = X2 * Y3 + X3 * Y1 + X1 * Y2 - (X2 * Y1 + X3 * Y2 + X1 * Y3);
+    double l1 = (X3 - X2) * (X3 - X2) + (Y3 - Y2) * (Y3 - Y2);
+    double l2 = (X1 - X3) * (X1 - X3) + (Y1 - Y3) * (Y1 - Y3);
+    double l3 = (X2 - X1) * (X2 - X1) + (Y2 - Y1) * (Y2 - Y1);
+    double l = l1 + l2 + l3;
+    return TWOSQRT3 * ar / l;
+}
+
+// an element's weight in laplace, 1/mu^2 (mLaplace.f90:120-148)
+__device__ inline double lap_weight(double X1, double X2, double X3, double Y1, double Y2, double Y3) {
+    const double mu = quality_mu(X1, X2, X3, Y1, Y2, Y3);
+    return 1.0 / (mu * mu);
+}
+// an element's two terms of gcl.f90:218-236: its W's divergence by area/3 now,
+// and the old W's by the old area's
+__device__ inline double2 gcl_terms(const double* nx, const double* ny, int n0, int n1, int n2,
+                                    const double* Wx, const double* wy, const double* Wxo,
+                                    const double* wyo, double area, double area_old) {
+    const double divW = nx[0] * Wx[n0] + nx[1] * Wx[n1] + nx[2] * Wx[n2] + ny[0] * wy[n0] +
+                        ny[1] * wy[n1] + ny[2] * wy[n2];
+    const double divWo = nx[0] * Wxo[n0] + nx[1] * Wxo[n1] + nx[2] * Wxo[n2] + ny[0] * wyo[n0] +
+                         ny[1] * wyo[n1] + ny[2] * wyo[n2];
+    return make_double2(divW * area / 3.0, divWo * area_old / 3.0);
+}
+
+// subrutinas.f90:99-125, and what else the nodes' kernel needs of an element:
+// its weight in laplace and (kGcl) its terms of the GCL, formed once here
+// instead of by each of its nodes
+template <bool kGcl>
 __global__ void __launch_bounds__(kBlock)
 k_deriv(const int* __restrict__ inpoel, const double* __restrict__ X, const double* __restrict__ Y,
         double* __restrict__ area, double* __restrict__ dNx, double* __restrict__ dNy,
         double* __restrict__ HH, double* __restrict__ HHX, double* __restrict__ HHY, int nelem,
-        double* __restrict__ partials, double* __restrict__ area_old) {
+        double* __restrict__ partials, ElemTerms x) {
     double hm = __builtin_huge_val();
     for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < nelem; e += gridDim.x * blockDim.x) {
         int n1 = inpoel[3 * e] - 1, n2 = inpoel[3 * e + 1] - 1, n3 = inpoel[3 * e + 2] - 1;
         double X1 = X[n1], X2 = X[n2], X3 = X[n3];
         double Y1 = Y[n1], Y2 = Y[n2], Y3 = Y[n3];
         double a = (X2 * Y3 + X3 * Y1 + X1 * Y2 - (X2 * Y1 + X3 * Y2 + X1 * Y3)) / 2.0;
-        if (area_old) area_old[e] = area[e];
+        const double old = kGcl ? area[e] : 0.0;
         area[e] = a;
         double a2 = 2.0 * a;
-        dNx[3 * e + 0] = (Y2 - Y3) / a2;
-        dNx[3 * e + 1] = (Y3 - Y1) / a2;
-        dNx[3 * e + 2] = (Y1 - Y2) / a2;
-        dNy[3 * e + 0] = (X3 - X2) / a2;
-        dNy[3 * e + 1] = (X1 - X3) / a2;
-        dNy[3 * e + 2] = (X2 - X1) / a2;
+        const double nx[3] = {(Y2 - Y3) / a2, (Y3 - Y1) / a2, (Y1 - Y2) / a2};
+        const double ny[3] = {(X3 - X2) / a2, (X1 - X3) / a2, (X2 - X1) / a2};
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            dNx[3 * e + j] = nx[j];
+            dNy[3 * e + j] = ny[j];
+        }
+        if (x.lapw) x.lapw[e] = lap_weight(X1, X2, X3, Y1, Y2, Y3);
+        if (kGcl) {
+            x.area_old[e] = old;
+            x.gcl[e] = gcl_terms(nx, ny, n1, n2, n3, x.Wx, x.mode ? x.Wy : x.Wx, x.Wxo,
+                                 x.mode ? x.Wyo : x.Wxo, a, old);
+        }
         double h = sqrt(a);
         HH[e] = h;
         if (h < hm) hm = h;
@@ -51,6 +89,15 @@ k_deriv(const int* __restrict__ inpoel, const double* __restrict__ X, const doub
     block_partial(hm, OpMin(), partials);
 }
 
+// the weights alone (the host entry's laplace)
+__global__ void k_lap_weights(const int* __restrict__ inpoel, const double* __restrict__ X,
+                              const double* __restrict__ Y, double* __restrict__ lapw, int nelem) {
+    const int e = blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= nelem) return;
+    const int n1 = inpoel[3 * e] - 1, n2 = inpoel[3 * e + 1] - 1, n3 = inpoel[3 * e + 2] - 1;
+    lapw[e] = lap_weight(X[n1], X[n2], X[n3], Y[n1], Y[n2], Y[n3]);
+}
+
 // subrutinas.f90:137-152: M(i) = sum of area/3 over i's elements, ascending
 __global__ void __launch_bounds__(kBlock)
 k_masas(const int* __restrict__ esup1, const int* __restrict__ esup2, const double* __restrict__ area,
@@ -62,17 +109,6 @@ k_masas(const int* __restrict__ esup1, const int* __restrict__ esup2, const doub
     M[i] = m;
 }
 
-// mLaplace.f90:188-200
-__device__ inline double quality_mu(double X1, double X2, double X3, double Y1, double Y2, double Y3) {
-    const double TWOSQRT3 = 3.46410161513775;
-    double ar = X2 * Y3 + X3 * Y1 + X1 * Y2 - (X2 * Y1 + X3 * Y2 + X1 * Y3);
-    double l1 = (X3 - X2) * (X3 - X2) + (Y3 - Y2) * (Y3 - Y2);
-    double l2 = (X1 - X3) * (X1 - X3) + (Y1 - Y3) * (Y1 - Y3);
-    double l3 = (X2 - X1) * (X2 - X1) + (Y2 - Y1) * (Y2 - Y1);
-    double l = l1 + l2 + l3;
-    return TWOSQRT3 * ar / l;
-}
-
 // mLaplace.f90:120-148, one row per thread; column positions from the slot
 // map.  A row of up to kLapRow entries accumulates in LDS (the same sequence
 // of additions per entry as in memory), column-major over the block's
@@ -82,42 +118,68 @@ __device__ inline double quality_mu(double X1, double X2, double X3, double Y1, 
 constexpr int kLapRow = 16;
 
 // row i's contributions in esup order; acc(k) is the accumulator of CSR
-// entry r0 + k
-template <class Acc>
-__device__ inline void laplace_row(int i, int r0, const int* __restrict__ inpoel,
-                                   const int* __restrict__ esup1, const int* __restrict__ esup2,
-                                   const int* __restrict__ lslot, const double* __restrict__ X,
-                                   const double* __restrict__ Y, const double* __restrict__ dNx,
-                                   const double* __restrict__ dNy, Acc acc) {
-    for (int s = esup2[i]; s < esup2[i + 1]; ++s) {
-        int e = esup1[s] - 1;
-        int n1 = inpoel[3 * e] - 1, n2 = inpoel[3 * e + 1] - 1, n3 = inpoel[3 * e + 2] - 1;
-        double mu = quality_mu(X[n1], X[n2], X[n3], Y[n1], Y[n2], Y[n3]);
-        double q = 1.0 / (mu * mu);
-        int li = (n1 == i) ? 0 : ((n2 == i) ? 1 : 2);
-        double ax = dNx[3 * e + li], ay = dNy[3 * e + li];
+// entry r0 + k, the first one the diagonal's; each(e): the node's other sums
+template <class Acc, class Each>
+__device__ inline void laplace_row(int r0, int s0, int s1, const int* __restrict__ esup1,
+                                   const int* __restrict__ lslot, const double* __restrict__ lapw,
+                                   const double* __restrict__ dNx, const double* __restrict__ dNy,
+                                   Acc acc, Each each) {
+    for (int s = s0; s < s1; ++s) {
+        const int e = esup1[s] - 1;
+        int slot[3];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) slot[j] = lslot[3 * s + j] - r0;
+        const int li = slot[0] == 0 ? 0 : slot[1] == 0 ? 1 : 2;  // the row's own node
+        const double q = lapw[e];
+        double nx[3], ny[3];
+#pragma unroll
         for (int j = 0; j < 3; ++j) {
-            double& a = acc(lslot[3 * s + j] - r0);
-            a = a + (ax * dNx[3 * e + j] + ay * dNy[3 * e + j]) * q;
+            nx[j] = dNx[3 * e + j];
+            ny[j] = dNy[3 * e + j];
         }
+        const double ax = li == 0 ? nx[0] : li == 1 ? nx[1] : nx[2];
+        const double ay = li == 0 ? ny[0] : li == 1 ? ny[1] : ny[2];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            double& a = acc(slot[j]);
+            a = a + (ax * nx[j] + ay * ny[j]) * q;
+        }
+        each(e);
     }
 }
 
+// laplace's rows, and the nodes' masses in the same pass over their elements:
+// MASAS, or the GCL's update from the terms that k_deriv left.
+// Bound by the loads of a node's six elements (scattered, from the caches).
+// With the quality formed per node and element from the coordinates, and the
+// GCL from the gradients and W, in launches of their own: 4,608 nodes 8.6 + 7.4
+// us, 524,288 nodes @LAP@.
+enum { kMassNone, kMassMasas, kMassGcl };
+template <int kMass>
 __global__ void __launch_bounds__(kBlock)
-k_laplace(const int* __restrict__ inpoel, const int* __restrict__ esup1, const int* __restrict__ esup2,
-          const int* __restrict__ rowptr, const int* __restrict__ lslot, const double* __restrict__ X,
-          const double* __restrict__ Y, const double* __restrict__ dNx, const double* __restrict__ dNy,
-          double* __restrict__ lap, double* __restrict__ diag, int npoin, int width,
-          double* __restrict__ ell) {
+k_laplace(const int* __restrict__ esup1, const int* __restrict__ esup2,
+          const int* __restrict__ rowptr, const int* __restrict__ lslot,
+          const double* __restrict__ lapw, const double* __restrict__ dNx,
+          const double* __restrict__ dNy, double* __restrict__ lap, double* __restrict__ diag,
+          int npoin, int width, double* __restrict__ ell, NodeMass m) {
     __shared__ double srow[kLapRow * kBlock];
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= npoin) return;
-    const int r0 = rowptr[i], len = rowptr[i + 1] - r0;
+    const int r0 = rowptr[i], len = rowptr[i + 1] - r0, s0 = esup2[i], s1 = esup2[i + 1];
+    double tot1 = 0.0, tot2 = 0.0;
+    auto each = [&](int e) {
+        if (kMass == kMassMasas) tot1 = tot1 + m.area[e] / 3.0;  // subrutinas.f90:137-152
+        if (kMass == kMassGcl) {  // gcl.f90:218-236
+            const double2 g = m.gcl[e];
+            tot1 = tot1 + g.x;
+            tot2 = tot2 + g.y;
+        }
+    };
     if (len <= kLapRow) {
         double* sr = srow + threadIdx.x;
         for (int j = 0; j < len; ++j) sr[j * kBlock] = 0.0;
-        laplace_row(i, r0, inpoel, esup1, esup2, lslot, X, Y, dNx, dNy,
-                    [sr](int k) -> double& { return sr[k * kBlock]; });
+        laplace_row(r0, s0, s1, esup1, lslot, lapw, dNx, dNy,
+                    [sr](int k) -> double& { return sr[k * kBlock]; }, each);
         for (int j = 0; j < len; ++j) lap[r0 + j] = sr[j * kBlock];
         for (int j = 0; j < width; ++j)
             ell[(size_t)j * npoin + i] = j < len ? sr[j * kBlock] : 0.0;
@@ -125,14 +187,17 @@ k_laplace(const int* __restrict__ inpoel, const int* __restrict__ esup1, const i
     } else {
         double* row = lap + r0;
         for (int j = 0; j < len; ++j) row[j] = 0.0;
-        laplace_row(i, r0, inpoel, esup1, esup2, lslot, X, Y, dNx, dNy,
-                    [row](int k) -> double& { return row[k]; });
+        laplace_row(r0, s0, s1, esup1, lslot, lapw, dNx, dNy,
+                    [row](int k) -> double& { return row[k]; }, each);
         for (int j = 0; j < width; ++j) ell[(size_t)j * npoin + i] = j < len ? row[j] : 0.0;
         diag[i] = row[0];
     }
+    if (kMass == kMassMasas) m.M[i] = tot1;
+    if (kMass == kMassGcl) m.M[i] = m.M[i] + *m.dt * (tot1 + tot2) / 2.0;
 }
 
-// gcl.f90:218-236 per node: both divergence sums in ascending element order
+// gcl.f90:218-236 per node: both divergence sums in ascending element order (the
+// host entry, whose gradients come from the caller)
 __global__ void __launch_bounds__(kBlock)
 k_gcl(const int* __restrict__ inpoel, const int* __restrict__ esup1, const int* __restrict__ esup2,
       double* __restrict__ M, const double* __restrict__ Wx, const double* __restrict__ Wy,
@@ -147,15 +212,11 @@ k_gcl(const int* __restrict__ inpoel, const int* __restrict__ esup1, const int* 
     double tot1 = 0.0, tot2 = 0.0;
     for (int s = esup2[i]; s < esup2[i + 1]; ++s) {
         int e = esup1[s] - 1;
-        int n0 = inpoel[3 * e] - 1, n1 = inpoel[3 * e + 1] - 1, n2 = inpoel[3 * e + 2] - 1;
-        const double* nx = dNx + 3 * e;
-        const double* ny = dNy + 3 * e;
-        double divW = nx[0] * Wx[n0] + nx[1] * Wx[n1] + nx[2] * Wx[n2] + ny[0] * wy[n0] +
-                      ny[1] * wy[n1] + ny[2] * wy[n2];
-        double divWo = nx[0] * Wxo[n0] + nx[1] * Wxo[n1] + nx[2] * Wxo[n2] + ny[0] * wyo[n0] +
-                       ny[1] * wyo[n1] + ny[2] * wyo[n2];
-        tot1 = tot1 + divW * area[e] / 3.0;
-        tot2 = tot2 + divWo * area_old[e] / 3.0;
+        const int n0 = inpoel[3 * e] - 1, n1 = inpoel[3 * e + 1] - 1, n2 = inpoel[3 * e + 2] - 1;
+        const double2 g = gcl_terms(dNx + 3 * e, dNy + 3 * e, n0, n1, n2, Wx, wy, Wxo, wyo, area[e],
+                                    area_old[e]);
+        tot1 = tot1 + g.x;
+        tot2 = tot2 + g.y;
     }
     M[i] = M[i] + dt * (tot1 + tot2) / 2.0;
 }
@@ -370,10 +431,10 @@ __global__ void k_transf(int nedge, const int* __restrict__ iset, const double* 
 
 void launch_deriv(const Tables& t, const double* X, const double* Y, double* area, double* dNx,
                   double* dNy, double* HH, double* HHX, double* HHY, double* hmin_out,
-                  double* partials, hipStream_t s, double* area_old) {
+                  double* partials, hipStream_t s, const ElemTerms& x) {
     const unsigned g = grid_for(t.nelem);
-    k_deriv<<<g, kBlock, 0, s>>>(t.inpoel.p, X, Y, area, dNx, dNy, HH, HHX, HHY, t.nelem, partials,
-                                 area_old);
+    const auto kernel = x.gcl ? k_deriv<true> : k_deriv<false>;
+    kernel<<<g, kBlock, 0, s>>>(t.inpoel.p, X, Y, area, dNx, dNy, HH, HHX, HHY, t.nelem, partials, x);
     // hmin = minval(HH), capped at 1e10 (subrutinas.f90:124-125)
     k_min_finalize<<<1, 256, 0, s>>>(partials, (int)g, __builtin_huge_val(), 1.0e10, hmin_out);
     CFD_HIP(hipGetLastError());
@@ -384,11 +445,18 @@ void launch_masas(const Tables& t, const double* area, double* M, hipStream_t s)
     CFD_HIP(hipGetLastError());
 }
 
-void launch_laplace(const Tables& t, const double* X, const double* Y, const double* dNx,
-                    const double* dNy, double* lap, double* diag, hipStream_t s, EllLap* ell) {
-    k_laplace<<<grid_for(t.npoin), kBlock, 0, s>>>(t.inpoel.p, t.esup1.p, t.esup2.p, t.rowptr.p,
-                                                   t.lslot.p, X, Y, dNx, dNy, lap, diag, t.npoin,
-                                                   ell ? ell->width : 0, ell ? ell->val.p : nullptr);
+void launch_lap_weights(const Tables& t, const double* X, const double* Y, double* lapw,
+                        hipStream_t s) {
+    k_lap_weights<<<grid_for(t.nelem), kBlock, 0, s>>>(t.inpoel.p, X, Y, lapw, t.nelem);
+    CFD_HIP(hipGetLastError());
+}
+
+void launch_laplace(const Tables& t, const double* lapw, const double* dNx, const double* dNy,
+                    double* lap, double* diag, hipStream_t s, EllLap* ell, const NodeMass& m) {
+    const auto kernel = m.gcl ? k_laplace<kMassGcl> : m.area ? k_laplace<kMassMasas> : k_laplace<kMassNone>;
+    kernel<<<grid_for(t.npoin), kBlock, 0, s>>>(t.esup1.p, t.esup2.p, t.rowptr.p, t.lslot.p, lapw,
+                                                dNx, dNy, lap, diag, t.npoin, ell ? ell->width : 0,
+                                                ell ? ell->val.p : nullptr, m);
     CFD_HIP(hipGetLastError());
 }
 
