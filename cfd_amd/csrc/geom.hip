@@ -149,21 +149,28 @@ __device__ inline void laplace_row(int r0, int s0, int s1, const int* __restrict
 }
 
 // laplace's rows, and the nodes' masses in the same pass over their elements:
-// MASAS, or the GCL's update from the terms that k_deriv left.
-// Bound by the loads of a node's six elements (scattered, from the caches).
-// With the quality formed per node and element from the coordinates, and the
-// GCL from the gradients and W, in launches of their own: 4,608 nodes 8.6 + 7.4
-// us, 524,288 nodes @LAP@.
+// MASAS, or the GCL's update from the terms that k_deriv left.  Blocks of one
+// wave in XCD order (a node's elements are its ring neighbours' too).
+//
+// Formed from the coordinates, gradients and W per node and element, in launches
+// of their own (laplace + GCL / laplace + MASAS), and so, k_deriv's 15 us more for
+// the GCL's terms not counted: 4,608 nodes 8.6 + 7.4 / 8.6 + 4.2 us, now 5.7 / 5.6;
+// 524,288 nodes 100 + 91 / 100 + 10 us, now 95 / 85 (blocks of 256 in natural order
+// 102 / 92, 7.4 us on the small mesh).  Bound by the lines that a node's scattered
+// elements share with others: 520 MB are fetched past the L2s for 150 MB of
+// tables.  Fewer loads (a packed slot record, the products instead of the
+// gradients) and rows staged for coalesced CSR stores left it at 88-92.
+constexpr int kLapThreads = 64;
 enum { kMassNone, kMassMasas, kMassGcl };
 template <int kMass>
-__global__ void __launch_bounds__(kBlock)
+__global__ void __launch_bounds__(kLapThreads)
 k_laplace(const int* __restrict__ esup1, const int* __restrict__ esup2,
           const int* __restrict__ rowptr, const int* __restrict__ lslot,
           const double* __restrict__ lapw, const double* __restrict__ dNx,
           const double* __restrict__ dNy, double* __restrict__ lap, double* __restrict__ diag,
           int npoin, int width, double* __restrict__ ell, NodeMass m) {
-    __shared__ double srow[kLapRow * kBlock];
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ double srow[kLapRow * kLapThreads];
+    const int i = xcd_block(blockIdx.x, gridDim.x) * kLapThreads + threadIdx.x;
     if (i >= npoin) return;
     const int r0 = rowptr[i], len = rowptr[i + 1] - r0, s0 = esup2[i], s1 = esup2[i + 1];
     double tot1 = 0.0, tot2 = 0.0;
@@ -177,12 +184,12 @@ k_laplace(const int* __restrict__ esup1, const int* __restrict__ esup2,
     };
     if (len <= kLapRow) {
         double* sr = srow + threadIdx.x;
-        for (int j = 0; j < len; ++j) sr[j * kBlock] = 0.0;
+        for (int j = 0; j < len; ++j) sr[j * kLapThreads] = 0.0;
         laplace_row(r0, s0, s1, esup1, lslot, lapw, dNx, dNy,
-                    [sr](int k) -> double& { return sr[k * kBlock]; }, each);
-        for (int j = 0; j < len; ++j) lap[r0 + j] = sr[j * kBlock];
+                    [sr](int k) -> double& { return sr[k * kLapThreads]; }, each);
+        for (int j = 0; j < len; ++j) lap[r0 + j] = sr[j * kLapThreads];
         for (int j = 0; j < width; ++j)
-            ell[(size_t)j * npoin + i] = j < len ? sr[j * kBlock] : 0.0;
+            ell[(size_t)j * npoin + i] = j < len ? sr[j * kLapThreads] : 0.0;
         diag[i] = sr[0];
     } else {
         double* row = lap + r0;
@@ -454,7 +461,7 @@ void launch_lap_weights(const Tables& t, const double* X, const double* Y, doubl
 void launch_laplace(const Tables& t, const double* lapw, const double* dNx, const double* dNy,
                     double* lap, double* diag, hipStream_t s, EllLap* ell, const NodeMass& m) {
     const auto kernel = m.gcl ? k_laplace<kMassGcl> : m.area ? k_laplace<kMassMasas> : k_laplace<kMassNone>;
-    kernel<<<grid_for(t.npoin), kBlock, 0, s>>>(t.esup1.p, t.esup2.p, t.rowptr.p, t.lslot.p, lapw,
+    kernel<<<(t.npoin + kLapThreads - 1) / kLapThreads, kLapThreads, 0, s>>>(t.esup1.p, t.esup2.p, t.rowptr.p, t.lslot.p, lapw,
                                                 dNx, dNy, lap, diag, t.npoin, ell ? ell->width : 0,
                                                 ell ? ell->val.p : nullptr, m);
     CFD_HIP(hipGetLastError());
