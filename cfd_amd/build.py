@@ -20,7 +20,7 @@ LIB = os.path.join(PKG, "libcfd_amd.so")
 SOURCES = ["tables.hip", "geom.hip", "flow.hip", "pcg.hip", "patches.hip", "mlp.hip",
            "warmstart.hip", "state.hip", "batch.hip", "api.hip", "restart.hip",
            "smooth.hip"]
-HEADERS = ["cfd_internal.hpp", "reduce.hpp", "crmath.hpp", "stepctl.hpp"]
+HEADERS = ["cfd_internal.hpp", "reduce.hpp", "crmath.hpp", "stepctl.hpp", "forces.hpp"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"

@@ -705,6 +705,7 @@ struct cfd_session {
     // would be DTMIN everywhere, and no kernel of theirs reads DT or DTL);
     // the two fields are formed when a caller reads them (dt_stale).
     bool dt_stale = false;
+    bool forces_due = false;  // the step before left its forces to this step's deltat
     bool lazy_dt() const { return fused() && d.itlocal == 0; }
     // timing
     bool timing = false;
@@ -863,9 +864,19 @@ struct cfd_session {
         CFD_HIP(hipGetLastError());
     }
 
+    // FORCES (and FORCE_VISC: the viscous terms) of a mesh at rest as one block's
+    // work, with the solves' zero counts
+    ForceIn still_forces() {
+        return ForceIn{d.nsetedges, ISET.p, X.p, Y.p, P.p, d.xref, d.yref,
+                       ViscIn{m->t.inpoel.p, T.p, VX.p, VY.p, DNX.p, DNY.p, c.t_inf},
+                       scal(CFD_S_FX), scal(CFD_S_FVX), scal(CFD_S_PCG_ITX)};
+    }
+
     // One time step, queued on the stream without waiting for the device
     // (except inside the mesh solves: the host polls PCG's done flag).
-    void step() {
+    // more: another step follows in the same call, whose deltat may form this
+    // step's forces beside its patches (nothing it reads or writes differs).
+    void step(bool more) {
         const Tables& t = m->t;
         tb(CFD_K_STEP);
         // deltat, DTMIN with its hysteresis, DTL, the clock (ns2DComp.ALE.f90:142-166)
@@ -877,11 +888,14 @@ struct cfd_session {
         const double* wy = fu ? WY.p : nullptr;
         const bool in_patches = fused() && patches.npatch <= (int)partials.n;
         const bool fold_ctl = in_patches && d.itlocal == 0 && patches.npatch <= kStepFoldMax;
+        const ForceIn due = still_forces();
         const int nb = in_patches
                            ? launch_deltat_patch(patches, c, AREA.p, T.p, VX.p, VY.p, wx, wy,
-                                                 DT.p, partials.p, s, fold_ctl ? ctl.p : nullptr)
+                                                 DT.p, partials.p, s, fold_ctl ? ctl.p : nullptr,
+                                                 forces_due ? &due : nullptr, c.fmu != 0.0)
                            : launch_deltat_partials(t, c, AREA.p, T.p, VX.p, VY.p, WX.p, WY.p,
                                                     DT.p, partials.p, s);
+        forces_due = false;
         const StepFold fold{partials.p, nb, ctl.p, d.itlocal, d.motion, d.motion_amp,
                             d.motion_omega};
         if (!fold_ctl)
@@ -956,9 +970,12 @@ struct cfd_session {
         static_assert(CFD_S_PCG_ITY == CFD_S_PCG_ITX + 1 && CFD_S_PCG_RZX == CFD_S_PCG_ITX + 2 &&
                           CFD_S_PCG_RZY == CFD_S_PCG_ITX + 3,
                       "mesh-solve scalars are contiguous");
-        launch_forces(d.nsetedges, ISET.p, X.p, Y.p, P.p, d.xref, d.yref, scal(CFD_S_FX),
-                      fvisc && still ? &visc : nullptr, scal(CFD_S_FVX), FPART.p,
-                      still ? scal(CFD_S_PCG_ITX) : nullptr, s);
+        forces_due = more && still && in_patches && d.nsetedges > 0 &&
+                     d.nsetedges <= 64 * kForcesOne;
+        if (!forces_due)
+            launch_forces(d.nsetedges, ISET.p, X.p, Y.p, P.p, d.xref, d.yref, scal(CFD_S_FX),
+                          fvisc && still ? &visc : nullptr, scal(CFD_S_FVX), FPART.p,
+                          still ? scal(CFD_S_PCG_ITX) : nullptr, s);
         if (!still) {
             // TRANSF's displacements reach the solves only through moving nodes
             if (d.nmove > 0)
@@ -1295,7 +1312,7 @@ int cfd_session_init_freestream(cfd_session* S) {
 int cfd_session_step(cfd_session* S, int nsteps) {
     CFD_TRY({
         CFD_ARG(S && nsteps >= 0, "arguments");
-        for (int k = 0; k < nsteps; ++k) S->step();
+        for (int k = 0; k < nsteps; ++k) S->step(k + 1 < nsteps);
     })
 }
 

@@ -235,11 +235,28 @@ int launch_deltat_partials(const Tables& t, const Consts& c, const double* area,
 // LDS): the same DT bits, one min partial per patch; returns ps.npatch.  A
 // batch's patches take their case's constants.
 struct PatchSet;
+// FORCES and FORCE_VISC on one edge set by one block (forces.hpp): up to
+// kForcesOne pieces of 64 edges
+constexpr int kForcesOne = 8;
+struct ViscIn {
+    const int* inpoel;
+    const double *T, *VX, *VY, *dNx, *dNy;
+    double t_inf;
+};
+struct ForceIn {
+    int nedge;
+    const int* iset;
+    const double *X, *Y, *P;
+    double xref, yref;
+    ViscIn v;
+    double *out, *outv, *zero4;  // FX, FY, RM; F_VX, F_VY; four zeros (null: none)
+};
 // ctl (may be null): the session scalars, of which DTMIN1 and BANDERA are copied
 // aside for step control inside ESTAB (StepFold).
 int launch_deltat_patch(const PatchSet& ps, const Consts& c, const double* area, const double* T,
                         const double* VX, const double* VY, const double* WX, const double* WY,
-                        double* DT, double* partials, hipStream_t s, double* ctl = nullptr);
+                        double* DT, double* partials, hipStream_t s, double* ctl = nullptr,
+                        const ForceIn* forces = nullptr, bool visc = false);
 // Step control (launch_step_ctl) inside launch_estab_patch: every block forms
 // DTMIN from deltat's partials, the first one stores the step's scalars.
 struct StepFold {
@@ -584,11 +601,6 @@ void launch_gather_field(const double* caller, double* state, const int* map, in
 // meshMove.f90 FORCES (out3 = FX, FY, RM; skipped when null) and, when visc
 // is given, FORCE_VISC (ns2DComp.ALE.f90:819-893; out2 = F_VX, F_VY) in the
 // same launch; device scalars out
-struct ViscIn {
-    const int* inpoel;
-    const double *T, *VX, *VY, *dNx, *dNy;
-    double t_inf;
-};
 // part: device scratch of forces_part_size(nedge) doubles; zero4 (may be
 // null): four device scalars set to 0 in the same launches
 size_t forces_part_size(int nedge);

@@ -22,6 +22,7 @@
 
 #include "cfd_internal.hpp"
 #include "crmath.hpp"
+#include "forces.hpp"
 #include "reduce.hpp"
 #include "stepctl.hpp"
 
@@ -89,9 +90,16 @@ k_deltat(const int* __restrict__ inpoel, const double* __restrict__ area, const 
 // (the same values as k_deltat), one min partial per patch.  Batches: the
 // constants of the patch's case (32 cases of a sweep, 3.1M triangles: 46 us,
 // against 76 in element order with 15 gathers an element).
+//
+// kForces: one more block forms the forces that the step before has left to this
+// launch (1: FORCES, 2: FORCE_VISC too), beside the patches instead of in a launch
+// of its own between the steps (a chain of loads of 4.5 us; us a step without / so:
+// FP64 42 patches 49.0 / 45.8, 675 patches 92.4 / 89.3; FP32 32 patches 47.0 / 43.5,
+// 505 patches 67.7 / 63.0).
 struct DtNode {
     double T, vu, vv;
 };
+template <int kForces>
 __global__ void __launch_bounds__(512)
 k_deltat_patch(const int* __restrict__ node_base, const int* __restrict__ elem_base,
                const int* __restrict__ pnode, const uint32_t* __restrict__ loc,
@@ -100,10 +108,14 @@ k_deltat_patch(const int* __restrict__ node_base, const int* __restrict__ elem_b
                const double* __restrict__ VY, const double* __restrict__ WX,
                const double* __restrict__ WY, double* __restrict__ DT, double t_inf, double fsafe,
                double* __restrict__ partials, const int* __restrict__ pcase,
-               const Consts* __restrict__ cases, double* __restrict__ ctl) {
+               const Consts* __restrict__ cases, double* __restrict__ ctl, ForceIn forces) {
+    if (kForces && (int)blockIdx.x == npatch) {
+        forces_block<true, kForces == 2>(forces);
+        return;
+    }
     extern __shared__ double4 smem4[];
     DtNode* sN = reinterpret_cast<DtNode*>(smem4);
-    const int p = xcd_block(blockIdx.x, npatch);  // grid = npatch: logical patch
+    const int p = xcd_block(blockIdx.x, npatch);  // blocks below npatch: logical patch
     if (pcase) {
         const Consts& q = cases[pcase[p]];
         t_inf = q.t_inf;
@@ -1205,13 +1217,16 @@ inline int patch_pass_block(int pe, int npatch) {
 
 int launch_deltat_patch(const PatchSet& ps, const Consts& c, const double* area, const double* T,
                         const double* VX, const double* VY, const double* WX, const double* WY,
-                        double* DT, double* partials, hipStream_t s, double* ctl) {
+                        double* DT, double* partials, hipStream_t s, double* ctl,
+                        const ForceIn* forces, bool visc) {
     CFD_CHECK(ps.npatch > 0 && ps.max_nodes <= kPatchMaxNodes, "internal: deltat patches");
+    CFD_CHECK(!forces || forces->nedge <= 64 * kForcesOne, "internal: forces of one block");
     const size_t lds = (size_t)ps.max_nodes * sizeof(DtNode);
-    k_deltat_patch<<<ps.npatch, patch_pass_block(ps.pe, ps.npatch), lds, s>>>(ps.node_base.p, ps.elem_base.p, ps.pnode.p,
-                                                  ps.loc.p, ps.perm.p, ps.npatch, area, T, VX, VY,
-                                                  WX, WY, DT, c.t_inf, c.fsafe, partials,
-                                                  ps.cases ? ps.pcase.p : nullptr, ps.cases, ctl);
+    const auto kernel = !forces ? k_deltat_patch<0> : visc ? k_deltat_patch<2> : k_deltat_patch<1>;
+    kernel<<<ps.npatch + (forces ? 1 : 0), patch_pass_block(ps.pe, ps.npatch), lds, s>>>(
+        ps.node_base.p, ps.elem_base.p, ps.pnode.p, ps.loc.p, ps.perm.p, ps.npatch, area, T, VX, VY,
+        WX, WY, DT, c.t_inf, c.fsafe, partials, ps.cases ? ps.pcase.p : nullptr, ps.cases, ctl,
+        forces ? *forces : ForceIn{});
     CFD_HIP(hipGetLastError());
     return ps.npatch;
 }

@@ -10,6 +10,7 @@
 #include <type_traits>
 
 #include "cfd_internal.hpp"
+#include "forces.hpp"
 #include "reduce.hpp"
 #include "crmath.hpp"
 
@@ -277,60 +278,6 @@ __global__ void k_normalvel(const int* __restrict__ bcidx, const int* __restrict
     VY[i] = nx * p + wy;
 }
 
-// meshMove.f90:167-192 FORCES and ns2DComp.ALE.f90:839-887 FORCE_VISC, one
-// set.  FORCE_VISC's traction is that of the full stress tensor (-p I +
-// viscous, with the element-average pressure), Sutherland mu at the
-// edge-average temperature, on the edge normal (Y2-Y1, -(X2-X1)) / |edge|.
-// r = FX, FY, RM, F_VX, F_VY terms of edge i.
-template <bool kPress, bool kVisc>
-__device__ __forceinline__ void force_terms(int i, const int* __restrict__ iset,
-                                            const double* __restrict__ X,
-                                            const double* __restrict__ Y,
-                                            const double* __restrict__ P, double xref,
-                                            double yref, const ViscIn& v, double r[5]) {
-    const int n1 = iset[3 * i] - 1, n2 = iset[3 * i + 1] - 1;
-    if (kPress) {
-        const double d_press = (P[n1] + P[n2]) / 2.0;
-        const double rlx = X[n1] - X[n2];
-        const double rly = Y[n2] - Y[n1];
-        const double dfx = d_press * rly, dfy = d_press * rlx;
-        const double xc = (X[n1] + X[n2]) / 2.0;
-        const double yc = (Y[n2] + Y[n1]) / 2.0;
-        r[0] = dfx;
-        r[1] = dfy;
-        r[2] = dfy * (xc - xref) - dfx * (yc - yref);
-    }
-    if (kVisc) {
-        const int ie = iset[3 * i + 2] - 1;
-        const double temp = (v.T[n1] + v.T[n2]) / 2.0;
-        const double smu = 110.0;
-        const double fmu = 0.017 * pow_3_2(temp / v.t_inf) * (v.t_inf + smu) / (temp + smu);
-        double rly = -(X[n2] - X[n1]);
-        double rlx = Y[n2] - Y[n1];
-        const double rmod = sqrt(rlx * rlx + rly * rly);
-        rlx = rlx / rmod;
-        rly = rly / rmod;
-        double dux = 0.0, duy = 0.0, dvx = 0.0, dvy = 0.0, press = 0.0;
-#pragma unroll
-        for (int jj = 0; jj < 3; ++jj) {
-            const int nn = v.inpoel[3 * ie + jj] - 1;
-            const double nx = v.dNx[3 * ie + jj], ny = v.dNy[3 * ie + jj];
-            const double vx = v.VX[nn], vy = v.VY[nn];
-            dux = dux + nx * vx;
-            duy = duy + ny * vx;
-            dvx = dvx + nx * vy;
-            dvy = dvy + ny * vy;
-            press = press + P[nn];
-        }
-        press = press / 3.0;
-        const double txx = -press - fmu * (2.0 / 3.0 * (dux + dvy) - 2.0 * dux);
-        const double txy = fmu * (duy + dvx);
-        const double tyy = -press - fmu * (2.0 / 3.0 * (dux + dvy) - 2.0 * dvy);
-        r[3] = (txx * rlx + txy * rly) * rmod;
-        r[4] = (txy * rlx + tyy * rly) * rmod;
-    }
-}
-
 // One wave per 64 edges: lane l forms edge 64 b + l, the wave sums the terms
 // by a fixed shuffle tree and lane 0 stores the block's five partials at
 // part[q * nb + b].
@@ -383,38 +330,10 @@ k_forces_fin(int nb, const double* __restrict__ part, double* __restrict__ out,
 // pieces (us a step with / without: 128 edges 49.5 / 52.0, 512 edges 93.8 /
 // 94.1); above, one CU's gathers take longer than a launch (1,024 edges 232 /
 // 226, 2,048 866 / 852).
-constexpr int kForcesOne = 8;
 template <bool kPress, bool kVisc>
 __global__ void __launch_bounds__(64 * kForcesOne)
-k_forces_one(int nedge, const int* __restrict__ iset, const double* __restrict__ X,
-             const double* __restrict__ Y, const double* __restrict__ P, double xref, double yref,
-             ViscIn v, double* __restrict__ out, double* __restrict__ outv,
-             double* __restrict__ zero4) {
-    __shared__ double part[5][kForcesOne];
-    const int nb = (nedge + 63) / 64, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    for (int b = w; b < nb; b += blockDim.x >> 6) {
-        const int i = b * 64 + lane;
-        double r[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-        if (i < nedge) force_terms<kPress, kVisc>(i, iset, X, Y, P, xref, yref, v, r);
-#pragma unroll
-        for (int q = 0; q < 5; ++q) {
-            if (q < 3 && !kPress) continue;
-            if (q >= 3 && !kVisc) continue;
-            const double t = wave_reduce(r[q], OpSum());
-            if (lane == 0) part[q][b] = t;
-        }
-    }
-    __syncthreads();
-    if (w < 5 && (w < 3 ? kPress : kVisc)) {  // wave w: sum w
-        double a = 0.0;
-        for (int k = lane; k < nb; k += 64) a = a + part[w][k];
-        a = wave_reduce(a, OpSum());
-        if (lane == 0) {
-            if (w < 3) out[w] = a;
-            else outv[w - 3] = a;
-        }
-    }
-    if (zero4 && threadIdx.x < 4) zero4[threadIdx.x] = 0.0;
+k_forces_one(ForceIn f) {
+    forces_block<kPress, kVisc>(f);
 }
 
 // meshMove.f90:378-389, one set
@@ -510,9 +429,8 @@ void launch_forces(int nedge, const int* iset, const double* X, const double* Y,
     auto go = [&](auto press, auto vis) {
         constexpr bool kP = decltype(press)::value, kV = decltype(vis)::value;
         if (nb <= kForcesOne) {
-            const int threads = 64 * std::max(5, nb);
-            k_forces_one<kP, kV><<<1, threads, 0, s>>>(nedge, iset, X, Y, P, xref, yref, v, out3,
-                                                       out2, zero4);
+            k_forces_one<kP, kV><<<1, 64 * std::max(5, nb), 0, s>>>(
+                ForceIn{nedge, iset, X, Y, P, xref, yref, v, out3, out2, zero4});
             return;
         }
         k_forces_part<kP, kV><<<nb, 64, 0, s>>>(nedge, iset, X, Y, P, xref, yref, v, part);

@@ -96,3 +96,29 @@ def test_fp64_step_from_the_oracle(moving, pe, block):
             a, b = got[name][:, k], ref[name][:, k]
             assert np.linalg.norm(a - b) <= 1e-12 * np.linalg.norm(b), (name, k)
     assert got["DTMIN"] == ref["DTMIN"] and got["TIME"] == ref["TIME"]
+
+
+@pytest.mark.parametrize("nr, nt, precision, viscous", [
+    (9, 33, 0, True), (24, 64, 1, True), (20, 65, 0, False), (150, 512, 0, True),
+    (150, 513, 1, True), (30, 96, 2, True),
+])
+def test_forces_of_many_steps_in_one_call(nr, nt, precision, viscous):
+    """The steps of one call leave their forces to the next step's deltat (up to
+    512 edges): after every number of steps they are those of steps called one
+    by one, with and without FORCE_VISC, bit for bit."""
+    from cfd_amd.solver import Session
+    cs = cylinder_case(nr, nt)
+    if not viscous:
+        cs.fmu = cs.fk = 0.0
+    print(f"forces on {nt} edges, precision {precision}", flush=True)
+    one, many = Session(cs, precision=precision), Session(cs, precision=precision)
+    names = ("FX1", "FY1", "RM1", "FVX1", "FVY1", "PCG_ITX", "PCG_ITY", "TIME")
+    for n in (1, 2, 5, 1):
+        for _ in range(n):
+            one.step(1)
+        many.step(n)
+        a, b = one.scalars(), many.scalars()
+        assert np.isfinite([a[k] for k in names]).all()
+        assert [a[k] for k in names] == [b[k] for k in names]
+    # (after the first step the pressure is uniform and its force closes to 0)
+    assert a["FX1"] != 0.0 and (a["FVX1"] != 0.0) == viscous
