@@ -774,12 +774,13 @@ struct cfd_session {
         bc.normales(X.p, Y.p, s);
         ElemTerms x;
         x.lapw = LAPW.p;
-        launch_deriv(t, X.p, Y.p, AREA.p, DNX.p, DNY.p, HH.p, HHX.p, HHY.p, scal(CFD_S_HMIN),
-                     partials.p, s, x);
+        launch_deriv(t, X.p, Y.p, AREA.p, DNX.p, DNY.p, HH.p, HHX.p, HHY.p, nullptr, partials.p, s,
+                     x);
         refresh_patch_geometry();
         launch_laplace(t, LAPW.p, DNX.p, DNY.p, LAP.p, LDIAG.p, s, ell_on ? &ell : nullptr,
-                       NodeMass{M.p, AREA.p, nullptr, nullptr});
+                       NodeMass{M.p, AREA.p, nullptr, nullptr}, hmin_fold());
     }
+    HminFold hmin_fold() { return {partials.p, scal(CFD_S_HMIN), (int)grid_for(ne)}; }
 
     // the fused paths' ESTAB outputs (patch order)
     template <class R>
@@ -864,9 +865,9 @@ struct cfd_session {
         CFD_HIP(hipGetLastError());
     }
 
-    // FORCES (and FORCE_VISC: the viscous terms) of a mesh at rest as one block's
-    // work, with the solves' zero counts
-    ForceIn still_forces() {
+    // FORCES (and FORCE_VISC: the viscous terms) as one block's work, with the zero
+    // counts of the solves of a mesh at rest
+    ForceIn force_in() {
         return ForceIn{d.nsetedges, ISET.p, X.p, Y.p, P.p, d.xref, d.yref,
                        ViscIn{m->t.inpoel.p, T.p, VX.p, VY.p, DNX.p, DNY.p, c.t_inf},
                        scal(CFD_S_FX), scal(CFD_S_FVX), scal(CFD_S_PCG_ITX)};
@@ -888,7 +889,7 @@ struct cfd_session {
         const double* wy = fu ? WY.p : nullptr;
         const bool in_patches = fused() && patches.npatch <= (int)partials.n;
         const bool fold_ctl = in_patches && d.itlocal == 0 && patches.npatch <= kStepFoldMax;
-        const ForceIn due = still_forces();
+        const ForceIn due = force_in();
         const int nb = in_patches
                            ? launch_deltat_patch(patches, c, AREA.p, T.p, VX.p, VY.p, wx, wy,
                                                  DT.p, partials.p, s, fold_ctl ? ctl.p : nullptr,
@@ -970,17 +971,21 @@ struct cfd_session {
         static_assert(CFD_S_PCG_ITY == CFD_S_PCG_ITX + 1 && CFD_S_PCG_RZX == CFD_S_PCG_ITX + 2 &&
                           CFD_S_PCG_RZY == CFD_S_PCG_ITX + 3,
                       "mesh-solve scalars are contiguous");
-        forces_due = more && still && in_patches && d.nsetedges > 0 &&
-                     d.nsetedges <= 64 * kForcesOne;
-        if (!forces_due)
+        // TRANSF's displacements reach the solves only through moving nodes
+        const bool transf = !still && d.nmove > 0;
+        const bool one = d.nsetedges > 0 && d.nsetedges <= 64 * kForcesOne;
+        forces_due = more && still && in_patches && one;
+        if (!forces_due && !(transf && one))
             launch_forces(d.nsetedges, ISET.p, X.p, Y.p, P.p, d.xref, d.yref, scal(CFD_S_FX),
                           fvisc && still ? &visc : nullptr, scal(CFD_S_FVX), FPART.p,
                           still ? scal(CFD_S_PCG_ITX) : nullptr, s);
+        if (transf) {
+            ForceIn f = force_in();
+            f.zero4 = nullptr;
+            launch_transf(d.nsetedges, ISET.p, X.p, Y.p, scal(X_CA), 0.0, d.xref, d.yref, DXPOS.p,
+                          DYPOS.p, s, one ? &f : nullptr);
+        }
         if (!still) {
-            // TRANSF's displacements reach the solves only through moving nodes
-            if (d.nmove > 0)
-                launch_transf(d.nsetedges, ISET.p, X.p, Y.p, scal(X_CA), 0.0, d.xref, d.yref,
-                              DXPOS.p, DYPOS.p, s);
             mesh_solves();
             move_normalized = true;
             if (fvisc)
@@ -995,12 +1000,12 @@ struct cfd_session {
             tb(CFD_K_GEOM);
             if (d.gcl >= 0) {
                 bc.normales(X.p, Y.p, s);
-                launch_deriv(t, X.p, Y.p, AREA.p, DNX.p, DNY.p, HH.p, HHX.p, HHY.p,
-                             scal(CFD_S_HMIN), partials.p, s,
+                launch_deriv(t, X.p, Y.p, AREA.p, DNX.p, DNY.p, HH.p, HHX.p, HHY.p, nullptr,
+                             partials.p, s,
                              ElemTerms{LAPW.p, GCLT.p, AREA_OLD.p, WX.p, WY.p, WXO.p, WYO.p, d.gcl});
                 refresh_patch_geometry();
                 launch_laplace(t, LAPW.p, DNX.p, DNY.p, LAP.p, LDIAG.p, s, ell_on ? &ell : nullptr,
-                               NodeMass{M.p, nullptr, GCLT.p, dtmin});
+                               NodeMass{M.p, nullptr, GCLT.p, dtmin}, hmin_fold());
             } else {
                 geometry();
             }

@@ -190,8 +190,8 @@ struct ElemTerms {
     const double *Wx = nullptr, *Wy = nullptr, *Wxo = nullptr, *Wyo = nullptr;
     int mode = 0;
 };
-// deriv (subrutinas.f90:88-126); hmin_out: device double; partials holds
-// grid_for(nelem) doubles
+// deriv (subrutinas.f90:88-126); hmin_out: device double (null: left to
+// launch_laplace, see HminFold); partials holds grid_for(nelem) doubles
 void launch_deriv(const Tables& t, const double* X, const double* Y, double* area, double* dNx,
                   double* dNy, double* HH, double* HHX, double* HHY, double* hmin_out,
                   double* partials, hipStream_t s, const ElemTerms& x = ElemTerms{});
@@ -208,12 +208,19 @@ struct NodeMass {
     const double2* gcl = nullptr;
     const double* dt = nullptr;
 };
+// hmin from the partials that launch_deriv left, by one more block of laplace's
+// launch (out null: none)
+struct HminFold {
+    const double* partials = nullptr;
+    double* out = nullptr;
+    int nb = 0;
+};
 // mLaplace.f90:7-58 values (structure comes from Tables); ell (when given): the
 // ELL copy's values too (EllLap::refresh in the same pass)
 struct EllLap;
 void launch_laplace(const Tables& t, const double* lapw, const double* dNx, const double* dNy,
                     double* lap, double* diag, hipStream_t s, EllLap* ell = nullptr,
-                    const NodeMass& m = NodeMass{});
+                    const NodeMass& m = NodeMass{}, HminFold h = HminFold{});
 // gcl.f90:8-46 main; mode 0 = as written, 1 = corrected y-divergence; dt is a
 // device scalar
 void launch_gcl(const Tables& t, double* M, const double* Wx, const double* Wy,
@@ -607,10 +614,11 @@ size_t forces_part_size(int nedge);
 void launch_forces(int nedge, const int* iset, const double* X, const double* Y, const double* P,
                    double xref, double yref, double* out3, const ViscIn* visc, double* out2,
                    double* part, double* zero4, hipStream_t s);
-// cs: device scalars cos(alpha), sin(alpha)
+// cs: device scalars cos(alpha), sin(alpha); forces (when given): FORCES of at
+// most 64 kForcesOne edges in the same launch
 void launch_transf(int nedge, const int* iset, const double* X, const double* Y, const double* cs,
                    double yposr, double xref, double yref, double* DXPOS, double* DYPOS,
-                   hipStream_t s);
+                   hipStream_t s, const ForceIn* forces = nullptr);
 
 // ---------------------------------------------------------------------------
 // PCG (biconjGrad.f90:8-62)

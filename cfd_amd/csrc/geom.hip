@@ -150,8 +150,8 @@ __device__ inline void laplace_row(int r0, int s0, int s1, const int* __restrict
 }
 
 // laplace's rows, and the nodes' masses in the same pass over their elements:
-// MASAS, or the GCL's update from the terms that k_deriv left.  Blocks of one
-// wave in XCD order (a node's elements are its ring neighbours' too).
+// MASAS, or the GCL's update from the terms that k_deriv left; one more block
+// folds k_deriv's minima of HH (a launch of 4.7 us less).  Blocks of one wave in XCD order (a node's elements are its ring neighbours' too).
 //
 // Formed from the coordinates, gradients and W per node and element, in launches
 // of their own (laplace + GCL / laplace + MASAS), and so, k_deriv's 15 us more for
@@ -169,9 +169,15 @@ k_laplace(const int* __restrict__ esup1, const int* __restrict__ esup2,
           const int* __restrict__ rowptr, const int* __restrict__ lslot,
           const double* __restrict__ lapw, const double* __restrict__ dNx,
           const double* __restrict__ dNy, double* __restrict__ lap, double* __restrict__ diag,
-          int npoin, int width, double* __restrict__ ell, NodeMass m) {
+          int npoin, int width, double* __restrict__ ell, NodeMass m, HminFold h) {
     __shared__ double srow[kLapRow * kLapThreads];
-    const int i = xcd_block(blockIdx.x, gridDim.x) * kLapThreads + threadIdx.x;
+    const int nblk = (npoin + kLapThreads - 1) / kLapThreads;
+    if ((int)blockIdx.x == nblk) {  // subrutinas.f90:124-125: hmin = min(minval(HH), 1e10)
+        const double v = combine_partials(h.partials, h.nb, __builtin_huge_val(), OpMin());
+        if (threadIdx.x == 0) *h.out = v > 1.0e10 ? 1.0e10 : v;
+        return;
+    }
+    const int i = xcd_block(blockIdx.x, nblk) * kLapThreads + threadIdx.x;
     if (i >= npoin) return;
     const int r0 = rowptr[i], len = rowptr[i + 1] - r0, s0 = esup2[i], s1 = esup2[i + 1];
     double tot1 = 0.0, tot2 = 0.0;
@@ -336,11 +342,17 @@ k_forces_one(ForceIn f) {
     forces_block<kPress, kVisc>(f);
 }
 
-// meshMove.f90:378-389, one set
-__global__ void k_transf(int nedge, const int* __restrict__ iset, const double* __restrict__ X,
-                         const double* __restrict__ Y, const double* __restrict__ cs,
-                         double yposr, double xref, double yref, double* __restrict__ DXPOS,
-                         double* __restrict__ DYPOS) {
+// meshMove.f90:378-389, one set; kForces: the last block forms FORCES instead (two
+// chains of loads side by side: a step of a small moving mesh 4.4 us less)
+template <bool kForces>
+__global__ void __launch_bounds__(kBlock)
+k_transf(int nedge, const int* __restrict__ iset, const double* __restrict__ X,
+         const double* __restrict__ Y, const double* __restrict__ cs, double yposr, double xref,
+         double yref, double* __restrict__ DXPOS, double* __restrict__ DYPOS, ForceIn forces) {
+    if (kForces && blockIdx.x == gridDim.x - 1) {
+        forces_block<true, false>(forces);
+        return;
+    }
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= nedge) return;
     const double ca = cs[0], sa = cs[1];
@@ -362,7 +374,8 @@ void launch_deriv(const Tables& t, const double* X, const double* Y, double* are
     const auto kernel = x.gcl ? k_deriv<true> : k_deriv<false>;
     kernel<<<g, kBlock, 0, s>>>(t.inpoel.p, X, Y, area, dNx, dNy, HH, HHX, HHY, t.nelem, partials, x);
     // hmin = minval(HH), capped at 1e10 (subrutinas.f90:124-125)
-    k_min_finalize<<<1, 256, 0, s>>>(partials, (int)g, __builtin_huge_val(), 1.0e10, hmin_out);
+    if (hmin_out)
+        k_min_finalize<<<1, 256, 0, s>>>(partials, (int)g, __builtin_huge_val(), 1.0e10, hmin_out);
     CFD_HIP(hipGetLastError());
 }
 
@@ -378,11 +391,12 @@ void launch_lap_weights(const Tables& t, const double* X, const double* Y, doubl
 }
 
 void launch_laplace(const Tables& t, const double* lapw, const double* dNx, const double* dNy,
-                    double* lap, double* diag, hipStream_t s, EllLap* ell, const NodeMass& m) {
+                    double* lap, double* diag, hipStream_t s, EllLap* ell, const NodeMass& m, HminFold h) {
     const auto kernel = m.gcl ? k_laplace<kMassGcl> : m.area ? k_laplace<kMassMasas> : k_laplace<kMassNone>;
-    kernel<<<(t.npoin + kLapThreads - 1) / kLapThreads, kLapThreads, 0, s>>>(t.esup1.p, t.esup2.p, t.rowptr.p, t.lslot.p, lapw,
+    const int nblk = (t.npoin + kLapThreads - 1) / kLapThreads + (h.out ? 1 : 0);
+    kernel<<<nblk, kLapThreads, 0, s>>>(t.esup1.p, t.esup2.p, t.rowptr.p, t.lslot.p, lapw,
                                                 dNx, dNy, lap, diag, t.npoin, ell ? ell->width : 0,
-                                                ell ? ell->val.p : nullptr, m);
+                                                ell ? ell->val.p : nullptr, m, h);
     CFD_HIP(hipGetLastError());
 }
 
@@ -444,10 +458,11 @@ void launch_forces(int nedge, const int* iset, const double* X, const double* Y,
 
 void launch_transf(int nedge, const int* iset, const double* X, const double* Y, const double* cs,
                    double yposr, double xref, double yref, double* DXPOS, double* DYPOS,
-                   hipStream_t s) {
+                   hipStream_t s, const ForceIn* forces) {
     if (nedge == 0) return;
-    k_transf<<<grid_for(nedge), kBlock, 0, s>>>(nedge, iset, X, Y, cs, yposr, xref, yref, DXPOS,
-                                                DYPOS);
+    const auto kernel = forces ? k_transf<true> : k_transf<false>;
+    kernel<<<grid_for(nedge) + (forces ? 1 : 0), kBlock, 0, s>>>(
+        nedge, iset, X, Y, cs, yposr, xref, yref, DXPOS, DYPOS, forces ? *forces : ForceIn{});
     CFD_HIP(hipGetLastError());
 }
 
