@@ -340,8 +340,10 @@ struct EllRows {
 
 // r = -1*(A x) + b with fixed rows y = 1e30 x and r(fix) = 0; partials of r.r
 // and, in relative mode, of rd.rd and rd.(rd/diag) for the residual rd of the
-// guess that is zero off the fixed nodes
-template <class Rows, int NS>
+// guess that is zero off the fixed nodes.  kFirst: the first preconditioned
+// residual too, z = r/diag with the partials of r.z (used only when the first
+// test does not end the solve; a launch of its own for it costs 4.5 us)
+template <class Rows, int NS, bool kFirst>
 __global__ void __launch_bounds__(kBlock)
 k_cg_residual(int n, Rows rows, const double* __restrict__ diag, CgBoth sys, int rel, int nb) {
     const CgArgs<NS> a(sys);
@@ -368,7 +370,7 @@ k_cg_residual(int n, Rows rows, const double* __restrict__ diag, CgBoth sys, int
 #pragma unroll
     for (int k = 0; k < NS; ++k) {
         const CgSys& q = a.s[k];
-        double v = 0.0, vdr = 0.0, vdz = 0.0;
+        double v = 0.0, vdr = 0.0, vdz = 0.0, vz = 0.0;
         if (act) {
             double ri = 0.0;
             if (row[k]) {
@@ -381,8 +383,14 @@ k_cg_residual(int n, Rows rows, const double* __restrict__ diag, CgBoth sys, int
             }
             q.r[i] = ri;
             v = ri * ri;
+            if (kFirst) {
+                const double zi = ri / diag[i];
+                q.z[i] = zi;
+                vz = ri * zi;
+            }
         }
         block_partial(v, OpSum(), q.prr, lb);
+        if (kFirst) block_partial(vz, OpSum(), q.prz, lb);
         if (rel) {
             block_partial(vdr, OpSum(), q.prr + nb, lb);
             block_partial(vdz, OpSum(), q.prr + 2 * nb, lb);
@@ -413,26 +421,6 @@ k_cg_test(CgBoth a, int nb, int rel) {
             scal[S_CONV] = 1.0;
             scal[S_EOLD] = rr;
         }
-    }
-}
-
-// first preconditioned residual: z = r/diag, partials of r.z
-template <int NS>
-__global__ void __launch_bounds__(kBlock)
-k_cg_first_z(int n, const double* __restrict__ diag, CgBoth sys) {
-    const CgArgs<NS> a(sys);
-    const int i = blockIdx.x * kBlock + threadIdx.x;
-#pragma unroll
-    for (int k = 0; k < NS; ++k) {
-        const CgSys& q = a.s[k];
-        if (q.scal[S_DONE] != 0.0) continue;  // uniform over the grid
-        double v = 0.0;
-        if (i < n) {
-            double zi = q.r[i] / diag[i];
-            q.z[i] = zi;
-            v = q.r[i] * zi;
-        }
-        block_partial(v, OpSum(), q.prz);
     }
 }
 
@@ -785,7 +773,7 @@ void pcg_initial_rr(const PcgSystem (&sys)[2], int npoin, const double* A, const
     for (auto& q : a.s) q.x = q.z;
     if (nfix > 0) k_cg_fix<1><<<dim3(grid_for(nfix), 2), kBlock, 0, s>>>(a);
     with_rows(npoin, A, idx, rowptr, ell, [&](auto rows) {
-        k_cg_residual<decltype(rows), 1><<<dim3(nb, 2), kBlock, 0, s>>>(npoin, rows, diag, a, 0, nb);
+        k_cg_residual<decltype(rows), 1, false><<<dim3(nb, 2), kBlock, 0, s>>>(npoin, rows, diag, a, 0, nb);
     });
     k_cg_rr<<<2, 256, 0, s>>>(a, nb, rr_out);
     CFD_HIP(hipGetLastError());
@@ -901,14 +889,12 @@ struct CgLaunch {
         k_cg_init<NS><<<g, blk, 0, s>>>(n, q, tol, maxit);
         const int nfix = std::max(q.s[0].nfix, q.s[1].nfix);
         if (nfix > 0) k_cg_fix<NS><<<dim3(grid_for(nfix), rows_y), blk, 0, s>>>(q);
-        k_cg_residual<Rows, NS><<<g, blk, 0, s>>>(n, rows, diag, q, rel, nb);
+        k_cg_residual<Rows, NS, true><<<g, blk, 0, s>>>(n, rows, diag, q, rel, nb);
         k_cg_test<<<NS * rows_y, 256, 0, s>>>(q, nb, rel);
-        k_cg_first_z<NS><<<g, blk, 0, s>>>(n, diag, q);
     }
     void start(const CgBoth& q, int nsys, double tol, int maxit, int rel) const {
         if (apart(nsys)) start_ns<1>(q, nsys, tol, maxit, rel);
         else start_ns<2>(q, 1, tol, maxit, rel);
-        b(q, nsys, 1);
     }
     template <int NS>
     void a_ns(const CgBoth& q, int rows_y, int both) const {
@@ -1312,7 +1298,12 @@ void pcg_launch_multi(const PcgSystem* sys, int nsys, int npoin, const double* A
     };
     with_rows(npoin, A, idx, rowptr, ell, [&](auto rows) {
         const CgLaunch<decltype(rows)> go{npoin, nb, rows, diag, s};
-        go.start(args(), nsys, tol, maxit, rel);  // p0 = z0 into pbuf[0]
+        go.start(args(), nsys, tol, maxit, rel);
+        // the first poll before the first product, which only solves that go on
+        // need: a solve that the first test ends is known 5 us earlier
+        int chunk = 4, slot = 0;
+        ask(slot);
+        go.b(args(), nsys, 1);  // p0 = z0 into pbuf[0]
         cur = 0;
         CFD_HIP(hipGetLastError());
         int both = 0;
@@ -1332,9 +1323,7 @@ void pcg_launch_multi(const PcgSystem* sys, int nsys, int npoin, const double* A
         // about 15 us, the batch queued in vain at the end about 50.
         constexpr long kAsyncFrom = 128;
         constexpr int kAsyncBatch = 8;
-        int chunk = 4, slot = 0;
         long launched = 0;
-        ask(slot);
         while (!told(slot)) {
             CFD_CHECK(launched <= 4L * maxit + 64, "PCG did not terminate");
             if (pinned && launched >= kAsyncFrom) break;
