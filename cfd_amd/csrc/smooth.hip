@@ -360,7 +360,9 @@ struct SmNode {
 // one follows that far behind, taking the positions and marks that it left.
 // Every update then reads exactly the values and marks that it would read with
 // the passes one after the other.  Block 0 waits for nothing and block w only
-// for block w - 1, which was started before it, so each wait ends.  On a ring by
+// for block w - 1, and the twelve blocks of every launch in flight (one a stream,
+// a few streams on the hardware's queues) are far fewer than the CUs: each has a
+// CU as soon as other kernels' blocks leave one, so each wait ends.  On a ring by
 // ring numbering the passes run one ring and a chunk apart; on one where every
 // node has a far neighbour they run one after the other.
 //
