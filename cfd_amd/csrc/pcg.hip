@@ -398,6 +398,14 @@ k_cg_residual(int n, Rows rows, const double* __restrict__ diag, CgBoth sys, int
     }
 }
 
+// The first residual test.  A residual that is exactly zero ends the solve too: in
+// relative mode the threshold is zero where the residual that it refers to is (no
+// fixed node displaced and b = 0, or every row fixed).
+__device__ __forceinline__ bool cg_solved(double rr, double tolr) { return rr < tolr || rr == 0.0; }
+// The step length e / p.y; none where a residual that has become exactly zero has
+// left no direction (p and p.y are zero then, or underflowed to it).
+__device__ __forceinline__ double cg_step(double e, double py) { return py == 0.0 ? 0.0 : e / py; }
+
 // the first residual test (block k: system k)
 __global__ void __launch_bounds__(256)
 k_cg_test(CgBoth a, int nb, int rel) {
@@ -416,7 +424,7 @@ k_cg_test(CgBoth a, int nb, int rel) {
         scal[S_TOLR] = tolr;
         scal[S_TOLZ] = tolz;
         scal[S_RR] = rr;
-        if (rr < tolr) {
+        if (cg_solved(rr, tolr)) {
             scal[S_DONE] = 1.0;
             scal[S_CONV] = 1.0;
             scal[S_EOLD] = rr;
@@ -444,7 +452,7 @@ struct CgScalars {
 // A's step length, and whether the loop goes on
 __device__ __forceinline__ double cg_alfa(const CgScalars& c, double py, bool& more) {
     more = fabs(c.enew) > c.tolz && c.k < c.maxit;
-    return c.enew / py;
+    return cg_step(c.enew, py);
 }
 
 // Kernel A of an iteration (see the file header).  both: x takes the previous
@@ -1128,7 +1136,7 @@ k_cg_whole(int n, EllMat m, const double* __restrict__ diag, CgBoth sys, double 
     const double rr = total(0);
     const double tolr = rel ? tol * tol * total(1) : tol, tolz = rel ? tol * tol * total(2) : tol;
     double e = rr, k = 0.0, conv = 1.0;
-    if (!(rr < tolr)) {
+    if (!cg_solved(rr, tolr)) {
         __syncthreads();  // sums are read
 #pragma unroll
         for (int s = 0; s < kR; ++s) {
@@ -1166,7 +1174,7 @@ k_cg_whole(int n, EllMat m, const double* __restrict__ diag, CgBoth sys, double 
             put(1, v);
             __syncthreads();
             // A: x += alfa p, r -= alfa y, z = r / diag
-            const double alfa = e / total(1), eold = e;
+            const double alfa = cg_step(e, total(1)), eold = e;
             const bool more = fabs(e) > tolz && k < (double)maxit;
 #pragma unroll
             for (int s = 0; s < kR; ++s) {
