@@ -113,18 +113,23 @@ struct cfd_batch {
             nes[k] = ebase[k + 1] - ebase[k];
             nps[k] = nbase[k + 1] - nbase[k];
         }
-        build_patches_batch(patches, ncases, ip.data(), xs.data(), ys.data(), nes.data(), nps.data(),
-                            pe, block, precision == 1, s);
-        patches.cases = cases.p;
+        // beside the present ones: a shape that does not fit leaves the batch as it is
+        PatchSet ps;
+        build_patches_batch(ps, ncases, ip.data(), xs.data(), ys.data(), nes.data(), nps.data(), pe,
+                            block, precision == 1, s);
+        ps.cases = cases.p;
         std::vector<int> base(1, 0);
         for (int k = 0; k < ncases; ++k) base.push_back(base.back() + (nes[k] + pe - 1) / pe);
-        CFD_CHECK(base.back() == patches.npatch, "internal: batch patches");
-        pb.alloc(base.size());
-        pb.upload(base.data(), base.size(), s);
-        partials.alloc(std::max<size_t>(grid_for(ne), patches.npatch));
+        CFD_CHECK(base.back() == ps.npatch, "internal: batch patches");
+        DBuf<int> pb_new(base.size());
+        pb_new.upload(base.data(), base.size(), s);
+        DBuf<double> part_new(std::max<size_t>(grid_for(ne), ps.npatch));
         CFD_HIP(hipStreamSynchronize(s));
+        drop_graphs();  // they name the present ones
+        patches = std::move(ps);
+        pb = std::move(pb_new);
+        partials = std::move(part_new);
         refresh_patch_geometry();
-        drop_graphs();
     }
 
     // One time step of every case (ns2DComp.ALE.f90:140-182 on a fixed mesh)

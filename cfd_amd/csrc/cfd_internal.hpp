@@ -87,11 +87,11 @@ struct DBuf {
         return *this;
     }
     ~DBuf() { release(); }
+    // empty when the allocation fails: callers that keep a buffer go by its n
     void alloc(size_t count) {
         release();
-        n = count;
-        owned = true;
         if (count) CFD_HIP(hipMalloc(&p, sizeof(T) * count));
+        n = count;
     }
     void borrow(T* ptr, size_t count) {
         release();

@@ -839,8 +839,8 @@ void EllLap::refresh(const int* rowptr, const double* A, hipStream_t s) {
 }
 
 void PcgWork::ensure(int npoin) {
-    if (npoin == n && r.p) return;
-    n = npoin;
+    if (npoin == n) return;
+    n = 0;  // until every part is there
     nblocks = (int)grid_for(npoin);
     r.alloc(npoin);
     z.alloc(npoin);
@@ -853,6 +853,7 @@ void PcgWork::ensure(int npoin) {
     hpin.alloc(2 * S_NSCAL);
     for (auto& e : ev)
         if (!e) CFD_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    n = npoin;
 }
 
 PcgWork::~PcgWork() {

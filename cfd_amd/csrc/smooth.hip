@@ -675,14 +675,14 @@ bool smooth_check(const Tables& t, SmoothPlan& plan, double* X, double* Y, doubl
 // order 0 (see k_sm_passes)
 static int smooth_run_seq(const Tables& t, SmoothPlan& plan, const SmDev& d, hipStream_t s) {
     const int n = t.npoin, nw = sm_words(n);
-    if (plan.ring.n != 9 * (size_t)t.nelem) {  // kept with the mesh's plan
-        plan.ring.alloc(9 * (size_t)t.nelem);
+    if (plan.ring.n != 9 * (size_t)t.nelem) {  // kept with the mesh's plan (ring, the last: all of it)
         plan.need.alloc(n);
         plan.xy.alloc(n);
         plan.hist.alloc((size_t)kSmPasses * n);
         plan.dmax_pass.alloc(kSmPasses);
         plan.rows.alloc((size_t)(kSmPasses + 2) * nw);
         plan.prog.alloc(kSmPasses);
+        plan.ring.alloc(9 * (size_t)t.nelem);
     }
     k_sm_ring<<<grid_for(n), kBlock, 0, s>>>(t.inpoel.p, t.esup1.p, t.esup2.p, plan.ring.p,
                                              plan.need.p, n);
