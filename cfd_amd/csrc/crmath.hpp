@@ -7,17 +7,24 @@
 //   recip(b)       Newton's iteration on the hardware's reciprocal;
 //   quot(a, r)     q = a r, corrected by its exact remainder a - b q (Markstein,
 //                  "Computation of elementary functions on the IBM RISC
-//                  System/6000 processor", 1990); zeros, infinities and NaNs as
-//                  '/' gives them;
+//                  System/6000 processor", 1990);
 //   third(a)       a / 3 from the rounded constant 1/3, the same way;
 //   sqrt_rn(x)     Goldschmidt's iteration on the hardware's reciprocal square
 //                  root, corrected twice by the exact remainder x - s^2.
-// Exponents: quot is exact for |a|, |b| and |a/b| within 2^+-900 or so (a
-// remainder below the smallest normal number would be lost); sqrt_rn hands x
-// below 2^-700 to sqrt().  Instructions: '/' 11, quot 4 and recip 5, third 4;
-// sqrt() 17, sqrt_rn 12.  Compared with '/' and sqrt() on gfx950 over 5 10^8
-// random operands in each of five exponent ranges up to 2^+-450: no
-// difference.
+// Where quot is not '/': a dividend below 2^-968 (2.5e-292; its remainder is a
+// multiple of 2^-106 |a| and would have to be one of 2^-1074) may give an ulp more or
+// less, and a divisor of at most 2^-1024 gives an infinity for every dividend but
+// zero.  Quotients that overflow, zeros, infinities and NaNs are as '/' gives them.
+// Callers divide by states (density, temperature), lengths, time steps and norms
+// kept above 1e-20, or a constant by a sum of velocities (where '/' overflows too);
+// a dividend that small is a momentum or a product of velocities, far from what
+// moves in a gas at rest, and its ulp is that of a velocity of 1e-292 or is lost in
+// what it is added to.  On gfx950 over 1.4 10^6 pairs from all of the exponent range,
+// subnormal numbers included: no other difference (third: none).
+// sqrt_rn hands x below 2^-700 to sqrt().  Compared with '/' and sqrt() on gfx950
+// over 5 10^8 random operands in each of five exponent ranges up to 2^+-450: no
+// difference.  Instructions: '/' 11, quot 4 and recip 5, third 4; sqrt() 17,
+// sqrt_rn 12.
 //
 // The powers are correctly rounded (round to nearest) up to a 2^-100 relative
 // window around rounding midpoints: each starts from an approximation and adds
