@@ -26,15 +26,16 @@
 // difference.  Instructions: '/' 11, quot 4 and recip 5, third 4; sqrt() 17,
 // sqrt_rn 12.
 //
-// The powers are correctly rounded (round to nearest) up to a 2^-100 relative
-// window around rounding midpoints: each starts from an approximation and adds
-// one correction carried in double-double with error-free products (fma), so
-// the approximation's own last bits do not reach the result:
-//   x^(-1/2) = y (1 + r/2),   r = 1 - x y^2 (exact to 2^-106)
-//   x^(3/2)  = x * sqrt(x),   sqrt(x) = s + (x - s*s)/(2 s), s = x y
+// The powers are correctly rounded (round to nearest) up to a 2^-103 relative
+// window around rounding midpoints, and exactly where x^(3/2) is a midpoint (x a
+// square): each starts from an approximation and adds one correction carried in
+// double-double with error-free products (fma):
+//   x^(-1/2) = y (1 + r/2 + 3 r^2/8),   r = 1 - x y^2 (exact to 2^-103)
+//   x^(3/2)  = x * sqrt(x),   sqrt(x) = s + (x - s*s) h
 // with y from the hardware's reciprocal square root and one third-order step
-// (relative error about 2^-52; the corrections' neglected terms are y's error
-// squared).  They replace pow(x, 1.5) (calcRHS.f90:50-51, subrutinas.f90:196,400)
+// (relative error about 2^-52), s = sqrt(x) correctly rounded (an s an ulp off
+// misrounds 2,772 of the 27,040 squares whose 3/2 power is a midpoint) and
+// h = 1/(2 s) within an ulp.  They replace pow(x, 1.5) (calcRHS.f90:50-51, subrutinas.f90:196,400)
 // and pow(x, -0.5) (subrutinas.f90:429,438-439): fewer instructions than a
 // general pow, and closer to the exact value than either the device pow or
 // glibc's.
@@ -61,15 +62,21 @@ __device__ __forceinline__ double quot(double a, const Recip& k) {
 __device__ __forceinline__ double quot(double a, double b) { return quot(a, recip(b)); }
 __device__ __forceinline__ double third(double a) { return quot(a, Recip{3.0, 1.0 / 3.0}); }
 
-__device__ __forceinline__ double sqrt_rn(double x) {
-    if (__any(x < 0x1p-700 && x != 0.0)) return sqrt(x);
+// sqrt(x), correctly rounded, for x > 2^-700; h: 1/(2 sqrt(x)) within 2^-44
+__device__ __forceinline__ double sqrt_core(double x, double& h) {
     const double y = __builtin_amdgcn_rsq(x);
-    double s = x * y, h = 0.5 * y;
+    double s = x * y;
+    h = 0.5 * y;
     const double e = __builtin_fma(-h, s, 0.5);
     s = __builtin_fma(s, e, s);
     h = __builtin_fma(h, e, h);
     s = __builtin_fma(__builtin_fma(-s, s, x), h, s);
-    s = __builtin_fma(__builtin_fma(-s, s, x), h, s);
+    return __builtin_fma(__builtin_fma(-s, s, x), h, s);
+}
+__device__ __forceinline__ double sqrt_rn(double x) {
+    if (__any(x < 0x1p-700 && x != 0.0)) return sqrt(x);
+    double h;
+    const double s = sqrt_core(x, h);
     return x == 0.0 || x == __builtin_huge_val() ? x : s;
 }
 
@@ -82,11 +89,10 @@ __device__ __forceinline__ double rsqrt_near(double x, double* edge) {
 }
 
 __device__ __forceinline__ double pow_3_2(double x) {
-    double edge;
-    const double y = rsqrt_near(x, &edge);
-    const double s = x * y;
-    const double d = __builtin_fma(-s, s, x);
-    const double sl = d * (0.5 * y);
+    double h;
+    const double s = sqrt_core(x, h);
+    h = __builtin_fma(h, __builtin_fma(-h, s, 0.5), h);
+    const double sl = __builtin_fma(-s, s, x) * h;  // sqrt(x) = s + sl
     const double p = x * s;
     const double pe = __builtin_fma(x, s, -p);  // x*s = p + pe, exact
     const double r = p + (pe + x * sl);
@@ -99,7 +105,7 @@ __device__ __forceinline__ double pow_m1_2(double x) {
     const double p = y * y, pe = __builtin_fma(y, y, -p);   // y^2 = p + pe
     const double q = x * p, qe = __builtin_fma(x, p, -q);   // x p = q + qe
     const double r = ((1.0 - q) - qe) - x * pe;             // 1 - x y^2
-    const double z = y + y * (0.5 * r);
+    const double z = y + y * (r * __builtin_fma(r, 0.375, 0.5));
     // 0 -> inf, inf -> 0, NaN -> NaN as pow(x, -0.5) gives for x >= 0
     return (x == 0.0 || !(x < __builtin_huge_val())) ? edge : z;
 }
