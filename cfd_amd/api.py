@@ -191,6 +191,11 @@ class MeshContext:
         """smoothing.f90:386-401 setTol_move: tol_move = |dX| + |dY|"""
         check(lib().cfd_smoothing_set_tol_move(self._h, dptr(_f64(dX)), dptr(_f64(dY))))
 
+    def set_smoothing_wait(self, seconds):
+        """The longest that a pass of order 0 waits without progress of the one
+        before (default 10 s); smoothing then fails."""
+        check(lib().cfd_smoothing_set_wait(self._h, C.c_double(seconds)))
+
     def force_visc(self, iset, X, Y, P, T, VEL_X, VEL_Y, dNx, dNy, t_inf):
         """ns2DComp.ALE.f90:819-893 for one set of edges (n1, n2, elem):
         (F_VX, F_VY)"""

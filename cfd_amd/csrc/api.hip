@@ -359,6 +359,13 @@ int cfd_smoothing_set_tol_move(cfd_mesh* m, const double* dX, const double* dY) 
     })
 }
 
+int cfd_smoothing_set_wait(cfd_mesh* m, double seconds) {
+    CFD_TRY({
+        CFD_ARG(m && seconds > 0.0 && seconds <= 3600.0, "seconds must be in (0, 3600]");
+        m->smooth.wait_s = seconds;
+    })
+}
+
 int cfd_smoothing(cfd_mesh* m, double* X, double* Y, const int* fixed, const double* dX,
                   const double* dY, int order, int* sweeps, double* hmin) {
     CFD_TRY({

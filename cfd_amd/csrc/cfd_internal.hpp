@@ -516,6 +516,7 @@ constexpr int kSmoothSeqMaxNodes = 65536;  // order 0 (a wave per pass) above th
 struct SmoothPlan {
     int max_elems = 0;              // most elements around one node
     double hmin = 1.0;              // H_MIN_GLOBAL of the last check
+    double wait_s = 10.0;           // order 0: the longest wait without progress
     std::vector<int> colour_ptr;    // free nodes of colour c: colour_nodes[ptr[c], ptr[c+1])
     DBuf<int> colour_nodes, fixed, smoothable;
     DBuf<double> dmove, partials, scal;

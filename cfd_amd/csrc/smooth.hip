@@ -362,9 +362,12 @@ struct SmNode {
 // the passes one after the other.  Block 0 waits for nothing and block w only
 // for block w - 1, and the twelve blocks of every launch in flight (one a stream,
 // a few streams on the hardware's queues) are far fewer than the CUs: each has a
-// CU as soon as other kernels' blocks leave one, so each wait ends.  On a ring by
-// ring numbering the passes run one ring and a chunk apart; on one where every
-// node has a far neighbour they run one after the other.
+// CU as soon as other kernels' blocks leave one, so each wait ends.  Should one not
+// (its predecessor has no CU for so long, or is lost), the block gives up when it has
+// seen no progress for `limit`, says so behind prog, and the call fails; those behind
+// it see no progress either.  On a ring by ring numbering the passes run one ring and
+// a chunk apart; on one where every node has a far neighbour they run one after the
+// other.
 //
 // Marks: a sweep that moves node i marks its ring.  Nodes after i take their
 // turn in the same sweep (the block's own marks), those before i in the next
@@ -395,9 +398,10 @@ struct SmSeq {
     // rows of a bit per node: row 0 the marks before the first sweep, row w + 1
     // those that pass w leaves to the next; then the free nodes
     unsigned* rows;
-    int* prog;             // per pass: nodes done
+    int* prog;             // per pass: nodes done; then 1 when a pass gave up
     double* dmax;          // per pass: the largest squared move
     int n, npass, nlap;    // passes of the launch, Laplacian ones first
+    long long limit;       // of a wait without progress, ticks of wall_clock64()
 };
 __host__ __device__ constexpr int sm_words(int n) { return (n + 63) / 64 * 2; }
 
@@ -428,9 +432,23 @@ k_sm_passes(SmSeq q) {
             int need = in ? q.need[node] : 0;
             for (int off = 32; off > 0; off >>= 1) need = max(need, __shfl_xor(need, off, 64));
             if (w > 0) {
-                while (__hip_atomic_load(&q.prog[w - 1], __ATOMIC_RELAXED,
-                                         __HIP_MEMORY_SCOPE_AGENT) < need)
+                long long since = wall_clock64();
+                for (int at, seen = -1;;) {
+                    at = __builtin_amdgcn_readfirstlane(__hip_atomic_load(
+                        &q.prog[w - 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+                    if (at >= need) break;
+                    const long long now = wall_clock64();
+                    if (at != seen) {
+                        seen = at;
+                        since = now;
+                    } else if (now - since > q.limit) {
+                        if (lane == 0)
+                            __hip_atomic_store(&q.prog[kSmPasses], 1, __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_AGENT);
+                        return;
+                    }
                     __builtin_amdgcn_s_sleep(16);
+                }
                 __threadfence();
             }
             for (int i = taken + lane; i < need; i += 64) xy[i] = src[i];
@@ -505,7 +523,7 @@ k_sm_passes(SmSeq q) {
 __global__ void k_sm_rows(const int* __restrict__ smoothable, const int* __restrict__ fixed,
                           unsigned* __restrict__ rows, int* __restrict__ prog, int n, int last) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x, nw = sm_words(n);
-    if (i < kSmPasses) prog[i] = 0;
+    if (i <= kSmPasses) prog[i] = 0;
     if (i >= nw) return;
     unsigned m = 0, f = 0;
     for (int b = 0; b < 32 && 32 * i + b < n; ++b) {
@@ -681,7 +699,7 @@ static int smooth_run_seq(const Tables& t, SmoothPlan& plan, const SmDev& d, hip
         plan.hist.alloc((size_t)kSmPasses * n);
         plan.dmax_pass.alloc(kSmPasses);
         plan.rows.alloc((size_t)(kSmPasses + 2) * nw);
-        plan.prog.alloc(kSmPasses);
+        plan.prog.alloc(kSmPasses + 1);
         plan.ring.alloc(9 * (size_t)t.nelem);
     }
     k_sm_ring<<<grid_for(n), kBlock, 0, s>>>(t.inpoel.p, t.esup1.p, t.esup2.p, plan.ring.p,
@@ -696,6 +714,9 @@ static int smooth_run_seq(const Tables& t, SmoothPlan& plan, const SmDev& d, hip
     if (lds)
         CFD_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_sm_passes<true>),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)full));
+    int khz = 0;
+    CFD_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev));
+    const long long limit = (long long)(1.0e3 * khz * plan.wait_s);
     const double tol_dist = kSmTolDist * plan.hmin;
     const double2* result = plan.xy.p;
     int sweep = 0, nlap = 2, last = 0;
@@ -703,17 +724,21 @@ static int smooth_run_seq(const Tables& t, SmoothPlan& plan, const SmDev& d, hip
         const int nsw = std::min(kSmPasses - nlap, kSmSweeps - sweep), np = nlap + nsw;
         if (last > 0)  // the next passes start from the last one's positions
             CFD_HIP(hipMemcpyAsync(plan.xy.p, result, sizeof(double2) * n, hipMemcpyDeviceToDevice, s));
-        k_sm_rows<<<grid_for(std::max(nw, kSmPasses)), kBlock, 0, s>>>(
+        k_sm_rows<<<grid_for(std::max(nw, kSmPasses + 1)), kBlock, 0, s>>>(
             plan.smoothable.p, plan.fixed.p, plan.rows.p, plan.prog.p, n, last);
         const SmSeq q{d, plan.ring.p, plan.need.p, plan.xy.p, plan.hist.p, plan.rows.p,
-                      plan.prog.p, plan.dmax_pass.p, n, np, nlap};
+                      plan.prog.p, plan.dmax_pass.p, n, np, nlap, limit};
         if (lds) k_sm_passes<true><<<np, 64, full, s>>>(q);
         else k_sm_passes<false><<<np, 64, base, s>>>(q);
         CFD_HIP(hipGetLastError());
         last = np;
         double dmax[kSmPasses];
+        int lost = 0;
         CFD_HIP(hipMemcpyAsync(dmax, plan.dmax_pass.p, sizeof(dmax), hipMemcpyDeviceToHost, s));
+        CFD_HIP(hipMemcpyAsync(&lost, plan.prog.p + kSmPasses, sizeof(lost), hipMemcpyDeviceToHost, s));
         CFD_HIP(hipStreamSynchronize(s));
+        CFD_CHECK(!lost, "smoothing: a pass saw no progress of the one before for " +
+                             std::to_string(plan.wait_s) + " s");
         for (int k = nlap; k < np && !end; ++k) {
             ++sweep;
             end = dmax[k] < tol_dist;

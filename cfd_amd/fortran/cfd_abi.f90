@@ -237,6 +237,12 @@ module cfd_abi
             type(c_ptr), value :: m
             real(c_double), intent(in) :: dx(*), dy(*)
         end function
+        integer(c_int) function cfd_smoothing_set_wait(m, seconds) &
+                bind(c, name='cfd_smoothing_set_wait')
+            import :: c_int, c_ptr, c_double
+            type(c_ptr), value :: m
+            real(c_double), value :: seconds
+        end function
         ! RK (subrutinas.f90:645-849, NGAS = 0)
         integer(c_int) function cfd_rk(m, c, bc, nrk, dtmin, dtl, nodes, elems) &
                 bind(c, name='cfd_rk')

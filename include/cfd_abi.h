@@ -172,6 +172,10 @@ int cfd_smoothing(cfd_mesh *m, double *X, double *Y, const int *fixed, const dou
 /* smoothing_mod::setTol_move (smoothing.f90:386-401): tol_move = |dX| + |dY|
  * per node; the tol_move mode stays on for this mesh context */
 int cfd_smoothing_set_tol_move(cfd_mesh *m, const double *dX, const double *dY);
+/* order 0's passes follow each other on the GPU; a pass that has seen no progress
+ * of the one before for so long (default 10 s, kept with the mesh context) gives
+ * up: cfd_smoothing then fails with CFD_ERR_DEVICE and leaves X and Y as they were */
+int cfd_smoothing_set_wait(cfd_mesh *m, double seconds);
 
 /* BiconjGrad::biCG (biconjGrad.f90:8-62): Jacobi-PCG on a CSR matrix with
  * Dirichlet nodes; x is the initial guess in, the solution out.  Extensions
