@@ -1221,9 +1221,12 @@ void launch_whole(int n, const EllMat& m, const double* diag, const CgBoth& q, i
                   int maxit, int rel, hipStream_t s) {
     const auto kernel = k_cg_whole<kT, kW, kR, kKeep, kLds, kX>;
     const size_t lds = (size_t)n * ((kX ? 1 + kLds : 2 + kLds) * sizeof(double) + 1);
-    if (lds > 48 * 1024)
+    // the kernel's limit holds for the process: always that of its largest n, so
+    // that threads with systems of different sizes set the same
+    constexpr int kMost = std::min(kT * kR, kWholeRows) * ((kX ? 1 + kLds : 2 + kLds) * 8 + 1);
+    if (kMost > 48 * 1024)
         CFD_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, kMost));
     kernel<<<nsys, kT, lds, s>>>(n, m, diag, q, tol, maxit, rel);
     CFD_HIP(hipGetLastError());
 }

@@ -711,9 +711,9 @@ static int smooth_run_seq(const Tables& t, SmoothPlan& plan, const SmDev& d, hip
     CFD_HIP(hipGetDevice(&dev));
     CFD_HIP(hipDeviceGetAttribute(&most, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
     const bool lds = full <= (size_t)most;
-    if (lds)
+    if (lds)  // the limit holds for the process: the same for every mesh
         CFD_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_sm_passes<true>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)full));
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, most));
     int khz = 0;
     CFD_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev));
     const long long limit = (long long)(1.0e3 * khz * plan.wait_s);
