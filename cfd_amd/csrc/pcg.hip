@@ -234,6 +234,7 @@ __global__ void k_cg_fix(CgBoth sys) {
 // entries in CSR order, from the CSR arrays (staged; every thread of the
 // block calls it, rows without work with on = false) or the ELL copy.
 struct CsrRows {
+    static constexpr bool kFew = false, kMany = false, kAlone = false;
     const double* A;
     const int *idx, *rowptr;
     template <class F>
@@ -262,11 +263,14 @@ struct CsrRows {
 };
 // kW: most entries of a row; kShort: columns as 16-bit distances from the
 // row; kAhead: k_cg_b loads the entries (1), and gathers their p and z too
-// (2), ahead of the scalars
+// (2), ahead of the scalars.  The rows that with_rows takes each form for leave some
+// kernels without use: kFew: up to kFoldSmall partials, kMany: above, kAlone: a pair
+// of systems never shares a thread
 template <int kW, bool kShort, int kAhead>
 struct EllRows {
     EllMat m;
-    static constexpr bool kDeep = kAhead == 2;
+    static constexpr bool kDeep = kAhead == 2, kFew = kAhead > 0, kAlone = kDeep;
+    static constexpr bool kMany = kW == 8 && kShort && kAhead == 0;
     template <class F>
     __device__ __forceinline__ void visit(int n, int, int i, bool on, F f) const {
         if (!on) return;
@@ -751,6 +755,12 @@ CgSys cg_sys(const PcgSystem& q, int cur) {
 // 524,288 rows (bound by bandwidth: the registers cost waves) 21.2 / 31.9,
 // 24.7 / 38.6, 24.5 / 39.3.
 constexpr int kDeepRows = 160 * 1024, kAheadRows = 256 * 1024;
+// Two systems up to kRowsApart rows: a grid row of blocks each, since latency and
+// not the matrix's bytes is what an iteration costs (4,608 rows 12.6 us with both in
+// each thread); above, both in each thread, which reads the matrix once.
+constexpr int kRowsApart = 160 * 1024;
+static_assert(kAheadRows == kFoldSmall * kBlock && kDeepRows <= kRowsApart,
+              "the row readers' kFew, kMany and kAlone");
 // calls f with the row reader of the matrix: the ELL copy when there is one
 template <class F>
 void with_rows(int n, const double* A, const int* idx, const int* rowptr, const EllMat* ell, F f) {
@@ -878,11 +888,6 @@ struct CgLaunch {
     const double* diag;
     hipStream_t s;
     static constexpr bool kEll = !std::is_same<Rows, CsrRows>::value;
-    // Two systems up to kRowsApart rows: a grid row of blocks each, since
-    // latency and not the matrix's bytes is what an iteration costs (4,608
-    // rows 12.6 us with both in each thread); above, both in each thread,
-    // which reads the matrix once.
-    static constexpr int kRowsApart = 160 * 1024;
     // Up to kFoldSmall partials blocks of 256 threads that each combine them
     // all (4 loads a thread); up to kFoldMid blocks of 512 and up to kFoldMax
     // of 1024, so that fewer blocks read them (an iteration of one system /
@@ -890,7 +895,17 @@ struct CgLaunch {
     // 1024); above, the one-block kernels (524,288 rows: 23.0 / 34.7 us with
     // them, 19.8 / 31.2 without; 980,000 rows 38.8 / 57.5 either way).  CSR
     // rows are staged by 256 threads.
-    bool apart(int nsys) const { return nsys == 1 || n <= kRowsApart; }
+    // f(systems in a thread, grid rows of systems)
+    template <class F>
+    void shaped(int nsys, F f) const {
+        if constexpr (!Rows::kAlone) {
+            if (nsys == 2 && n > kRowsApart) {
+                f(std::integral_constant<int, 2>{}, 1);
+                return;
+            }
+        }
+        f(std::integral_constant<int, 1>{}, nsys);
+    }
 
     template <int NS>
     void start_ns(const CgBoth& q, int rows_y, double tol, int maxit, int rel) const {
@@ -902,8 +917,7 @@ struct CgLaunch {
         k_cg_test<<<NS * rows_y, 256, 0, s>>>(q, nb, rel);
     }
     void start(const CgBoth& q, int nsys, double tol, int maxit, int rel) const {
-        if (apart(nsys)) start_ns<1>(q, nsys, tol, maxit, rel);
-        else start_ns<2>(q, 1, tol, maxit, rel);
+        shaped(nsys, [&](auto ns, int y) { start_ns<decltype(ns)::value>(q, y, tol, maxit, rel); });
     }
     template <int NS>
     void a_ns(const CgBoth& q, int rows_y, int both) const {
@@ -919,34 +933,37 @@ struct CgLaunch {
         }
     }
     void a(const CgBoth& q, int nsys, int both) const {
-        if (apart(nsys)) a_ns<1>(q, nsys, both);
-        else a_ns<2>(q, 1, both);
+        shaped(nsys, [&](auto ns, int y) { a_ns<decltype(ns)::value>(q, y, both); });
     }
     template <int NS>
     void b_ns(const CgBoth& q, int rows_y, int first) const {
-        if (nb <= kFoldSmall) {
-            k_cg_b<1, Rows, NS, true><<<dim3(nb, rows_y), kBlock, 0, s>>>(n, rows, q, nb, first);
-            return;
-        }
-        if constexpr (kEll) {
-            if (nb <= kFoldMid) {
-                k_cg_b<2, Rows, NS, true>
-                    <<<dim3((nb + 1) / 2, rows_y), 2 * kBlock, 0, s>>>(n, rows, q, nb, first);
-                return;
-            }
-            if (nb <= kFoldMax) {
-                k_cg_b<4, Rows, NS, true>
-                    <<<dim3((nb + 3) / 4, rows_y), 4 * kBlock, 0, s>>>(n, rows, q, nb, first);
+        CFD_CHECK(nb <= kFoldSmall ? !Rows::kMany : !Rows::kFew, "internal: PCG row reader");
+        if constexpr (!Rows::kMany) {
+            if (nb <= kFoldSmall) {
+                k_cg_b<1, Rows, NS, true><<<dim3(nb, rows_y), kBlock, 0, s>>>(n, rows, q, nb, first);
                 return;
             }
         }
-        if (first) k_cg_fin_a<<<NS * rows_y, 256, 0, s>>>(q, nb, 1);
-        k_cg_b<1, Rows, NS, false><<<dim3(nb, rows_y), kBlock, 0, s>>>(n, rows, q, nb, first);
-        k_cg_fin_b<<<NS * rows_y, 256, 0, s>>>(q, nb);
+        if constexpr (!Rows::kFew) {
+            if constexpr (kEll) {
+                if (nb <= kFoldMid) {
+                    k_cg_b<2, Rows, NS, true>
+                        <<<dim3((nb + 1) / 2, rows_y), 2 * kBlock, 0, s>>>(n, rows, q, nb, first);
+                    return;
+                }
+                if (nb <= kFoldMax) {
+                    k_cg_b<4, Rows, NS, true>
+                        <<<dim3((nb + 3) / 4, rows_y), 4 * kBlock, 0, s>>>(n, rows, q, nb, first);
+                    return;
+                }
+            }
+            if (first) k_cg_fin_a<<<NS * rows_y, 256, 0, s>>>(q, nb, 1);
+            k_cg_b<1, Rows, NS, false><<<dim3(nb, rows_y), kBlock, 0, s>>>(n, rows, q, nb, first);
+            k_cg_fin_b<<<NS * rows_y, 256, 0, s>>>(q, nb);
+        }
     }
     void b(const CgBoth& q, int nsys, int first) const {
-        if (apart(nsys)) b_ns<1>(q, nsys, first);
-        else b_ns<2>(q, 1, first);
+        shaped(nsys, [&](auto ns, int y) { b_ns<decltype(ns)::value>(q, y, first); });
     }
 };
 

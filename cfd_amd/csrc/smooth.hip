@@ -400,7 +400,7 @@ struct SmSeq {
     unsigned* rows;
     int* prog;             // per pass: nodes done; then 1 when a pass gave up
     double* dmax;          // per pass: the largest squared move
-    int n, npass, nlap;    // passes of the launch, Laplacian ones first
+    int n, nlap;           // nodes; Laplacian passes of the launch, the first ones
     long long limit;       // of a wait without progress, ticks of wall_clock64()
 };
 __host__ __device__ constexpr int sm_words(int n) { return (n + 63) / 64 * 2; }
@@ -727,7 +727,7 @@ static int smooth_run_seq(const Tables& t, SmoothPlan& plan, const SmDev& d, hip
         k_sm_rows<<<grid_for(std::max(nw, kSmPasses + 1)), kBlock, 0, s>>>(
             plan.smoothable.p, plan.fixed.p, plan.rows.p, plan.prog.p, n, last);
         const SmSeq q{d, plan.ring.p, plan.need.p, plan.xy.p, plan.hist.p, plan.rows.p,
-                      plan.prog.p, plan.dmax_pass.p, n, np, nlap, limit};
+                      plan.prog.p, plan.dmax_pass.p, n, nlap, limit};
         if (lds) k_sm_passes<true><<<np, 64, full, s>>>(q);
         else k_sm_passes<false><<<np, 64, base, s>>>(q);
         CFD_HIP(hipGetLastError());
