@@ -779,6 +779,7 @@ struct cfd_session {
     void geometry() {  // NORMALES, DERIV, MASAS, laplace (ns2DComp.ALE.f90:88-100, 259-275)
         const Tables& t = m->t;
         bc.normales(X.p, Y.p, s);
+        if (!LAPW.n) LAPW.alloc(ne);
         ElemTerms x;
         x.lapw = LAPW.p;
         launch_deriv(t, X.p, Y.p, AREA.p, DNX.p, DNY.p, HH.p, HHX.p, HHY.p, nullptr, partials.p, s,
@@ -786,6 +787,7 @@ struct cfd_session {
         refresh_patch_geometry();
         launch_laplace(t, LAPW.p, DNX.p, DNY.p, LAP.p, LDIAG.p, s, ell_on ? &ell : nullptr,
                        NodeMass{M.p, AREA.p, nullptr, nullptr}, hmin_fold());
+        if (d.moving != 1) LAPW.release();  // this once; a moving mesh keeps it for its steps
     }
     HminFold hmin_fold() { return {partials.p, scal(CFD_S_HMIN), (int)grid_for(ne)}; }
 
@@ -1223,7 +1225,7 @@ int cfd_session_create(cfd_session** out, cfd_mesh* m, const cfd_case_desc* d) {
                         &S->WYO, &S->LDIAG, &S->DXPOS, &S->DYPOS, &S->BZERO})
             b->alloc(np);
         for (auto* b : {&S->DTL, &S->DT, &S->SHOC, &S->T1, &S->T2, &S->T3, &S->AREA, &S->HH, &S->HHX,
-                        &S->HHY, &S->AREA_OLD, &S->LAPW})
+                        &S->HHY, &S->AREA_OLD})
             b->alloc(ne);
         if (d->moving == 1 && d->gcl >= 0) S->GCLT.alloc(ne);
         S->DNX.alloc(3 * (size_t)ne);
