@@ -151,7 +151,8 @@ __device__ inline void laplace_row(int r0, int s0, int s1, const int* __restrict
 
 // laplace's rows, and the nodes' masses in the same pass over their elements:
 // MASAS, or the GCL's update from the terms that k_deriv left; one more block
-// folds k_deriv's minima of HH (a launch of 4.7 us less).  Blocks of one wave in XCD order (a node's elements are its ring neighbours' too).
+// folds k_deriv's minima of HH (a launch of 4.7 us less).  Blocks of one wave in XCD
+// order (a node's elements are its ring neighbours' too).
 //
 // Formed from the coordinates, gradients and W per node and element, in launches
 // of their own (laplace + GCL / laplace + MASAS), and so, k_deriv's 15 us more for
@@ -171,13 +172,16 @@ k_laplace(const int* __restrict__ esup1, const int* __restrict__ esup2,
           const double* __restrict__ dNy, double* __restrict__ lap, double* __restrict__ diag,
           int npoin, int width, double* __restrict__ ell, NodeMass m, HminFold h) {
     __shared__ double srow[kLapRow * kLapThreads];
-    const int nblk = (npoin + kLapThreads - 1) / kLapThreads;
-    if ((int)blockIdx.x == nblk) {  // subrutinas.f90:124-125: hmin = min(minval(HH), 1e10)
+    // the fold is the first block's: on a large mesh it takes longer than a row block
+    // and ends beside them instead of behind (33.5M triangles: 2,011 us, as the last
+    // block's 2,077, in a launch of its own 2,018 + 29)
+    const int nblk = (npoin + kLapThreads - 1) / kLapThreads, fold = h.out ? 1 : 0;
+    if ((int)blockIdx.x < fold) {  // subrutinas.f90:124-125: hmin = min(minval(HH), 1e10)
         const double v = combine_partials(h.partials, h.nb, __builtin_huge_val(), OpMin());
         if (threadIdx.x == 0) *h.out = v > 1.0e10 ? 1.0e10 : v;
         return;
     }
-    const int i = xcd_block(blockIdx.x, nblk) * kLapThreads + threadIdx.x;
+    const int i = xcd_block((int)blockIdx.x - fold, nblk) * kLapThreads + threadIdx.x;
     if (i >= npoin) return;
     const int r0 = rowptr[i], len = rowptr[i + 1] - r0, s0 = esup2[i], s1 = esup2[i + 1];
     double tot1 = 0.0, tot2 = 0.0;
