@@ -519,14 +519,25 @@ int cfd_bicg_ex(int npoin, const double* spMtx, const int* spIdx, const int* spR
         XF.upload(x_fix, nfix, s);
         FI.upload(x_fixIdx, nfix, s);
         PcgWork w;
-        // the ELL copy (bit for bit the CSR kernels' results): its two passes
-        // over the matrix cost less than the first two iterations gain
+        // the ELL copy (bit for bit the CSR kernels' results), of a solve that is long
+        // enough for it; where it finds no room the solve goes on without
         EllLap ell;
-        const bool el = ell.build(npoin, nnz, R.p, I.p, spRowptr, s);
-        if (el) ell.refresh(R.p, A.p, s);
-        const EllMat em = ell.mat();
-        pcg_launch(w, npoin, A.p, I.p, R.p, D.p, X.p, B.p, XF.p, FI.p, nfix, tol, maxit, rel, s,
-                   el ? &em : nullptr);
+        EllMat em;
+        const auto copy = [&]() -> const EllMat* {
+            try {
+                if (!ell.build(npoin, nnz, R.p, I.p, spRowptr, s)) return nullptr;
+            } catch (const Error&) {
+                (void)hipGetLastError();
+                return nullptr;
+            }
+            ell.refresh(R.p, A.p, s);
+            em = ell.mat();
+            return &em;
+        };
+        pcg_launch(w, npoin, A.p, I.p, R.p, D.p, X.p, B.p, XF.p, FI.p, nfix, tol, maxit, rel, s, copy);
+        // what the host has queued in vain behind the end: a copy from a stream that is
+        // still at work makes the next stream's creation 100 us slower
+        CFD_HIP(hipStreamSynchronize(s));
         PcgResult res = pcg_result(w, s);
         X.download(x, npoin, s);
         CFD_HIP(hipStreamSynchronize(s));

@@ -18,6 +18,7 @@
 #include <cmath>
 #include <cstdint>
 #include <cstdio>
+#include <functional>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -683,11 +684,14 @@ struct EllLap {
     EllMat mat() const { return EllMat{val.p, col.p, dcol.p, len.p, width}; }
 };
 // Several independent solves on one matrix, interleaved on stream s with
-// shared polls (small systems: a block each, without); ell (when given) is the same matrix in ELL order, used by
-// the SpMV kernels of the iterations (bit for bit the CSR kernels' results).
+// shared polls (small systems: a block each, without); ell (when given) is the same
+// matrix in ELL order, used by the SpMV kernels of the iterations (bit for bit the
+// CSR kernels' results).  late (when given, with no ell): makes that copy once the
+// solve has turned out to need it (see ell_from); null where there is none.
+using EllMaker = std::function<const EllMat*()>;
 void pcg_launch_multi(const PcgSystem* sys, int nsys, int npoin, const double* A, const int* idx,
                       const int* rowptr, const double* diag, double tol, int maxit, int rel,
-                      hipStream_t s, const EllMat* ell = nullptr);
+                      hipStream_t s, const EllMat* ell = nullptr, const EllMaker& late = {});
 // iterations of the last solve run by pcg_launch_multi on w: as its final poll
 // read them (host memory), or, of a solve without polls, from the device after
 // waiting for s
@@ -706,7 +710,7 @@ struct PcgResult {
 void pcg_launch(PcgWork& w, int npoin, const double* A, const int* idx, const int* rowptr,
                 const double* diag, double* x, const double* b, const double* x_fix,
                 const int* x_fix_idx, int nfix, double tol, int maxit, int rel, hipStream_t s,
-                const EllMat* ell = nullptr);
+                const EllMaker& late = {});
 // Waits for the stream and returns the last solve's outcome.
 PcgResult pcg_result(const PcgWork& w, hipStream_t s);
 // One axis of the mesh's move, and where its solve's outcome goes: X += pos,

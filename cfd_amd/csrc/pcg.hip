@@ -663,12 +663,12 @@ k_cg_fin_b(CgBoth a, int nb) {
     }
 }
 
-// ELL row lengths and columns (EllLap::build), *far = 1 when a column lies
-// more than 16 bits from its row
+// ELL row lengths and columns (EllLap::build): distances from the row (kShort,
+// *far = 1 when one has more than 16 bits) or column numbers
+template <bool kShort, class C>
 __global__ void k_ell_col(int n, int width, const int* __restrict__ rowptr,
-                          const int* __restrict__ idx, int* __restrict__ col,
-                          short* __restrict__ dcol, unsigned char* __restrict__ len,
-                          int* __restrict__ far) {
+                          const int* __restrict__ idx, C* __restrict__ col,
+                          unsigned char* __restrict__ len, int* __restrict__ far) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const int b = rowptr[i], cnt = rowptr[i + 1] - b;
@@ -676,12 +676,11 @@ __global__ void k_ell_col(int n, int width, const int* __restrict__ rowptr,
     bool out = false;
     for (int k = 0; k < width; ++k) {
         const int c = k < cnt ? idx[b + k] - 1 : i;
-        const int d = c - i;
+        const int d = kShort ? c - i : c;
         out = out || d < -32768 || d > 32767;
-        col[(size_t)k * n + i] = c;
-        dcol[(size_t)k * n + i] = (short)d;
+        col[(size_t)k * n + i] = (C)d;
     }
-    if (out) *far = 1;
+    if (kShort && out) *far = 1;
 }
 
 __global__ void k_ell_val(int n, int width, const int* __restrict__ rowptr,
@@ -811,27 +810,31 @@ bool EllLap::build(int npoin, long long nnz, const int* rowptr, const int* idx, 
     n = npoin;
     width = 0;
     if (n <= 0 || nnz <= 0) return false;
-    int w = 0;
+    int w = 0, least = 0;
     for (int i = 0; i < n; ++i) {
         const int l = rowptr_host[i + 1] - rowptr_host[i];
-        if (l < 0) return false;
         w = std::max(w, l);
+        least = std::min(least, l);
     }
-    if (w <= 0 || w > kEllMaxWidth || (double)w * n > 1.5 * (double)nnz) return false;
-    width = w;
-    col.alloc((size_t)w * n);
+    if (least < 0 || w <= 0 || w > kEllMaxWidth || (double)w * n > 1.5 * (double)nnz) return false;
     dcol.alloc((size_t)w * n);
     len.alloc(n);
     val.alloc((size_t)w * n);
     DBuf<int> far(1);
     far.zero(s);
-    k_ell_col<<<grid_for(n), kBlock, 0, s>>>(n, w, rowptr, idx, col.p, dcol.p, len.p, far.p);
+    k_ell_col<true><<<grid_for(n), kBlock, 0, s>>>(n, w, rowptr, idx, dcol.p, len.p, far.p);
     CFD_HIP(hipGetLastError());
     int out = 0;
     CFD_HIP(hipMemcpyAsync(&out, far.p, sizeof(int), hipMemcpyDeviceToHost, s));
     CFD_HIP(hipStreamSynchronize(s));
-    if (out) dcol.release();
-    else col.release();
+    if (out) {
+        dcol.release();
+        col.alloc((size_t)w * n);
+        k_ell_col<false><<<grid_for(n), kBlock, 0, s>>>(n, w, rowptr, idx, col.p, len.p, far.p);
+        CFD_HIP(hipGetLastError());
+        CFD_HIP(hipStreamSynchronize(s));  // far goes out of scope
+    }
+    width = w;
     return true;
 }
 
@@ -1232,6 +1235,12 @@ k_cg_whole(int n, EllMat m, const double* __restrict__ diag, CgBoth sys, double 
 // The rows up to which a solve runs in k_cg_whole (33 bytes of LDS a row in
 // its largest form), and the iteration cap (one launch of at most 0.15 s)
 constexpr int kWholeRows = 4864, kWholeIters = 20000;
+// A caller's matrix gets its ELL copy (EllMaker) when the first test has not ended the
+// solve of a small system, and from so many iterations on that of a larger one, about
+// where the copy has cost what it gains (us: the copy, an iteration from CSR rows and
+// from it: 8,192 rows 65, 9.2, 7.7; 32,768 rows 60, 9.1, 7.6; 180,000 130, 12.5, 11.0;
+// 524,288 1,400, 30, 19; 2.1M 2,700, 88, 66).
+inline long ell_from(int n) { return n <= 128 * 1024 ? 28 : 96; }
 
 template <int kT, int kW, int kR, int kKeep, int kLds, bool kX>
 void launch_whole(int n, const EllMat& m, const double* diag, const CgBoth& q, int nsys, double tol,
@@ -1252,13 +1261,16 @@ void launch_whole(int n, const EllMat& m, const double* diag, const CgBoth& q, i
 
 void pcg_launch_multi(const PcgSystem* sys, int nsys, int npoin, const double* A, const int* idx,
                       const int* rowptr, const double* diag, double tol, int maxit, int rel,
-                      hipStream_t s, const EllMat* ell) {
+                      hipStream_t s, const EllMat* ell, const EllMaker& late) {
     CFD_CHECK(npoin > 0, "arg: PCG needs npoin > 0");
     constexpr int kMaxSys = 2;
     CFD_CHECK(nsys >= 1 && nsys <= kMaxSys, "internal: PCG systems per launch");
     const int nb = (int)grid_for(npoin);
     for (int k = 0; k < nsys; ++k) sys[k].w->ensure(npoin);
-    if (ell && ell->width <= 8 && ell->dcol && npoin <= kWholeRows && maxit <= kWholeIters) {
+    const bool small = npoin <= kWholeRows && maxit <= kWholeIters;
+    // small systems: the whole solve in one launch; false where its rule does not hold
+    auto whole = [&]() {
+        if (!small || !ell || ell->width > 8 || !ell->dcol) return false;
         CgBoth q{};
         for (int k = 0; k < nsys; ++k) {
             q.s[k] = cg_sys(sys[k], 0);
@@ -1282,8 +1294,9 @@ void pcg_launch_multi(const PcgSystem* sys, int nsys, int npoin, const double* A
         const auto go = ell->width <= 7 ? pick(std::integral_constant<int, 7>{})
                                         : pick(std::integral_constant<int, 8>{});
         go(npoin, *ell, diag, q, nsys, tol, maxit, rel, s);
-        return;
-    }
+        return true;
+    };
+    if (whole()) return;
     // pbuf[cur] holds the current p; both systems' buffers flip together
     int cur = 1;
     bool done[kMaxSys] = {false, nsys == 1};
@@ -1325,17 +1338,28 @@ void pcg_launch_multi(const PcgSystem* sys, int nsys, int npoin, const double* A
         }
         return count() == 0;
     };
-    with_rows(npoin, A, idx, rowptr, ell, [&](auto rows) {
+    int chunk = 4, slot = 0, both = 0;
+    long launched = 0;
+    enum { kStart, kProduct, kLoop } at = kStart;
+    bool waits = (bool)late;
+    // from where the solve stands; false: not done, and now is the time for the late copy
+    auto solve = [&](auto rows) {
         const CgLaunch<decltype(rows)> go{npoin, nb, rows, diag, s};
-        go.start(args(), nsys, tol, maxit, rel);
-        // the first poll before the first product, which only solves that go on
-        // need: a solve that the first test ends is known 5 us earlier
-        int chunk = 4, slot = 0;
-        ask(slot);
-        go.b(args(), nsys, 1);  // p0 = z0 into pbuf[0]
-        cur = 0;
-        CFD_HIP(hipGetLastError());
-        int both = 0;
+        if (at == kStart) {
+            // the first poll before the first product, which only solves that go on
+            // need: a solve that the first test ends is known 5 us earlier
+            go.start(args(), nsys, tol, maxit, rel);
+            ask(slot);
+            at = kProduct;
+            if (waits && told(slot)) return true;
+            if (waits && small) return false;
+        }
+        if (at == kProduct) {
+            go.b(args(), nsys, 1);  // p0 = z0 into pbuf[0]
+            cur = 0;
+            at = kLoop;
+            CFD_HIP(hipGetLastError());
+        }
         auto iterate = [&](int m) {
             for (int q = 0; q < m; ++q) {
                 go.a(args(), count(), both);
@@ -1352,16 +1376,16 @@ void pcg_launch_multi(const PcgSystem* sys, int nsys, int npoin, const double* A
         // about 15 us, the batch queued in vain at the end about 50.
         constexpr long kAsyncFrom = 128;
         constexpr int kAsyncBatch = 8;
-        long launched = 0;
         while (!told(slot)) {
             CFD_CHECK(launched <= 4L * maxit + 64, "PCG did not terminate");
+            if (waits && launched >= ell_from(npoin)) return false;
             if (pinned && launched >= kAsyncFrom) break;
             iterate(chunk);
             launched += chunk;
             chunk = std::min(chunk * 2, 16);
             ask(slot);
         }
-        if (count() == 0) return;
+        if (count() == 0) return true;
         iterate(kAsyncBatch);
         ask(slot);
         for (bool end = false; !end; slot ^= 1) {
@@ -1371,7 +1395,16 @@ void pcg_launch_multi(const PcgSystem* sys, int nsys, int npoin, const double* A
             ask(slot ^ 1);
             end = told(slot);
         }
-    });
+        return true;
+    };
+    bool end = false;
+    with_rows(npoin, A, idx, rowptr, ell, [&](auto rows) { end = solve(rows); });
+    if (end) return;
+    // it goes on with the late copy: small systems in one launch, from the start (the
+    // one above has set the fixed values only), others where they stand
+    waits = false;
+    ell = late();
+    if (!whole()) with_rows(npoin, A, idx, rowptr, ell, [&](auto rows) { solve(rows); });
 }
 
 double pcg_polled_iterations(const PcgWork& w, hipStream_t s) {
@@ -1381,9 +1414,9 @@ double pcg_polled_iterations(const PcgWork& w, hipStream_t s) {
 void pcg_launch(PcgWork& w, int npoin, const double* A, const int* idx, const int* rowptr,
                 const double* diag, double* x, const double* b, const double* x_fix,
                 const int* x_fix_idx, int nfix, double tol, int maxit, int rel, hipStream_t s,
-                const EllMat* ell) {
+                const EllMaker& late) {
     PcgSystem sys{&w, x, b, x_fix, x_fix_idx, nfix};
-    pcg_launch_multi(&sys, 1, npoin, A, idx, rowptr, diag, tol, maxit, rel, s, ell);
+    pcg_launch_multi(&sys, 1, npoin, A, idx, rowptr, diag, tol, maxit, rel, s, nullptr, late);
 }
 
 PcgResult pcg_result(const PcgWork& w, hipStream_t s) {
