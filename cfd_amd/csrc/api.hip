@@ -718,7 +718,7 @@ struct cfd_session {
     // their first residual test; after a step whose two solves both did, the
     // next step skips the learned candidate (and its training), as nothing
     // can be gained.  The relative rule always uses it.
-    bool last_solves_trivial = false;
+    bool solves_asked = false;  // the last step's solves can say whether they did
     // With ITLOCAL = 0 the fused paths skip DT's clip and the DTL fill (DTL
     // would be DTMIN everywhere, and no kernel of theirs reads DT or DTL);
     // the two fields are formed when a caller reads them (dt_stale).
@@ -841,7 +841,9 @@ struct cfd_session {
         const int maxit = d.pcg_maxit > 0 ? d.pcg_maxit : 1000;
         WsSolve q;
         const EllMat em = ell.mat();
-        const bool ws_now = ws_on && !(d.pcg_rel == 0 && last_solves_trivial);
+        const bool trivial = solves_asked && pcg_told_iterations(pcg, pcg_y) == 0.0;
+        solves_asked = false;
+        const bool ws_now = ws_on && !trivial;
         if (ws_on) {
             q.XPOS = XPOS.p;
             q.YPOS = YPOS.p;
@@ -871,9 +873,10 @@ struct cfd_session {
                                   {&pcg_y, YPOS.p, BZERO.p, POSAUY.p, ILAUX.p, nn}};
         pcg_launch_multi(sys, 2, np, LAP.p, m->t.idx.p, m->t.rowptr.p, LDIAG.p, tol, maxit,
                          d.pcg_rel, s, ell_on ? &em : nullptr);
-        if (ws_on && d.pcg_rel == 0)  // else nothing asks
-            last_solves_trivial =
-                pcg_polled_iterations(pcg, s) == 0.0 && pcg_polled_iterations(pcg_y, s) == 0.0;
+        if (ws_on && d.pcg_rel == 0) {  // else nothing asks; read by the next step's solves
+            pcg_ask_iterations(pcg, pcg_y, s);
+            solves_asked = true;
+        }
         te(CFD_K_PCG);
         if (ws_on) ws.after_solves(q, s);
         const bool old = d.gcl >= 0;
@@ -1328,7 +1331,7 @@ int cfd_session_init_freestream(cfd_session* S) {
         S->put_scalars();
         S->w_dirty = false;
         S->move_normalized = false;
-        S->last_solves_trivial = false;
+        S->solves_asked = false;
         S->ws.nhist = 0;  // the learned start's history restarts with the run
         S->ws.predicted = S->ws.net_used = false;
     })

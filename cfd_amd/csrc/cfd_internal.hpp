@@ -692,10 +692,11 @@ using EllMaker = std::function<const EllMat*()>;
 void pcg_launch_multi(const PcgSystem* sys, int nsys, int npoin, const double* A, const int* idx,
                       const int* rowptr, const double* diag, double tol, int maxit, int rel,
                       hipStream_t s, const EllMat* ell = nullptr, const EllMaker& late = {});
-// iterations of the last solve run by pcg_launch_multi on w: as its final poll
-// read them (host memory), or, of a solve without polls, from the device after
-// waiting for s
-double pcg_polled_iterations(const PcgWork& w, hipStream_t s);
+// The iterations of the last pair of solves run by pcg_launch_multi, both together: as
+// its final poll read them, or, of solves without polls, asked for on s (true) and
+// read when told, where the host waits for them.
+bool pcg_ask_iterations(PcgWork& x, PcgWork& y, hipStream_t s);
+double pcg_told_iterations(PcgWork& x, PcgWork& y);
 struct PcgResult {
     int iters;
     double rz;

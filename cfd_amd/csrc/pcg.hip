@@ -978,8 +978,10 @@ struct CgLaunch {
 // the order of the kernels above (the same bits).  r, diag and z or y (never
 // both alive) stay in registers, p is in LDS for the gathers, the matrix in
 // registers and LDS as far as it fits.  The scalars never leave the block: no
-// launch, no round trip through memory and no poll between the iterations,
-// and a mesh that moves in steps never waits for the host.
+// launch, no round trip through memory and no poll between the iterations, and a
+// mesh that moves in steps does not wait for the host (under the absolute rule with
+// a learned start the host waits, at the next step's solves, for these to have ended:
+// pcg_ask_iterations).
 //
 // An iteration of one system / two against the two launches above (us): 768
 // rows 1.6 / 1.65 against 7.9 / 8.3, 2,048 rows 2.3 / 2.45, 3,072 rows 3.1 /
@@ -1407,8 +1409,23 @@ void pcg_launch_multi(const PcgSystem* sys, int nsys, int npoin, const double* A
     if (!whole()) with_rows(npoin, A, idx, rowptr, ell, [&](auto rows) { solve(rows); });
 }
 
-double pcg_polled_iterations(const PcgWork& w, hipStream_t s) {
-    return w.polled_iters >= 0.0 ? w.polled_iters : (double)pcg_result(w, s).iters;
+bool pcg_ask_iterations(PcgWork& x, PcgWork& y, hipStream_t s) {
+    if (x.polled_iters >= 0.0 && y.polled_iters >= 0.0) return false;
+    CgBoth q{};
+    q.s[0].scal = x.scal.p;
+    q.s[1].scal = y.scal.p;
+    k_cg_poll<<<2, S_NSCAL, 0, s>>>(q, x.hpin.p, y.hpin.p);
+    CFD_HIP(hipEventRecord(x.ev[0], s));
+    return true;
+}
+
+double pcg_told_iterations(PcgWork& x, PcgWork& y) {
+    if (x.polled_iters < 0.0 || y.polled_iters < 0.0) {
+        CFD_HIP(hipEventSynchronize(x.ev[0]));
+        x.polled_iters = x.hpin.p[S_K];
+        y.polled_iters = y.hpin.p[S_K];
+    }
+    return x.polled_iters + y.polled_iters;
 }
 
 void pcg_launch(PcgWork& w, int npoin, const double* A, const int* idx, const int* rowptr,
