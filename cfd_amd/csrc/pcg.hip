@@ -987,7 +987,9 @@ struct CgLaunch {
 // rows 1.6 / 1.65 against 7.9 / 8.3, 2,048 rows 2.3 / 2.45, 3,072 rows 3.1 /
 // 3.3, 3,840 rows 3.8 / 4.0, 4,608 rows 5.3 / 5.7 against 7.9 / 8.35.  Bound by
 // the one CU: FP64 instructions (about 0.35 us per 512 rows), three barriers and
-// two trees (1 us).  Above kWholeRows the matrix no longer fits beside p (6,144
+// two trees (1 us).  The forms of 512 threads (up to 3,072 rows) spill nothing; those
+// of 1,024 are at their 128 VGPRs and keep 23 (up to 4,096 rows) to 35 registers a
+// thread in scratch, which the 4,608 rows' time includes.  Above kWholeRows the matrix no longer fits beside p (6,144
 // rows 8.9 / 8.9, 8,192 rows 13 / 13 against 7.8 / 8.0).
 // ---------------------------------------------------------------------------
 
@@ -1282,8 +1284,8 @@ void pcg_launch_multi(const PcgSystem* sys, int nsys, int npoin, const double* A
         // to 3,072 rows all of it in registers; above, values beside p in LDS,
         // and above 4,096 rows x there too and two or three values a row read
         // from L2 (5.3 us an iteration at 4,608 rows; 6.1 with three in LDS and
-        // x in registers, which spill; 6.8 with x in place; 8.0 in 512 threads of
-        // ten rows).
+        // x in registers, which spills more; 6.8 with x in place; 8.0 in 512 threads
+        // of ten rows).
         const int half = (npoin + 511) / 512;
         const auto pick = [&](auto width) {
             constexpr int kW = decltype(width)::value;

@@ -124,7 +124,8 @@ __device__ inline double combine_partials(const double* partials, int n, double 
 // (A "last block combines" variant -- a device-scope fence and an atomic
 // arrival count per block -- measured 2.6x slower per PCG iteration than the
 // separate one-block finalize kernel on gfx950: each block's release fence
-// writes back its L2.  The finalize kernels stay separate.)
+// writes back its L2.  The next kernel's blocks combine the partials instead, each
+// for itself, or a one-block kernel where they are many.)
 
 namespace {
 // *out = min(init, partials[0..n)), then min(*out, cap) (one block of 256)
