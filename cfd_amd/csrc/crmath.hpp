@@ -33,9 +33,9 @@
 //   x^(-1/2) = y (1 + r/2 + 3 r^2/8),   r = 1 - x y^2 (exact to 2^-103)
 //   x^(3/2)  = x * sqrt(x),   sqrt(x) = s + (x - s*s) h
 // with y from the hardware's reciprocal square root and one third-order step
-// (relative error about 2^-52), s = sqrt(x) correctly rounded (an s an ulp off
-// misrounds 2,772 of the 27,040 squares whose 3/2 power is a midpoint) and
-// h = 1/(2 s) within an ulp.  They replace pow(x, 1.5) (calcRHS.f90:50-51, subrutinas.f90:196,400)
+// (relative error about 2^-52), s = sqrt(x) rounded from a value 2^-88 off, so exact
+// for squares (an s an ulp off misrounds 2,772 of the 27,040 squares whose 3/2 power
+// is a midpoint), and h = 1/(2 s) within an ulp.  They replace pow(x, 1.5) (calcRHS.f90:50-51, subrutinas.f90:196,400)
 // and pow(x, -0.5) (subrutinas.f90:429,438-439): fewer instructions than a
 // general pow, and closer to the exact value than either the device pow or
 // glibc's.
@@ -62,7 +62,7 @@ __device__ __forceinline__ double quot(double a, const Recip& k) {
 __device__ __forceinline__ double quot(double a, double b) { return quot(a, recip(b)); }
 __device__ __forceinline__ double third(double a) { return quot(a, Recip{3.0, 1.0 / 3.0}); }
 
-// sqrt(x), correctly rounded, for x > 2^-700; h: 1/(2 sqrt(x)) within 2^-44
+// sqrt(x) for x > 2^-700, rounded from a value 2^-88 off; h: 1/(2 sqrt(x)) within 2^-44
 __device__ __forceinline__ double sqrt_core(double x, double& h) {
     const double y = __builtin_amdgcn_rsq(x);
     double s = x * y;
@@ -70,13 +70,13 @@ __device__ __forceinline__ double sqrt_core(double x, double& h) {
     const double e = __builtin_fma(-h, s, 0.5);
     s = __builtin_fma(s, e, s);
     h = __builtin_fma(h, e, h);
-    s = __builtin_fma(__builtin_fma(-s, s, x), h, s);
     return __builtin_fma(__builtin_fma(-s, s, x), h, s);
 }
 __device__ __forceinline__ double sqrt_rn(double x) {
     if (__any(x < 0x1p-700 && x != 0.0)) return sqrt(x);
     double h;
-    const double s = sqrt_core(x, h);
+    double s = sqrt_core(x, h);
+    s = __builtin_fma(__builtin_fma(-s, s, x), h, s);
     return x == 0.0 || x == __builtin_huge_val() ? x : s;
 }
 
