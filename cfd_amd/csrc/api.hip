@@ -164,9 +164,7 @@ int cfd_laplace(cfd_mesh* m, const double* X, const double* Y, const double* dNx
         double* dny = m->put("dNy", dNy, 3 * (size_t)ne);
         double* lap = m->scratch("lap", m->t.nnz);
         double* diag = m->scratch("diag", np);
-        double* w = m->scratch("lapw", ne);
-        launch_lap_weights(m->t, dX, dY, w, m->s);
-        launch_laplace(m->t, w, dnx, dny, lap, diag, m->s);
+        launch_laplace(m->t, dX, dY, dnx, dny, lap, diag, m->s);
         m->get(lap_sparse, lap, m->t.nnz);
         m->get(lap_diag, diag, np);
         m->sync();

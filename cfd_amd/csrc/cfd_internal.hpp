@@ -198,9 +198,6 @@ void launch_deriv(const Tables& t, const double* X, const double* Y, double* are
                   double* partials, hipStream_t s, const ElemTerms& x = ElemTerms{});
 // MASAS (subrutinas.f90:128-153) as an ascending-element gather
 void launch_masas(const Tables& t, const double* area, double* M, hipStream_t s);
-// each element's weight in laplace, from the coordinates
-void launch_lap_weights(const Tables& t, const double* X, const double* Y, double* lapw,
-                        hipStream_t s);
 // The nodes' masses in laplace's pass: MASAS (area given), or the GCL's update
 // M += dt (sums of gcl) / 2 (gcl given; dt a device scalar)
 struct NodeMass {
@@ -220,8 +217,11 @@ struct HminFold {
 // ELL copy's values too (EllLap::refresh in the same pass)
 struct EllLap;
 void launch_laplace(const Tables& t, const double* lapw, const double* dNx, const double* dNy,
-                    double* lap, double* diag, hipStream_t s, EllLap* ell = nullptr,
-                    const NodeMass& m = NodeMass{}, HminFold h = HminFold{});
+                    double* lap, double* diag, hipStream_t s, EllLap* ell, const NodeMass& m,
+                    HminFold h);
+// the same alone, the weights from the coordinates
+void launch_laplace(const Tables& t, const double* X, const double* Y, const double* dNx,
+                    const double* dNy, double* lap, double* diag, hipStream_t s);
 // gcl.f90:8-46 main; mode 0 = as written, 1 = corrected y-divergence; dt is a
 // device scalar
 void launch_gcl(const Tables& t, double* M, const double* Wx, const double* Wy,

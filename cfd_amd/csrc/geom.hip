@@ -90,15 +90,6 @@ k_deriv(const int* __restrict__ inpoel, const double* __restrict__ X, const doub
     block_partial(hm, OpMin(), partials);
 }
 
-// the weights alone (the host entry's laplace)
-__global__ void k_lap_weights(const int* __restrict__ inpoel, const double* __restrict__ X,
-                              const double* __restrict__ Y, double* __restrict__ lapw, int nelem) {
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= nelem) return;
-    const int n1 = inpoel[3 * e] - 1, n2 = inpoel[3 * e + 1] - 1, n3 = inpoel[3 * e + 2] - 1;
-    lapw[e] = lap_weight(X[n1], X[n2], X[n3], Y[n1], Y[n2], Y[n3]);
-}
-
 // subrutinas.f90:137-152: M(i) = sum of area/3 over i's elements, ascending
 __global__ void __launch_bounds__(kBlock)
 k_masas(const int* __restrict__ esup1, const int* __restrict__ esup2, const double* __restrict__ area,
@@ -119,10 +110,11 @@ k_masas(const int* __restrict__ esup1, const int* __restrict__ esup2, const doub
 constexpr int kLapRow = 16;
 
 // row i's contributions in esup order; acc(k) is the accumulator of CSR
-// entry r0 + k, the first one the diagonal's; each(e): the node's other sums
-template <class Acc, class Each>
+// entry r0 + k, the first one the diagonal's; weight(e): the element's weight;
+// each(e): the node's other sums
+template <class Weight, class Acc, class Each>
 __device__ inline void laplace_row(int r0, int s0, int s1, const int* __restrict__ esup1,
-                                   const int* __restrict__ lslot, const double* __restrict__ lapw,
+                                   const int* __restrict__ lslot, Weight weight,
                                    const double* __restrict__ dNx, const double* __restrict__ dNy,
                                    Acc acc, Each each) {
     for (int s = s0; s < s1; ++s) {
@@ -131,7 +123,7 @@ __device__ inline void laplace_row(int r0, int s0, int s1, const int* __restrict
 #pragma unroll
         for (int j = 0; j < 3; ++j) slot[j] = lslot[3 * s + j] - r0;
         const int li = slot[0] == 0 ? 0 : slot[1] == 0 ? 1 : 2;  // the row's own node
-        const double q = lapw[e];
+        const double q = weight(e);
         double nx[3], ny[3];
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
@@ -163,12 +155,19 @@ __device__ inline void laplace_row(int r0, int s0, int s1, const int* __restrict
 // tables.  Fewer loads (a packed slot record, the products instead of the
 // gradients) and rows staged for coalesced CSR stores left it at 88-92.
 constexpr int kLapThreads = 64;
+// kMassNone: the host entry, without masses and with the weights formed here from the
+// coordinates (one matrix: a pass over the elements before it costs it more)
 enum { kMassNone, kMassMasas, kMassGcl };
+struct LapWeights {
+    const double* w;  // from k_deriv, or (kMassNone) null:
+    const int* inpoel;
+    const double *X, *Y;
+};
 template <int kMass>
 __global__ void __launch_bounds__(kLapThreads)
 k_laplace(const int* __restrict__ esup1, const int* __restrict__ esup2,
           const int* __restrict__ rowptr, const int* __restrict__ lslot,
-          const double* __restrict__ lapw, const double* __restrict__ dNx,
+          LapWeights lw, const double* __restrict__ dNx,
           const double* __restrict__ dNy, double* __restrict__ lap, double* __restrict__ diag,
           int npoin, int width, double* __restrict__ ell, NodeMass m, HminFold h) {
     __shared__ double srow[kLapRow * kLapThreads];
@@ -184,6 +183,11 @@ k_laplace(const int* __restrict__ esup1, const int* __restrict__ esup2,
     const int i = xcd_block((int)blockIdx.x - fold, nblk) * kLapThreads + threadIdx.x;
     if (i >= npoin) return;
     const int r0 = rowptr[i], len = rowptr[i + 1] - r0, s0 = esup2[i], s1 = esup2[i + 1];
+    const auto weight = [&lw](int e) {
+        if (kMass != kMassNone) return lw.w[e];
+        const int n1 = lw.inpoel[3 * e] - 1, n2 = lw.inpoel[3 * e + 1] - 1, n3 = lw.inpoel[3 * e + 2] - 1;
+        return lap_weight(lw.X[n1], lw.X[n2], lw.X[n3], lw.Y[n1], lw.Y[n2], lw.Y[n3]);
+    };
     double tot1 = 0.0, tot2 = 0.0;
     auto each = [&](int e) {
         if (kMass == kMassMasas) tot1 = tot1 + m.area[e] / 3.0;  // subrutinas.f90:137-152
@@ -196,7 +200,7 @@ k_laplace(const int* __restrict__ esup1, const int* __restrict__ esup2,
     if (len <= kLapRow) {
         double* sr = srow + threadIdx.x;
         for (int j = 0; j < len; ++j) sr[j * kLapThreads] = 0.0;
-        laplace_row(r0, s0, s1, esup1, lslot, lapw, dNx, dNy,
+        laplace_row(r0, s0, s1, esup1, lslot, weight, dNx, dNy,
                     [sr](int k) -> double& { return sr[k * kLapThreads]; }, each);
         for (int j = 0; j < len; ++j) lap[r0 + j] = sr[j * kLapThreads];
         for (int j = 0; j < width; ++j)
@@ -205,7 +209,7 @@ k_laplace(const int* __restrict__ esup1, const int* __restrict__ esup2,
     } else {
         double* row = lap + r0;
         for (int j = 0; j < len; ++j) row[j] = 0.0;
-        laplace_row(r0, s0, s1, esup1, lslot, lapw, dNx, dNy,
+        laplace_row(r0, s0, s1, esup1, lslot, weight, dNx, dNy,
                     [row](int k) -> double& { return row[k]; }, each);
         for (int j = 0; j < width; ++j) ell[(size_t)j * npoin + i] = j < len ? row[j] : 0.0;
         diag[i] = row[0];
@@ -388,20 +392,25 @@ void launch_masas(const Tables& t, const double* area, double* M, hipStream_t s)
     CFD_HIP(hipGetLastError());
 }
 
-void launch_lap_weights(const Tables& t, const double* X, const double* Y, double* lapw,
-                        hipStream_t s) {
-    k_lap_weights<<<grid_for(t.nelem), kBlock, 0, s>>>(t.inpoel.p, X, Y, lapw, t.nelem);
+static void laplace(const Tables& t, const LapWeights& w, const double* dNx, const double* dNy,
+                    double* lap, double* diag, hipStream_t s, EllLap* ell, const NodeMass& m, HminFold h) {
+    const auto kernel = m.gcl ? k_laplace<kMassGcl> : m.area ? k_laplace<kMassMasas> : k_laplace<kMassNone>;
+    const int nblk = (t.npoin + kLapThreads - 1) / kLapThreads + (h.out ? 1 : 0);
+    kernel<<<nblk, kLapThreads, 0, s>>>(t.esup1.p, t.esup2.p, t.rowptr.p, t.lslot.p, w, dNx, dNy, lap,
+                                        diag, t.npoin, ell ? ell->width : 0,
+                                        ell ? ell->val.p : nullptr, m, h);
     CFD_HIP(hipGetLastError());
 }
 
 void launch_laplace(const Tables& t, const double* lapw, const double* dNx, const double* dNy,
                     double* lap, double* diag, hipStream_t s, EllLap* ell, const NodeMass& m, HminFold h) {
-    const auto kernel = m.gcl ? k_laplace<kMassGcl> : m.area ? k_laplace<kMassMasas> : k_laplace<kMassNone>;
-    const int nblk = (t.npoin + kLapThreads - 1) / kLapThreads + (h.out ? 1 : 0);
-    kernel<<<nblk, kLapThreads, 0, s>>>(t.esup1.p, t.esup2.p, t.rowptr.p, t.lslot.p, lapw,
-                                                dNx, dNy, lap, diag, t.npoin, ell ? ell->width : 0,
-                                                ell ? ell->val.p : nullptr, m, h);
-    CFD_HIP(hipGetLastError());
+    CFD_CHECK(m.area || m.gcl, "internal: laplace with the masses");
+    laplace(t, {lapw, nullptr, nullptr, nullptr}, dNx, dNy, lap, diag, s, ell, m, h);
+}
+
+void launch_laplace(const Tables& t, const double* X, const double* Y, const double* dNx,
+                    const double* dNy, double* lap, double* diag, hipStream_t s) {
+    laplace(t, {nullptr, t.inpoel.p, X, Y}, dNx, dNy, lap, diag, s, nullptr, NodeMass{}, HminFold{});
 }
 
 void launch_gcl(const Tables& t, double* M, const double* Wx, const double* Wy, const double* Wxo,
