@@ -663,15 +663,8 @@ struct Renumbering {
     std::vector<int> node_old;      // node_old[i]: the caller's node at position i
     std::vector<int> elem_old;      // elem_old[q]: the caller's element at position q
     std::vector<int> lap_old;       // the caller's CSR entry of each Laplace entry
-    // the three on the device, and room for one field in the caller's order
-    // (grown to the largest field that crossed the boundary)
-    DBuf<int> d_node, d_elem, d_lap;
-    DBuf<double> stage;
-    std::mutex stage_mu;  // held while a field crosses
-    double* room(size_t n) {
-        if (stage.n < n) stage.alloc(n);
-        return stage.p;
-    }
+    DBuf<int> d_node, d_elem, d_lap;  // the three on the device
+    FieldStage stage;
     ~Renumbering() {
         if (mesh) cfd_mesh_destroy(mesh);
     }
@@ -1371,12 +1364,13 @@ static FieldKind field_kind(int f, int& width) {
     }
 }
 
-// the map of field f's entities to the caller's, their number and width
-static const int* field_map(const Renumbering& rn, int f, int& n, int& w) {
+// the map of field f's entities to the caller's
+static FieldMap field_map(const Renumbering& rn, int f) {
+    int w = 1;
     const FieldKind k = field_kind(f, w);
     const DBuf<int>& d = k == FK_NODE ? rn.d_node : k == FK_ELEM ? rn.d_elem : rn.d_lap;
-    n = (int)d.n;
-    return d.p;
+    const std::vector<int>& h = k == FK_NODE ? rn.node_old : k == FK_ELEM ? rn.elem_old : rn.lap_old;
+    return {h.data(), d.p, (int)h.size(), w};
 }
 
 extern "C" {
@@ -1399,18 +1393,12 @@ int cfd_session_get_field(cfd_session* S, int f, double* host_out) {
             launch_dt_finish(S->DT.p, S->DTL.p, S->ctl.p, nullptr, false, S->ne, S->s);
             S->dt_stale = false;
         }
-        const double* src = b->p;
-        std::unique_lock<std::mutex> hold;
-        if (S->rn) {  // in the caller's order, on the device
-            int m = 0, w = 1;
-            const int* map = field_map(*S->rn, f, m, w);
-            hold = std::unique_lock<std::mutex>(S->rn->stage_mu);
-            double* out = S->rn->room(n);
-            launch_scatter_field(src, out, map, m, w, S->s);
-            src = out;
+        if (S->rn) {
+            read_field(b->p, host_out, field_map(*S->rn, f), S->rn->stage, S->s);
+        } else {
+            b->download(host_out, n, S->s);
+            CFD_HIP(hipStreamSynchronize(S->s));
         }
-        CFD_HIP(hipMemcpyAsync(host_out, src, sizeof(double) * n, hipMemcpyDeviceToHost, S->s));
-        CFD_HIP(hipStreamSynchronize(S->s));
     })
 }
 
@@ -1419,18 +1407,12 @@ int cfd_session_set_field(cfd_session* S, int f, const double* host_in) {
         CFD_ARG(S && host_in, "null argument");
         long long n = 0;
         DBuf<double>* b = S->field(f, n);
-        std::unique_lock<std::mutex> hold;
         if (S->rn) {
-            int m = 0, w = 1;
-            const int* map = field_map(*S->rn, f, m, w);
-            hold = std::unique_lock<std::mutex>(S->rn->stage_mu);
-            double* in = S->rn->room(n);
-            CFD_HIP(hipMemcpyAsync(in, host_in, sizeof(double) * n, hipMemcpyHostToDevice, S->s));
-            launch_gather_field(in, b->p, map, m, w, S->s);
+            write_field(host_in, b->p, field_map(*S->rn, f), S->rn->stage, S->s);
         } else {
             b->upload(host_in, n, S->s);
+            CFD_HIP(hipStreamSynchronize(S->s));
         }
-        CFD_HIP(hipStreamSynchronize(S->s));
         if (f == CFD_F_W_X || f == CFD_F_W_Y || f == CFD_F_XPOS || f == CFD_F_YPOS) S->w_dirty = true;
         if (f == CFD_F_XPOS || f == CFD_F_YPOS) S->xpos_zero = false;
         if (f == CFD_F_X || f == CFD_F_Y || f == CFD_F_X1 || f == CFD_F_Y1 || f == CFD_F_W_X ||

@@ -50,8 +50,7 @@ struct cfd_batch {
     // per case: the caller's node / element at each patch-order position
     std::vector<std::vector<int>> node_old, elem_old;
     DBuf<int> d_node, d_elem;  // the same on the device, the cases one after the other
-    DBuf<double> stage;        // one case's field in the caller's order
-    std::mutex stage_mu;       // held while a field crosses
+    FieldStage stage;          // one case's field in the caller's order
     // With itlocal = 0 DT's clip and DTL (DTMIN everywhere) are formed when a
     // caller reads them: no kernel of a step does
     bool dt_stale = false;
@@ -495,13 +494,10 @@ int cfd_batch_get_field(cfd_batch* b, int icase, int field, double* host) {
         if (field == CFD_F_DT || field == CFD_F_DTL) b->finish_dt();
         const size_t o = node ? b->nbase[icase] : b->ebase[icase];
         const size_t n = node ? b->nbase[icase + 1] - o : b->ebase[icase + 1] - o;
-        // back to the caller's numbering of the case, on the device
-        std::lock_guard<std::mutex> hold(b->stage_mu);
-        if (b->stage.n < w * n) b->stage.alloc(w * n);
-        launch_scatter_field(buf->p + w * o, b->stage.p, (node ? b->d_node.p : b->d_elem.p) + o,
-                             (int)n, w, b->s);
-        CFD_HIP(hipMemcpyAsync(host, b->stage.p, sizeof(double) * w * n, hipMemcpyDeviceToHost, b->s));
-        CFD_HIP(hipStreamSynchronize(b->s));
+        // back to the caller's numbering of the case
+        const FieldMap map{(node ? b->node_old : b->elem_old)[icase].data(),
+                           (node ? b->d_node.p : b->d_elem.p) + o, (int)n, w};
+        read_field(buf->p + w * o, host, map, b->stage, b->s);
     })
 }
 

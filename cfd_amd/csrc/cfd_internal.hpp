@@ -19,6 +19,7 @@
 #include <cstdint>
 #include <cstdio>
 #include <functional>
+#include <mutex>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -599,13 +600,25 @@ void launch_step_ctl(const double* partials, const int* pb, int nb, double* ctl,
 void launch_dt_finish(double* DT, double* DTL, const double* ctl, const int* ecase, bool blend,
                       int nelem, hipStream_t s);
 
-// Fields between a renumbered state and the caller's numbering: entity i of
-// the state is the caller's map[i], w doubles each (4 for U, U1, RHS; 3 for
-// the gradients).  scatter: caller[map[i]] = state[i]; gather the other way.
-void launch_scatter_field(const double* state, double* caller, const int* map, int n, int w,
-                          hipStream_t s);
-void launch_gather_field(const double* caller, double* state, const int* map, int n, int w,
-                         hipStream_t s);
+// Fields between a renumbered state (device) and the caller's numbering (host):
+// entity i of the state is the caller's map[i], w doubles each (4 for U, U1, RHS; 3 for
+// the gradients).  Both wait for the stream.  The map is wanted on both sides; the
+// stage holds one field in the caller's order, grown to the largest that crossed by
+// the kernel, one call at a time.
+struct FieldMap {
+    const int *host, *dev;
+    int n, w;
+};
+struct FieldStage {
+    DBuf<double> buf;
+    std::mutex mu;
+    double* room(size_t n) {
+        if (buf.n < n) buf.alloc(n);
+        return buf.p;
+    }
+};
+void read_field(const double* state, double* host, const FieldMap& m, FieldStage& st, hipStream_t s);
+void write_field(const double* host, double* state, const FieldMap& m, FieldStage& st, hipStream_t s);
 
 // meshMove.f90 FORCES (out3 = FX, FY, RM; skipped when null) and, when visc
 // is given, FORCE_VISC (ns2DComp.ALE.f90:819-893; out2 = F_VX, F_VY) in the

@@ -70,7 +70,23 @@ __global__ void k_dt_finish(double* __restrict__ DT, double* __restrict__ DTL,
 
 // One thread per entity.  Bound by the scattered side (32-byte records of U
 // fill a memory sector each): U of 2,097,152 nodes 64 MB in, 64 MB out.  In
-// place of a loop on the host, which took 20 of the 24 ms of reading U.
+// place of a loop on the host, which took 20 of the 24 ms of reading U; up to
+// kRenumberHost doubles the loop takes less than the launch (us a read of U by the
+// loop / so: 1,152 nodes 26 / 39, 8,192 27 / 34, 16,000 48 / 44, 32,768 111 / 79).
+constexpr size_t kRenumberHost = 40000;
+template <int W, bool kScatter>
+void renumber_host_w(const double* in, double* out, const int* map, int n) {
+    for (int i = 0; i < n; ++i) {
+        const size_t a = W * (size_t)(kScatter ? i : map[i]), b = W * (size_t)(kScatter ? map[i] : i);
+        for (int c = 0; c < W; ++c) out[b + c] = in[a + c];
+    }
+}
+template <bool kScatter>
+void renumber_host(const double* in, double* out, const FieldMap& m) {
+    if (m.w == 4) renumber_host_w<4, kScatter>(in, out, m.host, m.n);
+    else if (m.w == 3) renumber_host_w<3, kScatter>(in, out, m.host, m.n);
+    else renumber_host_w<1, kScatter>(in, out, m.host, m.n);
+}
 template <int W, bool kScatter>
 __global__ void k_renumber(const double* __restrict__ in, double* __restrict__ out,
                            const int* __restrict__ map, int n) {
@@ -97,13 +113,36 @@ void renumber(const double* in, double* out, const int* map, int n, int w, hipSt
 
 }  // namespace
 
-void launch_scatter_field(const double* state, double* caller, const int* map, int n, int w,
-                          hipStream_t s) {
-    renumber<true>(state, caller, map, n, w, s);
+void read_field(const double* state, double* host, const FieldMap& m, FieldStage& st, hipStream_t s) {
+    const size_t n = (size_t)m.n * m.w;
+    if (n <= kRenumberHost) {
+        std::vector<double> tmp(n);
+        CFD_HIP(hipMemcpyAsync(tmp.data(), state, sizeof(double) * n, hipMemcpyDeviceToHost, s));
+        CFD_HIP(hipStreamSynchronize(s));
+        renumber_host<true>(tmp.data(), host, m);
+        return;
+    }
+    std::lock_guard<std::mutex> hold(st.mu);
+    double* out = st.room(n);
+    renumber<true>(state, out, m.dev, m.n, m.w, s);
+    CFD_HIP(hipMemcpyAsync(host, out, sizeof(double) * n, hipMemcpyDeviceToHost, s));
+    CFD_HIP(hipStreamSynchronize(s));
 }
-void launch_gather_field(const double* caller, double* state, const int* map, int n, int w,
-                         hipStream_t s) {
-    renumber<false>(caller, state, map, n, w, s);
+
+void write_field(const double* host, double* state, const FieldMap& m, FieldStage& st, hipStream_t s) {
+    const size_t n = (size_t)m.n * m.w;
+    if (n <= kRenumberHost) {
+        std::vector<double> tmp(n);
+        renumber_host<false>(host, tmp.data(), m);
+        CFD_HIP(hipMemcpyAsync(state, tmp.data(), sizeof(double) * n, hipMemcpyHostToDevice, s));
+        CFD_HIP(hipStreamSynchronize(s));
+        return;
+    }
+    std::lock_guard<std::mutex> hold(st.mu);
+    double* in = st.room(n);
+    CFD_HIP(hipMemcpyAsync(in, host, sizeof(double) * n, hipMemcpyHostToDevice, s));
+    renumber<false>(in, state, m.dev, m.n, m.w, s);
+    CFD_HIP(hipStreamSynchronize(s));
 }
 
 // ---------------------------------------------------------------------------
